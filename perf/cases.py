@@ -166,6 +166,14 @@ def _cloths(case, seed):
     return ctx
 
 
+def _moving(case, seed, kw):
+    ctx = _cloths(case, seed)
+    ctx.set_solver(**kw)
+    x, _ = ctx.state_save()
+    ctx.state_load(x, _velocity(seed, len(x)))
+    return ctx
+
+
 def _contact_scene(case, seed):
     if case["kind"] == "drape":
         sc = scenes.config2(n=case["n"], seed=seed % 1000003)
@@ -200,25 +208,21 @@ def _wavy_sheet(n, rng):
 def prepare(case, seed):
     kind = case["kind"]
     if kind in ("sheet", "scenes", "batch"):
-        ctx = _cloths(case, seed)
         kw = dict(dt=DT, iterations=case["iterations"], graph=case["graph"], tile_sweeps=case.get("tile_sweeps", 0),
                   tile_max_verts=case.get("tile_max_verts", 0))
-        ctx.set_solver(**kw)
-        x, _ = ctx.state_save()
-        v = _velocity(seed, len(x))
-        ctx.state_load(x, v)
+        ctx = _moving(case, seed, kw)
         if case.get("warm"):
-            # weights trained on samples the solver recorded on other cloths
-            other = _cloths(dict(case, count=12, layout=case["layout"] + 1), seed)
-            other.set_solver(**kw)
+            # weights trained on samples the solver recorded on other cloths, both sets some substeps into their fall
+            other = _moving(dict(case, count=16, layout=case["layout"] + 1), seed, kw)
             other.step(12)
             other.ws_init(seed % 1000)
             other.ws_collect(60, 1)
-            other.ws_train(2, 4096, 1e-3, 0)
+            other.ws_train(4, 4096, 1e-3, 0)
             ctx.ws_set_params(other.ws_params())
             ctx.ws_set_norm(other.ws_norm())
-            ctx.set_solver(warm_iterations=1, warm_rule=1, warm_gate=1e-4, **kw)
             other.close()
+            ctx.step(12)
+            ctx.set_solver(warm_iterations=1, warm_rule=1, warm_gate=1e-4, **kw)
             ctx.ws_enable(True)
         ctx.snapshot(False)
         return dict(kind="step", ctx=ctx)
