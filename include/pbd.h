@@ -85,11 +85,15 @@ typedef struct {
     double tol;             /* stop when max |d-L|/L <= tol after a check; < 0 = fixed sweeps */
     int check_every;        /* sweeps between residual checks (chunk length) */
     int path;               /* PBD_PATH_* */
-    int tile_sweeps;        /* sweeps per launch for multi-tile cloths (0 = check_every) */
-    int tile_max_verts;     /* LDS vertices per tile (0 = from the device's LDS size) */
-    int block_threads;      /* threads per workgroup of the tile kernel (0 = 1024) */
+    int tile_sweeps;        /* sweeps per launch for multi-tile cloths (0 = check_every, or up to four for grid
+                               cloths of distance prims when check_every is 1 and neither a tolerance, the warm
+                               start nor collisions are in use; results are identical) */
+    int tile_max_verts;     /* most LDS vertices per tile (0 = from the device's LDS size); tiles are smaller where
+                               the cloths would otherwise not fill the GPU */
+    int block_threads;      /* threads per workgroup of the tile kernel (0 = by the tiles' sizes, at most 1024) */
     int graph;              /* 1: pbd_step replays each substep from a captured hipGraph whenever the
-                               substep makes no host decision (fixed sweeps, no collisions, profiling off) */
+                               substep makes no host decision (fixed sweeps, no collisions, profiling off); a
+                               context of single-tile cloths runs its substeps in one launch instead */
     int warm_iterations;    /* with the warm start on: sweep budget of a cloth whose prediction was kept
                                (0 = iterations); a cloth whose prediction is discarded runs `iterations`,
                                exactly the plain solver's substep */

@@ -48,10 +48,11 @@ struct pbd_ctx {
     // tiles
     TilePlan plan;
     int plan_sweeps = 0, plan_max_load = 0, plan_split = 0;
+    bool plan_small = false;  // planned with tiles smaller than the budget on offer
     DBuf<TileDev> tiles;
     // launch orders: single-tile cloths' tiles, multi-tile cloths' tiles, and
     // both (the first launch of a substep runs them side by side)
-    DBuf<int> tverts, tcols, order_whole, order_partial, order_first, tile_ids;
+    DBuf<int> tverts, tcounts, order_whole, order_partial, order_first, tile_ids;
     // later chunks under per-cloth budgets: the multi-tile tiles still
     // needed, compacted on the device, and the list's length
     DBuf<int> order_follow, follow_len, order_partial_cloth;
@@ -70,8 +71,11 @@ struct pbd_ctx {
     // (kernel, threads, LDS) it was last asked for
     int walk_key_threads = 0, walk_key_bend = -1, walk_slots = 0;
     size_t walk_key_lds = 0;
-    DBuf<uint32_t> tdist, tbend, town;
-    DBuf<float> tdist_rest, tbend_rest, town_rest;
+    DBuf<int4> tphases;
+    DBuf<uint2> tdist;
+    DBuf<uint4> tbend;
+    DBuf<uint32_t> town;
+    DBuf<float> town_rest;
     bool any_whole = false, any_partial = false;
     // residual / sweep bookkeeping
     DBuf<unsigned long long> res_slots, rmax;
@@ -235,10 +239,28 @@ void fill_ktabs(pbd_ctx* c) {
     c->ktab_b.upload(kb, c->stream);
 }
 
+bool has_tolerance(const pbd_ctx* c);
+// Every cloth with prims is a grid with its own distance prims only.
+bool distance_grids(const pbd_ctx* c) {
+    for (auto& k : c->cloths)
+        if (k.np() > 0 && (k.rx == 0 || k.nb > 0 || k.has_user_pairs)) return false;
+    return true;
+}
+
 int effective_tile_sweeps(const pbd_ctx* c) {
     if (c->coll.enabled) return 1;  // contacts are resolved after every sweep
-    int s = c->sp.tile_sweeps > 0 ? c->sp.tile_sweeps : c->sp.check_every;
-    return std::max(1, s);
+    if (c->sp.tile_sweeps > 0) return c->sp.tile_sweeps;
+    // Unset and free to choose (fixed sweeps, no per-cloth budgets): four
+    // sweeps per launch for distance prims.  Bending prims touch four vertices
+    // and take three times the colours, so their cones grow too fast: one.
+    // Measured per substep of 20 sweeps at the best tile size for each: a
+    // 389 x 211 cloth 152 / 133 / 117 / 113 / 133 us at 1 / 2 / 3 / 4 / 5
+    // sweeps per launch, a 256 x 256 cloth with bending 721 us at 1 and 923 at 2.
+    // Meshes are tiled by vertex id, whose cones may grow faster than a grid's:
+    // they keep one.
+    if (c->sp.check_every <= 1 && !has_tolerance(c) && !c->ws.enabled && distance_grids(c))
+        return std::min(4, std::max(1, c->sp.iterations));
+    return std::max(1, c->sp.check_every);
 }
 
 int effective_max_load(const pbd_ctx* c) {
@@ -251,11 +273,11 @@ void upload_plan(pbd_ctx* c) {
     TilePlan& p = c->plan;
     c->tiles.upload(p.tiles, c->stream);
     c->tverts.upload(p.verts, c->stream);
-    c->tcols.upload(p.cols, c->stream);
-    c->tdist.upload(p.dist, c->stream);
-    c->tdist_rest.upload(p.dist_rest, c->stream);
-    c->tbend.upload(p.bend, c->stream);
-    c->tbend_rest.upload(p.bend_rest, c->stream);
+    c->tphases.upload(p.phases, c->stream);
+    c->tcounts.upload(p.counts, c->stream);
+    // never empty: the record prefetch of an empty phase reads record 0
+    c->tdist.upload(p.dist.empty() ? std::vector<uint2>(1, make_uint2(0, 0)) : p.dist, c->stream);
+    c->tbend.upload(p.bend.empty() ? std::vector<uint4>(1, make_uint4(0, 0, 0, 0)) : p.bend, c->stream);
     c->town.upload(p.own, c->stream);
     c->town_rest.upload(p.own_rest, c->stream);
     c->order_whole.upload(p.whole_order, c->stream);
@@ -327,7 +349,7 @@ void ensure_queue(pbd_ctx* c) {
 int walk_grid(pbd_ctx* c) {
     const bool bend = !c->plan.bend.empty();
     const int threads = c->sp.block_threads > 0 ? c->sp.block_threads : 1024;
-    const size_t lds = (size_t)std::max(1, c->plan_max_load) * sizeof(float4);
+    const size_t lds = (size_t)std::max(1, c->plan.max_loaded) * sizeof(float4);
     if (threads != c->walk_key_threads || lds != c->walk_key_lds || (int)bend != c->walk_key_bend) {
         c->walk_slots = std::max(1, c->num_cu) * tiles_per_cu(bend, threads, lds);
         c->walk_key_threads = threads;
@@ -337,16 +359,71 @@ int walk_grid(pbd_ctx* c) {
     return (c->walk_slots + 7) / 8 * 8;
 }
 
+// The form of a tile launch of `ntiles` tiles: threads per workgroup, LDS for
+// the vertices, and the records per thread and colour kept in registers (0:
+// records fetched phase by phase).
+struct TileShape {
+    int threads, regs;
+    size_t lds;
+};
+TileShape tile_shape(const pbd_ctx* c, int ntiles) {
+    TileShape t;
+    t.threads = c->sp.block_threads > 0 ? c->sp.block_threads : 1024;
+    t.regs = 0;
+    t.lds = (size_t)std::max(1, c->plan.max_loaded) * sizeof(float4);
+    if (!c->plan.bend.empty() || c->ncolors_max > REG_COLORS || ntiles > c->num_cu) return t;
+    const int m = c->plan.max_phase;
+    if (c->sp.block_threads == 0 && m <= 1024) t.threads = std::max(256, (m + 63) / 64 * 64);
+    for (int r : {1, 2})
+        if (m <= r * t.threads) {
+            t.regs = r;
+            break;
+        }
+    return t;
+}
+
 void replan_if_needed(pbd_ctx* c) {
     int s = effective_tile_sweeps(c), ml = effective_max_load(c), sp = c->sp.split_whole ? 1 : 0;
-    if (s == c->plan_sweeps && ml == c->plan_max_load && sp == c->plan_split) return;
+    // Tiles smaller than the budget where the multi-tile cloths would not fill
+    // the GPU: a launch takes as long as its largest tile, so the smallest
+    // tile size of at most one tile per CU is the fastest (a 389 x 211 cloth at
+    // 4 sweeps per launch: 113 us per substep with 213 tiles of up to 2048
+    // vertices, 265 us with 18 of up to 10,208).
+    // (Grids only: a mesh's tiles are id ranges, whose cones do not shrink with them.)
+    long long multi = 0;
+    bool grids = true;
+    for (auto& k : c->cloths)
+        if (k.nv > ml) {
+            multi += k.nv;
+            grids &= k.rx > 0 && !k.has_user_pairs;
+        }
+    std::vector<int> loads;
+    if (multi > 0 && grids && !c->ws.enabled)
+        for (int load : {512, 768, 1024, 1280, 1536, 2048, 2560, 3072, 3584, 4096, 4608})
+            if (load < ml && (long long)load * c->num_cu > multi) loads.push_back(load);
+    const bool small = !loads.empty();
+    if (s == c->plan_sweeps && ml == c->plan_max_load && sp == c->plan_split && small == c->plan_small) return;
     // a failed plan leaves no valid one behind: the next call plans again
     c->plan_sweeps = 0;
     c->plan_max_load = 0;
-    plan_tiles(c->cloths, ml, s, sp != 0, c->plan);
+    bool planned = false;
+    if (small) {
+        loads = fitting_loads(c->cloths, ml, loads, s, c->num_cu);
+        for (size_t i = 0; i < loads.size() && !planned; i++) {
+            try {
+                plan_tiles(c->cloths, ml, loads[i], s, sp != 0, c->plan);
+            } catch (const Error& e) {
+                if (e.code != PBD_ERR_LIMIT) throw;
+                continue;  // some cone does not fit tiles of this size
+            }
+            planned = (int)c->plan.tiles.size() <= c->num_cu;
+        }
+    }
+    if (!planned) plan_tiles(c->cloths, ml, ml, s, sp != 0, c->plan);
     c->plan_sweeps = s;
     c->plan_max_load = ml;
     c->plan_split = sp;
+    c->plan_small = small;
     upload_plan(c);
     fill_cloth_dev(c);
 }
@@ -560,7 +637,12 @@ void do_init(pbd_ctx* c, int color_rounds) {
     fill_ktabs(c);
     c->plan_sweeps = 0;
     c->plan_max_load = 0;
-    replan_if_needed(c);
+    // grids always have a plan: theirs waits for the solver parameters; a
+    // mesh that has none is refused here
+    bool mesh = false;
+    for (auto& k : c->cloths) mesh |= k.np() > 0 && (k.rx == 0 || k.has_user_pairs);
+    if (mesh) replan_if_needed(c);
+    else fill_cloth_dev(c);
     PBD_HIP(hipStreamSynchronize(s));
     c->inited = true;
 }
@@ -731,7 +813,6 @@ void ws_require_params(pbd_ctx* c) {
 // Whether a warm substep of `iterations` sweeps under per-cloth budgets folds
 // the keep decision into the queued tile launch's schedule (true), or makes
 // it before the projection (false).
-bool has_tolerance(const pbd_ctx* c);
 bool queue_folds(pbd_ctx* c, int iterations) {
     if (c->sp.path != PBD_PATH_AUTO || has_tolerance(c) || c->sp.per_chunk_launches == 1) return false;
     replan_if_needed(c);
@@ -1070,17 +1151,18 @@ bool project(pbd_ctx* c, int iterations, bool fused_whole, float dt, const int* 
         integrate_end && !any_tol && !(fused_whole && c->any_partial && (nchunks < 2 || cap != nullptr));
     ensure_slots(c, nchunks);
     if (!fold) launch_fill_u64(s, c->res_slots.ptr, (size_t)c->nslots * ncl, 0ull);
-    size_t lds = (size_t)std::max(1, c->plan_max_load) * sizeof(float4);
-    int threads = c->sp.block_threads > 0 ? c->sp.block_threads : 1024;
+    const size_t lds = (size_t)std::max(1, c->plan.max_loaded) * sizeof(float4);
+    const TileShape shape = tile_shape(c, (int)c->plan.tiles.size());
+    const int threads = c->sp.block_threads > 0 ? c->sp.block_threads : 1024;
     int cur = c->pcur;
     const bool bend = !c->plan.bend.empty();
     auto tiles = [&](int nblocks, const int* order, const float4* pin, float4* pout, const SolveArgs& sa,
                      const int* n_items = nullptr) {
         if (c->prof_on) PBD_HIP(hipEventRecord(next_event(c), s));
-        launch_tiles(s, nblocks, order, c->tiles.ptr, c->tverts.ptr, c->tdist.ptr, c->tdist_rest.ptr, c->tbend.ptr,
-                     c->tbend_rest.ptr, c->town.ptr, c->town_rest.ptr, c->tcols.ptr, c->cl.ptr, c->ktab_d.ptr,
+        launch_tiles(s, nblocks, order, c->tiles.ptr, c->tverts.ptr, c->tdist.ptr, c->tbend.ptr,
+                     c->town.ptr, c->town_rest.ptr, c->tphases.ptr, c->tcounts.ptr, c->cl.ptr, c->ktab_d.ptr,
                      c->ktab_b.ptr, c->x.ptr, c->v.ptr, pin, pout, c->res_slots.ptr, ncl, c->sweeps.ptr, cap, sa,
-                     threads, lds, bend, n_items);
+                     shape.threads, shape.lds, bend, shape.regs, n_items);
         if (c->prof_on) PBD_HIP(hipEventRecord(next_event(c), s));
     };
     // Under per-cloth budgets and no tolerance, a later chunk needs only the
@@ -1097,6 +1179,7 @@ bool project(pbd_ctx* c, int iterations, bool fused_whole, float dt, const int* 
         follow_grid = std::min(walk_grid(c), (int)c->order_partial.n);
     }
     SolveArgs a{};
+    a.substeps = 1;
     a.dt = dt;
     a.check_every = ce;
     a.tol = tol;
@@ -1159,8 +1242,8 @@ bool project(pbd_ctx* c, int iterations, bool fused_whole, float dt, const int* 
         a.nsweeps = std::min(ts, iterations);
         a.chunk = 0;
         if (c->prof_on) PBD_HIP(hipEventRecord(next_event(c), s));
-        launch_tiles_decide(s, walk_grid(c), c->tiles.ptr, c->tverts.ptr, c->tdist.ptr, c->tdist_rest.ptr,
-                            c->tbend.ptr, c->tbend_rest.ptr, c->town.ptr, c->town_rest.ptr, c->tcols.ptr, c->cl.ptr,
+        launch_tiles_decide(s, walk_grid(c), c->tiles.ptr, c->tverts.ptr, c->tdist.ptr, c->tbend.ptr,
+                     c->town.ptr, c->town_rest.ptr, c->tphases.ptr, c->tcounts.ptr, c->cl.ptr,
                             c->ktab_d.ptr, c->ktab_b.ptr, c->x.ptr, c->v.ptr, c->res_slots.ptr, ncl, c->sweeps.ptr,
                             cap, a, q, threads, lds, bend);
         if (c->prof_on) PBD_HIP(hipEventRecord(next_event(c), s));
@@ -1203,8 +1286,8 @@ bool project(pbd_ctx* c, int iterations, bool fused_whole, float dt, const int* 
         a.nsweeps = std::min(ts, iterations);
         a.chunk = 0;
         if (c->prof_on) PBD_HIP(hipEventRecord(next_event(c), s));
-        launch_tiles_queue(s, walk_grid(c), c->tiles.ptr, c->tverts.ptr, c->tdist.ptr, c->tdist_rest.ptr,
-                           c->tbend.ptr, c->tbend_rest.ptr, c->town.ptr, c->town_rest.ptr, c->tcols.ptr, c->cl.ptr,
+        launch_tiles_queue(s, walk_grid(c), c->tiles.ptr, c->tverts.ptr, c->tdist.ptr, c->tbend.ptr,
+                     c->town.ptr, c->town_rest.ptr, c->tphases.ptr, c->tcounts.ptr, c->cl.ptr,
                            c->ktab_d.ptr, c->ktab_b.ptr, c->x.ptr, c->v.ptr, c->res_slots.ptr, ncl, c->sweeps.ptr,
                            cap, a, q, threads, lds, bend);
         if (c->prof_on) PBD_HIP(hipEventRecord(next_event(c), s));
@@ -1307,11 +1390,11 @@ void ccd_sweeps(pbd_ctx* c, int n, float dt, const int* cap) {
     ensure_slots(c, 1);
     launch_fill_u64(s, c->res_slots.ptr, (size_t)c->nslots * ncl, 0ull);
     PBD_HIP(hipMemsetAsync(c->sweeps.ptr, 0, sizeof(int) * ncl, s));
-    size_t lds = (size_t)std::max(1, c->plan_max_load) * sizeof(float4);
-    int threads = c->sp.block_threads > 0 ? c->sp.block_threads : 1024;
+    const TileShape shape = tile_shape(c, (int)c->plan.tiles.size());
     bool coll = false;
     for (auto& k : c->cloths) coll |= (k.prm.sphere_on || k.prm.box_on);
     SolveArgs a{};
+    a.substeps = 1;
     a.dt = dt;
     a.check_every = 1;
     a.tol = -1.0;
@@ -1329,11 +1412,10 @@ void ccd_sweeps(pbd_ctx* c, int n, float dt, const int* cap) {
         a.sweep_base = ii;
         if (c->order_first.n) {
             if (c->prof_on) PBD_HIP(hipEventRecord(next_event(c), s));
-            launch_tiles(s, (int)c->order_first.n, c->order_first.ptr, c->tiles.ptr, c->tverts.ptr, c->tdist.ptr,
-                         c->tdist_rest.ptr, c->tbend.ptr, c->tbend_rest.ptr, c->town.ptr, c->town_rest.ptr,
-                         c->tcols.ptr, c->cl.ptr, c->ktab_d.ptr, c->ktab_b.ptr, c->x.ptr, c->v.ptr, c->pbuf[cur].ptr,
-                         c->pbuf[cur ^ 1].ptr, c->res_slots.ptr, ncl, c->sweeps.ptr, cap, a, threads, lds,
-                         !c->plan.bend.empty());
+            launch_tiles(s, (int)c->order_first.n, c->order_first.ptr, c->tiles.ptr, c->tverts.ptr, c->tdist.ptr, c->tbend.ptr,
+                     c->town.ptr, c->town_rest.ptr, c->tphases.ptr, c->tcounts.ptr, c->cl.ptr, c->ktab_d.ptr, c->ktab_b.ptr, c->x.ptr, c->v.ptr, c->pbuf[cur].ptr,
+                         c->pbuf[cur ^ 1].ptr, c->res_slots.ptr, ncl, c->sweeps.ptr, cap, a, shape.threads,
+                         shape.lds, !c->plan.bend.empty(), shape.regs);
             if (c->prof_on) PBD_HIP(hipEventRecord(next_event(c), s));
         }
         c->pcur = cur ^ 1;
@@ -1545,18 +1627,18 @@ void step_cloth(pbd_ctx* c, int ci, float dt) {
     ensure_slots(c, nchunks);
     launch_fill_u64(s, c->res_slots.ptr, (size_t)c->nslots * ncl, 0ull);
     launch_fill_int(s, c->sweeps.ptr + ci, 1, 0);
-    size_t lds = (size_t)std::max(1, c->plan_max_load) * sizeof(float4);
-    int threads = c->sp.block_threads > 0 ? c->sp.block_threads : 1024;
+    const TileShape shape = tile_shape(c, nblocks);
     SolveArgs a{};
+    a.substeps = 1;
     a.dt = dt;
     a.check_every = ce;
     a.tol = c->sp.tol;
     a.kmax = c->kmax;
     auto tiles = [&](const float4* pin, float4* pout) {
-        launch_tiles(s, nblocks, order, c->tiles.ptr, c->tverts.ptr, c->tdist.ptr, c->tdist_rest.ptr, c->tbend.ptr,
-                     c->tbend_rest.ptr, c->town.ptr, c->town_rest.ptr, c->tcols.ptr, c->cl.ptr, c->ktab_d.ptr,
+        launch_tiles(s, nblocks, order, c->tiles.ptr, c->tverts.ptr, c->tdist.ptr, c->tbend.ptr,
+                     c->town.ptr, c->town_rest.ptr, c->tphases.ptr, c->tcounts.ptr, c->cl.ptr, c->ktab_d.ptr,
                      c->ktab_b.ptr, c->x.ptr, c->v.ptr, pin, pout, c->res_slots.ptr, ncl, c->sweeps.ptr, nullptr, a,
-                     threads, lds, !c->plan.bend.empty());
+                     shape.threads, shape.lds, !c->plan.bend.empty(), shape.regs);
     };
     int cur = c->pcur;
     if (k.whole) {
@@ -1599,10 +1681,47 @@ void step_cloth(pbd_ctx* c, int ci, float dt) {
     }
 }
 
+// A context of single-tile cloths only, with nothing to do between their
+// substeps: each cloth's workgroup can run them all in one launch.
+bool whole_only(const pbd_ctx* c) {
+    return c->sp.path == PBD_PATH_AUTO && !c->coll.enabled && !c->ws.enabled && !c->prof_on && !has_tolerance(c) &&
+           c->any_whole && !c->any_partial;
+}
+
+// n substeps of such a context in one launch.
+void step_whole(pbd_ctx* c, int n, float dt) {
+    hipStream_t s = c->stream;
+    advect_prepare(c, dt);
+    const int ncl = (int)c->cloths.size();
+    ensure_slots(c, 1);
+    const TileShape shape = tile_shape(c, (int)c->plan.tiles.size());
+    SolveArgs a{};
+    a.substeps = n;
+    a.dt = dt;
+    a.check_every = std::max(1, c->sp.check_every);
+    a.tol = -1.0;
+    a.kmax = c->kmax;
+    a.nsweeps = a.whole_nsweeps = c->sp.iterations;
+    a.fused = 1;
+    const int cur = c->pcur;
+    launch_tiles(s, (int)c->order_whole.n, c->order_whole.ptr, c->tiles.ptr, c->tverts.ptr, c->tdist.ptr, c->tbend.ptr,
+                 c->town.ptr, c->town_rest.ptr, c->tphases.ptr, c->tcounts.ptr, c->cl.ptr, c->ktab_d.ptr, c->ktab_b.ptr,
+                 c->x.ptr, c->v.ptr, c->pbuf[cur].ptr, c->pbuf[cur ^ 1].ptr, c->res_slots.ptr, ncl, c->sweeps.ptr,
+                 nullptr, a, shape.threads, shape.lds, !c->plan.bend.empty(), shape.regs);
+    c->pcur = cur ^ 1;  // every cloth with a tile wrote it
+    c->pfinal_valid = false;
+    c->sweeps_pending = false;
+    for (auto& k : c->cloths) k.last_sweeps = c->sp.iterations;
+}
+
 // pbd_step's loop: graph replays where eligible, eager substeps otherwise.
 void run_substeps(pbd_ctx* c, int n) {
     replan_if_needed(c);
     const float dt = c->sp.dt;
+    if (whole_only(c)) {
+        for (int s = 0; s < n; s += 64) step_whole(c, std::min(64, n - s), dt);  // launches of bounded length
+        return;
+    }
     const bool graph = graph_eligible(c);
     if (graph) {
         // everything a capture must not do (allocations, uploads) happens first
@@ -1640,9 +1759,9 @@ int pbd_create(int device, pbd_ctx** out) {
             int lds = 0;
             PBD_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
             PBD_HIP(hipDeviceGetAttribute(&c->num_cu, hipDeviceAttributeMultiprocessorCount, device));
-            // lds_max - TILE_STATIC_LDS is what the tile kernel's dynamic LDS may reach
-            const size_t dyn = tiles_lds_optin((size_t)std::max(lds, 65536) - TILE_STATIC_LDS);
-            c->lds_max = (int)dyn + TILE_STATIC_LDS;
+            // the vertices' lds_max - TILE_STATIC_LDS and the tail are what a tile kernel's dynamic LDS may reach
+            const size_t dyn = tiles_lds_optin((size_t)std::max(lds, 65536) - (TILE_STATIC_LDS - TILE_TAIL_LDS));
+            c->lds_max = (int)dyn + (TILE_STATIC_LDS - TILE_TAIL_LDS);
         } catch (...) {
             delete c;
             throw;
@@ -1830,6 +1949,8 @@ int pbd_cloth_get_info(pbd_ctx* ctx, int id, pbd_cloth_info* info) {
         Cloth& c = cloth_of(ctx, id);
         PBD_CHECK(info, PBD_ERR_ARG, "null info");
         PBD_CHECK(ctx->inited, PBD_ERR_STATE, "call pbd_init first");
+        set_device(ctx);
+        replan_if_needed(ctx);  // the tile counts
         info->nv = c.nv;
         info->nt = c.nt;
         info->ne = c.ne;

@@ -484,20 +484,127 @@ struct Block { int x0, x1, y0, y1; };
 
 }  // namespace
 
-void plan_tiles(std::vector<Cloth>& cloths, int max_load, int sweeps, bool split_whole, TilePlan& plan) {
+// Runs f(i) for i in [0, n) on `threads` threads (each index once).
+template <class F>
+static void parallel_for(size_t n, unsigned threads, F&& f) {
+    std::atomic_size_t next{0};
+    auto work = [&]() {
+        for (size_t i; (i = next.fetch_add(1)) < n;) f(i);
+    };
+    std::vector<std::thread> pool;
+    for (unsigned t = 1; t < threads && t < n; t++) pool.emplace_back(work);
+    work();
+    for (auto& th : pool) th.join();
+}
+
+// Side of a grid cloth's nominal square block: the largest (in steps of 0.85)
+// whose central cone fits the loaded budget.
+static int grid_block_side(const Cloth& c, const ClothTopo& topo, int max_load, int phases, std::vector<int>& mark,
+                           std::vector<int>& entry, int& stamp) {
+    int T = std::max(4, (int)std::sqrt((double)max_load) - 2);
+    for (;;) {
+        int cx = std::max(0, c.rx / 2 - T / 2), cy = std::max(0, c.ry / 2 - T / 2);
+        std::vector<int> in;
+        for (int y = cy; y < std::min(c.ry, cy + T); y++)
+            for (int x = cx; x < std::min(c.rx, cx + T); x++) in.push_back(y * c.rx + x);
+        int n = plan_one(topo, in, phases, max_load, mark, entry, stamp++, nullptr);
+        if (n <= max_load || T <= 4) return T;
+        T = std::max(4, (int)(T * 0.85));
+    }
+}
+
+// The nominal interior blocks of a cloth: squares of a grid, id ranges of a
+// general mesh.
+static std::vector<Block> nominal_blocks(const Cloth& c, const ClothTopo& topo, int max_load, int phases,
+                                         std::vector<int>& mark, std::vector<int>& entry, int& stamp) {
+    std::vector<Block> todo;
+    if (c.rx > 0) {
+        const int T = grid_block_side(c, topo, max_load, phases, mark, entry, stamp);
+        for (int y0 = 0; y0 < c.ry; y0 += T)
+            for (int x0 = 0; x0 < c.rx; x0 += T) todo.push_back({x0, std::min(c.rx, x0 + T), y0, std::min(c.ry, y0 + T)});
+    } else {
+        int T = std::max(16, max_load / 3);
+        for (int a = 0; a < c.nv; a += T) todo.push_back({a, std::min(c.nv, a + T), 0, 1});
+    }
+    return todo;
+}
+
+// The tiles of one nominal block, split in halves until every cone fits.
+// Returns false when a single vertex's cone does not.
+static bool plan_block(const Cloth& c, const ClothTopo& topo, Block first, int max_load, int phases,
+                       std::vector<int>& mark, std::vector<int>& entry, int& stamp, std::vector<TileOut>& outs) {
+    std::vector<Block> todo(1, first);
+    while (!todo.empty()) {
+        Block b = todo.back();
+        todo.pop_back();
+        std::vector<int> in;
+        if (c.rx > 0) {
+            for (int y = b.y0; y < b.y1; y++)
+                for (int x = b.x0; x < b.x1; x++) in.push_back(y * c.rx + x);
+        } else {
+            for (int v = b.x0; v < b.x1; v++) in.push_back(v);
+        }
+        TileOut o;
+        int n = plan_one(topo, in, phases, max_load, mark, entry, stamp++, &o);
+        if (n <= max_load) {
+            outs.push_back(std::move(o));
+            continue;
+        }
+        int wx = b.x1 - b.x0, wy = b.y1 - b.y0;
+        if ((c.rx > 0 && wx * wy <= 1) || (c.rx == 0 && wx <= 1)) return false;
+        if (c.rx > 0 && wx >= wy) {
+            int m = b.x0 + wx / 2;
+            todo.push_back({b.x0, m, b.y0, b.y1});
+            todo.push_back({m, b.x1, b.y0, b.y1});
+        } else if (c.rx > 0) {
+            int m = b.y0 + wy / 2;
+            todo.push_back({b.x0, b.x1, b.y0, m});
+            todo.push_back({b.x0, b.x1, m, b.y1});
+        } else {
+            int m = b.x0 + wx / 2;
+            todo.push_back({b.x0, m, 0, 1});
+            todo.push_back({m, b.x1, 0, 1});
+        }
+    }
+    return true;
+}
+
+std::vector<int> fitting_loads(const std::vector<Cloth>& cloths, int whole_load, const std::vector<int>& loads, int sweeps,
+                               int max_tiles) {
+    const Cloth* big = nullptr;
+    for (const Cloth& c : cloths)
+        if (c.nv > whole_load && (!big || c.nv > big->nv)) big = &c;
+    if (!big || big->rx == 0) return {};
+    ClothTopo topo;
+    build_topo(*big, topo);
+    std::vector<int> mark((size_t)big->nv, -1), entry((size_t)big->nv, 0), fit;
+    int stamp = 0;
+    bool seen = false;
+    for (int load : loads) {
+        if (!seen) {
+            const int T = grid_block_side(*big, topo, load, std::max(1, sweeps) * big->ncolors, mark, entry, stamp);
+            long long n = 0;
+            for (const Cloth& c : cloths)
+                n += c.nv <= whole_load ? 1 : (long long)((c.rx + T - 1) / T) * ((c.ry + T - 1) / T);
+            seen = n <= max_tiles;
+        }
+        if (seen) fit.push_back(load);
+    }
+    return fit;
+}
+
+void plan_tiles(std::vector<Cloth>& cloths, int whole_load, int max_load, int sweeps, bool split_whole, TilePlan& plan) {
     plan = TilePlan();
     struct Pending { int cloth; std::vector<TileOut> outs; };
     std::vector<Pending> per(cloths.size());
-    std::vector<std::thread> pool;
-    unsigned hw = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    // Large cloths are planned in parallel; a small one is a single tile of
-    // all its vertices (no halo), whole unless split_whole asks for it to be
-    // stepped like a multi-tile cloth.
+    const unsigned hw = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
+    // A small cloth is a single tile of all its vertices (no halo), whole
+    // unless split_whole asks for it to be stepped like a multi-tile cloth.
     std::vector<int> work;
     for (size_t ci = 0; ci < cloths.size(); ci++) {
         Cloth& c = cloths[ci];
         per[ci].cloth = (int)ci;
-        const bool fits = c.nv <= max_load;
+        const bool fits = c.nv <= whole_load;
         c.whole = fits && !split_whole;
         c.max_loaded = 0;
         if (fits) {
@@ -519,88 +626,44 @@ void plan_tiles(std::vector<Cloth>& cloths, int max_load, int sweeps, bool split
             work.push_back((int)ci);
         }
     }
-    std::string err;
-    auto run_cloth = [&](int ci) {
+    // Many cloths are planned side by side, few cloths block by block.
+    std::atomic_bool failed{false};
+    const unsigned outer = work.size() >= hw ? hw : 1, inner = work.size() >= hw ? 1 : hw;
+    parallel_for(work.size(), outer, [&](size_t w) {
+        const int ci = work[w];
         Cloth& c = cloths[ci];
         ClothTopo topo;
         build_topo(c, topo);
-        std::vector<int> mark((size_t)c.nv, -1), entry((size_t)c.nv, 0);
-        int stamp = 0;
-        int phases = std::max(1, sweeps) * c.ncolors;
-        std::vector<Block> todo;
-        if (c.rx > 0) {
-            int T = std::max(4, (int)std::sqrt((double)max_load) - 2);
-            // shrink the nominal block until a central block's cone fits
-            for (;;) {
-                int cx = std::max(0, c.rx / 2 - T / 2), cy = std::max(0, c.ry / 2 - T / 2);
-                std::vector<int> in;
-                for (int y = cy; y < std::min(c.ry, cy + T); y++)
-                    for (int x = cx; x < std::min(c.rx, cx + T); x++) in.push_back(y * c.rx + x);
-                int n = plan_one(topo, in, phases, max_load, mark, entry, stamp++, nullptr);
-                if (n <= max_load || T <= 4) break;
-                T = std::max(4, (int)(T * 0.85));
-            }
-            for (int y0 = 0; y0 < c.ry; y0 += T)
-                for (int x0 = 0; x0 < c.rx; x0 += T)
-                    todo.push_back({x0, std::min(c.rx, x0 + T), y0, std::min(c.ry, y0 + T)});
-        } else {
-            int T = std::max(16, max_load / 3);
-            for (int a = 0; a < c.nv; a += T) todo.push_back({a, std::min(c.nv, a + T), 0, 1});
+        const int phases = std::max(1, sweeps) * c.ncolors;
+        std::vector<Block> blocks;
+        {
+            std::vector<int> mark((size_t)c.nv, -1), entry((size_t)c.nv, 0);
+            int stamp = 0;
+            blocks = nominal_blocks(c, topo, max_load, phases, mark, entry, stamp);
         }
-        std::vector<TileOut> outs;
-        while (!todo.empty()) {
-            Block b = todo.back();
-            todo.pop_back();
-            std::vector<int> in;
-            if (c.rx > 0) {
-                for (int y = b.y0; y < b.y1; y++)
-                    for (int x = b.x0; x < b.x1; x++) in.push_back(y * c.rx + x);
-            } else {
-                for (int v = b.x0; v < b.x1; v++) in.push_back(v);
-            }
-            TileOut o;
-            int n = plan_one(topo, in, phases, max_load, mark, entry, stamp++, &o);
-            if (n <= max_load) {
-                outs.push_back(std::move(o));
-                c.max_loaded = std::max(c.max_loaded, n);
-                continue;
-            }
-            int wx = b.x1 - b.x0, wy = b.y1 - b.y0;
-            if ((c.rx > 0 && wx * wy <= 1) || (c.rx == 0 && wx <= 1)) {
-                err = "a single vertex's dependency cone exceeds the tile budget; lower the sweeps per launch";
-                return;
-            }
-            if (c.rx > 0 && wx >= wy) {
-                int m = b.x0 + wx / 2;
-                todo.push_back({b.x0, m, b.y0, b.y1});
-                todo.push_back({m, b.x1, b.y0, b.y1});
-            } else if (c.rx > 0) {
-                int m = b.y0 + wy / 2;
-                todo.push_back({b.x0, b.x1, b.y0, m});
-                todo.push_back({b.x0, b.x1, m, b.y1});
-            } else {
-                int m = b.x0 + wx / 2;
-                todo.push_back({b.x0, m, 0, 1});
-                todo.push_back({m, b.x1, 0, 1});
-            }
-        }
-        // spatial order: by the first interior vertex
-        std::sort(outs.begin(), outs.end(), [](const TileOut& a, const TileOut& b) { return a.load[0] < b.load[0]; });
-        per[ci].outs = std::move(outs);
-    };
-    std::atomic_size_t next{0};
-    for (unsigned t = 0; t < hw; t++)
-        pool.emplace_back([&]() {
-            for (;;) {
-                size_t i = next.fetch_add(1);
-                if (i >= work.size()) break;
-                run_cloth(work[i]);
-            }
+        std::vector<std::vector<TileOut>> outs(blocks.size());
+        // runs of blocks share one set of marks
+        const size_t run = std::max<size_t>(1, (blocks.size() + 2 * inner - 1) / (2 * inner));
+        parallel_for((blocks.size() + run - 1) / run, inner, [&](size_t r) {
+            std::vector<int> mark((size_t)c.nv, -1), entry((size_t)c.nv, 0);
+            int stamp = 0;
+            for (size_t k = r * run; k < std::min(blocks.size(), (r + 1) * run); k++)
+                if (!plan_block(c, topo, blocks[k], max_load, phases, mark, entry, stamp, outs[k])) failed = true;
         });
-    for (auto& th : pool) th.join();
-    PBD_CHECK(err.empty(), PBD_ERR_LIMIT, err);
+        auto& all = per[ci].outs;
+        for (auto& o : outs)
+            for (auto& t : o) all.push_back(std::move(t));
+        for (auto& t : all) c.max_loaded = std::max(c.max_loaded, (int)t.load.size());
+        // spatial order: by the first interior vertex
+        std::sort(all.begin(), all.end(), [](const TileOut& a, const TileOut& b) { return a.load[0] < b.load[0]; });
+    });
+    PBD_CHECK(!failed, PBD_ERR_LIMIT,
+              "a single vertex's dependency cone exceeds the tile budget; lower the sweeps per launch");
 
-    // Flatten.
+    // Flatten: offsets first, then the tiles' records side by side.
+    struct Place { const Cloth* c; const TileOut* o; int own_at, vert_at, dist_at, bend_at; };
+    std::vector<Place> place;
+    size_t nverts = 0, ndist = 0, nbend = 0, nown = 0, nphase = 0, ncount = 0;
     for (size_t ci = 0; ci < cloths.size(); ci++) {
         Cloth& c = cloths[ci];
         c.tile_begin = (int)plan.tiles.size();
@@ -611,97 +674,127 @@ void plan_tiles(std::vector<Cloth>& cloths, int max_load, int sweeps, bool split
             TileDev td{};
             td.cloth = (int)ci;
             td.whole = c.whole ? 1 : 0;
-            td.load_off = (int)plan.verts.size();
+            td.load_off = (int)nverts;
             td.n_load = (int)o.load.size();
             td.n_int = o.n_int;
             td.ncolors = c.ncolors;
-            td.col_off = (int)plan.cols.size();
-            td.dist_off = (int)plan.dist_rest.size();
-            td.bend_off = (int)plan.bend_rest.size();
-            td.own_off = (int)plan.own_rest.size();
+            td.phase_off = (int)nphase;
+            td.count_off = (int)ncount;
+            td.own_off = (int)nown;
             td.n_own = (int)o.own.size();
-            std::vector<int> local((size_t)c.nv, -1);
-            for (size_t k = 0; k < o.load.size(); k++) {
-                local[o.load[k]] = (int)k;
-                plan.verts.push_back(c.vbase + o.load[k]);
-            }
-            PBD_CHECK(o.load.size() <= 65535, PBD_ERR_LIMIT, "tile exceeds 16-bit local indices");
-            int dsum = 0, bsum = 0;
-            for (int col = 0; col < c.ncolors; col++) {
-                plan.cols.push_back(dsum);
-                dsum += (int)o.dist_by_col[col].size();
-            }
-            plan.cols.push_back(dsum);
-            for (int col = 0; col < c.ncolors; col++) {
-                plan.cols.push_back(bsum);
-                bsum += (int)o.bend_by_col[col].size();
-            }
-            plan.cols.push_back(bsum);
-            // per-sweep prefixes of the partial tiles: sweeps x C distance
-            // counts, sweeps x C bending counts, then the loaded vertices of
-            // a launch of 1 .. sweeps sweeps
+            PBD_CHECK(o.load.size() <= (size_t)REC_MAX_VERTS, PBD_ERR_LIMIT, "tile exceeds 15-bit local indices");
             td.plan_sweeps = o.dcount.empty() ? 0 : (int)(o.dcount.size() / std::max(1, c.ncolors));
-            plan.cols.insert(plan.cols.end(), o.dcount.begin(), o.dcount.end());
-            plan.cols.insert(plan.cols.end(), o.bcount.begin(), o.bcount.end());
+            PBD_CHECK(!td.plan_sweeps || (int)o.lcount.size() == td.plan_sweeps, PBD_ERR_STATE,
+                      "internal: load prefix count");
+            place.push_back({&c, &o, (int)nown, (int)nverts, (int)ndist, (int)nbend});
+            nverts += o.load.size();
+            nown += o.own.size();
+            for (int col = 0; col < c.ncolors; col++) {
+                ndist += o.dist_by_col[col].size();
+                nbend += o.bend_by_col[col].size();
+            }
+            nphase += (size_t)std::max(1, td.plan_sweeps) * c.ncolors;
+            ncount += (size_t)td.plan_sweeps;
+            plan.max_loaded = std::max(plan.max_loaded, td.n_load);
+            plan.tiles.push_back(td);
+            c.tiles_loaded += (long long)o.load.size();
+            c.tiles_interior += o.n_int;
+            c.tiles_owned += (long long)o.own.size();
             if (td.plan_sweeps) {
-                PBD_CHECK((int)o.lcount.size() == td.plan_sweeps, PBD_ERR_STATE, "internal: load prefix count");
-                plan.cols.insert(plan.cols.end(), o.lcount.begin(), o.lcount.end());
                 for (int n = 1; n <= td.plan_sweeps && n < (int)c.tile_loaded_by_sweeps.size(); n++)
                     c.tile_loaded_by_sweeps[n] += o.lcount[(size_t)n - 1];
             } else {
                 for (size_t n = 1; n < c.tile_loaded_by_sweeps.size(); n++)
                     c.tile_loaded_by_sweeps[n] += (double)o.load.size();
             }
-            c.tiles_loaded += (long long)o.load.size();
-            c.tiles_interior += o.n_int;
-            c.tiles_owned += (long long)o.own.size();
-            if (o.dcount.empty()) {
-                // every prim at every sweep: the bytes of one sweep
-                double b = 0.0;
-                for (int col = 0; col < c.ncolors; col++)
-                    b += 8.0 * o.dist_by_col[col].size() + 12.0 * o.bend_by_col[col].size();
-                c.tile_record_bytes[1] += b;
-            } else {
-                const int ps = td.plan_sweeps;
-                for (int n = 1; n <= ps && n < (int)c.tile_record_bytes.size(); n++) {
-                    double b = 0.0;
-                    for (int sw = 0; sw < n; sw++)
-                        for (int col = 0; col < c.ncolors; col++) {
-                            const size_t q = (size_t)(sw + ps - n) * c.ncolors + col;
-                            b += 8.0 * o.dcount[q] + 12.0 * o.bcount[q];
-                        }
-                    c.tile_record_bytes[n] += b;
-                }
-            }
             plan.stat_loaded += (long long)o.load.size();
             plan.stat_interior += o.n_int;
-            for (int col = 0; col < c.ncolors; col++) plan.stat_dist_loaded += (long long)o.dist_by_col[col].size();
-            for (size_t q = 0; q < o.dcount.size(); q++) plan.stat_dist_phase_needed += o.dcount[q];
-            if (o.dcount.empty())
-                for (int col = 0; col < c.ncolors; col++)
-                    plan.stat_dist_phase_needed += (long long)sweeps * o.dist_by_col[col].size();
-            for (int col = 0; col < c.ncolors; col++)
-                for (int p : o.dist_by_col[col]) {
-                    const int* ix = &c.indices[c.prim_list[2 * p]];
-                    plan.dist.push_back((uint32_t)local[ix[0]] | ((uint32_t)local[ix[1]] << 16));
-                    plan.dist_rest.push_back(c.rest[p]);
+            if (o.dcount.empty()) {
+                // every prim at every sweep: the bytes of one sweep
+                for (int col = 0; col < c.ncolors; col++) {
+                    const size_t nd = o.dist_by_col[col].size(), nb = o.bend_by_col[col].size();
+                    c.tile_record_bytes[1] += 8.0 * nd + 16.0 * nb;
+                    plan.stat_dist_loaded += (long long)nd;
+                    plan.stat_dist_phase_needed += (long long)sweeps * nd;
+                    plan.max_phase = std::max(plan.max_phase, (int)std::max(nd, nb));
                 }
-            for (int col = 0; col < c.ncolors; col++)
-                for (int p : o.bend_by_col[col]) {
-                    const int* ix = &c.indices[c.prim_list[2 * p]];
-                    plan.bend.push_back((uint32_t)local[ix[0]] | ((uint32_t)local[ix[1]] << 16));
-                    plan.bend.push_back((uint32_t)local[ix[2]] | ((uint32_t)local[ix[3]] << 16));
-                    plan.bend_rest.push_back(c.rest[p]);
+            } else {
+                const int ps = td.plan_sweeps;
+                for (int col = 0; col < c.ncolors; col++) plan.stat_dist_loaded += (long long)o.dist_by_col[col].size();
+                for (size_t q = 0; q < o.dcount.size(); q++) {
+                    plan.stat_dist_phase_needed += o.dcount[q];
+                    plan.max_phase = std::max(plan.max_phase, std::max(o.dcount[q], o.bcount[q]));
+                    // row q / ncolors runs in the launches of at least ps - row sweeps
+                    for (int n = ps - (int)(q / c.ncolors); n <= ps && n < (int)c.tile_record_bytes.size(); n++)
+                        c.tile_record_bytes[n] += 8.0 * o.dcount[q] + 16.0 * o.bcount[q];
                 }
-            for (int p : o.own) {
-                const int* ix = &c.indices[c.prim_list[2 * p]];
-                plan.own.push_back((uint32_t)local[ix[0]] | ((uint32_t)local[ix[1]] << 16));
-                plan.own_rest.push_back(c.rest[p]);
             }
-            plan.tiles.push_back(td);
         }
         c.tile_end = (int)plan.tiles.size();
     }
+    PBD_CHECK(nverts < (1ull << 31) && ndist < (1ull << 31) && nbend < (1ull << 31) && nphase < (1ull << 31),
+              PBD_ERR_LIMIT, "tile plan exceeds 2^31 records");
+    plan.verts.resize(nverts);
+    plan.dist.resize(ndist);
+    plan.bend.resize(nbend);
+    plan.own.resize(nown);
+    plan.own_rest.resize(nown);
+    plan.phases.resize(nphase);
+    plan.counts.resize(ncount);
+    const size_t runs = std::min<size_t>(place.size(), 4 * hw);
+    parallel_for(runs, hw, [&](size_t r) {
+        std::vector<int> local;  // cloth vertex -> slot; only entries of the tile at hand are read
+        for (size_t t = r * place.size() / runs; t < (r + 1) * place.size() / runs; t++) {
+            const TileDev& td = plan.tiles[t];
+            const Cloth& c = *place[t].c;
+            const TileOut& o = *place[t].o;
+            if (local.size() < (size_t)c.nv) local.resize((size_t)c.nv);
+            for (size_t k = 0; k < o.load.size(); k++) {
+                local[o.load[k]] = (int)k;
+                plan.verts[(size_t)td.load_off + k] = c.vbase + o.load[k];
+            }
+            auto pair = [&](int a, int b) { return (uint32_t)local[a] | ((uint32_t)local[b] << 16); };
+            size_t at = (size_t)place[t].dist_at;
+            for (int col = 0; col < c.ncolors; col++)
+                for (int p : o.dist_by_col[col]) {
+                    const int* ix = &c.indices[c.prim_list[2 * p]];
+                    const float w0 = c.w[ix[0]], w1 = c.w[ix[1]];
+                    const uint32_t general = (w0 == w1 && w0 != 0.0f) ? 0u : REC_GENERAL;
+                    uint32_t rest;
+                    memcpy(&rest, &c.rest[p], 4);
+                    plan.dist[at++] = make_uint2(pair(ix[0], ix[1]) | general, rest);
+                }
+            at = (size_t)place[t].bend_at;
+            for (int col = 0; col < c.ncolors; col++)
+                for (int p : o.bend_by_col[col]) {
+                    const int* ix = &c.indices[c.prim_list[2 * p]];
+                    uint32_t rest;
+                    memcpy(&rest, &c.rest[p], 4);
+                    plan.bend[at++] = make_uint4(pair(ix[0], ix[1]), pair(ix[2], ix[3]), rest, 0u);
+                }
+            at = (size_t)td.own_off;
+            for (int p : o.own) {
+                const int* ix = &c.indices[c.prim_list[2 * p]];
+                plan.own[at] = pair(ix[0], ix[1]);
+                plan.own_rest[at++] = c.rest[p];
+            }
+            // record ranges of every colour phase: the prefix of the colour's
+            // records that the row's sweep needs (whole tiles: all of them)
+            at = (size_t)td.phase_off;
+            for (int row = 0; row < std::max(1, td.plan_sweeps); row++) {
+                int db = place[t].dist_at, bb = place[t].bend_at;
+                for (int col = 0; col < c.ncolors; col++) {
+                    const size_t q = (size_t)row * c.ncolors + col;
+                    const int nd = (int)o.dist_by_col[col].size(), nb = (int)o.bend_by_col[col].size();
+                    plan.phases[at++] = make_int4(db, db + (td.plan_sweeps ? o.dcount[q] : nd), bb,
+                                                  bb + (td.plan_sweeps ? o.bcount[q] : nb));
+                    db += nd;
+                    bb += nb;
+                }
+            }
+            std::copy(o.lcount.begin(), o.lcount.end(), plan.counts.begin() + td.count_off);
+        }
+    });
     // Tile neighbours: t and n are neighbours when one loads a vertex of the
     // other's interior (a later chunk of t reads what n wrote, or writes what
     // n read).  Only tiles of the same cloth share vertices.

@@ -111,16 +111,14 @@ struct TileDev {
     int load_off;        // offset into tile_verts
     int n_load;
     int n_int;           // interior vertices = first n_int of the loaded list
-    int dist_off;        // offset into tile_dist of colour 0
-    int bend_off;        // offset into tile_bend of colour 0
     int own_off;         // offset into tile_own (distance prims owned by the tile)
     int n_own;
-    int col_off;         // offset into tile_cols: (ncolors+1) dist offsets, (ncolors+1) bend offsets, then for
-                         // partial tiles plan_sweeps x ncolors dist counts and as many bend counts
+    int phase_off;       // offset into tile_phases: one int4 (distance begin, end, bending begin, end) per colour
+                         // phase, ncolors per sweep row; partial tiles hold plan_sweeps rows, whole tiles one
+    int count_off;       // offset into tile_counts: the vertices a launch of 1 .. plan_sweeps sweeps loads
     int ncolors;
     int plan_sweeps;     // partial tiles: sweeps per launch the cone was planned for; sweep s of an n-sweep
-                         // launch runs the first counts[(s + plan_sweeps - n) * ncolors + c] prims of colour c
-                         // (0: whole tiles, every prim of the colour)
+                         // launch runs the phases of row s + plan_sweeps - n (0: whole tiles, row 0 every sweep)
 };
 
 // Kernel-wide parameters of one solver launch.
@@ -145,6 +143,8 @@ struct SolveArgs {
                          //    a launch where this can happen reads x
     int coherent_load;   // 1: p_in was written earlier in this launch by other workgroups (a queued
                          //    later chunk): loaded past every cache
+    int substeps;        // fused single-tile cloths: substeps this launch runs
+    int lds_slots;       // vertices of dynamic LDS before the tail (set by the launch functions)
     int queue_ts;        // queued launches: sweeps per chunk; a tile whose cloth has a further chunk
                          //    stores p_out write-through for it (0: not queued)
 };
@@ -347,17 +347,23 @@ void ws_apply(hipStream_t s, const int* vcloth, float4* p, const float4* delta, 
 void ws_target(hipStream_t s, const ClothDev* cl, const int* vcloth, const float4* pa, const float4* pb, int nv,
                float* y);
 
+// Set in a distance record whose weights are not the same nonzero value on
+// both vertices (a pin, unequal masses): the projection then takes the general form.
+constexpr uint32_t REC_GENERAL = 0x80000000u;
+constexpr int REC_MAX_VERTS = 1 << 15;  // local vertex indices of a tile
+
 // Tile plan for the whole batch.
 struct TilePlan {
     std::vector<TileDev> tiles;
     std::vector<int> verts;               // global vertex ids
-    std::vector<uint32_t> dist;           // packed (i0 | i1 << 16), local indices
-    std::vector<float> dist_rest;
-    std::vector<uint32_t> bend;           // 2 words per prim: (i0|i1<<16), (i2|i3<<16)
-    std::vector<float> bend_rest;
+    std::vector<uint2> dist;              // (i0 | i1 << 16 | REC_GENERAL, rest bits), local indices of 15 bits
+    std::vector<uint4> bend;              // (i0 | i1 << 16, i2 | i3 << 16, rest bits, 0)
     std::vector<uint32_t> own;            // owned distance prims (local pair)
     std::vector<float> own_rest;
-    std::vector<int> cols;                // per tile colour offsets
+    std::vector<int4> phases;             // per tile, sweep row and colour: record ranges (see TileDev)
+    std::vector<int> counts;              // per partial tile: loaded vertices of a launch of 1 .. sweeps sweeps
+    int max_loaded = 0;                   // most vertices one tile loads
+    int max_phase = 0;                    // most records of one kind in one colour phase of one tile
     std::vector<int> partial_order;       // launch order of the partial tiles only
     std::vector<int> whole_order;         // launch order of the whole tiles only
     // neighbours of each partial tile (CSR over tiles): the tiles of its
@@ -368,9 +374,15 @@ struct TilePlan {
     // and distance prim updates of one launch of `sweeps` sweeps
     long long stat_loaded = 0, stat_interior = 0, stat_dist_loaded = 0, stat_dist_phase_needed = 0;
 };
-// split_whole: a cloth that fits one tile still gets a (single, halo-free)
-// multi-launch tile instead of a whole tile.
-void plan_tiles(std::vector<Cloth>& cloths, int max_load, int sweeps_per_launch, bool split_whole, TilePlan& plan);
+// The budgets of `loads` (ascending) from the first at which a batch of grid
+// cloths takes about max_tiles tiles or fewer.
+std::vector<int> fitting_loads(const std::vector<Cloth>& cloths, int whole_load, const std::vector<int>& loads,
+                               int sweeps_per_launch, int max_tiles);
+// A cloth of at most whole_load vertices is one tile; the others' tiles load
+// at most max_load.  split_whole: a cloth that fits one tile still gets a
+// (single, halo-free) multi-launch tile instead of a whole tile.
+void plan_tiles(std::vector<Cloth>& cloths, int whole_load, int max_load, int sweeps_per_launch, bool split_whole,
+                TilePlan& plan);
 
 // ---------------------------------------------------------------------------
 // Kernel launchers (implemented in the .hip files)
@@ -421,13 +433,12 @@ void launch_jacobi(hipStream_t s, const JacobiDev& J, const ClothDev* cloths, co
 void launch_residual(hipStream_t s, const int4* dist, int n, const float4* p,
                      unsigned long long* rmax, double* rsum, int* rcnt);
 void launch_tiles(hipStream_t s, int nblocks, const int* order, const TileDev* tiles,
-                  const int* verts, const uint32_t* dist, const float* dist_rest,
-                  const uint32_t* bend, const float* bend_rest, const uint32_t* own,
-                  const float* own_rest, const int* cols, const ClothDev* cloths,
+                  const int* verts, const uint2* dist, const uint4* bend, const uint32_t* own,
+                  const float* own_rest, const int4* phases, const int* counts, const ClothDev* cloths,
                   const float* ktab_d, const float* ktab_b, float4* x, float4* v,
                   const float4* p_in, float4* p_out, unsigned long long* res_slots,
                   int nslots_cloth, int* sweeps_out, const int* sweep_cap, const SolveArgs& a,
-                  int threads, size_t lds_bytes, bool with_bend, const int* n_items = nullptr);
+                  int threads, size_t lds_bytes, bool with_bend, int regs = 0, const int* n_items = nullptr);
 // One launch for every chunk of a substep under per-cloth budgets: the
 // workgroups take (tile, chunk) items from a queue in which every item comes
 // after the items it depends on (its neighbour tiles' previous chunk).
@@ -488,15 +499,15 @@ enum {
 // goes on from the kept prediction or from the unwarmed start.  A cloth's
 // tiles wait for each other, so the launch needs every multi-tile cloth's
 // tiles resident at once (at most nblocks - 1 tiles per cloth).
-void launch_tiles_decide(hipStream_t s, int nblocks, const TileDev* tiles, const int* verts, const uint32_t* dist,
-                         const float* dist_rest, const uint32_t* bend, const float* bend_rest, const uint32_t* own,
-                         const float* own_rest, const int* cols, const ClothDev* cloths, const float* ktab_d,
+void launch_tiles_decide(hipStream_t s, int nblocks, const TileDev* tiles, const int* verts, const uint2* dist,
+                         const uint4* bend, const uint32_t* own, const float* own_rest, const int4* phases,
+                         const int* counts, const ClothDev* cloths, const float* ktab_d,
                          const float* ktab_b, float4* x, float4* v, unsigned long long* res_slots, int ncl,
                          int* sweeps_out, const int* sweep_cap, const SolveArgs& a, const TileQueue& q, int threads,
                          size_t lds_bytes, bool with_bend);
-void launch_tiles_queue(hipStream_t s, int nblocks, const TileDev* tiles, const int* verts, const uint32_t* dist,
-                        const float* dist_rest, const uint32_t* bend, const float* bend_rest, const uint32_t* own,
-                        const float* own_rest, const int* cols, const ClothDev* cloths, const float* ktab_d,
+void launch_tiles_queue(hipStream_t s, int nblocks, const TileDev* tiles, const int* verts, const uint2* dist,
+                        const uint4* bend, const uint32_t* own, const float* own_rest, const int4* phases,
+                        const int* counts, const ClothDev* cloths, const float* ktab_d,
                         const float* ktab_b, float4* x, float4* v, unsigned long long* res_slots, int ncl,
                         int* sweeps_out, const int* sweep_cap, const SolveArgs& a, const TileQueue& q, int threads,
                         size_t lds_bytes, bool with_bend);
@@ -526,7 +537,17 @@ int tiles_per_cu(bool with_bend, int threads, size_t lds_bytes);
 // Opts the tile kernels in to `bytes` of dynamic LDS on the current device;
 // returns what they may use (bytes, or 64 KiB if the runtime refuses).
 size_t tiles_lds_optin(size_t bytes);
-constexpr int TILE_STATIC_LDS = 256;  // bytes reserved for the tile kernel's static LDS (block reductions)
+// A tile launch's dynamic LDS: the tile's vertices, then a tail of
+// TILE_TAIL_LDS bytes (16 doubles of block reductions, an idle vertex pair, a
+// word), so that vertex 0 sits at LDS address 0.  TILE_STATIC_LDS bytes of the
+// CU's LDS are kept from the vertices: the tail, and the few static words of
+// the deciding kernels.
+constexpr int TILE_TAIL_LDS = 256;
+constexpr int TILE_STATIC_LDS = 512;
+constexpr int TILE_IDLE_SLOT = 8, TILE_WORD_SLOT = 10;  // in float4 slots after the vertices
+// The launch form that keeps a tile's distance records in registers
+// (k_tiles_regs<R>): colours and records per thread and colour it holds.
+constexpr int REG_COLORS = 8;
 void launch_fill_u64(hipStream_t s, unsigned long long* p, size_t n, unsigned long long v);
 void launch_fill_int(hipStream_t s, int* p, size_t n, int v);
 void launch_min_sweeps(hipStream_t s, int* sweeps, const int* cap, int sw, int n);

@@ -42,22 +42,16 @@ PBD_HD V3 cross(V3 a, V3 b) {
 }
 PBD_HD V3 scale(float s, V3 a) { return V3{s * a.x, s * a.y, s * a.z}; }
 
-// Correctly rounded square root for x in [2^-96, 2^96]: the hardware
-// estimate s (within 1 ulp) is replaced by its neighbour s - ulp or s + ulp
-// when the fused residual x - s' * s shows that neighbour is nearer
-// (Markstein's correction).  In that range it is the sequence a correctly
-// rounded sqrtf runs without its rescaling of small inputs, so the result
-// equals sqrtf bit for bit; an exhaustive test over every float of the range
-// checks it.
+// Correctly rounded square root for x in [2^-96, 2^96]: g = x y from the
+// hardware reciprocal square root y (within 1 ulp), then one step
+// g + (x - g^2) y / 2 with the residual fused and exact (Markstein 1990).
+// Equal to sqrtf on every float of the range, checked exhaustively by a test.
+// Five operations, one of them transcendental; choosing between the
+// neighbours of the hardware square root took nine.
 __device__ __forceinline__ float sqrt_rn(float x) {
-    float s = __builtin_amdgcn_sqrtf(x);
-    const float sd = __int_as_float(__float_as_int(s) - 1);
-    const float su = __int_as_float(__float_as_int(s) + 1);
-    const float rd = __builtin_fmaf(-sd, s, x);
-    const float ru = __builtin_fmaf(-su, s, x);
-    s = rd <= 0.0f ? sd : s;
-    s = ru > 0.0f ? su : s;
-    return s;
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y, h = 0.5f * y;
+    return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
 }
 
 // Correctly rounded 1/d for d in [2^-48, 2^48]: one Newton step on the

@@ -421,10 +421,97 @@ __device__ __forceinline__ double block_max(double v, double* red) {
 // loading or storing its tile while the other projects).
 template <bool BEND>
 struct TileFetch {
-    static constexpr int dist = BEND ? 8 : 4;
-    static constexpr int bend = 4;
+    static constexpr int dist = 2;
+    static constexpr int bend = 2;
     static constexpr int vert = 4;
 };
+
+typedef float f32x4l __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) f32x4l* lds_vec;
+
+// Projects N distance prims of one colour on the vertices at LDS byte
+// addresses a0, a1; the prims share no vertex, so all are read before any is
+// written and their instruction chains overlap.  A prim of two free vertices
+// of equal weight and a length in [2^-48, 2^48] takes the short form of
+// project_distance: q0 = -1/2 and q1 = 1/2 there, so both vertices move by the
+// same vector m = ((d - L) / 2 * r) * k and negation is exact.  A wave with a
+// prim of the other kind (general, bit 31: a pin or unequal weights; a
+// collapsed edge) projects all its prims in the general form; the results are
+// the same.  One branch per wave in place of the general form's nested
+// per-lane ones.
+template <int N>
+__device__ __forceinline__ void project_pairs(const unsigned* a0, const unsigned* a1, const float* rest, float k,
+                                              unsigned general) {
+    f32x4l A[N], B[N];
+    float vx[N], vy[N], vz[N], d2[N];
+#pragma unroll
+    for (int u = 0; u < N; u++) {
+        A[u] = *(lds_vec)(size_t)a0[u];
+        B[u] = *(lds_vec)(size_t)a1[u];
+    }
+    constexpr unsigned lo = (127u - 96u) << 23, hi = (127u + 96u) << 23;  // 2^-96, 2^96
+    unsigned out = 0;
+#pragma unroll
+    for (int u = 0; u < N; u++) {
+        vx[u] = A[u].x - B[u].x;
+        vy[u] = A[u].y - B[u].y;
+        vz[u] = A[u].z - B[u].z;
+        d2[u] = vx[u] * vx[u] + vy[u] * vy[u] + vz[u] * vz[u];
+        const unsigned o = __float_as_uint(d2[u]) - lo;
+        out = u ? max(out, o) : o;
+    }
+    out |= general;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(out > hi - lo) == 0, 1)) {
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            const float d = sqrt_rn(d2[u]), inv = rcp_rn(d);
+            const float h = 0.5f * (d - rest[u]);
+            vx[u] = h * (vx[u] * inv);
+            vy[u] = h * (vy[u] * inv);
+            vz[u] = h * (vz[u] * inv);
+        }
+        if (k != 1.0f) {  // uniform: a branch, not selects
+            asm volatile("");
+#pragma unroll
+            for (int u = 0; u < N; u++) {
+                vx[u] = vx[u] * k;
+                vy[u] = vy[u] * k;
+                vz[u] = vz[u] * k;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            A[u].x -= vx[u];
+            A[u].y -= vy[u];
+            A[u].z -= vz[u];
+            B[u].x += vx[u];
+            B[u].y += vy[u];
+            B[u].z += vz[u];
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            float4 q0 = make_float4(A[u].x, A[u].y, A[u].z, A[u].w), q1 = make_float4(B[u].x, B[u].y, B[u].z, B[u].w);
+            project_distance(q0, q1, rest[u], k);
+            A[u] = f32x4l{q0.x, q0.y, q0.z, q0.w};
+            B[u] = f32x4l{q1.x, q1.y, q1.z, q1.w};
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < N; u++) {
+        // 16-byte stores: a 12-byte LDS store takes 9.4 cycles per wave against 6.5
+        // (the compiler would leave out the unchanged weight)
+        asm("" : "+v"(A[u]), "+v"(B[u]));
+        *(lds_vec)(size_t)a0[u] = A[u];
+        *(lds_vec)(size_t)a1[u] = B[u];
+    }
+}
+__device__ __forceinline__ unsigned lds_address(const float4* P) {
+    return (unsigned)(size_t)(__attribute__((address_space(3))) const float4*)P;
+}
+// LDS byte addresses of a distance record's vertices (base: of vertex 0).
+__device__ __forceinline__ unsigned rec_a0(uint2 r, unsigned base) { return ((r.x & 0xffffu) << 4) + base; }
+__device__ __forceinline__ unsigned rec_a1(uint2 r, unsigned base) { return ((r.x >> 12) & 0x7fff0u) + base; }
 
 // This thread's max relative residual over the tile's owned distance prims
 // (records fetched PF at a time).
@@ -451,14 +538,14 @@ __device__ __forceinline__ double own_residual(const float4* P, const uint32_t* 
 
 #define TILE_PARAMS                                                                                              \
     const int *__restrict__ order, const TileDev *__restrict__ tiles, const int *__restrict__ verts,              \
-        const uint32_t *__restrict__ dist, const float *__restrict__ dist_rest, const uint32_t *__restrict__ bend, \
-        const float *__restrict__ bend_rest, const uint32_t *__restrict__ own, const float *__restrict__ own_rest, \
-        const int *__restrict__ cols, const ClothDev *__restrict__ cloths, const float *__restrict__ ktab_d,       \
+        const uint2 *__restrict__ dist, const uint4 *__restrict__ bend, const uint32_t *__restrict__ own,           \
+        const float *__restrict__ own_rest, const int4 *__restrict__ phases, const int *__restrict__ counts,       \
+        const ClothDev *__restrict__ cloths, const float *__restrict__ ktab_d,                                     \
         const float *__restrict__ ktab_b, float4 *__restrict__ x, float4 *__restrict__ v,                          \
         const float4 *__restrict__ p_in, float4 *__restrict__ p_out, unsigned long long *__restrict__ res_slots,   \
         int ncl, int *__restrict__ sweeps_out, const int *__restrict__ sweep_cap, SolveArgs a
 #define TILE_ARGS                                                                                               \
-    order, tiles, verts, dist, dist_rest, bend, bend_rest, own, own_rest, cols, cloths, ktab_d, ktab_b, x, v, p_in, \
+    order, tiles, verts, dist, bend, own, own_rest, phases, counts, cloths, ktab_d, ktab_b, x, v, p_in, \
         p_out, res_slots, ncl, sweeps_out, sweep_cap, a
 
 // The hand-off of positions between chunks of one queued launch, whose
@@ -683,7 +770,13 @@ __device__ __forceinline__ bool cloth_decide(const TileQueue& q, const TileDev& 
 // decision itself (qd, see cloth_decide), and every budget is read from qd
 // (the launch writes it; sweep_cap is unused).  Returns the cloth's sweep
 // budget.  slot: the tile (< 0: none).
-template <bool BEND, bool DECIDE = false>
+//
+// REGS > 0 (no bending prims, at most REG_COLORS colours and REGS x threads
+// records per colour, which the host checks): the tile's records stay in
+// registers for the whole launch, REGS per thread and colour.  A phase then
+// waits for nothing but LDS and runs no loop: with the few waves of a small
+// tile its time is the length of its instruction chain.
+template <bool BEND, bool DECIDE = false, int REGS = 0>
 __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, double* red,
                                           const TileQueue* qd = nullptr) {
     constexpr int PREFETCH = TileFetch<BEND>::dist;
@@ -737,15 +830,12 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
         return budget_c;
     }
     const int C = td.ncolors;
-    const int* dc = cols + td.col_off;
-    const int* bc = dc + C + 1;
-    // partial tiles run, at sweep s of this launch, the prefix of each colour
-    // list that the cone of the launch's last nsweeps sweeps needs (the index
-    // is kept within the tile's plan_sweeps rows of counts), and load the
-    // prefix of the vertex list that cone reads
-    const int* dn = bc + C + 1;
-    const int* bn = dn + td.plan_sweeps * C;
-    const int* ln = bn + td.plan_sweeps * C;
+    // partial tiles run, at sweep s of this launch, the phases of the row that
+    // the cone of the launch's last nsweeps sweeps needs, and load the prefix
+    // of the vertex list that cone reads
+    const int4* ph = phases + td.phase_off;
+    const int rows = max(td.plan_sweeps, 1);
+    const int* ln = counts + td.count_off;
     auto cone = [&](int n) { return (td.plan_sweeps && n < td.plan_sweeps) ? ln[n - 1] : td.n_load; };
     bool loaded = false;
     if (deciding) {
@@ -790,6 +880,42 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
     const int n_load = cone(nsweeps);
     // the kept warm-start prediction enters here, on the substep's first load
     const bool add_delta = !loaded && a.delta != nullptr && a.keep[td.cloth] != 0;
+    const int4* ph0 = ph + min(shift, rows - 1) * C;  // the first sweep's row: its ranges hold the later rows'
+    const unsigned base = lds_address(P);
+    constexpr int RN = REGS > 0 ? REGS : 1;
+    unsigned ra[REG_COLORS][RN], rb[REG_COLORS][RN];
+    float rl[REG_COLORS][RN];
+    unsigned any = 0, gen = 0;  // wave-uniform, bit c * RN + u: some lane holds a record, a general one
+    if (REGS > 0) {
+        // lanes without a record project a pair of their own far from every
+        // vertex: two slots at rest length 1, which no projection moves
+        const int idle = a.lds_slots + TILE_IDLE_SLOT;
+        if (tid < 2) P[idle + tid] = make_float4((float)tid, 0.0f, 0.0f, 1.0f);
+#pragma unroll
+        for (int c = 0; c < REG_COLORS; c++) {
+            const int4 r = c < C ? ph0[c] : make_int4(0, 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < RN; u++) {
+                const int j = r.x + u * T + tid;
+                uint2 d = make_uint2((unsigned)idle | ((unsigned)(idle + 1) << 16), __float_as_uint(1.0f));
+                if (j < r.y) d = dist[(unsigned)j];
+                const unsigned bit = 1u << (c * RN + u);
+                if (__builtin_amdgcn_ballot_w64(j < r.y)) any |= bit;
+                if (__builtin_amdgcn_ballot_w64((d.x & REC_GENERAL) != 0)) gen |= bit;
+                ra[c][u] = rec_a0(d, base);
+                rb[c][u] = rec_a1(d, base);
+                rl[c][u] = __uint_as_float(d.y);
+            }
+        }
+    }
+    // A context of single-tile cloths runs several substeps in one launch:
+    // each thread stores and loads the same vertices, so x and v carry over
+    // through memory without a barrier of their own.
+    const int nsub = (td.whole && a.fused) ? a.substeps : 1;
+    int sw = 0;
+    double resid = -1.0;
+    for (int ss = 0; ss < nsub; ss++) {
+    sw = 0;
     for (int i0 = tid; !loaded && i0 < n_load; i0 += VERT_PREFETCH * T) {
         int g[VERT_PREFETCH];
 #pragma unroll
@@ -835,72 +961,105 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
     }
     __syncthreads();
 
-    const uint32_t* D = dist + td.dist_off;
-    const float* DR = dist_rest + td.dist_off;
-    const uint32_t* B = bend + 2 * (size_t)td.bend_off;
-    const float* BR = bend_rest + td.bend_off;
     const bool coll = (cd.sphere_on || cd.box_on) && !a.no_coll;
-    int sw = 0;
-    double resid = -1.0;
+    // The phases run as a pipeline of stages: a stage is up to PREFETCH
+    // distance records per thread of one phase (and, with the phase's last
+    // stage, its bending records).  A stage's records are fetched while the
+    // stage before it projects, across the phase barrier, and the ranges of a
+    // phase two phases ahead, so that a phase waits for LDS only.
+    auto phase_at = [&](int sw, int c) { return ph[min(sw + shift, rows - 1) * C + c]; };
+    auto fetch_dist = [&](uint2* r, int j, int e) {
+#pragma unroll
+        for (int u = 0; u < PREFETCH; u++) r[u] = dist[(unsigned)max(min(j + u * T, e - 1), 0)];
+    };
+    auto fetch_bend = [&](uint4* r, int j, int e) {
+#pragma unroll
+        for (int u = 0; u < BEND_PREFETCH; u++) r[u] = bend[(unsigned)max(min(j + u * T, e - 1), 0)];
+    };
+    int4 now = make_int4(0, 0, 0, 0), next = now;
+    uint2 dr[PREFETCH];
+    uint4 br[BEND_PREFETCH];
+    if (REGS == 0 && C > 0 && nsweeps > 0) {
+        now = phase_at(0, 0);
+        next = C > 1 ? phase_at(0, 1) : phase_at(1, 0);
+        fetch_dist(dr, now.x + tid, now.y);
+        if (BEND) fetch_bend(br, now.z + tid, now.w);
+    }
     for (; sw < nsweeps;) {
         int gs = a.sweep_base + sw;
         int ks = gs < a.kmax ? gs : a.kmax - 1;
         float kd = ktab_d[cd.ktab + ks];
         float kb = ktab_b[cd.ktab + ks];
-        const int* dnow = td.plan_sweeps ? dn + min(sw + shift, td.plan_sweeps - 1) * C : nullptr;
-        const int* bnow = td.plan_sweeps ? bn + min(sw + shift, td.plan_sweeps - 1) * C : nullptr;
-        for (int c = 0; c < C; c++) {
-            // the prim records of a phase are fetched from global memory
-            // in batches of PREFETCH per thread before any is processed, so
-            // the phase waits for one round trip instead of one per prim
-            const int je = dnow ? dc[c] + dnow[c] : dc[c + 1];
-            for (int j0 = dc[c] + tid; j0 < je; j0 += PREFETCH * T) {
-                uint32_t pr[PREFETCH];
-                float rl[PREFETCH];
+        if (REGS > 0) {
 #pragma unroll
-                for (int u = 0; u < PREFETCH; u++) {
-                    const int j = j0 + u * T;
-                    pr[u] = j < je ? D[j] : 0u;
-                    rl[u] = j < je ? DR[j] : 0.0f;
-                }
+            for (int c = 0; c < REG_COLORS; c++) {
+                if (c < C) {
 #pragma unroll
-                for (int u = 0; u < PREFETCH; u++) {
-                    if (j0 + u * T >= je) break;
-                    const int i0 = pr[u] & 0xffffu, i1 = pr[u] >> 16;
-                    float4 p0 = P[i0], p1 = P[i1];
-                    project_distance(p0, p1, rl[u], kd);
-                    P[i0] = p0;
-                    P[i1] = p1;
+                    for (int u = 0; u < RN; u += 2) {
+                        const unsigned bit = 1u << (c * RN + u), both = RN > 1 ? bit * 3 : bit;
+                        const unsigned g = (gen & both) ? REC_GENERAL : 0u;
+                        constexpr int N2 = RN > 1 ? 2 : 1;
+                        if (RN > 1 && (any & (bit << 1)))
+                            project_pairs<N2>(&ra[c][u], &rb[c][u], &rl[c][u], kd, g);
+                        else if (any & bit)
+                            project_pairs<1>(&ra[c][u], &rb[c][u], &rl[c][u], kd, g);
+                    }
+                    __syncthreads();
                 }
             }
-            const int be = !BEND ? bc[c] : bnow ? bc[c] + bnow[c] : bc[c + 1];
-            for (int j0 = bc[c] + tid; BEND && j0 < be; j0 += BEND_PREFETCH * T) {
-                uint2 bw[BEND_PREFETCH];
-                float br[BEND_PREFETCH];
+        }
+        for (int c = 0; REGS == 0 && c < C; c++) {
+            const int4 after = c + 2 < C ? phase_at(sw, c + 2)
+                                         : C > 1 ? phase_at(sw + 1, c + 2 - C) : phase_at(sw + 2, 0);
+            for (int j0 = now.x;; j0 += PREFETCH * T) {
+                const bool last = j0 + PREFETCH * T >= now.y;
+                uint2 dn[PREFETCH];
+                fetch_dist(dn, (last ? next.x : j0 + PREFETCH * T) + tid, last ? next.y : now.y);
 #pragma unroll
-                for (int u = 0; u < BEND_PREFETCH; u++) {
-                    const int j = j0 + u * T;
-                    bw[u] = j < be ? make_uint2(B[2 * j], B[2 * j + 1]) : make_uint2(0u, 0u);
-                    br[u] = j < be ? BR[j] : 0.0f;
+                for (int u = 0; u < PREFETCH; u++)
+                    if (j0 + u * T + tid < now.y) {
+                        const unsigned a0 = rec_a0(dr[u], base), a1 = rec_a1(dr[u], base);
+                        const float rest = __uint_as_float(dr[u].y);
+                        project_pairs<1>(&a0, &a1, &rest, kd, dr[u].x & REC_GENERAL);
+                    }
+#pragma unroll
+                for (int u = 0; u < PREFETCH; u++) dr[u] = dn[u];
+                if (last) break;
+            }
+            if (BEND) {
+                uint4 bn[BEND_PREFETCH];
+                fetch_bend(bn, next.z + tid, next.w);
+                for (int j0 = now.z; j0 < now.w; j0 += BEND_PREFETCH * T) {
+                    if (j0 > now.z) fetch_bend(br, j0 + tid, now.w);
+#pragma unroll
+                    for (int u = 0; u < BEND_PREFETCH; u++) {
+                        if (j0 + u * T + tid >= now.w) break;
+                        const int i0 = br[u].x & 0xffffu, i1 = br[u].x >> 16, i2 = br[u].y & 0xffffu,
+                                  i3 = br[u].y >> 16;
+                        float4 q0 = P[i0], q1 = P[i1], q2 = P[i2], q3 = P[i3];
+                        project_bending(q0, q1, q2, q3, __uint_as_float(br[u].z), kb);
+                        P[i0] = q0;
+                        P[i1] = q1;
+                        P[i2] = q2;
+                        P[i3] = q3;
+                    }
                 }
 #pragma unroll
-                for (int u = 0; u < BEND_PREFETCH; u++) {
-                    if (j0 + u * T >= be) break;
-                    const int i0 = bw[u].x & 0xffffu, i1 = bw[u].x >> 16, i2 = bw[u].y & 0xffffu,
-                              i3 = bw[u].y >> 16;
-                    float4 q0 = P[i0], q1 = P[i1], q2 = P[i2], q3 = P[i3];
-                    project_bending(q0, q1, q2, q3, br[u], kb);
-                    P[i0] = q0;
-                    P[i1] = q1;
-                    P[i2] = q2;
-                    P[i3] = q3;
-                }
+                for (int u = 0; u < BEND_PREFETCH; u++) br[u] = bn[u];
             }
             __syncthreads();
+            now = next;
+            next = after;
         }
         if (coll) {
             for (int i = tid; i < n_load; i += T) {
                 float4 q = P[i];
+                if (!cd.box_on) {
+                    // well outside the sphere (its test is d - r > 0.001): no square root
+                    const float dx = q.x - cd.sphere_c[0], dy = q.y - cd.sphere_c[1], dz = q.z - cd.sphere_c[2];
+                    const float reach = cd.sphere_r + 0.001f;
+                    if (dx * dx + dy * dy + dz * dz > 1.001f * (reach * reach)) continue;
+                }
                 collide_point(q, cd.sphere_on, cd.sphere_c, cd.sphere_r, cd.box_on, cd.box_lo, cd.box_hi);
                 P[i] = q;
             }
@@ -916,7 +1075,7 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
     // tolerance (a fixed budget) nothing reads it, and it is not computed
     if (tol >= 0.0 && (!td.whole || resid < 0.0 || (sw % a.check_every) != 0))
         resid = block_max(own_residual<PREFETCH>(P, own + td.own_off, own_rest + td.own_off, td.n_own), red);
-    if (tid == 0) {
+    if (tid == 0 && ss == nsub - 1) {
         if (tol >= 0.0)
             atomicMax(&res_slots[(size_t)a.chunk * ncl + td.cloth], (unsigned long long)__double_as_longlong(resid));
         atomicMax(&sweeps_out[td.cloth], a.sweep_base + sw);
@@ -941,7 +1100,7 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
                     const float4 Q = P[i0 + u * T];
                     v[g[u]] = make_float4((Q.x - X[u].x) / a.dt, (Q.y - X[u].y) / a.dt, (Q.z - X[u].z) / a.dt, 0.0f);
                     x[g[u]] = make_float4(Q.x, Q.y, Q.z, X[u].w);
-                    p_out[g[u]] = Q;
+                    if (ss == nsub - 1) p_out[g[u]] = Q;
                 }
         } else if (handoff) {
 #pragma unroll
@@ -953,6 +1112,7 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
                 if (g[u] >= 0) p_out[g[u]] = P[i0 + u * T];
         }
     }
+    }  // substeps
     return budget_c;
 }
 
@@ -961,12 +1121,13 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
 // workgroup takes entries blockIdx.x, blockIdx.x + gridDim.x, ... .  With
 // gridDim.x a multiple of 8 every entry a workgroup takes sits at its own
 // position mod 8, the XCD the list's layout meant it for.
-template <bool BEND>
-__device__ __forceinline__ void tiles_walk(TILE_PARAMS, const int* __restrict__ n_items, float4* P, double* red) {
+template <bool BEND, int REGS = 0>
+__device__ __forceinline__ void tiles_walk(TILE_PARAMS, const int* __restrict__ n_items, float4* P) {
+    double* red = (double*)(P + a.lds_slots);
     // one loop for both forms, so the body is inlined once
     const int n = n_items ? *n_items : (int)gridDim.x;
     for (int it = blockIdx.x; it < n; it += gridDim.x) {
-        tiles_body<BEND>(TILE_ARGS, order[it], P, red);
+        tiles_body<BEND, false, REGS>(TILE_ARGS, order[it], P, red);
         __syncthreads();  // the tile's stores have read LDS before the next tile loads
     }
 }
@@ -975,14 +1136,19 @@ __device__ __forceinline__ void tiles_walk(TILE_PARAMS, const int* __restrict__ 
 // two 1024-thread workgroups fit a CU when their tiles fit half its LDS.
 __global__ __launch_bounds__(1024, 8) void k_tiles(TILE_PARAMS, const int* __restrict__ n_items) {
     extern __shared__ float4 P[];
-    __shared__ double red[16];
-    tiles_walk<false>(TILE_ARGS, n_items, P, red);
+    tiles_walk<false>(TILE_ARGS, n_items, P);
 }
 
 __global__ __launch_bounds__(1024) void k_tiles_bend(TILE_PARAMS, const int* __restrict__ n_items) {
     extern __shared__ float4 P[];
-    __shared__ double red[16];
-    tiles_walk<true>(TILE_ARGS, n_items, P, red);
+    tiles_walk<true>(TILE_ARGS, n_items, P);
+}
+
+// The form with the records in registers (one workgroup of 1024 threads per CU).
+template <int REGS>
+__global__ __launch_bounds__(1024) void k_tiles_regs(TILE_PARAMS, const int* __restrict__ n_items) {
+    extern __shared__ float4 P[];
+    tiles_walk<false, REGS>(TILE_ARGS, n_items, P);
 }
 
 // The tiles of a later chunk: the entries of `order` (the multi-tile launch
@@ -1062,13 +1228,14 @@ __global__ __launch_bounds__(512) void k_follow_list(const int* __restrict__ ord
 // instead of hanging.
 
 template <bool BEND>
-__device__ __forceinline__ void tiles_queue(TILE_PARAMS, const TileQueue& q, float4* P, double* red) {
-    __shared__ int s_item;
+__device__ __forceinline__ void tiles_queue(TILE_PARAMS, const TileQueue& q, float4* P) {
+    double* red = (double*)(P + a.lds_slots);
+    int& s_item = *(int*)(P + a.lds_slots + TILE_WORD_SLOT);
     const int n = *q.n_items;
     for (;;) {
         if (threadIdx.x == 0) s_item = atomicAdd(q.head, 1);
         __syncthreads();
-        const int idx = s_item;
+        const int idx = __builtin_amdgcn_readfirstlane(s_item);
         if (idx >= n) break;
         const int slot = q.item_tile[idx], c = q.item_chunk[idx];
         const TileDev& td = tiles[slot];
@@ -1105,7 +1272,7 @@ __device__ __forceinline__ void tiles_queue(TILE_PARAMS, const TileQueue& q, flo
             b.coherent_load = 1;
         }
         const bool odd = ((q.start ^ c) & 1) != 0;
-        tiles_body<BEND>(q.item_tile, tiles, verts, dist, dist_rest, bend, bend_rest, own, own_rest, cols, cloths,
+        tiles_body<BEND>(q.item_tile, tiles, verts, dist, bend, own, own_rest, phases, counts, cloths,
                          ktab_d, ktab_b, x, v, odd ? q.pbuf1 : q.pbuf0, odd ? q.pbuf0 : q.pbuf1, res_slots, ncl,
                          sweeps_out, sweep_cap, b, slot, P, red);
         const bool more = !td.whole && sweep_cap && sweep_cap[td.cloth] > (c + 1) * q.ts;
@@ -1118,14 +1285,12 @@ __device__ __forceinline__ void tiles_queue(TILE_PARAMS, const TileQueue& q, flo
 
 __global__ __launch_bounds__(1024, 8) void k_tiles_queue(TILE_PARAMS, TileQueue q) {
     extern __shared__ float4 P[];
-    __shared__ double red[16];
-    tiles_queue<false>(TILE_ARGS, q, P, red);
+    tiles_queue<false>(TILE_ARGS, q, P);
 }
 
 __global__ __launch_bounds__(1024) void k_tiles_queue_bend(TILE_PARAMS, TileQueue q) {
     extern __shared__ float4 P[];
-    __shared__ double red[16];
-    tiles_queue<true>(TILE_ARGS, q, P, red);
+    tiles_queue<true>(TILE_ARGS, q, P);
 }
 
 // The queued launch that decides (see cloth_decide): a workgroup takes an
@@ -1137,7 +1302,8 @@ __global__ __launch_bounds__(1024) void k_tiles_queue_bend(TILE_PARAMS, TileQueu
 // tiles leave a workgroup free for its remaining ones, and a later chunk
 // waits only for items taken before it.
 template <bool BEND>
-__device__ __forceinline__ void tiles_decide_walk(TILE_PARAMS, const TileQueue& q, float4* P, double* red) {
+__device__ __forceinline__ void tiles_decide_walk(TILE_PARAMS, const TileQueue& q, float4* P) {
+    double* red = (double*)(P + a.lds_slots);
     __shared__ int s_slot, s_chunk;
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(q.launches, 1);
     for (;;) {
@@ -1216,7 +1382,7 @@ __device__ __forceinline__ void tiles_decide_walk(TILE_PARAMS, const TileQueue& 
             }
         }
         __syncthreads();
-        const int slot = s_slot, c = s_chunk;
+        const int slot = __builtin_amdgcn_readfirstlane(s_slot), c = __builtin_amdgcn_readfirstlane(s_chunk);
         if (slot < 0) break;
         if (c > 0) {
             // the neighbour tiles' previous chunk, polled by one thread in turn
@@ -1248,8 +1414,8 @@ __device__ __forceinline__ void tiles_decide_walk(TILE_PARAMS, const TileQueue& 
             b.coherent_load = 1;
         }
         const bool odd = ((q.start ^ c) & 1) != 0;
-        const int budget = tiles_body<BEND, true>(order, tiles, verts, dist, dist_rest, bend, bend_rest, own,
-                                                  own_rest, cols, cloths, ktab_d, ktab_b, x, v,
+        const int budget = tiles_body<BEND, true>(order, tiles, verts, dist, bend, own, own_rest, phases,
+                                                  counts, cloths, ktab_d, ktab_b, x, v,
                                                   odd ? q.pbuf1 : q.pbuf0, odd ? q.pbuf0 : q.pbuf1, res_slots, ncl,
                                                   sweeps_out, nullptr, b, slot, P, red, &q);
         const bool more = !tiles[slot].whole && budget > (c + 1) * q.ts;
@@ -1262,14 +1428,12 @@ __device__ __forceinline__ void tiles_decide_walk(TILE_PARAMS, const TileQueue& 
 
 __global__ __launch_bounds__(1024, 8) void k_tiles_decide(TILE_PARAMS, TileQueue q) {
     extern __shared__ float4 P[];
-    __shared__ double red[16];
-    tiles_decide_walk<false>(TILE_ARGS, q, P, red);
+    tiles_decide_walk<false>(TILE_ARGS, q, P);
 }
 
 __global__ __launch_bounds__(1024) void k_tiles_decide_bend(TILE_PARAMS, TileQueue q) {
     extern __shared__ float4 P[];
-    __shared__ double red[16];
-    tiles_decide_walk<true>(TILE_ARGS, q, P, red);
+    tiles_decide_walk<true>(TILE_ARGS, q, P);
 }
 
 // Block-wide exclusive prefix of a 0/1 flag over up to 1024 threads (16
@@ -1383,7 +1547,8 @@ size_t tiles_lds_optin(size_t bytes) {
     if (bytes <= 65536) return bytes;
     for (const void* k : {(const void*)k_tiles, (const void*)k_tiles_bend, (const void*)k_tiles_queue,
                           (const void*)k_tiles_queue_bend, (const void*)k_tiles_decide,
-                          (const void*)k_tiles_decide_bend}) {
+                          (const void*)k_tiles_decide_bend, (const void*)k_tiles_regs<1>,
+                          (const void*)k_tiles_regs<2>}) {
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         if (e != hipSuccess) {
             (void)hipGetLastError();  // the refusal is handled by the smaller limit
@@ -1394,45 +1559,52 @@ size_t tiles_lds_optin(size_t bytes) {
 }
 
 void launch_tiles(hipStream_t s, int nblocks, const int* order, const TileDev* tiles, const int* verts,
-                  const uint32_t* dist, const float* dist_rest, const uint32_t* bend, const float* bend_rest,
-                  const uint32_t* own, const float* own_rest, const int* cols, const ClothDev* cloths,
+                  const uint2* dist, const uint4* bend, const uint32_t* own, const float* own_rest,
+                  const int4* phases, const int* counts, const ClothDev* cloths,
                   const float* ktab_d, const float* ktab_b, float4* x, float4* v, const float4* p_in,
                   float4* p_out, unsigned long long* res_slots, int ncl, int* sweeps_out, const int* sweep_cap,
-                  const SolveArgs& a, int threads, size_t lds_bytes, bool with_bend, const int* n_items) {
+                  const SolveArgs& args, int threads, size_t lds_bytes, bool with_bend, int regs, const int* n_items) {
     if (nblocks <= 0) return;
-    hipLaunchKernelGGL(with_bend ? k_tiles_bend : k_tiles, dim3(nblocks), dim3(threads), lds_bytes, s, order, tiles,
-                       verts, dist, dist_rest, bend, bend_rest, own, own_rest, cols, cloths, ktab_d, ktab_b, x, v,
+    SolveArgs a = args;
+    a.lds_slots = (int)(lds_bytes / sizeof(float4));
+    auto* kernel = with_bend ? k_tiles_bend : regs == 1 ? k_tiles_regs<1> : regs == 2 ? k_tiles_regs<2> : k_tiles;
+    hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(threads), lds_bytes + TILE_TAIL_LDS, s, order, tiles,
+                       verts, dist, bend, own, own_rest, phases, counts, cloths, ktab_d, ktab_b, x, v,
                        p_in, p_out, res_slots, ncl, sweeps_out, sweep_cap, a, n_items);
     PBD_HIP(hipGetLastError());
 }
 
-void launch_tiles_queue(hipStream_t s, int nblocks, const TileDev* tiles, const int* verts, const uint32_t* dist,
-                        const float* dist_rest, const uint32_t* bend, const float* bend_rest, const uint32_t* own,
-                        const float* own_rest, const int* cols, const ClothDev* cloths, const float* ktab_d,
+void launch_tiles_queue(hipStream_t s, int nblocks, const TileDev* tiles, const int* verts, const uint2* dist,
+                        const uint4* bend, const uint32_t* own, const float* own_rest, const int4* phases,
+                        const int* counts, const ClothDev* cloths, const float* ktab_d,
                         const float* ktab_b, float4* x, float4* v, unsigned long long* res_slots, int ncl,
-                        int* sweeps_out, const int* sweep_cap, const SolveArgs& a, const TileQueue& q, int threads,
+                        int* sweeps_out, const int* sweep_cap, const SolveArgs& args, const TileQueue& q, int threads,
                         size_t lds_bytes, bool with_bend) {
     if (nblocks <= 0) return;
+    SolveArgs a = args;
+    a.lds_slots = (int)(lds_bytes / sizeof(float4));
     // order, p_in and p_out of the common parameter list are unused: the
     // queue carries the items and the two buffers
-    hipLaunchKernelGGL(with_bend ? k_tiles_queue_bend : k_tiles_queue, dim3(nblocks), dim3(threads), lds_bytes, s,
-                       q.item_tile, tiles, verts, dist, dist_rest, bend, bend_rest, own, own_rest, cols, cloths,
+    hipLaunchKernelGGL(with_bend ? k_tiles_queue_bend : k_tiles_queue, dim3(nblocks), dim3(threads), lds_bytes + TILE_TAIL_LDS, s,
+                       q.item_tile, tiles, verts, dist, bend, own, own_rest, phases, counts, cloths,
                        ktab_d, ktab_b, x, v, (const float4*)q.pbuf0, q.pbuf1, res_slots, ncl, sweeps_out, sweep_cap,
                        a, q);
     PBD_HIP(hipGetLastError());
 }
 
-void launch_tiles_decide(hipStream_t s, int nblocks, const TileDev* tiles, const int* verts, const uint32_t* dist,
-                         const float* dist_rest, const uint32_t* bend, const float* bend_rest, const uint32_t* own,
-                         const float* own_rest, const int* cols, const ClothDev* cloths, const float* ktab_d,
+void launch_tiles_decide(hipStream_t s, int nblocks, const TileDev* tiles, const int* verts, const uint2* dist,
+                         const uint4* bend, const uint32_t* own, const float* own_rest, const int4* phases,
+                         const int* counts, const ClothDev* cloths, const float* ktab_d,
                          const float* ktab_b, float4* x, float4* v, unsigned long long* res_slots, int ncl,
-                         int* sweeps_out, const int* sweep_cap, const SolveArgs& a, const TileQueue& q, int threads,
-                         size_t lds_bytes, bool with_bend) {
+                        int* sweeps_out, const int* sweep_cap, const SolveArgs& args, const TileQueue& q, int threads,
+                        size_t lds_bytes, bool with_bend) {
     if (nblocks <= 0) return;
+    SolveArgs a = args;
+    a.lds_slots = (int)(lds_bytes / sizeof(float4));
     // order, p_in and p_out of the common parameter list are unused: the
     // queue carries the items and the two buffers
-    hipLaunchKernelGGL(with_bend ? k_tiles_decide_bend : k_tiles_decide, dim3(nblocks), dim3(threads), lds_bytes, s,
-                       q.stat_item, tiles, verts, dist, dist_rest, bend, bend_rest, own, own_rest, cols, cloths,
+    hipLaunchKernelGGL(with_bend ? k_tiles_decide_bend : k_tiles_decide, dim3(nblocks), dim3(threads), lds_bytes + TILE_TAIL_LDS, s,
+                       q.stat_item, tiles, verts, dist, bend, own, own_rest, phases, counts, cloths,
                        ktab_d, ktab_b, x, v, (const float4*)q.pbuf0, q.pbuf1, res_slots, ncl, sweeps_out, sweep_cap,
                        a, q);
     PBD_HIP(hipGetLastError());
@@ -1469,7 +1641,7 @@ void launch_follow_list(hipStream_t s, const int* order, const int* order_cloth,
 int tiles_per_cu(bool with_bend, int threads, size_t lds_bytes) {
     int n = 0;
     PBD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, with_bend ? k_tiles_bend : k_tiles, threads,
-                                                         lds_bytes));
+                                                         lds_bytes + TILE_TAIL_LDS));
     return std::max(1, n);
 }
 
