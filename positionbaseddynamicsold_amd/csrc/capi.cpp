@@ -84,9 +84,11 @@ struct pbd_ctx {
     int nslots = 0;
     // standalone broadphase / CCD (parity-test entry points)
     Broadphase sbp;
-    DBuf<float4> sx, sp4;
+    DBuf<float4> sx, sp4, sres;
     DBuf<int> stris;
     int snv = 0, snt = 0;
+    float s_th = 0.0f;       // thickness of the standalone scene
+    bool sh_stale = false;   // the sorted table of the standalone scene is yet to be built
     uint64_t scene_hash = 0;  // of the standalone scene and its detection settings (scene_fingerprint)
     bool sh_built = false, ccd_built = false;
     // in-solver collision
@@ -95,6 +97,7 @@ struct pbd_ctx {
     Broadphase cbp;
     DBuf<int> gtris;
     int gnt = 0;
+    float mean_edge = 0.0f;  // of gtris, at rest
     // learned warm start
     struct WarmStart {
         bool params_ready = false, enabled = false, nbr_built = false;
@@ -748,26 +751,56 @@ void upload_scene(pbd_ctx* c, const float* x, const float* p, const float* w, in
     c->sx.upload(X, c->stream);
     c->sp4.upload(P, c->stream);
     c->stris.upload(std::vector<int>(tris, tris + 3ll * nt), c->stream);
+    c->sbp.set_triangles(c->stream, c->stris.ptr, nt, nv);
     c->snv = nv;
     c->snt = nt;
+    c->s_th = th;
     c->scene_hash = scene_fingerprint(x, p, nv, tris, nt, th, d ? *d : pbd_hash_desc{});
+}
+
+// The grid of the swept-box table: the caller's cells taken m at a time per
+// axis so that they are about as large as a face's widened box.  Faces are then
+// entered in a few cells each and vertices look in one or two, whatever the
+// caller's cell (the candidates do not depend on it).
+HashCfg swept_cfg(const HashCfg& g, float mean_edge, float th) {
+    HashCfg w = g;
+    const float target = mean_edge + 8.0f * th;
+    for (int k = 0; k < 3; k++) {
+        const float r = std::ceil(target / g.cell[k]);
+        const int m = r >= 1.0f ? (int)std::min(r, 1048576.0f) : 1;
+        w.cell[k] = g.cell[k] * (float)m;
+        if (g.mode == 0) w.size[k] = (g.size[k] + m - 1) / m + 1;
+    }
+    return w;
+}
+
+// Mean edge length of (a sample of) a triangle list over 3-float positions.
+float mean_edge_length(const float* x, const int* tris, int nt) {
+    double sum = 0.0;
+    long long n = 0;
+    const int step = std::max(1, nt / 1024);
+    for (int t = 0; t < nt; t += step)
+        for (int k = 0; k < 3; k++) {
+            const float* a = x + 3 * (size_t)tris[3 * (size_t)t + k];
+            const float* b = x + 3 * (size_t)tris[3 * (size_t)t + (k + 1) % 3];
+            const double dx = a[0] - b[0], dy = a[1] - b[1], dz = a[2] - b[2], d = std::sqrt(dx * dx + dy * dy + dz * dz);
+            if (std::isfinite(d)) {
+                sum += d;
+                n++;
+            }
+        }
+    return n ? (float)(sum / n) : 0.0f;
 }
 
 // Contact detection for the whole context (all cloths, global vertex ids).
 void detect_contacts(pbd_ctx* c, const float4* p) {
     hipStream_t s = c->stream;
-    if (c->coll.broadphase == 1) {
-        c->cbp.pairs_swept(s, c->ccfg, c->x.ptr, p, c->gtris.ptr, c->gnt, c->nv_total, c->coll.thickness);
-    } else {
-        c->cbp.build(s, c->ccfg, p, c->gtris.ptr, c->gnt);
-        c->cbp.pairs(s, p, c->gtris.ptr, c->nv_total);
-    }
-    c->cbp.narrow(s, c->x.ptr, p, c->gtris.ptr, c->coll.thickness);
+    HashCfg swept = c->ccfg;
+    if (c->coll.broadphase == 1) swept = swept_cfg(c->ccfg, c->mean_edge, c->coll.thickness);
+    c->cbp.detect(s, c->ccfg, c->coll.broadphase == 1 ? &swept : nullptr, c->x.ptr, p, c->gtris.ptr, c->gnt,
+                  c->nv_total, c->coll.thickness, false);
     if (c->coll.edge_edge) {
-        // edge-edge candidates come from the centroid-cell table
-        if (c->coll.broadphase == 1) c->cbp.build(s, c->ccfg, p, c->gtris.ptr, c->gnt);
-        c->cbp.ee_pairs(s, p, c->gtris.ptr);
-        c->cbp.ee_narrow(s, c->x.ptr, p, c->coll.thickness);
+        c->cbp.detect_ee(s, c->ccfg, c->x.ptr, p, c->gtris.ptr, c->gnt, c->coll.thickness, false);
     } else {
         c->cbp.ee_npairs = 0;
         c->cbp.ee_ncontacts = 0;
@@ -1419,7 +1452,7 @@ void ccd_sweeps(pbd_ctx* c, int n, float dt, const int* cap) {
             if (c->prof_on) PBD_HIP(hipEventRecord(next_event(c), s));
         }
         c->pcur = cur ^ 1;
-        c->cbp.resolve(s, c->x.ptr, c->pbuf[c->pcur].ptr, c->gtris.ptr, c->nv_total, c->coll.thickness,
+        c->cbp.resolve(s, c->x.ptr, c->pbuf[c->pcur].ptr, c->nv_total, c->coll.thickness,
                        c->coll.resolve_passes, c->coll.min_normal2 > 0.0f ? c->coll.min_normal2 : 1e-6f);
         if (coll) launch_colliders(s, c->cl.ptr, c->vcloth.ptr, c->pbuf[c->pcur].ptr, 0, c->nv_total, cap, ii);
     }
@@ -2092,6 +2125,7 @@ int pbd_sh_build(pbd_ctx* ctx, const pbd_hash_desc* d, const float* pos, int nv,
         upload_scene(ctx, pos, pos, nullptr, nv, tris, nt);
         ctx->sbp.build(ctx->stream, g, ctx->sp4.ptr, ctx->stris.ptr, nt);
         PBD_HIP(hipStreamSynchronize(ctx->stream));
+        ctx->sh_stale = false;
         ctx->sh_built = true;
         ctx->ccd_built = false;
     });
@@ -2140,6 +2174,8 @@ int pbd_sh_get(pbd_ctx* ctx, int* keys, int* ids, int* raw, int* cstart, int* ce
         set_device(ctx);
         hipStream_t s = ctx->stream;
         Broadphase& b = ctx->sbp;
+        if (ctx->sh_stale) b.build(s, b.cfg, ctx->sp4.ptr, ctx->stris.ptr, ctx->snt);
+        ctx->sh_stale = false;
         int nt = b.nt;
         if (nt > 0) {
             std::vector<uint32_t> k1;
@@ -2163,7 +2199,7 @@ int pbd_sh_pairs(pbd_ctx* ctx, long long cap, int64_t* out, long long* count) {
         PBD_CHECK(ctx->sh_built, PBD_ERR_STATE, "call pbd_sh_build first");
         set_device(ctx);
         hipStream_t s = ctx->stream;
-        long long n = ctx->sbp.pairs(s, ctx->sp4.ptr, ctx->stris.ptr, ctx->snv);
+        long long n = ctx->sbp.list_pairs(s, ctx->sbp.cfg, ctx->sp4.ptr, ctx->stris.ptr, ctx->snt, ctx->snv);
         *count = n;
         if (out && n > 0) {
             long long m = std::min(n, cap);
@@ -2185,12 +2221,12 @@ int pbd_ccd_detect(pbd_ctx* ctx, const pbd_hash_desc* d, const float* x, const f
         hipStream_t s = ctx->stream;
         HashCfg g = make_hash_cfg(*d);
         upload_scene(ctx, x, p, nullptr, nv, tris, nt, th, d);
-        ctx->sbp.build(s, g, ctx->sp4.ptr, ctx->stris.ptr, nt);
-        ctx->sbp.pairs(s, ctx->sp4.ptr, ctx->stris.ptr, nv);
-        *nc = ctx->sbp.narrow(s, ctx->sx.ptr, ctx->sp4.ptr, ctx->stris.ptr, th);
+        ctx->sbp.detect(s, g, nullptr, ctx->sx.ptr, ctx->sp4.ptr, ctx->stris.ptr, nt, nv, th, true);
+        *nc = ctx->sbp.ncontacts;
         ctx->sbp.ee_npairs = 0;
         ctx->sbp.ee_ncontacts = 0;
         ctx->sh_built = true;
+        ctx->sh_stale = true;
         ctx->ccd_built = true;
     });
 }
@@ -2208,7 +2244,10 @@ int pbd_ccd_detect_ee(pbd_ctx* ctx, const pbd_hash_desc* d, const float* x, cons
         // at another thickness or grid, do not carry over
         upload_scene(ctx, x, p, nullptr, nv, tris, nt, th, d);
         bool same = ctx->ccd_built && ctx->scene_hash == prev_hash;
-        if (!same) {
+        if (same) {
+            // their list shares a buffer with the edge pairs
+            ctx->sbp.list_detected(s, ctx->sp4.ptr, ctx->stris.ptr, nv);
+        } else {
             ctx->sbp.npairs = 0;
             ctx->sbp.ncontacts = 0;
         }
@@ -2216,10 +2255,12 @@ int pbd_ccd_detect_ee(pbd_ctx* ctx, const pbd_hash_desc* d, const float* x, cons
         std::vector<int2> ed;
         build_edge_table(tris, nt, te, ed);
         ctx->sbp.set_edges(s, te, ed);
-        ctx->sbp.build(s, g, ctx->sp4.ptr, ctx->stris.ptr, nt);
-        long long np = ctx->sbp.ee_pairs(s, ctx->sp4.ptr, ctx->stris.ptr);
-        if (npairs) *npairs = np;
-        *nc = ctx->sbp.ee_narrow(s, ctx->sx.ptr, ctx->sp4.ptr, th);
+        ctx->sbp.cfg = g;
+        ctx->sbp.nt = nt;
+        ctx->sbp.detect_ee(s, g, ctx->sx.ptr, ctx->sp4.ptr, ctx->stris.ptr, nt, th, true);
+        if (npairs) *npairs = ctx->sbp.ee_npairs;
+        *nc = ctx->sbp.ee_ncontacts;
+        ctx->sh_stale = true;
         ctx->sh_built = true;
         ctx->ccd_built = true;
     });
@@ -2235,6 +2276,7 @@ int pbd_ccd_get_ee_pairs(pbd_ctx* ctx, long long cap, int* quads, long long* cou
         *count = b.ee_npairs;
         long long m = std::min(cap, b.ee_npairs);
         if (m <= 0 || !quads) return;
+        b.list_detected_ee(s, b.cfg, ctx->sx.ptr, ctx->sp4.ptr, ctx->stris.ptr, ctx->s_th);
         std::vector<uint32_t> ea(m), eb(m);
         std::vector<int2> ed;
         PBD_HIP(hipMemcpyAsync(ea.data(), b.eua.ptr, 4 * m, hipMemcpyDeviceToHost, s));
@@ -2279,9 +2321,10 @@ int pbd_ccd_detect_swept(pbd_ctx* ctx, const pbd_hash_desc* d, const float* x, c
         hipStream_t s = ctx->stream;
         HashCfg g = make_hash_cfg(*d);
         upload_scene(ctx, x, p, nullptr, nv, tris, nt, th, d);
-        long long np = ctx->sbp.pairs_swept(s, g, ctx->sx.ptr, ctx->sp4.ptr, ctx->stris.ptr, nt, nv, th);
-        if (npairs) *npairs = np;
-        *nc = ctx->sbp.narrow(s, ctx->sx.ptr, ctx->sp4.ptr, ctx->stris.ptr, th);
+        const HashCfg swept = swept_cfg(g, mean_edge_length(x, tris, nt), th);
+        ctx->sbp.detect(s, g, &swept, ctx->sx.ptr, ctx->sp4.ptr, ctx->stris.ptr, nt, nv, th, true);
+        if (npairs) *npairs = ctx->sbp.npairs;
+        *nc = ctx->sbp.ncontacts;
         ctx->sbp.ee_npairs = 0;
         ctx->sbp.ee_ncontacts = 0;
         ctx->sh_built = false;  // the cell table holds swept entries, not centroid keys
@@ -2298,6 +2341,7 @@ int pbd_ccd_get_pairs(pbd_ctx* ctx, long long cap, int64_t* out, long long* coun
         const long long n = ctx->sbp.npairs;
         *count = n;
         if (out && n > 0) {
+            ctx->sbp.list_detected(s, ctx->sp4.ptr, ctx->stris.ptr, ctx->snv);
             long long m = std::min(n, cap);
             std::vector<uint32_t> v(m), f(m);
             PBD_HIP(hipMemcpyAsync(v.data(), ctx->sbp.uv.ptr, 4 * m, hipMemcpyDeviceToHost, s));
@@ -2317,16 +2361,7 @@ int pbd_ccd_get_contacts(pbd_ctx* ctx, long long cap, int* vf, float* t, float* 
         Broadphase& b = ctx->sbp;
         long long m = std::min(cap, b.ncontacts);
         if (m <= 0) return;
-        if (vf) {
-            std::vector<int> v(m), f(m);
-            PBD_HIP(hipMemcpyAsync(v.data(), b.cv.ptr, 4 * m, hipMemcpyDeviceToHost, s));
-            PBD_HIP(hipMemcpyAsync(f.data(), b.cf.ptr, 4 * m, hipMemcpyDeviceToHost, s));
-            PBD_HIP(hipStreamSynchronize(s));
-            for (long long i = 0; i < m; i++) {
-                vf[2 * i] = v[i];
-                vf[2 * i + 1] = f[i];
-            }
-        }
+        if (vf) PBD_HIP(hipMemcpyAsync(vf, b.ckey.ptr, 8 * m, hipMemcpyDeviceToHost, s));
         if (t) PBD_HIP(hipMemcpyAsync(t, b.ct.ptr, 4 * m, hipMemcpyDeviceToHost, s));
         if (n) PBD_HIP(hipMemcpyAsync(n, b.cn.ptr, 12 * m, hipMemcpyDeviceToHost, s));
         if (w) PBD_HIP(hipMemcpyAsync(w, b.cw.ptr, 32 * m, hipMemcpyDeviceToHost, s));
@@ -2350,10 +2385,10 @@ int pbd_ccd_resolve(pbd_ctx* ctx, float* p, const float* w, float th, int passes
             P[i] = make_float4(p[3 * i], p[3 * i + 1], p[3 * i + 2], wi);
             X[i].w = wi;
         }
-        ctx->sp4.upload(P, s);
+        ctx->sres.upload(P, s);
         ctx->sx.upload(X, s);
-        ctx->sbp.resolve(s, ctx->sx.ptr, ctx->sp4.ptr, ctx->stris.ptr, nv, th, passes, 1e-6f);
-        ctx->sp4.download(P, s);
+        ctx->sbp.resolve(s, ctx->sx.ptr, ctx->sres.ptr, nv, th, passes, 1e-6f);
+        ctx->sres.download(P, s);
         PBD_HIP(hipStreamSynchronize(s));
         for (int i = 0; i < nv; i++) {
             p[3 * i] = P[i].x;
@@ -2396,6 +2431,10 @@ int pbd_set_collision(pbd_ctx* ctx, const pbd_collision_params* cp) {
             for (int i : k.tris) gt.push_back(i + k.vbase);
         ctx->gtris.upload(gt, ctx->stream);
         ctx->gnt = (int)gt.size() / 3;
+        ctx->cbp.set_triangles(ctx->stream, ctx->gtris.ptr, ctx->gnt, ctx->nv_total);
+        double edge_sum = 0.0;
+        for (auto& k : ctx->cloths) edge_sum += (double)k.nt * mean_edge_length(k.pos0.data(), k.tris.data(), k.nt);
+        ctx->mean_edge = ctx->gnt ? (float)(edge_sum / ctx->gnt) : 0.0f;
         if (cp->edge_edge) {
             std::vector<int> te;
             std::vector<int2> ed;

@@ -1,12 +1,16 @@
 // Spatial-hash broadphase and vertex-face CCD for gfx950.
 //
-// Broadphase (SpatialHashSystem, SpatialHashSystem.cpp:88-187, 276-413):
+// Broadphase build (SpatialHashSystem, SpatialHashSystem.cpp:88-121, 276-413):
 //   triangle centroid -> cell coordinates -> key (dense grid index or -1
 //   outside, or a hashed table slot) -> stable radix sort of (key, id) ->
-//   cell ranges [start, end] -> candidate (vertex, face) pairs from the 27
-//   cells around each triangle's cell, de-duplicated by a 64-bit radix sort.
-// Narrowphase: ExtendedVFTest (CCD.cpp:1733-1808) per candidate, FP64 only in
-//   the coplanarity cubic / time-of-impact solve (CCD.cpp:48-113).
+//   cell ranges [start, end].
+// Candidates: an unsorted table of the faces by cell, built with one atomic
+//   per entry; each vertex (edge) visits the cells around it once, so that
+//   every distinct pair comes up exactly once and no list of pairs is sorted
+//   or stored to be de-duplicated.
+// Narrowphase: ExtendedVFTest (CCD.cpp:1733-1808) per candidate whose swept
+//   boxes meet, FP64 only in the coplanarity cubic / time-of-impact solve
+//   (CCD.cpp:48-113).
 // Response: VFResolveTest/VFResolveNew (CCD.cpp:1996-2090) evaluated for all
 //   contacts against the same positions, fixes summed per vertex in 2^-32 m
 //   fixed point (integer sums are order independent, so the result does not
@@ -125,7 +129,7 @@ __device__ __forceinline__ void tri_cell(const HashCfg& g, const P* __restrict__
 __global__ __launch_bounds__(256) void k_tri_keys(HashCfg g, const float4* __restrict__ p,
                                                   const int* __restrict__ tris, int nt,
                                                   uint32_t* __restrict__ keys1, uint32_t* __restrict__ ids,
-                                                  int* __restrict__ raw, int4* __restrict__ tcell) {
+                                                  int* __restrict__ raw) {
     int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nt) return;
     int gp[3];
@@ -134,7 +138,6 @@ __global__ __launch_bounds__(256) void k_tri_keys(HashCfg g, const float4* __res
     keys1[t] = (uint32_t)(k + 1);  // -1 sorts first, as the reference's signed sort
     ids[t] = (uint32_t)t;
     raw[t] = k;
-    tcell[t] = make_int4(gp[0], gp[1], gp[2], 0);
 }
 
 __global__ __launch_bounds__(256) void k_fill_i32(int* __restrict__ a, int n, int v) {
@@ -154,191 +157,35 @@ __global__ __launch_bounds__(256) void k_cell_ranges(const uint32_t* __restrict_
     if (i == n - 1 || keys1[i + 1] != keys1[i]) cend[k] = i;
 }
 
-// Candidate (v, f): v a vertex of triangle t whose cell is valid, f != t in
-// the 27 cells around t's cell (FindNeighbors, SpatialHashSystem.cpp:134-187),
-// v not a vertex of f.  A face is taken only from the slot of its own cell,
-// so hashed tables give the same set at every size (other cells that share
-// the slot are skipped); dense keys are one slot per cell already.
-// mode 0 counts, mode 1 writes at off[t].
-template <int EMIT>
-__global__ __launch_bounds__(256) void k_pairs(HashCfg g, const float4* __restrict__ p,
-                                               const int* __restrict__ tris, int nt,
-                                               const int* __restrict__ raw, const uint32_t* __restrict__ sids,
-                                               const int* __restrict__ cstart, const int* __restrict__ cend,
-                                               const int4* __restrict__ tcell, int* __restrict__ cnt_or_off,
-                                               uint32_t* __restrict__ ov, uint32_t* __restrict__ of) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nt) return;
-    int n = 0, off = EMIT ? cnt_or_off[t] : 0;
-    if (raw[t] >= 0) {
-        int gp[3];
-        tri_cell(g, p, tris, t, gp);
-        int tv[3] = {tris[3 * t], tris[3 * t + 1], tris[3 * t + 2]};
-        for (int z = -1; z <= 1; z++)
-            for (int y = -1; y <= 1; y++)
-                for (int x = -1; x <= 1; x++) {
-                    const int qx = gp[0] + x, qy = gp[1] + y, qz = gp[2] + z;
-                    int h = cell_key(g, qx, qy, qz);
-                    if (h < 0) continue;
-                    int s = cstart[h];
-                    if (s < 0) continue;
-                    int e = cend[h];
-                    for (int i = s; i <= e; i++) {
-                        int f = (int)sids[i];
-                        if (f == t) continue;
-                        int4 fc = tcell[f];
-                        if (fc.x != qx || fc.y != qy || fc.z != qz) continue;
-                        int f0 = tris[3 * f], f1 = tris[3 * f + 1], f2 = tris[3 * f + 2];
-                        for (int k = 0; k < 3; k++) {
-                            int v = tv[k];
-                            if (v == f0 || v == f1 || v == f2) continue;
-                            if (EMIT) {
-                                ov[off + n] = (uint32_t)v;
-                                of[off + n] = (uint32_t)f;
-                            }
-                            n++;
-                        }
-                    }
-                }
-    }
-    if (!EMIT) cnt_or_off[t] = n;
-}
-
-constexpr int EE_RING = 40;  // LDS slots per thread for a triangle's vertices and their neighbours
-
-// True when a vertex of edge a is a mesh neighbour of a vertex of edge b
-// (vertex -> neighbour CSR voff / vnbr).
-__device__ __forceinline__ bool ring_neighbours(int2 a, int2 b, const int* __restrict__ voff,
-                                                const int* __restrict__ vnbr) {
-    const int ends[2] = {a.x, a.y};
-    for (int k = 0; k < 2; k++)
-        for (int j = voff[ends[k]]; j < voff[ends[k] + 1]; j++) {
-            int u = vnbr[j];
-            if (u == b.x || u == b.y) return true;
-        }
-    return false;
-}
-
-// Edge-edge candidates (new: the reference declares Contact::EE, CCD_Basic.h:14,
-// and leaves it unimplemented, CCD.cpp:925-928).  From the triangle pairs
-// k_pairs visits (centroid cells within one cell, the neighbour's own cell
-// checked), taken once (t < f): every edge of t against every edge of f that
-// shares no vertex with it and has no vertex that is a mesh neighbour of one
-// of its vertices (pairs that close in the mesh are material neighbours, not
-// contacts), as (lower edge id, higher edge id).
-template <int EMIT>
-__global__ __launch_bounds__(256) void k_ee_pairs(HashCfg g, const float4* __restrict__ p,
-                                                  const int* __restrict__ tris, int nt, const int* __restrict__ raw,
-                                                  const uint32_t* __restrict__ sids, const int* __restrict__ cstart,
-                                                  const int* __restrict__ cend, const int4* __restrict__ tcell,
-                                                  const int* __restrict__ tedge, const int2* __restrict__ edges,
-                                                  const int* __restrict__ voff, const int* __restrict__ vnbr,
-                                                  int* __restrict__ cnt_or_off, uint32_t* __restrict__ oa,
-                                                  uint32_t* __restrict__ ob) {
-    // t's vertices and their mesh neighbours, per thread in LDS: a triangle f
-    // with no vertex in this set shares no vertex with, and is outside the
-    // 2-ring of, every edge of t, so its edge pairs skip the exact tests
-    __shared__ int ring[256][EE_RING + 1];
-    int* rt = ring[threadIdx.x];
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nt) return;
-    int n = 0, off = EMIT ? cnt_or_off[t] : 0;
-    if (raw[t] >= 0) {
-        int gp[3];
-        tri_cell(g, p, tris, t, gp);
-        int te[3] = {tedge[3 * t], tedge[3 * t + 1], tedge[3 * t + 2]};
-        int2 tv[3] = {edges[te[0]], edges[te[1]], edges[te[2]]};
-        int nr = 0;
-        bool exact_all = false;
-        for (int k = 0; k < 3 && !exact_all; k++) {
-            const int v = tris[3 * t + k];
-            const int b0 = voff[v], b1 = voff[v + 1];
-            if (nr + 1 + (b1 - b0) > EE_RING) {
-                exact_all = true;
-                break;
-            }
-            rt[nr++] = v;
-            for (int j = b0; j < b1; j++) rt[nr++] = vnbr[j];
-        }
-        for (int z = -1; z <= 1; z++)
-            for (int y = -1; y <= 1; y++)
-                for (int x = -1; x <= 1; x++) {
-                    const int qx = gp[0] + x, qy = gp[1] + y, qz = gp[2] + z;
-                    int h = cell_key(g, qx, qy, qz);
-                    if (h < 0) continue;
-                    int s = cstart[h];
-                    if (s < 0) continue;
-                    int e = cend[h];
-                    for (int i = s; i <= e; i++) {
-                        int f = (int)sids[i];
-                        if (f <= t) continue;
-                        int4 fc = tcell[f];
-                        if (fc.x != qx || fc.y != qy || fc.z != qz) continue;
-                        bool exact = exact_all;
-                        if (!exact) {
-                            const int f0 = tris[3 * f], f1 = tris[3 * f + 1], f2 = tris[3 * f + 2];
-                            for (int k = 0; k < nr; k++) {
-                                const int u = rt[k];
-                                if (u == f0 || u == f1 || u == f2) {
-                                    exact = true;
-                                    break;
-                                }
-                            }
-                        }
-                        for (int kb = 0; kb < 3; kb++) {
-                            int eb = tedge[3 * f + kb];
-                            int2 bv = edges[eb];
-                            for (int ka = 0; ka < 3; ka++) {
-                                int2 av = tv[ka];
-                                if (exact) {
-                                    if (av.x == bv.x || av.x == bv.y || av.y == bv.x || av.y == bv.y) continue;
-                                    if (ring_neighbours(av, bv, voff, vnbr)) continue;
-                                }
-                                if (EMIT) {
-                                    int ea = te[ka];
-                                    oa[off + n] = (uint32_t)(ea < eb ? ea : eb);
-                                    ob[off + n] = (uint32_t)(ea < eb ? eb : ea);
-                                }
-                                n++;
-                            }
-                        }
-                    }
-                }
-    }
-    if (!EMIT) cnt_or_off[t] = n;
-}
-
-__global__ __launch_bounds__(256) void k_unique_flags(const uint32_t* __restrict__ hi, const uint32_t* __restrict__ lo,
-                                                      int n, int* __restrict__ flag) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    flag[i] = (i == 0 || hi[i] != hi[i - 1] || lo[i] != lo[i - 1]) ? 1 : 0;
-}
-
-__global__ __launch_bounds__(256) void k_compact_pairs(const uint32_t* __restrict__ hi, const uint32_t* __restrict__ lo,
-                                                       int n, const int* __restrict__ flag,
-                                                       const int* __restrict__ pos, uint32_t* __restrict__ ohi,
-                                                       uint32_t* __restrict__ olo) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !flag[i]) return;
-    ohi[pos[i]] = hi[i];
-    olo[pos[i]] = lo[i];
-}
-
 // ---------------------------------------------------------------------------
-// Swept-box broadphase (a conservative alternative to the centroid-cell
-// candidate set above, which misses faces larger than a cell).  Candidate
-// (v, f): v is a vertex of some triangle, v not in f, and v's box over the
-// substep, AABB(x_v, p_v), meets f's box over the substep, AABB of the six
-// points x_f*, p_f*, widened per side by 4 thickness plus 1e-6 |bound|.  The
-// narrowphase accepts a vertex within 2 thickness of the face plane and
+// Candidate pairs.
+//
+// Centroid cells (FindNeighbors over every triangle as CCD_SH_Extended
+// consumes it, SpatialHashSystem.cpp:134-187, CCD.cpp:1541-1586): (v, f) with
+// v a vertex of some triangle t whose cell is valid, f in the 27 cells around
+// t's cell, v not in f.  Edge pairs likewise from the cells of two triangles.
+//
+// Swept boxes (a conservative alternative, since the centroid cells miss faces
+// larger than a cell): v is a vertex of some triangle, v not in f, and v's box
+// over the substep, AABB(x_v, p_v), meets f's box over the substep, AABB of the
+// six points x_f*, p_f*, widened per side by 4 thickness plus 1e-6 |bound|.
+// The narrowphase accepts a vertex within 2 thickness of the face plane and
 // inside the face's barycentric band of width thickness / mean edge, i.e.
 // within sqrt(13) thickness of the face, at an interpolated position inside
-// both boxes, so every pair it accepts is a candidate: the contact set
-// equals that of the all-pairs test (CCD_N2, CCD.cpp:1040-1098).  The cell
-// grid only accelerates the box tests and does not change the set.
+// both boxes, so every pair it accepts is a candidate: the contact set equals
+// that of the all-pairs test (CCD_N2, CCD.cpp:1040-1098).
+//
+// Faces go into a hash table by cell: slot counts (one atomic per entry, whose
+// return value is the entry's place in its slot), slot offsets (one scan
+// pass), the entries.  A group of 32 lanes takes a vertex (an edge): its lanes
+// look up one cell each, then share the cells' entries evenly.  Each cell is
+// visited once per vertex, so a pair comes up once.  The form this replaces
+// made the pairs of every triangle (3.7 times as many on a folded 256 x 256
+// cloth), stored them, sorted them twice and compacted them: 2.6 ms per
+// detection there against 0.6 ms for the table, the visit and the narrowphase.
 // ---------------------------------------------------------------------------
-constexpr int SWEPT_MAX_CELLS = 4096;  // cells one box may span
+constexpr int SWEPT_MAX_CELLS = 4096;  // cells of the caller's grid one box may span
+constexpr int ENTRY_MAX_CELLS = 64;    // cells of the table's own grid a face is entered in
 
 __device__ __forceinline__ float widen_lo(float v, float m) { return v - (m + 1e-6f * fabsf(v)); }
 __device__ __forceinline__ float widen_hi(float v, float m) { return v + (m + 1e-6f * fabsf(v)); }
@@ -355,24 +202,12 @@ struct SweptBox {
     float lo[3], hi[3];
 };
 
-__device__ __forceinline__ SweptBox face_box(const float4* __restrict__ x, const float4* __restrict__ p,
-                                             const int* __restrict__ tris, int f, float margin) {
-    SweptBox b;
-    const float4 a[6] = {x[tris[3 * f]], x[tris[3 * f + 1]], x[tris[3 * f + 2]],
-                         p[tris[3 * f]], p[tris[3 * f + 1]], p[tris[3 * f + 2]]};
-    float lo[3] = {a[0].x, a[0].y, a[0].z}, hi[3] = {a[0].x, a[0].y, a[0].z};
-    for (int i = 1; i < 6; i++) {
-        const float c[3] = {a[i].x, a[i].y, a[i].z};
-        for (int k = 0; k < 3; k++) {
-            lo[k] = fminf(lo[k], c[k]);
-            hi[k] = fmaxf(hi[k], c[k]);
-        }
-    }
+__device__ __forceinline__ void box_add(SweptBox& b, float4 a) {
+    const float c[3] = {a.x, a.y, a.z};
     for (int k = 0; k < 3; k++) {
-        b.lo[k] = widen_lo(lo[k], margin);
-        b.hi[k] = widen_hi(hi[k], margin);
+        b.lo[k] = fminf(b.lo[k], c[k]);
+        b.hi[k] = fmaxf(b.hi[k], c[k]);
     }
-    return b;
 }
 
 __device__ __forceinline__ SweptBox vertex_box(const float4 X, const float4 P) {
@@ -383,114 +218,502 @@ __device__ __forceinline__ SweptBox vertex_box(const float4 X, const float4 P) {
     return b;
 }
 
-// Face boxes, their cell ranges and cell counts; err[0] = 1 if a face spans
-// more than SWEPT_MAX_CELLS cells (its count is then 0).
-__global__ __launch_bounds__(256) void k_swept_faces(HashCfg g, const float4* __restrict__ x, const float4* __restrict__ p,
-                                                     const int* __restrict__ tris, int nt, float margin,
-                                                     float4* __restrict__ fbox, int4* __restrict__ fcell,
-                                                     int* __restrict__ cnt, int* __restrict__ err) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= nt) return;
-    const SweptBox b = face_box(x, p, tris, f, margin);
-    int lo[3], hi[3];
-    long long n = 1;
-    for (int k = 0; k < 3; k++) {
-        lo[k] = cell_coord(g, b.lo[k], k);
-        hi[k] = cell_coord(g, b.hi[k], k);
-        // per-axis bound first: the product of three spans of up to 2^31 overflows
-        n *= (long long)min(hi[k] - lo[k] + 1, SWEPT_MAX_CELLS + 1);
-    }
-    fbox[2 * f] = make_float4(b.lo[0], b.lo[1], b.lo[2], 0.0f);
-    fbox[2 * f + 1] = make_float4(b.hi[0], b.hi[1], b.hi[2], 0.0f);
-    fcell[2 * f] = make_int4(lo[0], lo[1], lo[2], 0);
-    fcell[2 * f + 1] = make_int4(hi[0], hi[1], hi[2], 0);
-    if (n > SWEPT_MAX_CELLS) {
-        err[0] = 1;
-        n = 0;
-    }
-    cnt[f] = (int)n;
+// Slot of a cell in the table (any hash does: entries carry their cell).
+__device__ __forceinline__ unsigned cell_slot(int x, int y, int z, unsigned mask) {
+    unsigned h = ((unsigned)x * 73856093u) ^ ((unsigned)y * 19349663u) ^ ((unsigned)z * 83492791u);
+    h ^= h >> 15;
+    return h & mask;
 }
 
-// One (cell key + 1, face) entry per cell of each face box, x fastest.
-__global__ __launch_bounds__(256) void k_swept_entries(HashCfg g, int nt, const int4* __restrict__ fcell,
-                                                       const int* __restrict__ off, uint32_t* __restrict__ keys,
-                                                       uint32_t* __restrict__ ids) {
+// A face as the visits read it, one cache line: its widened swept box, its
+// vertices, and whether the box may rule pairs out (face_cullable).
+struct alignas(64) FaceRec {
+    float lo[3];
+    int v0;
+    float hi[3];
+    int v1;
+    int v2, cull;
+    int pad[6];
+};
+
+// Whether a vertex outside the face's swept box widened by 6 thickness cannot
+// pass the narrowphase's floating-point tests: the face keeps a good shape
+// over the whole step (doubled area at least 0.05 of its longest edge squared,
+// bounded below from the start's area and the edges' changes), so barycentric
+// coordinates carry a relative error of about 1e-4, and the thickness is not
+// tiny beside the edges, so the widening covers that error with room to spare.
+// Pairs with other faces always go to the narrowphase.
+__device__ __forceinline__ bool face_cullable(const float4* X, const float4* P, float th) {
+    const V3 e1 = mk(X[1].x - X[0].x, X[1].y - X[0].y, X[1].z - X[0].z);
+    const V3 e2 = mk(X[2].x - X[0].x, X[2].y - X[0].y, X[2].z - X[0].z);
+    const V3 d1 = mk(P[1].x - P[0].x - e1.x, P[1].y - P[0].y - e1.y, P[1].z - P[0].z - e1.z);
+    const V3 d2 = mk(P[2].x - P[0].x - e2.x, P[2].y - P[0].y - e2.y, P[2].z - P[0].z - e2.z);
+    const V3 c = cross(e1, e2);
+    const float l1 = sqrtf(dot(e1, e1)), l2 = sqrtf(dot(e2, e2)), m1 = sqrtf(dot(d1, d1)), m2 = sqrtf(dot(d2, d2));
+    const V3 e3 = sub(e2, e1);
+    const float longest = fmaxf(fmaxf(l1, l2), sqrtf(dot(e3, e3))) + m1 + m2;
+    const float area = sqrtf(dot(c, c)) - (l1 * m2 + l2 * m1 + m1 * m2);
+    return area >= 0.05f * (longest * longest) && th >= 4e-3f * longest;  // false for NaN
+}
+
+__device__ __forceinline__ void write_face(FaceRec* __restrict__ rec, int f, const float4* __restrict__ x,
+                                           const float4* __restrict__ p, const int* __restrict__ tris, float th,
+                                           float margin) {
+    FaceRec r;
+    r.v0 = tris[3 * f];
+    r.v1 = tris[3 * f + 1];
+    r.v2 = tris[3 * f + 2];
+    const float4 X[3] = {x[r.v0], x[r.v1], x[r.v2]}, P[3] = {p[r.v0], p[r.v1], p[r.v2]};
+    SweptBox b = vertex_box(X[0], X[0]);
+    for (int k = 1; k < 3; k++) box_add(b, X[k]);
+    for (int k = 0; k < 3; k++) box_add(b, P[k]);
+    for (int k = 0; k < 3; k++) {
+        r.lo[k] = widen_lo(b.lo[k], margin);
+        r.hi[k] = widen_hi(b.hi[k], margin);
+    }
+    r.cull = face_cullable(X, P, th) ? 1 : 0;
+    rec[f] = r;
+}
+
+__device__ __forceinline__ bool box_misses(const SweptBox& b, const FaceRec& r) {
+    return b.lo[0] > r.hi[0] || r.lo[0] > b.hi[0] || b.lo[1] > r.hi[1] || r.lo[1] > b.hi[1] || b.lo[2] > r.hi[2] ||
+           r.lo[2] > b.hi[2];
+}
+
+// Centroid cells: the face's cell and place in its slot, and its record.
+// tcell[t] = (cell, slot), slot -1 outside a dense grid.
+__global__ __launch_bounds__(256) void k_face_cells(HashCfg g, const float4* __restrict__ x, const float4* __restrict__ p,
+                                                    const int* __restrict__ tris, int nt, float th, unsigned mask,
+                                                    int* __restrict__ cnt, int4* __restrict__ tcell,
+                                                    int* __restrict__ rank, FaceRec* __restrict__ rec) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nt) return;
+    int gp[3];
+    tri_cell(g, p, tris, t, gp);
+    const bool in = cell_key(g, gp[0], gp[1], gp[2]) >= 0;
+    const unsigned slot = cell_slot(gp[0], gp[1], gp[2], mask);
+    tcell[t] = make_int4(gp[0], gp[1], gp[2], in ? (int)slot : -1);
+    rank[t] = in ? atomicAdd(&cnt[slot], 1) : 0;
+    write_face(rec, t, x, p, tris, th, 6.0f * th);
+}
+
+__global__ __launch_bounds__(256) void k_cell_fill(int nt, const int4* __restrict__ tcell, const int* __restrict__ rank,
+                                                   const int* __restrict__ cnt, const int* __restrict__ end,
+                                                   int4* __restrict__ ent) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nt) return;
+    const int4 c = tcell[t];
+    if (c.w >= 0) ent[end[c.w] - cnt[c.w] + rank[t]] = make_int4(c.x, c.y, c.z, t);
+}
+
+// Each slot's place among the entries: end[slot] (END) or its start.  Order
+// among workgroups is whatever their atomics make it.
+template <bool END>
+__global__ __launch_bounds__(256) void k_slot_places(const int* __restrict__ cnt, int nslots, int* __restrict__ place,
+                                                     unsigned* __restrict__ total) {
+    __shared__ int wave[4], base;
+    const int i = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int c = i < nslots ? cnt[i] : 0;
+    int run = c;
+    for (int off = 1; off < 64; off <<= 1) {
+        const int o = __shfl_up(run, off);
+        if (lane >= off) run += o;
+    }
+    if (lane == 63) wave[wv] = run;
+    __syncthreads();
+    if (threadIdx.x == 0) base = (int)atomicAdd(total, (unsigned)(wave[0] + wave[1] + wave[2] + wave[3]));
+    __syncthreads();
+    for (int w = 0; w < wv; w++) run += wave[w];
+    if (i < nslots) place[i] = base + (END ? run : run - c);
+}
+
+// Swept boxes: face records (their margin defines the candidate set), the
+// cells of the table's own grid gi they cover counted per slot.  A face over
+// more than ENTRY_MAX_CELLS of them goes to the list of large faces, which
+// every vertex tests.
+__global__ __launch_bounds__(256) void k_swept_faces(HashCfg g, HashCfg gi, const float4* __restrict__ x,
+                                                     const float4* __restrict__ p, const int* __restrict__ tris, int nt,
+                                                     float th, unsigned mask, int* __restrict__ cnt,
+                                                     int4* __restrict__ fcell, FaceRec* __restrict__ rec,
+                                                     int* __restrict__ large, DetectCounts* __restrict__ c) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= nt) return;
-    int o = off[f];
-    if (off[f + 1] == o) return;
+    write_face(rec, f, x, p, tris, th, 4.0f * th);
+    const FaceRec& r = rec[f];
+    int lo[3], hi[3];
+    long long span = 1, n = 1;
+    for (int k = 0; k < 3; k++) {
+        // per-axis bounds first: the product of three spans of up to 2^31 overflows
+        span *= (long long)min(cell_coord(g, r.hi[k], k) - cell_coord(g, r.lo[k], k) + 1, SWEPT_MAX_CELLS + 1);
+        lo[k] = cell_coord(gi, r.lo[k], k);
+        hi[k] = cell_coord(gi, r.hi[k], k);
+        n *= (long long)min(hi[k] - lo[k] + 1, ENTRY_MAX_CELLS + 1);
+    }
+    if (span > SWEPT_MAX_CELLS) c->face_span = 1;
+    fcell[2 * f] = make_int4(lo[0], lo[1], lo[2], n > ENTRY_MAX_CELLS ? 1 : 0);
+    fcell[2 * f + 1] = make_int4(hi[0], hi[1], hi[2], 0);
+    if (n > ENTRY_MAX_CELLS) {
+        large[atomicAdd(&c->large, 1u)] = f;
+        return;
+    }
+    for (int z = lo[2]; z <= hi[2]; z++)
+        for (int y = lo[1]; y <= hi[1]; y++)
+            for (int xx = lo[0]; xx <= hi[0]; xx++) atomicAdd(&cnt[cell_slot(xx, y, z, mask)], 1);
+}
+
+// The cell of an entry, 9 bits per axis (a face covers at most ENTRY_MAX_CELLS
+// cells, so it cannot cover two that agree in them), and per axis whether it is
+// the face's lowest cell.
+__device__ __forceinline__ int cell_code(int x, int y, int z) { return (x & 511) | ((y & 511) << 9) | ((z & 511) << 18); }
+
+// place: each slot's start, moved up by every entry stored; it ends at the
+// slot's end.
+__global__ __launch_bounds__(256) void k_swept_fill(int nt, const int4* __restrict__ fcell, unsigned mask,
+                                                    int* __restrict__ place, int2* __restrict__ ent, int cap) {
+    const int f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= nt) return;
     const int4 lo = fcell[2 * f], hi = fcell[2 * f + 1];
+    if (lo.w) return;
     for (int z = lo.z; z <= hi.z; z++)
         for (int y = lo.y; y <= hi.y; y++)
             for (int xx = lo.x; xx <= hi.x; xx++) {
-                keys[o] = (uint32_t)(cell_key(g, xx, y, z) + 1);
-                ids[o] = (uint32_t)f;
-                o++;
+                const int at = atomicAdd(&place[cell_slot(xx, y, z, mask)], 1);
+                const int first = (xx == lo.x ? 1 << 27 : 0) | (y == lo.y ? 1 << 28 : 0) | (z == lo.z ? 1 << 29 : 0);
+                if (at < cap) ent[at] = make_int2(f, cell_code(xx, y, z) | first);
             }
 }
 
-__global__ __launch_bounds__(256) void k_mark_vertices(const int* __restrict__ tris, int nt, int* __restrict__ vin) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < 3 * nt) vin[tris[i]] = 1;
+// Pairs a wave has found, appended to the global list in runs: one atomic on
+// the list's length per run.
+constexpr int VISIT_WAVES = 4, VISIT_BUF = 256;
+struct PairSink {
+    int2* buf;       // this wave's LDS
+    int n;           // wave-uniform
+    unsigned* len;
+    int2* out;
+    unsigned cap;
+    __device__ __forceinline__ void flush() {
+        const int lane = threadIdx.x & 63;
+        unsigned at = 0;
+        if (lane == 0) at = atomicAdd(len, (unsigned)n);
+        at = __shfl(at, 0);
+        for (int i = lane; i < n; i += 64)
+            if (at + i < cap) out[at + i] = buf[i];
+        n = 0;
+    }
+    // Called by all lanes of the wave.
+    __device__ __forceinline__ void add(bool hit, int a, int b) {
+        const unsigned long long m = __ballot(hit);
+        if (!m) return;
+        const int lane = threadIdx.x & 63;
+        if (hit) buf[n + __popcll(m & ((1ull << lane) - 1ull))] = make_int2(a, b);
+        n += __popcll(m);
+        if (n > VISIT_BUF - 64) flush();
+    }
+};
+
+// One round of a group's visit: lane l (of 32) of the group holds a run of
+// `mine` entries starting at `start` (0 entries: none); calls f(e, l) for every
+// entry e of every lane l's run, the lanes taking them in turn, and f(-1, l)
+// for the lanes left over.  Both groups of a wave stay in the loop until the
+// longer is done, so f may use wave-wide operations.
+template <class F>
+__device__ __forceinline__ void visit_runs(int start, int mine, F&& f) {
+    const int l = threadIdx.x & 31;
+    int sum = mine;
+    for (int off = 1; off < 32; off <<= 1) {
+        const int o = __shfl_up(sum, off, 32);
+        if (l >= off) sum += o;
+    }
+    const int total = __shfl(sum, 31, 32);
+    const int before = sum - mine;
+    const int longest = max(total, __shfl_xor(total, 32));
+    for (int b = 0; b < longest; b += 32) {
+        const int i = b + l;
+        int at = 0;  // the last lane whose runs before it do not exceed i
+        for (int step = 16; step > 0; step >>= 1)
+            if (__shfl(before, at + step, 32) <= i) at += step;
+        const int e = __shfl(start, at, 32) + i - __shfl(before, at, 32);
+        f(i < total ? e : -1, at);
+    }
 }
 
-// Per vertex: faces found in the cells of its box whose boxes meet it.  A
-// pair is taken at the lowest cell of the two cell ranges' intersection
-// only (a face stored twice in one slot is removed by the later unique
-// pass).  err[1] = 1 if a vertex box spans more than SWEPT_MAX_CELLS cells.
-template <int EMIT>
-__global__ __launch_bounds__(256) void k_swept_pairs(HashCfg g, const float4* __restrict__ x,
-                                                     const float4* __restrict__ p, const int* __restrict__ vin, int nv,
-                                                     const int* __restrict__ tris, const float4* __restrict__ fbox,
-                                                     const int4* __restrict__ fcell, const uint32_t* __restrict__ sids,
-                                                     const int* __restrict__ cstart, const int* __restrict__ cend,
-                                                     int* __restrict__ cnt_or_off, uint32_t* __restrict__ ov,
-                                                     uint32_t* __restrict__ of, int* __restrict__ err) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nv) return;
-    int n = 0;
-    const int base = EMIT ? cnt_or_off[v] : 0;
-    if (vin[v]) {
-        const SweptBox b = vertex_box(x[v], p[v]);
-        int lo[3], hi[3];
-        long long span = 1;
-        for (int k = 0; k < 3; k++) {
-            lo[k] = cell_coord(g, b.lo[k], k);
-            hi[k] = cell_coord(g, b.hi[k], k);
-            span *= (long long)min(hi[k] - lo[k] + 1, SWEPT_MAX_CELLS + 1);
-        }
-        if (span > SWEPT_MAX_CELLS) {
-            if (!EMIT) err[1] = 1;
-        } else {
-            for (int qz = lo[2]; qz <= hi[2]; qz++)
-                for (int qy = lo[1]; qy <= hi[1]; qy++)
-                    for (int qx = lo[0]; qx <= hi[0]; qx++) {
-                        const int h = cell_key(g, qx, qy, qz);
-                        if (h < 0) continue;
-                        const int s = cstart[h];
-                        if (s < 0) continue;
-                        const int e = cend[h];
-                        for (int i = s; i <= e; i++) {
-                            const int f = (int)sids[i];
-                            const int4 fl = fcell[2 * f], fh = fcell[2 * f + 1];
-                            // the pair's first shared cell, and f really covers it
-                            if (qx != max(lo[0], fl.x) || qy != max(lo[1], fl.y) || qz != max(lo[2], fl.z)) continue;
-                            if (qx > fh.x || qy > fh.y || qz > fh.z) continue;
-                            const float4 flo = fbox[2 * f], fhi = fbox[2 * f + 1];
-                            if (b.lo[0] > fhi.x || flo.x > b.hi[0] || b.lo[1] > fhi.y || flo.y > b.hi[1] ||
-                                b.lo[2] > fhi.z || flo.z > b.hi[2])
-                                continue;
-                            if (tris[3 * f] == v || tris[3 * f + 1] == v || tris[3 * f + 2] == v) continue;
-                            if (EMIT) {
-                                ov[base + n] = (uint32_t)v;
-                                of[base + n] = (uint32_t)f;
-                            }
-                            n++;
+// Whether c is a valid cell and (x, y, z) is within one cell of it.
+__device__ __forceinline__ bool near_cell(int4 c, int x, int y, int z) {
+    return c.w >= 0 && abs(c.x - x) <= 1 && abs(c.y - y) <= 1 && abs(c.z - z) <= 1;
+}
+// Cell l (0..26) of the 27 around c.
+__device__ __forceinline__ int3 around(int4 c, int l) {
+    return make_int3(c.x + l % 3 - 1, c.y + l / 3 % 3 - 1, c.z + l / 9 - 1);
+}
+
+__device__ __forceinline__ unsigned long long wave_total(int n) {
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
+    return (unsigned long long)n;
+}
+
+// Vertex-face candidates by centroid cells.  Group = 32 lanes = one vertex:
+// for its triangles in turn, lanes 0..26 take the cells around the triangle's
+// own that no earlier triangle of the vertex has covered.  All candidates are
+// counted; listed are all of them (LIST) or those that no box rules out.
+template <bool LIST>
+__global__ __launch_bounds__(64 * VISIT_WAVES) void k_vf_candidates(
+    HashCfg g, const float4* __restrict__ x, const float4* __restrict__ p, int nv, const int* __restrict__ vtoff,
+    const int* __restrict__ vtri, const int4* __restrict__ tcell, const int* __restrict__ cnt,
+    const int* __restrict__ end, unsigned mask, const int4* __restrict__ ent, const FaceRec* __restrict__ rec,
+    DetectCounts* __restrict__ c, int2* __restrict__ out, unsigned cap) {
+    __shared__ int2 buf[VISIT_WAVES][VISIT_BUF];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 31;
+    PairSink sink{buf[wv], 0, &c->near, out, cap};
+    int pairs = 0;
+    const int stride = (int)gridDim.x * VISIT_WAVES * 2;
+    for (int v0 = ((int)blockIdx.x * VISIT_WAVES + wv) * 2; v0 < nv; v0 += stride) {
+        const int v = v0 + (lane >> 5), at = min(v, nv - 1);
+        const int o = vtoff[at], deg = v < nv ? vtoff[at + 1] - o : 0;
+        const SweptBox b = vertex_box(x[at], p[at]);
+        const int most = max(deg, __shfl_xor(deg, 32));
+        for (int i = 0; i < most; i++) {
+            const int4 tc = i < deg ? tcell[vtri[o + i]] : make_int4(0, 0, 0, -1);
+            const int3 q = around(tc, l);
+            bool mine = tc.w >= 0 && l < 27 && cell_key(g, q.x, q.y, q.z) >= 0;
+            for (int j = 0; j < min(i, deg); j++)
+                if (near_cell(tcell[vtri[o + j]], q.x, q.y, q.z)) mine = false;
+            if (!__any(mine)) continue;
+            const unsigned slot = cell_slot(q.x, q.y, q.z, mask);
+            const int n = mine ? cnt[slot] : 0;
+            visit_runs(n ? end[slot] - n : 0, n, [&](int e, int from) {
+                bool hit = false;
+                int f = 0;
+                if (e >= 0) {
+                    const int4 ec = ent[e];
+                    const int3 fq = around(tc, from);
+                    f = ec.w;
+                    // a slot may hold other cells' faces too
+                    if (ec.x == fq.x && ec.y == fq.y && ec.z == fq.z) {
+                        const FaceRec r = rec[f];
+                        if (v != r.v0 && v != r.v1 && v != r.v2) {
+                            pairs++;
+                            hit = LIST || !(r.cull && box_misses(b, r));
                         }
                     }
+                }
+                sink.add(hit, v, f);
+            });
         }
     }
-    if (!EMIT) cnt_or_off[v] = n;
+    if (sink.n) sink.flush();
+    const unsigned long long t = wave_total(pairs);
+    if (!LIST && lane == 0 && t) atomicAdd(&c->pairs, t);
+}
+
+// Vertex-face candidates by swept boxes: the faces entered in the cells of the
+// vertex's box, taken at the lowest cell that the two boxes' cell ranges share,
+// and the large faces.
+__global__ __launch_bounds__(64 * VISIT_WAVES) void k_swept_candidates(
+    HashCfg g, HashCfg gi, const float4* __restrict__ x, const float4* __restrict__ p, int nv,
+    const int* __restrict__ vtoff, const int* __restrict__ cnt, const int* __restrict__ end, unsigned mask,
+    const int2* __restrict__ ent, int ent_cap, const FaceRec* __restrict__ rec, const int* __restrict__ large,
+    DetectCounts* __restrict__ c, int2* __restrict__ out, unsigned cap) {
+    __shared__ int2 buf[VISIT_WAVES][VISIT_BUF];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 31;
+    PairSink sink{buf[wv], 0, &c->near, out, cap};
+    const int nlarge = (int)c->large;
+    int pairs = 0;
+    const int stride = (int)gridDim.x * VISIT_WAVES * 2;
+    for (int v0 = ((int)blockIdx.x * VISIT_WAVES + wv) * 2; v0 < nv; v0 += stride) {
+        const int v = v0 + (lane >> 5), at = min(v, nv - 1);
+        const bool used = v < nv && vtoff[at + 1] > vtoff[at];
+        const SweptBox b = vertex_box(x[at], p[at]);
+        int lo[3], w[3];
+        long long span = 1;
+        for (int k = 0; k < 3; k++) {
+            span *= (long long)min(cell_coord(g, b.hi[k], k) - cell_coord(g, b.lo[k], k) + 1, SWEPT_MAX_CELLS + 1);
+            lo[k] = cell_coord(gi, b.lo[k], k);
+            w[k] = min(cell_coord(gi, b.hi[k], k) - lo[k] + 1, SWEPT_MAX_CELLS + 1);
+        }
+        const bool over = span > SWEPT_MAX_CELLS;
+        if (used && over) c->vertex_span = 1;
+        const int cells = used && !over ? w[0] * w[1] * w[2] : 0;
+        auto cell_of = [&](int i) { return make_int3(lo[0] + i % w[0], lo[1] + i / w[0] % w[1], lo[2] + i / (w[0] * w[1])); };
+        auto test = [&](bool in, int f) {
+            bool hit = false;
+            if (in) {
+                const FaceRec r = rec[f];
+                hit = !box_misses(b, r) && v != r.v0 && v != r.v1 && v != r.v2;
+                pairs += hit;
+            }
+            sink.add(hit, v, f);
+        };
+        const int most = max(cells, __shfl_xor(cells, 32));
+        for (int c0 = 0; c0 < most; c0 += 32) {
+            const int3 q = cell_of(c0 + l);
+            const unsigned slot = cell_slot(q.x, q.y, q.z, mask);
+            int n = c0 + l < cells ? cnt[slot] : 0;
+            const int e1 = n ? end[slot] : 0;
+            if (e1 > ent_cap) n = 0;  // the table did not fit: the caller starts over
+            visit_runs(e1 - n, n, [&](int e, int from) {
+                bool in = false;
+                int f = 0;
+                if (e >= 0) {
+                    const int2 en = ent[e];
+                    const int3 fq = cell_of(c0 + from);
+                    f = en.x;
+                    in = (en.y & 0x7ffffff) == cell_code(fq.x, fq.y, fq.z) && ((en.y >> 27 & 1) || fq.x == lo[0]) &&
+                         ((en.y >> 28 & 1) || fq.y == lo[1]) && ((en.y >> 29 & 1) || fq.z == lo[2]);
+                }
+                test(in, f);
+            });
+        }
+        for (int i = 0; i < nlarge; i += 32) test(used && !over && i + l < nlarge, large[min(i + l, nlarge - 1)]);
+    }
+    if (sink.n) sink.flush();
+    const unsigned long long t = wave_total(pairs);
+    if (lane == 0 && t) atomicAdd(&c->pairs, t);
+}
+
+// Swept boxes of the edges (four points each), not widened.
+__global__ __launch_bounds__(256) void k_edge_boxes(const int2* __restrict__ edges, int ne, const float4* __restrict__ x,
+                                                    const float4* __restrict__ p, float4* __restrict__ box) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= ne) return;
+    const int2 v = edges[e];
+    SweptBox b = vertex_box(x[v.x], p[v.x]);
+    box_add(b, x[v.y]);
+    box_add(b, p[v.y]);
+    box[2 * e] = make_float4(b.lo[0], b.lo[1], b.lo[2], 0.0f);
+    box[2 * e + 1] = make_float4(b.hi[0], b.hi[1], b.hi[2], 0.0f);
+}
+
+// Whether two edges' swept boxes lie further apart along an axis than the
+// contact distance and the rounding of the closest points' coordinates: every
+// point the narrowphase measures between lies in the boxes, so such a pair is
+// no contact.  (False for NaN.)
+__device__ __forceinline__ bool edges_apart(float4 alo, float4 ahi, float4 blo, float4 bhi, float th) {
+    auto apart = [&](float hi, float lo) { return lo - hi > 2.0f * th + 2e-6f * (fabsf(lo) + fabsf(hi)); };
+    return apart(ahi.x, blo.x) || apart(bhi.x, alo.x) || apart(ahi.y, blo.y) || apart(bhi.y, alo.y) ||
+           apart(ahi.z, blo.z) || apart(bhi.z, alo.z);
+}
+
+// Edge-edge candidates (new: the reference declares Contact::EE, CCD_Basic.h:14,
+// and leaves it unimplemented, CCD.cpp:925-928): every pair of edges of two
+// triangles whose centroid cells are at most one cell apart that shares no
+// vertex and has no vertex that is a mesh neighbour of the other edge's (pairs
+// that close in the mesh are material neighbours, not contacts), once, as
+// (lower edge id, higher edge id).  Group = 32 lanes = the lower edge a: the
+// cells around its triangles, each once; a face found there offers its edges b
+// of higher id, and an edge b of several faces counts at the first of them (in
+// the order of b's list) that lies around a's triangles.
+constexpr int RING_MAX = 64;
+
+template <bool LIST>
+__global__ __launch_bounds__(64 * VISIT_WAVES) void k_ee_candidates(
+    HashCfg g, int ne, const int2* __restrict__ edges, const int* __restrict__ etoff, const int* __restrict__ etri,
+    const int* __restrict__ tedge, const int* __restrict__ voff, const int* __restrict__ vnbr,
+    const int4* __restrict__ tcell, const int* __restrict__ cnt, const int* __restrict__ end, unsigned mask,
+    const int4* __restrict__ ent, const FaceRec* __restrict__ rec, const float4* __restrict__ box, float th,
+    DetectCounts* __restrict__ c, int2* __restrict__ out, unsigned cap) {
+    __shared__ int2 buf[VISIT_WAVES][VISIT_BUF];
+    __shared__ int ring_s[VISIT_WAVES][2][RING_MAX];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 31;
+    int* ring = ring_s[wv][lane >> 5];
+    PairSink sink{buf[wv], 0, &c->ee_near, out, cap};
+    int pairs = 0;
+    const int stride = (int)gridDim.x * VISIT_WAVES * 2;
+    for (int a0 = ((int)blockIdx.x * VISIT_WAVES + wv) * 2; a0 < ne; a0 += stride) {
+        const int a = a0 + (lane >> 5), at = min(a, ne - 1);
+        const int2 av = edges[at];
+        const int o = etoff[at], deg = a < ne ? etoff[at + 1] - o : 0;
+        const float4 alo = box[2 * at], ahi = box[2 * at + 1];
+        // a's vertices and their mesh neighbours: an edge with a vertex among them is no candidate
+        const int r0 = voff[av.x], n0 = voff[av.x + 1] - r0, r1 = voff[av.y], n1 = voff[av.y + 1] - r1;
+        const bool fits = n0 + n1 + 2 <= RING_MAX;
+        __builtin_amdgcn_wave_barrier();  // the round before has read the lists
+        if (fits)
+            for (int i = l; i < n0 + n1 + 2; i += 32)
+                ring[i] = i == 0 ? av.x : i == 1 ? av.y : i < n0 + 2 ? vnbr[r0 + i - 2] : vnbr[r1 + i - 2 - n0];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        auto in_ring = [&](int u) {
+            if (fits) {
+                bool in = false;
+                for (int i = 0; i < n0 + n1 + 2; i++) in |= ring[i] == u;
+                return in;
+            }
+            bool in = u == av.x || u == av.y;
+            for (int i = 0; i < n0; i++) in |= vnbr[r0 + i] == u;
+            for (int i = 0; i < n1; i++) in |= vnbr[r1 + i] == u;
+            return in;
+        };
+        const int most = max(deg, __shfl_xor(deg, 32));
+        for (int i = 0; i < most; i++) {
+            const int4 tc = i < deg ? tcell[etri[o + i]] : make_int4(0, 0, 0, -1);
+            const int3 q = around(tc, l);
+            bool mine = tc.w >= 0 && l < 27 && cell_key(g, q.x, q.y, q.z) >= 0;
+            for (int j = 0; j < min(i, deg); j++)
+                if (near_cell(tcell[etri[o + j]], q.x, q.y, q.z)) mine = false;
+            if (!__any(mine)) continue;
+            const unsigned slot = cell_slot(q.x, q.y, q.z, mask);
+            const int n = mine ? cnt[slot] : 0;
+            visit_runs(n ? end[slot] - n : 0, n, [&](int e, int from) {
+                bool face = false, out_of[3] = {false, false, false};
+                int f = 0;
+                if (e >= 0) {
+                    const int4 ec = ent[e];
+                    const int3 fq = around(tc, from);
+                    f = ec.w;
+                    face = ec.x == fq.x && ec.y == fq.y && ec.z == fq.z;
+                    if (face) {
+                        out_of[0] = !in_ring(rec[f].v0);
+                        out_of[1] = !in_ring(rec[f].v1);
+                        out_of[2] = !in_ring(rec[f].v2);
+                    }
+                }
+                for (int k = 0; k < 3; k++) {
+                    bool hit = false;
+                    int eb = 0;
+                    if (face && out_of[k] && out_of[k == 2 ? 0 : k + 1]) {
+                        eb = tedge[3 * f + k];
+                        bool cand = eb > a;
+                        // a face with a repeated vertex has an edge twice
+                        for (int m = 0; m < k; m++) cand = cand && eb != tedge[3 * f + m];
+                        for (int j = etoff[eb]; cand && j < etoff[eb + 1]; j++) {
+                            const int f2 = etri[j];
+                            if (f2 == f) break;
+                            const int4 c2 = tcell[f2];
+                            for (int m = 0; c2.w >= 0 && m < deg; m++)
+                                if (near_cell(tcell[etri[o + m]], c2.x, c2.y, c2.z)) cand = false;
+                        }
+                        if (cand) {
+                            pairs++;
+                            hit = LIST || !edges_apart(alo, ahi, box[2 * eb], box[2 * eb + 1], th);
+                        }
+                    }
+                    sink.add(hit, a, eb);
+                }
+            });
+        }
+    }
+    if (sink.n) sink.flush();
+    const unsigned long long t = wave_total(pairs);
+    if (!LIST && lane == 0 && t) atomicAdd(&c->ee_pairs, t);
+}
+
+// Vertex -> triangles (CSR, any order within a vertex).
+__global__ __launch_bounds__(256) void k_vt_count(const int* __restrict__ tris, int n, int* __restrict__ cnt) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) atomicAdd(&cnt[tris[i]], 1);
+}
+__global__ __launch_bounds__(256) void k_vt_fill(const int* __restrict__ tris, int n, const int* __restrict__ off,
+                                                 int* __restrict__ cnt, int* __restrict__ vtri) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) vtri[off[tris[i]] + atomicSub(&cnt[tris[i]], 1) - 1] = i / 3;
+}
+__global__ __launch_bounds__(256) void k_unzip(const int2* __restrict__ a, int n, uint32_t* __restrict__ hi,
+                                               uint32_t* __restrict__ lo) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    hi[i] = (uint32_t)a[i].x;
+    lo[i] = (uint32_t)a[i].y;
 }
 
 // ---------------------------------------------------------------------------
@@ -631,51 +854,73 @@ __device__ bool vf_ccd(V3 x0, V3 x1, V3 x2, V3 x3, V3 p0, V3 p1, V3 p2, V3 p3, f
     return false;
 }
 
-__global__ __launch_bounds__(256) void k_narrow(const uint32_t* __restrict__ cv, const uint32_t* __restrict__ cf,
-                                                int n, const int* __restrict__ tris, const float4* __restrict__ x,
-                                                const float4* __restrict__ p, float th, int* __restrict__ flag,
+// The narrowphase over the listed pairs (their number is on the device), its
+// contacts appended in any order.  STORE: time, normal and weights too (the
+// response needs only the vertices).
+template <bool STORE>
+__global__ __launch_bounds__(256) void k_narrow(const int2* __restrict__ near, unsigned near_cap,
+                                                const int* __restrict__ tris, const float4* __restrict__ x,
+                                                const float4* __restrict__ p, float th, DetectCounts* __restrict__ c,
+                                                unsigned cap, int4* __restrict__ vquad, int2* __restrict__ vf,
                                                 float* __restrict__ ct, float* __restrict__ cn,
                                                 double* __restrict__ cw) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int v = (int)cv[i], f = (int)cf[i];
-    int a = tris[3 * f], b = tris[3 * f + 1], c = tris[3 * f + 2];
-    float t;
-    V3 nr, wg;
-    bool hit = vf_ccd(v3(x[v]), v3(x[a]), v3(x[b]), v3(x[c]), v3(p[v]), v3(p[a]), v3(p[b]), v3(p[c]), th, &t, &nr, &wg);
-    flag[i] = hit ? 1 : 0;
-    if (hit) {
-        ct[i] = t;
-        cn[3 * i] = nr.x;
-        cn[3 * i + 1] = nr.y;
-        cn[3 * i + 2] = nr.z;
-        cw[4 * i] = 1.0;
-        cw[4 * i + 1] = wg.x;
-        cw[4 * i + 2] = wg.y;
-        cw[4 * i + 3] = wg.z;
+    const unsigned n = min(c->near, near_cap);
+    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+        const int2 q = near[i];
+        const int a = tris[3 * q.y], b = tris[3 * q.y + 1], d = tris[3 * q.y + 2];
+        float t;
+        V3 nr, wg;
+        if (!vf_ccd(v3(x[q.x]), v3(x[a]), v3(x[b]), v3(x[d]), v3(p[q.x]), v3(p[a]), v3(p[b]), v3(p[d]), th, &t, &nr, &wg))
+            continue;
+        const unsigned o = atomicAdd(&c->contacts, 1u);
+        if (o >= cap) continue;
+        vquad[o] = make_int4(q.x, a, b, d);
+        if (STORE) {
+            vf[o] = q;
+            ct[o] = t;
+            cn[3 * o] = nr.x;
+            cn[3 * o + 1] = nr.y;
+            cn[3 * o + 2] = nr.z;
+            cw[4 * o] = 1.0;
+            cw[4 * o + 1] = wg.x;
+            cw[4 * o + 2] = wg.y;
+            cw[4 * o + 3] = wg.z;
+        }
     }
 }
 
-__global__ __launch_bounds__(256) void k_compact_contacts(int n, const int* __restrict__ flag,
-                                                          const int* __restrict__ pos,
-                                                          const uint32_t* __restrict__ cv,
-                                                          const uint32_t* __restrict__ cf, const float* __restrict__ ct,
-                                                          const float* __restrict__ cn, const double* __restrict__ cw,
-                                                          int* __restrict__ ov, int* __restrict__ of,
-                                                          float* __restrict__ ot, float* __restrict__ on,
-                                                          double* __restrict__ ow) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !flag[i]) return;
-    int o = pos[i];
-    ov[o] = (int)cv[i];
-    of[o] = (int)cf[i];
-    ot[o] = ct[i];
-    for (int k = 0; k < 3; k++) on[3 * o + k] = cn[3 * i + k];
-    for (int k = 0; k < 4; k++) ow[4 * o + k] = cw[4 * i + k];
+// Contacts in ascending (first, second) order, for callers that read them:
+// counted by their first id, scanned, dealt to their first id's run, and each
+// placed by the number of smaller second ids in its run.
+__global__ __launch_bounds__(256) void k_first_count(const int2* __restrict__ key, int n, int* __restrict__ cnt) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) atomicAdd(&cnt[key[i].x], 1);
+}
+__global__ __launch_bounds__(256) void k_first_deal(const int2* __restrict__ key, int n, const int* __restrict__ off,
+                                                    int* __restrict__ cnt, int* __restrict__ idx) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) idx[off[key[i].x] + atomicSub(&cnt[key[i].x], 1) - 1] = i;
+}
+__global__ __launch_bounds__(256) void k_contact_order(const int2* __restrict__ key, int n, const int* __restrict__ off,
+                                                       const int* __restrict__ idx, const float* __restrict__ t,
+                                                       const float* __restrict__ nr, const double* __restrict__ w,
+                                                       const int4* __restrict__ quad, int2* __restrict__ okey,
+                                                       float* __restrict__ ot, float* __restrict__ on,
+                                                       double* __restrict__ ow, int4* __restrict__ oquad) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int2 k = key[i];
+    int at = off[k.x];
+    for (int j = off[k.x]; j < off[k.x + 1]; j++) at += key[idx[j]].y < k.y;
+    okey[at] = k;
+    ot[at] = t[i];
+    for (int a = 0; a < 3; a++) on[3 * at + a] = nr[3 * i + a];
+    for (int a = 0; a < 4; a++) ow[4 * at + a] = w[4 * i + a];
+    if (quad) oquad[at] = quad[i];
 }
 
 // ---------------------------------------------------------------------------
-// edge-edge narrowphase and response (new; see k_ee_pairs)
+// edge-edge narrowphase and response (new; see k_ee_candidates)
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ long long to_fixed(float f) { return (long long)rint((double)f * 4294967296.0); }
 __device__ __forceinline__ float clamp01(float v) { return v < 0.0f ? 0.0f : (v > 1.0f ? 1.0f : v); }
@@ -793,42 +1038,34 @@ __device__ bool ee_ccd(V3 x0, V3 x1, V3 x2, V3 x3, V3 p0, V3 p1, V3 p2, V3 p3, f
     return false;
 }
 
-__global__ __launch_bounds__(256) void k_narrow_ee(const uint32_t* __restrict__ ua, const uint32_t* __restrict__ ub,
-                                                   int n, const int2* __restrict__ edges,
-                                                   const float4* __restrict__ x, const float4* __restrict__ p,
-                                                   float th, int* __restrict__ flag, float* __restrict__ ct,
-                                                   float* __restrict__ cn, double* __restrict__ cw) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int2 ea = edges[ua[i]], eb = edges[ub[i]];
-    float t, w[4];
-    V3 nr;
-    bool hit = ee_ccd(v3(x[ea.x]), v3(x[ea.y]), v3(x[eb.x]), v3(x[eb.y]), v3(p[ea.x]), v3(p[ea.y]), v3(p[eb.x]),
-                      v3(p[eb.y]), th, &t, &nr, w);
-    flag[i] = hit ? 1 : 0;
-    if (hit) {
-        ct[i] = t;
-        cn[3 * i] = nr.x;
-        cn[3 * i + 1] = nr.y;
-        cn[3 * i + 2] = nr.z;
-        for (int k = 0; k < 4; k++) cw[4 * i + k] = w[k];
+template <bool STORE>
+__global__ __launch_bounds__(256) void k_narrow_ee(const int2* __restrict__ near, unsigned near_cap,
+                                                   const int2* __restrict__ edges, const float4* __restrict__ x,
+                                                   const float4* __restrict__ p, float th, DetectCounts* __restrict__ c,
+                                                   unsigned cap, int2* __restrict__ ab, int4* __restrict__ quad,
+                                                   float* __restrict__ ct, float* __restrict__ cn,
+                                                   double* __restrict__ cw) {
+    const unsigned n = min(c->ee_near, near_cap);
+    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+        const int2 q = near[i];
+        const int2 ea = edges[q.x], eb = edges[q.y];
+        float t, w[4];
+        V3 nr;
+        if (!ee_ccd(v3(x[ea.x]), v3(x[ea.y]), v3(x[eb.x]), v3(x[eb.y]), v3(p[ea.x]), v3(p[ea.y]), v3(p[eb.x]),
+                    v3(p[eb.y]), th, &t, &nr, w))
+            continue;
+        const unsigned o = atomicAdd(&c->ee_contacts, 1u);
+        if (o >= cap) continue;
+        quad[o] = make_int4(ea.x, ea.y, eb.x, eb.y);
+        if (STORE) {
+            ab[o] = q;
+            ct[o] = t;
+            cn[3 * o] = nr.x;
+            cn[3 * o + 1] = nr.y;
+            cn[3 * o + 2] = nr.z;
+            for (int k = 0; k < 4; k++) cw[4 * o + k] = w[k];
+        }
     }
-}
-
-__global__ __launch_bounds__(256) void k_compact_ee(int n, const int* __restrict__ flag, const int* __restrict__ pos,
-                                                    const uint32_t* __restrict__ ua, const uint32_t* __restrict__ ub,
-                                                    const int2* __restrict__ edges, const float* __restrict__ ct,
-                                                    const float* __restrict__ cn, const double* __restrict__ cw,
-                                                    int4* __restrict__ oq, float* __restrict__ ot,
-                                                    float* __restrict__ on, double* __restrict__ ow) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !flag[i]) return;
-    int o = pos[i];
-    int2 ea = edges[ua[i]], eb = edges[ub[i]];
-    oq[o] = make_int4(ea.x, ea.y, eb.x, eb.y);
-    ot[o] = ct[i];
-    for (int k = 0; k < 3; k++) on[3 * o + k] = cn[3 * i + k];
-    for (int k = 0; k < 4; k++) ow[4 * o + k] = cw[4 * i + k];
 }
 
 // Edge-edge response on the current positions, for separable edges
@@ -857,62 +1094,25 @@ __device__ bool ee_fix(const V3* X, const V3* q, float th, V3* d) {
     return true;
 }
 
-__global__ __launch_bounds__(256) void k_resolve_ee_acc(const int4* __restrict__ cq, int nc,
-                                                        const float4* __restrict__ x, const float4* __restrict__ p,
-                                                        float th, unsigned long long* __restrict__ acc,
-                                                        int* __restrict__ cnt) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nc) return;
-    int4 c = cq[i];
-    int id[4] = {c.x, c.y, c.z, c.w};
-    float4 P[4];
-    V3 X[4], q[4], d[4];
-    for (int k = 0; k < 4; k++) {
-        P[k] = p[id[k]];
-        X[k] = v3(x[id[k]]);
-        q[k] = v3(P[k]);
-    }
-    if (!ee_fix(X, q, th, d)) return;
-    bool a_static = P[0].w == 0.0f && P[1].w == 0.0f, b_static = P[2].w == 0.0f && P[3].w == 0.0f;
-    for (int k = 0; k < 4; k++) {
-        if (P[k].w == 0.0f) continue;
-        float sc = (k < 2 ? b_static : a_static) ? 2.0f : 1.0f;
-        atomicAdd(&acc[3 * (size_t)id[k]], (unsigned long long)to_fixed(d[k].x * sc));
-        atomicAdd(&acc[3 * (size_t)id[k] + 1], (unsigned long long)to_fixed(d[k].y * sc));
-        atomicAdd(&acc[3 * (size_t)id[k] + 2], (unsigned long long)to_fixed(d[k].z * sc));
-        atomicAdd(&cnt[id[k]], 1);
-    }
-}
-
 // ---------------------------------------------------------------------------
 // response
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void k_resolve_acc(const int* __restrict__ cvv, const int* __restrict__ cff, int nc,
-                                                     const int* __restrict__ tris, const float4* __restrict__ x,
-                                                     const float4* __restrict__ p, float th, float min_n2,
-                                                     unsigned long long* __restrict__ acc, int* __restrict__ cnt) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nc) return;
-    int f = cff[i];
-    int id[4] = {cvv[i], tris[3 * f], tris[3 * f + 1], tris[3 * f + 2]};
-    float4 P[4];
-    V3 X[4], q[4];
-    for (int k = 0; k < 4; k++) {
-        P[k] = p[id[k]];
-        X[k] = v3(x[id[k]]);
-        q[k] = v3(P[k]);
-    }
-    // VFResolveTest (CCD.cpp:1996-2032)
+// The side of the face that the vertex was on at the start of the step.
+__device__ __forceinline__ bool vf_front(const V3* X) {
     V3 n0 = vnormalize(cross(sub(X[2], X[1]), sub(X[3], X[1])));
-    bool dir = dot(sub(X[0], X[1]), n0) >= 0;
+    return dot(sub(X[0], X[1]), n0) >= 0;
+}
+
+__device__ __forceinline__ bool vf_fix(bool front, const V3* q, float th, float min_n2, V3* d) {
+    // VFResolveTest (CCD.cpp:1996-2032)
     V3 cr = cross(sub(q[2], q[1]), sub(q[3], q[1]));
-    if (dot(cr, cr) <= min_n2) return;
+    if (dot(cr, cr) <= min_n2) return false;
     V3 pn = vnormalize(cr);
-    float s = dir ? 1.0f : -1.0f;
+    float s = front ? 1.0f : -1.0f;
     V3 sn = V3{pn.x * s, pn.y * s, pn.z * s};
     float depth0 = dot(sub(q[0], q[1]), sn) - 2.0 * th;
-    if (!(depth0 < -1e-6)) return;
+    if (!(depth0 < -1e-6)) return false;
     // VFResolveNew (CCD.cpp:2034-2090)
     V3 proj = V3{q[1].x + ((pn.x * s) * 2.0f) * th, q[1].y + ((pn.y * s) * 2.0f) * th, q[1].z + ((pn.z * s) * 2.0f) * th};
     float depth = dot(sub(proj, q[0]), sn) * 0.5;
@@ -921,37 +1121,172 @@ __global__ __launch_bounds__(256) void k_resolve_acc(const int* __restrict__ cvv
     float wf[3] = {wg.x, wg.y, wg.z};
     float snv[3] = {sn.x, sn.y, sn.z}, pnv[3] = {pn.x, pn.y, pn.z};
     float qa[4][3] = {{q[0].x, q[0].y, q[0].z}, {q[1].x, q[1].y, q[1].z}, {q[2].x, q[2].y, q[2].z}, {q[3].x, q[3].y, q[3].z}};
-    float qb[4][3];
+    float fix[4][3];
     for (int a = 0; a < 3; a++) {
         float vfix = depth * snv[a];
         float ffix = depth * (pnv[a] * -s);
-        qb[0][a] = qa[0][a] + vfix;
-        qb[1][a] = qa[1][a] + (ffix * wf[0]) / sw;
-        qb[2][a] = qa[2][a] + (ffix * wf[1]) / sw;
-        qb[3][a] = qa[3][a] + (ffix * wf[2]) / sw;
+        fix[0][a] = (qa[0][a] + vfix) - qa[0][a];
+        fix[1][a] = (qa[1][a] + (ffix * wf[0]) / sw) - qa[1][a];
+        fix[2][a] = (qa[2][a] + (ffix * wf[1]) / sw) - qa[2][a];
+        fix[3][a] = (qa[3][a] + (ffix * wf[2]) / sw) - qa[3][a];
     }
-    bool face_static = (P[1].w == 0.0f) && (P[2].w == 0.0f) && (P[3].w == 0.0f);
+    for (int k = 0; k < 4; k++) d[k] = V3{fix[k][0], fix[k][1], fix[k][2]};
+    return true;
+}
+
+// A contact's corners: vertex-face contacts (vertex, face) first, edge-edge
+// ones (two edges) behind them.
+__device__ __forceinline__ int4 contact_at(const int4* __restrict__ vquad, int nc, const int4* __restrict__ quad, int i) {
+    return i < nc ? vquad[i] : quad[i - nc];
+}
+__device__ __forceinline__ int corner(int4 c, int k) { return k == 0 ? c.x : k == 1 ? c.y : k == 2 ? c.z : c.w; }
+
+// The fix of corner k of a contact: doubled where the other side (face or
+// vertex, or the other edge) is static as a whole.  `still`: bit per static corner.
+__device__ __forceinline__ float fix_scale(bool vertex_face, unsigned still, int k) {
+    if (vertex_face) return (k == 0 ? (still & 14) == 14 : (still & 1)) ? 2.0f : 1.0f;
+    return (k < 2 ? (still & 12) == 12 : (still & 3) == 3) ? 2.0f : 1.0f;
+}
+
+__device__ __forceinline__ float mean_fix(unsigned long long sum, double c) {
+    return (float)((double)(long long)sum / 4294967296.0 / c);
+}
+
+__global__ __launch_bounds__(256) void k_resolve_acc(const int4* __restrict__ vquad, int nc,
+                                                     const int4* __restrict__ quad, int ne, const float4* __restrict__ x,
+                                                     const float4* __restrict__ p, float th, float min_n2,
+                                                     unsigned long long* __restrict__ acc, int* __restrict__ cnt) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nc + ne) return;
+    const int4 c = contact_at(vquad, nc, quad, i);
+    V3 X[4], q[4], d[4];
+    unsigned still = 0;
     for (int k = 0; k < 4; k++) {
-        if (P[k].w == 0.0f) continue;
-        float sc = 1.0f;
-        if (k == 0 && face_static) sc = 2.0f;
-        if (k > 0 && P[0].w == 0.0f) sc = 2.0f;
-        for (int a = 0; a < 3; a++)
-            atomicAdd(&acc[3 * (size_t)id[k] + a], (unsigned long long)to_fixed((qb[k][a] - qa[k][a]) * sc));
-        atomicAdd(&cnt[id[k]], 1);
+        const float4 P = p[corner(c, k)];
+        X[k] = v3(x[corner(c, k)]);
+        q[k] = v3(P);
+        if (P.w == 0.0f) still |= 1u << k;
+    }
+    if (!(i < nc ? vf_fix(vf_front(X), q, th, min_n2, d) : ee_fix(X, q, th, d))) return;
+    for (int k = 0; k < 4; k++) {
+        if (still >> k & 1) continue;
+        const float sc = fix_scale(i < nc, still, k);
+        const size_t v = corner(c, k);
+        atomicAdd(&acc[3 * v], (unsigned long long)to_fixed(d[k].x * sc));
+        atomicAdd(&acc[3 * v + 1], (unsigned long long)to_fixed(d[k].y * sc));
+        atomicAdd(&acc[3 * v + 2], (unsigned long long)to_fixed(d[k].z * sc));
+        atomicAdd(&cnt[v], 1);
     }
 }
 
-__global__ __launch_bounds__(256) void k_resolve_apply(const unsigned long long* __restrict__ acc,
-                                                       const int* __restrict__ cnt, float4* __restrict__ p, int nv) {
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nv || !cnt[v]) return;
+// Applies the mean fix of every vertex that a contact touches and clears its
+// sums for the next pass.  A vertex of several contacts is applied by the
+// thread that takes its count.
+__global__ __launch_bounds__(256) void k_resolve_apply(const int4* __restrict__ vquad, int nc,
+                                                       const int4* __restrict__ quad, int ne,
+                                                       unsigned long long* __restrict__ acc, int* __restrict__ cnt,
+                                                       float4* __restrict__ p) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= 4 * (nc + ne)) return;
+    const int v = corner(contact_at(vquad, nc, quad, i >> 2), i & 3);
+    const int n = atomicExch(&cnt[v], 0);
+    if (!n) return;
     float4 q = p[v];
-    double c = (double)cnt[v];
-    q.x = q.x + (float)((double)(long long)acc[3 * (size_t)v] / 4294967296.0 / c);
-    q.y = q.y + (float)((double)(long long)acc[3 * (size_t)v + 1] / 4294967296.0 / c);
-    q.z = q.z + (float)((double)(long long)acc[3 * (size_t)v + 2] / 4294967296.0 / c);
+    const double c = (double)n;
+    q.x = q.x + mean_fix(atomicExch(&acc[3 * (size_t)v], 0ull), c);
+    q.y = q.y + mean_fix(atomicExch(&acc[3 * (size_t)v + 1], 0ull), c);
+    q.z = q.z + mean_fix(atomicExch(&acc[3 * (size_t)v + 2], 0ull), c);
     p[v] = q;
+}
+
+// Every pass of a few contacts in one workgroup, one contact per thread, with
+// the touched vertices' positions and sums in an LDS table (open addressing by
+// vertex id).  The contacts must have at most `slots` corners.
+// The sums are integers, so this order gives the bits of any other.
+constexpr int RESOLVE_BLOCK = 1024, RESOLVE_SLOTS = 3712, RESOLVE_SLOT_BYTES = 44;
+
+__device__ __forceinline__ int resolve_slot(int* __restrict__ key, int slots, int v) {
+    int s = (int)__umulhi((unsigned)v * 0x9E3779B1u, (unsigned)slots);
+    for (;;) {  // ends: there are no more distinct vertices than slots
+        const int old = atomicCAS(&key[s], -1, v);
+        if (old == -1 || old == v) return s;
+        s = s + 1 == slots ? 0 : s + 1;
+    }
+}
+
+__global__ __launch_bounds__(RESOLVE_BLOCK) void k_resolve_few(const int4* __restrict__ vquad, int nc,
+                                                               const int4* __restrict__ quad, int ne,
+                                                               const float4* __restrict__ x, float4* __restrict__ p,
+                                                               float th, float min_n2, int passes, int slots) {
+    extern __shared__ unsigned long long lds_sums[];
+    unsigned long long* sum = lds_sums;                       // 3 per slot
+    float* at = reinterpret_cast<float*>(sum + 3 * slots);    // 3 per slot
+    int* count = reinterpret_cast<int*>(at + 3 * slots);
+    int* key = count + slots;
+    const int i = threadIdx.x;
+    const bool mine = i < nc + ne;
+    const int4 c = mine ? contact_at(vquad, nc, quad, i) : make_int4(0, 0, 0, 0);
+    for (int s = threadIdx.x; s < slots; s += blockDim.x) {
+        sum[3 * s] = sum[3 * s + 1] = sum[3 * s + 2] = 0;
+        count[s] = 0;
+        key[s] = -1;
+    }
+    V3 X[4];
+    float4 P[4];
+    unsigned still = 0;
+    if (mine)
+        for (int k = 0; k < 4; k++) {
+            P[k] = p[corner(c, k)];
+            X[k] = v3(x[corner(c, k)]);
+            if (P[k].w == 0.0f) still |= 1u << k;
+        }
+    __syncthreads();
+    int slot[4] = {0, 0, 0, 0};
+    bool front = false;
+    if (mine) {
+        front = vf_front(X);
+        for (int k = 0; k < 4; k++) {
+            slot[k] = resolve_slot(key, slots, corner(c, k));
+            at[3 * slot[k]] = P[k].x;
+            at[3 * slot[k] + 1] = P[k].y;
+            at[3 * slot[k] + 2] = P[k].z;
+        }
+    }
+    __syncthreads();
+    for (int ps = 0; ps < passes; ps++) {
+        V3 q[4], d[4];
+        if (mine)
+            for (int k = 0; k < 4; k++) q[k] = V3{at[3 * slot[k]], at[3 * slot[k] + 1], at[3 * slot[k] + 2]};
+        if (mine && (i < nc ? vf_fix(front, q, th, min_n2, d) : ee_fix(X, q, th, d)))
+            for (int k = 0; k < 4; k++) {
+                if (still >> k & 1) continue;
+                const float sc = fix_scale(i < nc, still, k);
+                atomicAdd(&sum[3 * slot[k]], (unsigned long long)to_fixed(d[k].x * sc));
+                atomicAdd(&sum[3 * slot[k] + 1], (unsigned long long)to_fixed(d[k].y * sc));
+                atomicAdd(&sum[3 * slot[k] + 2], (unsigned long long)to_fixed(d[k].z * sc));
+                atomicAdd(&count[slot[k]], 1);
+            }
+        __syncthreads();
+        for (int s = threadIdx.x; s < slots; s += blockDim.x) {
+            const int n = count[s];
+            if (!n) continue;
+            const double cn = (double)n;
+            for (int a = 0; a < 3; a++) {
+                at[3 * s + a] = at[3 * s + a] + mean_fix(sum[3 * s + a], cn);
+                sum[3 * s + a] = 0;
+            }
+            count[s] = 0;
+        }
+        __syncthreads();
+    }
+    // w was not changed; a static vertex has no sum and its position is the one read
+    for (int s = threadIdx.x; s < slots; s += blockDim.x) {
+        const int v = key[s];
+        if (v < 0) continue;
+        p[v].x = at[3 * s];
+        p[v].y = at[3 * s + 1];
+        p[v].z = at[3 * s + 2];
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -972,14 +1307,12 @@ void Broadphase::build(hipStream_t s, const HashCfg& g, const float4* p, const i
     grow(keys, std::max(1, nt));
     grow(ids, std::max(1, nt));
     grow(raw, std::max(1, nt));
-    grow(tcell, std::max(1, nt));
     grow(k2, std::max(1, nt));
     grow(v2, std::max(1, nt));
     grow(hist, radix_hist_ints(nt));
     grow(cstart, std::max(1, g.ncells));
     grow(cend, std::max(1, g.ncells));
-    if (nt > 0) hipLaunchKernelGGL(k_tri_keys, dim3(blocks(nt)), dim3(256), 0, s, g, p, tris, nt, keys.ptr, ids.ptr, raw.ptr,
-                                  tcell.ptr);
+    if (nt > 0) hipLaunchKernelGGL(k_tri_keys, dim3(blocks(nt)), dim3(256), 0, s, g, p, tris, nt, keys.ptr, ids.ptr, raw.ptr);
     int bits = 1;
     while (bits < 32 && ((1ll << bits) < (long long)g.ncells + 1)) bits++;
     radix_sort_pairs(s, keys.ptr, ids.ptr, k2.ptr, v2.ptr, nt, bits, hist.ptr);
@@ -989,73 +1322,18 @@ void Broadphase::build(hipStream_t s, const HashCfg& g, const float4* p, const i
     PBD_HIP(hipGetLastError());
 }
 
-long long Broadphase::pairs(hipStream_t s, const float4* p, const int* tris, int nv) {
-    npairs = 0;
-    if (nt <= 0) return 0;
-    grow(cnt, nt + 1);
-    grow(off, nt + 1);
-    grow(scan_tmp, (nt + SB) / SB + 2);
-    hipLaunchKernelGGL(k_pairs<0>, dim3(blocks(nt)), dim3(256), 0, s, cfg, p, tris, nt, raw.ptr, ids.ptr, cstart.ptr,
-                       cend.ptr, tcell.ptr, cnt.ptr, (uint32_t*)nullptr, (uint32_t*)nullptr);
-    PBD_HIP(hipMemsetAsync(cnt.ptr + nt, 0, sizeof(int), s));
-    device_scan(s, cnt.ptr, off.ptr, nt + 1, scan_tmp.ptr);
-    int total = 0;
-    PBD_HIP(hipMemcpyAsync(&total, off.ptr + nt, sizeof(int), hipMemcpyDeviceToHost, s));
-    PBD_HIP(hipStreamSynchronize(s));
-    PBD_CHECK(total >= 0, PBD_ERR_LIMIT, "candidate pair count overflows int32");
-    st_dets++;
-    st_tris += nt;
-    st_entries += nt;
-    st_raw += total;
-    if (total == 0) return 0;
-    grow(pv, total);
-    grow(pf, total);
-    grow(t1, total);
-    grow(t2, total);
-    grow(flag, total + 1);
-    grow(pos, total + 1);
-    hipLaunchKernelGGL(k_pairs<1>, dim3(blocks(nt)), dim3(256), 0, s, cfg, p, tris, nt, raw.ptr, ids.ptr, cstart.ptr,
-                       cend.ptr, tcell.ptr, off.ptr, pv.ptr, pf.ptr);
-    return unique_pairs(s, total, nt, nv);
-}
-
-// Sorts the `total` raw pairs in pv/pf by (v, f) and keeps one of each in uv/uf.
-long long Broadphase::unique_pairs(hipStream_t s, int total, int nt, int nv) {
-    long long uniq = unique_into(s, total, nt, nv, uv, uf);
-    npairs = uniq;
-    st_pairs += uniq;
-    return uniq;
-}
-
-// Sorts the `total` raw pairs in pv/pf by (pv, pf) (pv < nv, pf < nt) and
-// writes one of each to oa/ob.
-long long Broadphase::unique_into(hipStream_t s, int total, int nt, int nv, DBuf<uint32_t>& oa, DBuf<uint32_t>& ob) {
-    // sort by (v, f): by f first, then stably by v
-    int fb = 1, vb = 1;
-    while (fb < 31 && (1ll << fb) < nt) fb++;
-    while (vb < 31 && (1ll << vb) < nv) vb++;
-    grow(hist2, radix_hist_ints(total));
-    radix_sort_pairs(s, pf.ptr, pv.ptr, t1.ptr, t2.ptr, total, fb, hist2.ptr);
-    radix_sort_pairs(s, pv.ptr, pf.ptr, t1.ptr, t2.ptr, total, vb, hist2.ptr);
-    hipLaunchKernelGGL(k_unique_flags, dim3(blocks(total)), dim3(256), 0, s, pv.ptr, pf.ptr, total, flag.ptr);
-    PBD_HIP(hipMemsetAsync(flag.ptr + total, 0, sizeof(int), s));
-    grow(scan_tmp, (total + 1 + SB) / SB + 2);
-    device_scan(s, flag.ptr, pos.ptr, total + 1, scan_tmp.ptr);
-    int uniq = 0;
-    PBD_HIP(hipMemcpyAsync(&uniq, pos.ptr + total, sizeof(int), hipMemcpyDeviceToHost, s));
-    PBD_HIP(hipStreamSynchronize(s));
-    grow(oa, std::max(1, uniq));
-    grow(ob, std::max(1, uniq));
-    hipLaunchKernelGGL(k_compact_pairs, dim3(blocks(total)), dim3(256), 0, s, pv.ptr, pf.ptr, total, flag.ptr, pos.ptr,
-                       oa.ptr, ob.ptr);
-    PBD_HIP(hipGetLastError());
-    return uniq;
-}
-
 void Broadphase::set_edges(hipStream_t s, const std::vector<int>& te, const std::vector<int2>& ed) {
     tedge.upload(te, s);
     edges.upload(ed, s);
     nedges = (int)ed.size();
+    // edge -> triangles (CSR)
+    std::vector<int> eo(ed.size() + 1, 0), et(te.size());
+    for (int e : te) eo[(size_t)e + 1]++;
+    for (size_t e = 0; e < ed.size(); e++) eo[e + 1] += eo[e];
+    std::vector<int> at(eo.begin(), eo.end() - 1);
+    for (size_t i = 0; i < te.size(); i++) et[at[te[i]]++] = (int)(i / 3);
+    etoff.upload(eo, s);
+    etri.upload(et, s);
     // vertex -> neighbour CSR from the edges (each edge once, both directions)
     int nv = 0;
     for (const int2& e : ed) nv = std::max(nv, e.y + 1);
@@ -1075,183 +1353,335 @@ void Broadphase::set_edges(hipStream_t s, const std::vector<int>& te, const std:
     PBD_HIP(hipStreamSynchronize(s));
 }
 
-// Edge-edge candidates from the cell table of the last build() (see k_ee_pairs).
-long long Broadphase::ee_pairs(hipStream_t s, const float4* p, const int* tris) {
-    ee_npairs = 0;
-    ee_ncontacts = 0;
-    if (nt <= 0) return 0;
-    PBD_CHECK(tedge.n >= (size_t)3 * nt, PBD_ERR_STATE, "internal: edge table does not match the triangles");
-    grow(cnt, nt + 1);
-    grow(off, nt + 1);
-    grow(scan_tmp, (nt + SB) / SB + 2);
-    hipLaunchKernelGGL(k_ee_pairs<0>, dim3(blocks(nt)), dim3(256), 0, s, cfg, p, tris, nt, raw.ptr, ids.ptr,
-                       cstart.ptr, cend.ptr, tcell.ptr, tedge.ptr, edges.ptr, voff.ptr, vnbr.ptr, cnt.ptr,
-                       (uint32_t*)nullptr, (uint32_t*)nullptr);
-    PBD_HIP(hipMemsetAsync(cnt.ptr + nt, 0, sizeof(int), s));
-    device_scan(s, cnt.ptr, off.ptr, nt + 1, scan_tmp.ptr);
-    int total = 0;
-    PBD_HIP(hipMemcpyAsync(&total, off.ptr + nt, sizeof(int), hipMemcpyDeviceToHost, s));
-    PBD_HIP(hipStreamSynchronize(s));
-    PBD_CHECK(total >= 0, PBD_ERR_LIMIT, "edge-edge candidate count overflows int32");
-    st_ee_raw += total;
-    if (total == 0) return 0;
-    grow(pv, total);
-    grow(pf, total);
-    grow(t1, total);
-    grow(t2, total);
-    grow(flag, total + 1);
-    grow(pos, total + 1);
-    hipLaunchKernelGGL(k_ee_pairs<1>, dim3(blocks(nt)), dim3(256), 0, s, cfg, p, tris, nt, raw.ptr, ids.ptr,
-                       cstart.ptr, cend.ptr, tcell.ptr, tedge.ptr, edges.ptr, voff.ptr, vnbr.ptr, off.ptr, pv.ptr,
-                       pf.ptr);
-    ee_npairs = unique_into(s, total, nedges, nedges, eua, eub);
-    st_ee_pairs += ee_npairs;
-    return ee_npairs;
-}
-
-long long Broadphase::ee_narrow(hipStream_t s, const float4* x, const float4* p, float th) {
-    ee_ncontacts = 0;
-    if (ee_npairs <= 0) return 0;
-    long long n = ee_npairs;
-    grow(flag, n + 1);
-    grow(pos, n + 1);
-    grow(ctmp_t, n);
-    grow(ctmp_n, 3 * n);
-    grow(ctmp_w, 4 * n);
-    hipLaunchKernelGGL(k_narrow_ee, dim3(blocks(n)), dim3(256), 0, s, eua.ptr, eub.ptr, (int)n, edges.ptr, x, p, th,
-                       flag.ptr, ctmp_t.ptr, ctmp_n.ptr, ctmp_w.ptr);
-    PBD_HIP(hipMemsetAsync(flag.ptr + n, 0, sizeof(int), s));
-    grow(scan_tmp, (n + 1 + SB) / SB + 2);
-    device_scan(s, flag.ptr, pos.ptr, (int)n + 1, scan_tmp.ptr);
-    int nc = 0;
-    PBD_HIP(hipMemcpyAsync(&nc, pos.ptr + n, sizeof(int), hipMemcpyDeviceToHost, s));
-    PBD_HIP(hipStreamSynchronize(s));
-    grow(ecq, std::max(1, nc));
-    grow(ect, std::max(1, nc));
-    grow(ecn, 3 * std::max(1, nc));
-    grow(ecw, 4 * std::max(1, nc));
-    hipLaunchKernelGGL(k_compact_ee, dim3(blocks(n)), dim3(256), 0, s, (int)n, flag.ptr, pos.ptr, eua.ptr, eub.ptr,
-                       edges.ptr, ctmp_t.ptr, ctmp_n.ptr, ctmp_w.ptr, ecq.ptr, ect.ptr, ecn.ptr, ecw.ptr);
+// Vertex -> triangles of a triangle list.
+void Broadphase::set_triangles(hipStream_t s, const int* tris, int nt_, int nv) {
+    grow(vtoff, (size_t)nv + 1);
+    grow(vtri, (size_t)3 * std::max(1, nt_));
+    grow(cnt, (size_t)nv + 1);
+    grow(scan_tmp, ((size_t)nv + 1) / SB + 2);
+    PBD_HIP(hipMemsetAsync(cnt.ptr, 0, sizeof(int) * ((size_t)nv + 1), s));
+    if (nt_ > 0) hipLaunchKernelGGL(k_vt_count, dim3(blocks(3ll * nt_)), dim3(256), 0, s, tris, 3 * nt_, cnt.ptr);
+    device_scan(s, cnt.ptr, vtoff.ptr, nv + 1, scan_tmp.ptr);
+    if (nt_ > 0)
+        hipLaunchKernelGGL(k_vt_fill, dim3(blocks(3ll * nt_)), dim3(256), 0, s, tris, 3 * nt_, vtoff.ptr, cnt.ptr, vtri.ptr);
     PBD_HIP(hipGetLastError());
-    ee_ncontacts = nc;
-    st_ee_contacts += nc;
-    return nc;
 }
 
-long long Broadphase::pairs_swept(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris,
-                                  int nt_, int nv, float th) {
+// Table sizes for n entries: at least one slot per entry.
+static int table_bits_for(long long n) {
+    int b = 10;
+    while (b < 26 && (1ll << b) < n) b++;
+    return b;
+}
+
+// The cleared table (slot counts after the counters, one fill for both).
+void Broadphase::clear_table(hipStream_t s, int bits) {
+    table_bits = bits;
+    const size_t head = sizeof(DetectCounts) / sizeof(int);
+    static_assert(sizeof(DetectCounts) % 16 == 0, "counters before the table");
+    grow(table, head + (1ull << bits));
+    grow(place, 1ull << bits);
+    PBD_HIP(hipMemsetAsync(table.ptr, 0, sizeof(int) * (head + (1ull << bits)), s));
+}
+static DetectCounts* counts_of(const DBuf<int>& table) { return reinterpret_cast<DetectCounts*>(table.ptr); }
+static int* slots_of(const DBuf<int>& table) { return table.ptr + sizeof(DetectCounts) / sizeof(int); }
+
+// The counters as of this point of the stream (waits).
+DetectCounts Broadphase::read_counts(hipStream_t s) {
+    if (!counts_h) PBD_HIP(hipHostMalloc(&counts_h, sizeof(DetectCounts), hipHostMallocDefault));
+    PBD_HIP(hipMemcpyAsync(counts_h, table.ptr, sizeof(DetectCounts), hipMemcpyDeviceToHost, s));
+    PBD_HIP(hipStreamSynchronize(s));
+    return *reinterpret_cast<DetectCounts*>(counts_h);
+}
+
+// Workgroups of the candidate visits: each wave takes two vertices (edges) at
+// a time, and enough waves to fill the GPU take them in turn.
+static int visit_blocks(int n) { return std::max(1, std::min(2048, (n + 2 * VISIT_WAVES - 1) / (2 * VISIT_WAVES))); }
+
+// The centroid-cell table of the faces at p.
+void Broadphase::cells(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt_,
+                       float th) {
+    cfg = g;
+    nt = nt_;
+    grow(tcell, std::max(1, nt));
+    grow(raw_rank, std::max(1, nt));
+    grow(rec, (size_t)std::max(1, nt) * sizeof(FaceRec));
+    grow(ent, 2 * (size_t)std::max(1, nt));
+    const int bits = table_bits_for(2ll * nt);
+    clear_table(s, bits);
+    const unsigned mask = (1u << table_bits) - 1;
+    hipLaunchKernelGGL(k_face_cells, dim3(blocks(nt)), dim3(256), 0, s, g, x, p, tris, nt, th, mask, slots_of(table),
+                       tcell.ptr, raw_rank.ptr, (FaceRec*)rec.ptr);
+    hipLaunchKernelGGL(k_slot_places<true>, dim3((1 << table_bits) / 256), dim3(256), 0, s, slots_of(table),
+                       1 << table_bits, place.ptr, &counts_of(table)->entries);
+    hipLaunchKernelGGL(k_cell_fill, dim3(blocks(nt)), dim3(256), 0, s, nt, tcell.ptr, raw_rank.ptr, slots_of(table),
+                       place.ptr, (int4*)ent.ptr);
+    PBD_HIP(hipGetLastError());
+}
+
+void Broadphase::check_pairs(unsigned long long n, const char* what) {
+    PBD_CHECK(n < (1ull << 31), PBD_ERR_LIMIT, std::string(what) + " overflows int32");
+}
+
+// Vertex-face contacts of one substep: candidates, narrowphase.  Lists that
+// turn out too short are grown and the detection runs again.
+void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, const float4* x, const float4* p,
+                        const int* tris, int nt_, int nv, float th, bool store) {
+    npairs = ncontacts = 0;
+    listed = false;
+    cfg = g;
+    nt = nt_;
+    by_box = swept != nullptr;
+    if (nt <= 0 || nv <= 0) return;
+    grow(near_, std::max<size_t>(1 << 16, (size_t)nv));
+    grow_contacts(std::max<size_t>(1 << 14, (size_t)nv / 4), store);
+    DetectCounts c{};
+    for (;;) {
+        const unsigned near_cap = (unsigned)std::min<size_t>(near_.n, 0x7fffffff), cap = (unsigned)vquad.n;
+        if (swept) {
+            swept_table(s, g, *swept, x, p, tris, th);
+            hipLaunchKernelGGL(k_swept_candidates, dim3(visit_blocks(nv)), dim3(64 * VISIT_WAVES), 0, s, g, *swept, x, p,
+                               nv, vtoff.ptr, slots_of(table), place.ptr, (1u << table_bits) - 1, ent.ptr,
+                               (int)std::min<size_t>(ent.n, 0x7fffffff), (const FaceRec*)rec.ptr, large.ptr,
+                               counts_of(table), near_.ptr, near_cap);
+        } else {
+            cells(s, g, x, p, tris, nt, th);
+            hipLaunchKernelGGL(k_vf_candidates<false>, dim3(visit_blocks(nv)), dim3(64 * VISIT_WAVES), 0, s, g, x, p, nv,
+                               vtoff.ptr, vtri.ptr, tcell.ptr, slots_of(table), place.ptr, (1u << table_bits) - 1,
+                               (const int4*)ent.ptr, (const FaceRec*)rec.ptr, counts_of(table), near_.ptr,
+                               near_cap);
+        }
+        auto* narrow = store ? k_narrow<true> : k_narrow<false>;
+        hipLaunchKernelGGL(narrow, dim3(1024), dim3(256), 0, s, near_.ptr, near_cap, tris, x, p, th,
+                           counts_of(table), cap, vquad.ptr, vf.ptr, rt.ptr, rn.ptr, rw.ptr);
+        PBD_HIP(hipGetLastError());
+        c = read_counts(s);
+        if (swept) {
+            PBD_CHECK(!c.face_span, PBD_ERR_LIMIT, "a face's swept box spans more than 4096 cells: use a larger cell");
+            PBD_CHECK(c.entries < (1u << 31), PBD_ERR_LIMIT, "swept-box cell entries overflow int32");
+        }
+        const bool table_short = swept && c.entries > ent.n;
+        if (!table_short) {
+            PBD_CHECK(!c.vertex_span, PBD_ERR_LIMIT,
+                      "a vertex's swept box spans more than 4096 cells: use a larger cell");
+            check_pairs(c.pairs, "candidate pair count");
+        }
+        if (!table_short && c.near <= near_cap && c.contacts <= cap) break;
+        if (table_short) grow(ent, (size_t)c.entries + c.entries / 4);
+        else if (c.near > near_cap) grow(near_, (size_t)c.near + c.near / 4);
+        else grow_contacts((size_t)c.contacts + c.contacts / 4, store);
+    }
+    npairs = (long long)c.pairs;
+    ncontacts = c.contacts;
+    st_dets++;
+    st_tris += nt;
+    st_entries += swept ? (long long)c.entries : (long long)nt;
+    st_raw += npairs;
+    st_pairs += npairs;
+    st_contacts += ncontacts;
+    if (store) order_contacts(s, vf, nullptr, ncontacts, nv, ckey, nullptr);
+}
+
+void Broadphase::swept_table(hipStream_t s, const HashCfg& g, const HashCfg& gi, const float4* x, const float4* p,
+                             const int* tris, float th) {
+    grow(rec, (size_t)nt * sizeof(FaceRec));
+    grow(sw_cell, 2 * (size_t)nt);
+    grow(large, nt);
+    grow(ent, 12 * (size_t)nt);
+    clear_table(s, table_bits_for(2ll * nt));
+    const unsigned mask = (1u << table_bits) - 1;
+    hipLaunchKernelGGL(k_swept_faces, dim3(blocks(nt)), dim3(256), 0, s, g, gi, x, p, tris, nt, th, mask,
+                       slots_of(table), sw_cell.ptr, (FaceRec*)rec.ptr, large.ptr, counts_of(table));
+    hipLaunchKernelGGL(k_slot_places<false>, dim3((1 << table_bits) / 256), dim3(256), 0, s, slots_of(table),
+                       1 << table_bits, place.ptr, &counts_of(table)->entries);
+    hipLaunchKernelGGL(k_swept_fill, dim3(blocks(nt)), dim3(256), 0, s, nt, sw_cell.ptr, mask, place.ptr,
+                       ent.ptr, (int)std::min<size_t>(ent.n, 0x7fffffff));
+    PBD_HIP(hipGetLastError());
+}
+
+void Broadphase::grow_contacts(size_t n, bool store) {
+    grow(vquad, n);
+    if (!store) return;
+    grow(vf, vquad.n);
+    grow(rt, vquad.n);
+    grow(rn, 3 * vquad.n);
+    grow(rw, 4 * vquad.n);
+}
+
+// The n contacts of rt / rn / rw with ids `key` in ascending order of their
+// ids, into okey (and oquad) / ct / cn / cw or their edge-edge counterparts.
+void Broadphase::order_contacts(hipStream_t s, const DBuf<int2>& key, const int4* quad, long long n, int nfirst,
+                                DBuf<int2>& okey, DBuf<int4>* oquad) {
+    const size_t m = (size_t)std::max(1ll, n);
+    DBuf<float>& ot = oquad ? ect : ct;
+    DBuf<float>& on = oquad ? ecn : cn;
+    DBuf<double>& ow = oquad ? ecw : cw;
+    grow(okey, m);
+    grow(ot, m);
+    grow(on, 3 * m);
+    grow(ow, 4 * m);
+    if (oquad) grow(*oquad, m);
+    if (n <= 0) return;
+    grow(cnt, (size_t)nfirst + 1);
+    grow(off, (size_t)nfirst + 1);
+    grow(idx, m);
+    grow(scan_tmp, ((size_t)nfirst + 1) / SB + 2);
+    PBD_HIP(hipMemsetAsync(cnt.ptr, 0, sizeof(int) * ((size_t)nfirst + 1), s));
+    hipLaunchKernelGGL(k_first_count, dim3(blocks(n)), dim3(256), 0, s, key.ptr, (int)n, cnt.ptr);
+    device_scan(s, cnt.ptr, off.ptr, nfirst + 1, scan_tmp.ptr);
+    hipLaunchKernelGGL(k_first_deal, dim3(blocks(n)), dim3(256), 0, s, key.ptr, (int)n, off.ptr, cnt.ptr, idx.ptr);
+    hipLaunchKernelGGL(k_contact_order, dim3(blocks(n)), dim3(256), 0, s, key.ptr, (int)n, off.ptr, idx.ptr, rt.ptr,
+                       rn.ptr, rw.ptr, quad, okey.ptr, ot.ptr, on.ptr, ow.ptr, oquad ? oquad->ptr : nullptr);
+    PBD_HIP(hipGetLastError());
+}
+
+// Sorts the n pairs in `near` by (first, second) into hi / lo.
+void Broadphase::sort_near(hipStream_t s, long long n, int nfirst, int nsecond, DBuf<uint32_t>& hi, DBuf<uint32_t>& lo) {
+    grow(hi, (size_t)std::max(1ll, n));
+    grow(lo, (size_t)std::max(1ll, n));
+    if (n <= 0) return;
+    grow(k2, n);
+    grow(v2, n);
+    grow(hist, radix_hist_ints(n));
+    hipLaunchKernelGGL(k_unzip, dim3(blocks(n)), dim3(256), 0, s, near_.ptr, (int)n, hi.ptr, lo.ptr);
+    int fb = 1, vb = 1;
+    while (fb < 31 && (1ll << fb) < nsecond) fb++;
+    while (vb < 31 && (1ll << vb) < nfirst) vb++;
+    radix_sort_pairs(s, lo.ptr, hi.ptr, k2.ptr, v2.ptr, (int)n, fb, hist.ptr);
+    radix_sort_pairs(s, hi.ptr, lo.ptr, k2.ptr, v2.ptr, (int)n, vb, hist.ptr);
+}
+
+// The centroid-cell candidates of the faces at p as sorted lists uv / uf.
+long long Broadphase::list_pairs(hipStream_t s, const HashCfg& g, const float4* p, const int* tris, int nt_, int nv) {
     cfg = g;
     nt = nt_;
     npairs = 0;
     if (nt <= 0 || nv <= 0) return 0;
-    grow(sw_box, 2 * (size_t)nt);
-    grow(sw_cell, 2 * (size_t)nt);
-    grow(cnt, (size_t)std::max(nt, nv) + 1);
-    grow(off, (size_t)std::max(nt, nv) + 1);
-    grow(sw_err, 2);
-    grow(sw_vin, nv);
-    grow(scan_tmp, (std::max(nt, nv) + SB) / SB + 2);
-    PBD_HIP(hipMemsetAsync(sw_err.ptr, 0, 2 * sizeof(int), s));
-    hipLaunchKernelGGL(k_swept_faces, dim3(blocks(nt)), dim3(256), 0, s, g, x, p, tris, nt, 4.0f * th, sw_box.ptr,
-                       sw_cell.ptr, cnt.ptr, sw_err.ptr);
-    PBD_HIP(hipMemsetAsync(cnt.ptr + nt, 0, sizeof(int), s));
-    device_scan(s, cnt.ptr, off.ptr, nt + 1, scan_tmp.ptr);
-    int hst[3] = {0, 0, 0};
-    PBD_HIP(hipMemcpyAsync(&hst[0], off.ptr + nt, sizeof(int), hipMemcpyDeviceToHost, s));
-    PBD_HIP(hipMemcpyAsync(&hst[1], sw_err.ptr, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
-    PBD_HIP(hipStreamSynchronize(s));
-    PBD_CHECK(!hst[1], PBD_ERR_LIMIT, "a face's swept box spans more than 4096 cells: use a larger cell");
-    const int ne = hst[0];
-    PBD_CHECK(ne >= 0, PBD_ERR_LIMIT, "swept-box cell entries overflow int32");
-    grow(keys, ne);
-    grow(ids, ne);
-    grow(k2, ne);
-    grow(v2, ne);
-    grow(hist, radix_hist_ints(ne));
-    grow(cstart, std::max(1, g.ncells));
-    grow(cend, std::max(1, g.ncells));
-    hipLaunchKernelGGL(k_swept_entries, dim3(blocks(nt)), dim3(256), 0, s, g, nt, sw_cell.ptr, off.ptr, keys.ptr, ids.ptr);
-    int bits = 1;
-    while (bits < 32 && ((1ll << bits) < (long long)g.ncells + 1)) bits++;
-    radix_sort_pairs(s, keys.ptr, ids.ptr, k2.ptr, v2.ptr, ne, bits, hist.ptr);
-    hipLaunchKernelGGL(k_fill_i32, dim3(blocks(g.ncells)), dim3(256), 0, s, cstart.ptr, g.ncells, -1);
-    hipLaunchKernelGGL(k_fill_i32, dim3(blocks(g.ncells)), dim3(256), 0, s, cend.ptr, g.ncells, -1);
-    if (ne > 0) hipLaunchKernelGGL(k_cell_ranges, dim3(blocks(ne)), dim3(256), 0, s, keys.ptr, ne, cstart.ptr, cend.ptr);
-    PBD_HIP(hipMemsetAsync(sw_vin.ptr, 0, sizeof(int) * (size_t)nv, s));
-    hipLaunchKernelGGL(k_mark_vertices, dim3(blocks(3ll * nt)), dim3(256), 0, s, tris, nt, sw_vin.ptr);
-    hipLaunchKernelGGL(k_swept_pairs<0>, dim3(blocks(nv)), dim3(256), 0, s, g, x, p, sw_vin.ptr, nv, tris, sw_box.ptr,
-                       sw_cell.ptr, ids.ptr, cstart.ptr, cend.ptr, cnt.ptr, (uint32_t*)nullptr, (uint32_t*)nullptr,
-                       sw_err.ptr);
-    PBD_HIP(hipMemsetAsync(cnt.ptr + nv, 0, sizeof(int), s));
-    device_scan(s, cnt.ptr, off.ptr, nv + 1, scan_tmp.ptr);
-    PBD_HIP(hipMemcpyAsync(&hst[0], off.ptr + nv, sizeof(int), hipMemcpyDeviceToHost, s));
-    PBD_HIP(hipMemcpyAsync(&hst[1], sw_err.ptr, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
-    PBD_HIP(hipStreamSynchronize(s));
-    PBD_CHECK(!hst[2], PBD_ERR_LIMIT, "a vertex's swept box spans more than 4096 cells: use a larger cell");
-    const int total = hst[0];
-    PBD_CHECK(total >= 0, PBD_ERR_LIMIT, "candidate pair count overflows int32");
-    st_dets++;
-    st_tris += nt;
-    st_entries += ne;
-    st_raw += total;
-    if (total == 0) return 0;
-    grow(pv, total);
-    grow(pf, total);
-    grow(t1, total);
-    grow(t2, total);
-    grow(flag, total + 1);
-    grow(pos, total + 1);
-    hipLaunchKernelGGL(k_swept_pairs<1>, dim3(blocks(nv)), dim3(256), 0, s, g, x, p, sw_vin.ptr, nv, tris, sw_box.ptr,
-                       sw_cell.ptr, ids.ptr, cstart.ptr, cend.ptr, off.ptr, pv.ptr, pf.ptr, sw_err.ptr);
-    return unique_pairs(s, total, nt, nv);
+    if (!near_.n) grow(near_, 1 << 16);
+    for (;;) {
+        const unsigned cap = (unsigned)std::min<size_t>(near_.n, 0x7fffffff);
+        cells(s, g, p, p, tris, nt, 0.0f);
+        hipLaunchKernelGGL(k_vf_candidates<true>, dim3(visit_blocks(nv)), dim3(64 * VISIT_WAVES), 0, s, g, p, p, nv,
+                           vtoff.ptr, vtri.ptr, tcell.ptr, slots_of(table), place.ptr, (1u << table_bits) - 1,
+                           (const int4*)ent.ptr, (const FaceRec*)rec.ptr, counts_of(table), near_.ptr, cap);
+        const DetectCounts c = read_counts(s);
+        check_pairs(c.near, "candidate pair count");
+        npairs = c.near;
+        if (c.near <= cap) break;
+        grow(near_, c.near);
+    }
+    sort_near(s, npairs, nv, nt, uv, uf);
+    return npairs;
 }
 
-long long Broadphase::narrow(hipStream_t s, const float4* x, const float4* p, const int* tris, float th) {
-    ncontacts = 0;
-    if (npairs <= 0) return 0;
-    long long n = npairs;
-    grow(flag, n + 1);
-    grow(pos, n + 1);
-    grow(ctmp_t, n);
-    grow(ctmp_n, 3 * n);
-    grow(ctmp_w, 4 * n);
-    hipLaunchKernelGGL(k_narrow, dim3(blocks(n)), dim3(256), 0, s, uv.ptr, uf.ptr, (int)n, tris, x, p, th, flag.ptr,
-                       ctmp_t.ptr, ctmp_n.ptr, ctmp_w.ptr);
-    PBD_HIP(hipMemsetAsync(flag.ptr + n, 0, sizeof(int), s));
-    grow(scan_tmp, (n + 1 + SB) / SB + 2);
-    device_scan(s, flag.ptr, pos.ptr, (int)n + 1, scan_tmp.ptr);
-    int nc = 0;
-    PBD_HIP(hipMemcpyAsync(&nc, pos.ptr + n, sizeof(int), hipMemcpyDeviceToHost, s));
-    PBD_HIP(hipStreamSynchronize(s));
-    grow(cv, std::max(1, nc));
-    grow(cf, std::max(1, nc));
-    grow(ct, std::max(1, nc));
-    grow(cn, 3 * std::max(1, nc));
-    grow(cw, 4 * std::max(1, nc));
-    hipLaunchKernelGGL(k_compact_contacts, dim3(blocks(n)), dim3(256), 0, s, (int)n, flag.ptr, pos.ptr, uv.ptr, uf.ptr,
-                       ctmp_t.ptr, ctmp_n.ptr, ctmp_w.ptr, cv.ptr, cf.ptr, ct.ptr, cn.ptr, cw.ptr);
+// The candidates of the last detect() as sorted lists uv / uf, made when first
+// asked for.
+void Broadphase::list_detected(hipStream_t s, const float4* p, const int* tris, int nv) {
+    if (listed) return;
+    const long long n = npairs;
+    if (by_box) sort_near(s, n, nv, nt, uv, uf);
+    else if (n > 0) list_pairs(s, cfg, p, tris, nt, nv);
+    npairs = n;
+    listed = true;
+}
+
+void Broadphase::ee_candidates(hipStream_t s, bool list, float th, unsigned cap) {
+    auto* k = list ? k_ee_candidates<true> : k_ee_candidates<false>;
+    hipLaunchKernelGGL(k, dim3(visit_blocks(nedges)), dim3(64 * VISIT_WAVES), 0, s, cfg, nedges, edges.ptr, etoff.ptr,
+                       etri.ptr, tedge.ptr, voff.ptr, vnbr.ptr, tcell.ptr, slots_of(table), place.ptr,
+                       (1u << table_bits) - 1, (const int4*)ent.ptr, (const FaceRec*)rec.ptr, ebox.ptr, th,
+                       counts_of(table), near_.ptr, cap);
     PBD_HIP(hipGetLastError());
-    ncontacts = nc;
-    st_contacts += nc;
-    return nc;
 }
 
-void Broadphase::resolve(hipStream_t s, const float4* x, float4* p, const int* tris, int nv, float th, int passes,
-                         float min_n2) {
-    if (ncontacts <= 0 && ee_ncontacts <= 0) return;
-    st_resolved += (ncontacts + ee_ncontacts) * passes;
-    grow(acc, (size_t)3 * nv);
-    grow(vcnt, nv);
+// Edge-edge contacts at p.
+void Broadphase::detect_ee(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt_,
+                           float th, bool store) {
+    ee_npairs = ee_ncontacts = 0;
+    ee_listed = false;
+    if (nt_ <= 0 || nedges <= 0) return;
+    PBD_CHECK(tedge.n >= (size_t)3 * nt_, PBD_ERR_STATE, "internal: edge table does not match the triangles");
+    grow(near_, std::max<size_t>(1 << 16, (size_t)nedges));
+    grow(ebox, 2 * (size_t)nedges);
+    auto grow_ee = [&](size_t n) {
+        grow(quad, n);
+        if (!store) return;
+        grow(eab, quad.n);
+        grow(rt, quad.n);
+        grow(rn, 3 * quad.n);
+        grow(rw, 4 * quad.n);
+    };
+    grow_ee(std::max<size_t>(1 << 14, (size_t)nedges / 8));
+    DetectCounts c{};
+    for (;;) {
+        const unsigned near_cap = (unsigned)std::min<size_t>(near_.n, 0x7fffffff), cap = (unsigned)quad.n;
+        cells(s, g, x, p, tris, nt_, th);
+        hipLaunchKernelGGL(k_edge_boxes, dim3(blocks(nedges)), dim3(256), 0, s, edges.ptr, nedges, x, p, ebox.ptr);
+        ee_candidates(s, false, th, near_cap);
+        auto* narrow = store ? k_narrow_ee<true> : k_narrow_ee<false>;
+        hipLaunchKernelGGL(narrow, dim3(1024), dim3(256), 0, s, near_.ptr, near_cap, edges.ptr, x, p, th,
+                           counts_of(table), cap, eab.ptr, quad.ptr, rt.ptr, rn.ptr, rw.ptr);
+        PBD_HIP(hipGetLastError());
+        c = read_counts(s);
+        check_pairs(c.ee_pairs, "edge-edge candidate count");
+        if (c.ee_near <= near_cap && c.ee_contacts <= cap) break;
+        if (c.ee_near > near_cap) grow(near_, (size_t)c.ee_near + c.ee_near / 4);
+        else grow_ee((size_t)c.ee_contacts + c.ee_contacts / 4);
+    }
+    ee_npairs = (long long)c.ee_pairs;
+    ee_ncontacts = c.ee_contacts;
+    st_ee_raw += ee_npairs;
+    st_ee_pairs += ee_npairs;
+    st_ee_contacts += ee_ncontacts;
+    if (store) order_contacts(s, eab, quad.ptr, ee_ncontacts, nedges, eabs, &ecq);
+}
+
+// The edge-edge candidates of the last detect_ee() as sorted lists eua / eub.
+void Broadphase::list_detected_ee(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris,
+                                  float th) {
+    if (ee_listed) return;
+    if (ee_npairs > 0) {
+        grow(near_, (size_t)ee_npairs);
+        cells(s, g, x, p, tris, nt, th);
+        ee_candidates(s, true, th, (unsigned)std::min<size_t>(near_.n, 0x7fffffff));
+        sort_near(s, ee_npairs, nedges, nedges, eua, eub);
+    }
+    ee_listed = true;
+}
+
+void Broadphase::resolve(hipStream_t s, const float4* x, float4* p, int nv, float th, int passes, float min_n2) {
+    const int nc = (int)ncontacts, ne = (int)ee_ncontacts, n = nc + ne;
+    if (n <= 0 || passes <= 0) return;
+    st_resolved += (long long)n * passes;
+    if (!few_slots) {
+        // the LDS one workgroup may take on this device, asked for once
+        few_slots = RESOLVE_SLOTS;
+        if (hipFuncSetAttribute((const void*)k_resolve_few, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                RESOLVE_SLOTS * RESOLVE_SLOT_BYTES) != hipSuccess) {
+            (void)hipGetLastError();  // the refusal is handled by the smaller limit
+            few_slots = 65536 / RESOLVE_SLOT_BYTES;
+        }
+    }
+    if (4 * n <= few_slots) {
+        // up to half of the slots stay free
+        const int slots = std::min(few_slots, std::max(64, 8 * n)), lds = slots * RESOLVE_SLOT_BYTES;
+        hipLaunchKernelGGL(k_resolve_few, dim3(1), dim3((n + 63) / 64 * 64), lds, s, vquad.ptr, nc, quad.ptr, ne, x, p,
+                           th, min_n2, passes, slots);
+        PBD_HIP(hipGetLastError());
+        return;
+    }
+    if (acc.n < (size_t)3 * nv || vcnt.n < (size_t)nv) {
+        // the passes leave both cleared
+        grow(acc, (size_t)3 * nv);
+        grow(vcnt, nv);
+        PBD_HIP(hipMemsetAsync(acc.ptr, 0, sizeof(unsigned long long) * acc.n, s));
+        PBD_HIP(hipMemsetAsync(vcnt.ptr, 0, sizeof(int) * vcnt.n, s));
+    }
     for (int ps = 0; ps < passes; ps++) {
-        PBD_HIP(hipMemsetAsync(acc.ptr, 0, sizeof(unsigned long long) * 3 * (size_t)nv, s));
-        PBD_HIP(hipMemsetAsync(vcnt.ptr, 0, sizeof(int) * (size_t)nv, s));
-        if (ncontacts > 0)
-            hipLaunchKernelGGL(k_resolve_acc, dim3(blocks(ncontacts)), dim3(256), 0, s, cv.ptr, cf.ptr, (int)ncontacts,
-                               tris, x, (const float4*)p, th, min_n2, acc.ptr, vcnt.ptr);
-        if (ee_ncontacts > 0)
-            hipLaunchKernelGGL(k_resolve_ee_acc, dim3(blocks(ee_ncontacts)), dim3(256), 0, s, ecq.ptr,
-                               (int)ee_ncontacts, x, (const float4*)p, th, acc.ptr, vcnt.ptr);
-        hipLaunchKernelGGL(k_resolve_apply, dim3(blocks(nv)), dim3(256), 0, s, acc.ptr, vcnt.ptr, p, nv);
+        hipLaunchKernelGGL(k_resolve_acc, dim3(blocks(n)), dim3(256), 0, s, vquad.ptr, nc, quad.ptr, ne, x,
+                           (const float4*)p, th, min_n2, acc.ptr, vcnt.ptr);
+        hipLaunchKernelGGL(k_resolve_apply, dim3(blocks(4ll * n)), dim3(256), 0, s, vquad.ptr, nc, quad.ptr, ne,
+                           acc.ptr, vcnt.ptr, p);
     }
     PBD_HIP(hipGetLastError());
 }

@@ -233,52 +233,98 @@ struct HashCfg {
     int ncells;          // dense: size product; hashed: 1 << table_bits
 };
 
+// Counters of a detection, cleared with the table's slot counts.
+struct DetectCounts {
+    unsigned long long pairs, ee_pairs;  // distinct candidates
+    unsigned near, ee_near;              // candidates that go to the narrowphase
+    unsigned contacts, ee_contacts;
+    unsigned entries, large;             // table entries; faces kept out of the table
+    unsigned face_span, vertex_span;     // 1: a box over the allowed cells of the caller's grid
+};
+
 // Broadphase + CCD working set (device buffers reused between calls).
 struct Broadphase {
+    Broadphase() = default;
+    ~Broadphase() {
+        if (counts_h) (void)hipHostFree(counts_h);
+    }
     HashCfg cfg{};
     int nt = 0;
     long long npairs = 0, ncontacts = 0;
-    DBuf<uint32_t> keys, ids, k2, v2, pv, pf, t1, t2, uv, uf;
-    DBuf<int> raw, hist, hist2, cstart, cend, cnt, off, scan_tmp, flag, pos, cv, cf, vcnt;
-    DBuf<float> ctmp_t, ctmp_n, ct, cn;
-    DBuf<double> ctmp_w, cw;
-    DBuf<unsigned long long> acc;
-    DBuf<int4> tcell;    // centroid cell coordinates per triangle
-    DBuf<float4> sw_box; // swept-box broadphase: face boxes (lo, hi)
-    DBuf<int4> sw_cell;  // and their cell ranges (lo, hi)
-    DBuf<int> sw_err, sw_vin;
-    // running counts (host values the drivers read anyway): detections,
-    // triangles, cell entries, raw pairs, distinct pairs, contacts
+    // sorted table of build()
+    DBuf<uint32_t> keys, ids, k2, v2;
+    DBuf<int> raw, hist, cstart, cend;
+    DBuf<int> cnt, off, scan_tmp, idx;
+    // vertex -> triangles of the current triangle list
+    DBuf<int> vtoff, vtri;
+    // unsorted table of the faces by cell: counters and slot counts, slot
+    // places, entries (int4 cell and face, or int2 face and cell code), face
+    // records, per-face cells
+    DBuf<int> table, place, raw_rank, large;
+    int table_bits = 0;
+    DBuf<int2> ent;
+    DBuf<unsigned char> rec;
+    DBuf<int4> tcell, sw_cell;
+    void* counts_h = nullptr;  // pinned
+    // candidates that go to the narrowphase; contacts in any order (the
+    // response reads these) and, when asked for, in ascending order
+    DBuf<int2> near_;
+    DBuf<int4> vquad;
+    DBuf<int2> vf, ckey;
+    DBuf<float> rt, rn, ct, cn;
+    DBuf<double> rw, cw;
+    // sorted candidate lists, made when first asked for
+    DBuf<uint32_t> uv, uf, eua, eub;
+    bool by_box = false, listed = false, ee_listed = false;
+    DBuf<unsigned long long> acc;  // response sums and counts, zero between passes
+    DBuf<int> vcnt;
+    int few_slots = 0;  // LDS table of the response in one workgroup, 0 before the first use
+    // running counts: detections, triangles, cell entries, raw pairs, distinct pairs, contacts
     long long st_dets = 0, st_tris = 0, st_entries = 0, st_raw = 0, st_pairs = 0, st_contacts = 0, st_resolved = 0;
-    // edge-edge: per-triangle edge ids, edge endpoints (lower, higher), the
-    // distinct candidate edge pairs and the contacts (a0, a1, b0, b1)
-    DBuf<int> tedge;
+    // edge-edge: per-triangle edge ids, edge endpoints (lower, higher), edge ->
+    // triangles, vertex -> mesh neighbours, swept boxes, and the contacts
+    // (a0, a1, b0, b1) with their edge ids
+    DBuf<int> tedge, etoff, etri, voff, vnbr;
     DBuf<int2> edges;
-    DBuf<int> voff, vnbr;  // vertex -> mesh neighbours (CSR) of the edge table
     int nedges = 0;
-    DBuf<uint32_t> eua, eub;
-    DBuf<int4> ecq;
+    DBuf<float4> ebox;
+    DBuf<int4> quad, ecq;
+    DBuf<int2> eab, eabs;
     DBuf<float> ect, ecn;
     DBuf<double> ecw;
     long long ee_npairs = 0, ee_ncontacts = 0;
     long long st_ee_raw = 0, st_ee_pairs = 0, st_ee_contacts = 0;
     void build(hipStream_t s, const HashCfg& g, const float4* p, const int* tris, int nt);
-    long long pairs(hipStream_t s, const float4* p, const int* tris, int nv);
-    long long unique_pairs(hipStream_t s, int total, int nt, int nv);
-    long long unique_into(hipStream_t s, int total, int nt, int nv, DBuf<uint32_t>& oa, DBuf<uint32_t>& ob);
+    void set_triangles(hipStream_t s, const int* tris, int nt, int nv);
     void set_edges(hipStream_t s, const std::vector<int>& tedge, const std::vector<int2>& edges);
-    // after build(): edge-edge candidates and contacts (contacts resolved with
-    // the vertex-face ones by resolve())
-    long long ee_pairs(hipStream_t s, const float4* p, const int* tris);
-    long long ee_narrow(hipStream_t s, const float4* x, const float4* p, float th);
-    // Swept-box candidate set (replaces build + pairs); x = start of substep.
-    long long pairs_swept(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt,
-                          int nv, float th);
-    long long narrow(hipStream_t s, const float4* x, const float4* p, const int* tris, float th);
+    // Vertex-face contacts (after set_triangles): candidates by the centroid
+    // cells of g, or by swept boxes (swept: the table's own grid, whose ranges
+    // contain g's).  store: contacts with time, normal and weights, in order.
+    void detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, const float4* x, const float4* p, const int* tris,
+                int nt, int nv, float th, bool store);
+    // Edge-edge contacts (after set_edges) by the centroid cells of g; the
+    // response takes them with the vertex-face ones.
+    void detect_ee(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt, float th,
+                   bool store);
+    long long list_pairs(hipStream_t s, const HashCfg& g, const float4* p, const int* tris, int nt, int nv);
+    void list_detected(hipStream_t s, const float4* p, const int* tris, int nv);
+    void list_detected_ee(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, float th);
     // min_n2: faces with |(p2 - p1) x (p3 - p1)|^2 <= min_n2 are skipped
     // (VFResolveTest's degenerate-face test, 1e-6 in the reference)
-    void resolve(hipStream_t s, const float4* x, float4* p, const int* tris, int nv, float th, int passes,
-                 float min_n2);
+    void resolve(hipStream_t s, const float4* x, float4* p, int nv, float th, int passes, float min_n2);
+
+private:
+    void clear_table(hipStream_t s, int bits);
+    DetectCounts read_counts(hipStream_t s);
+    void cells(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt, float th);
+    void swept_table(hipStream_t s, const HashCfg& g, const HashCfg& gi, const float4* x, const float4* p,
+                     const int* tris, float th);
+    void check_pairs(unsigned long long n, const char* what);
+    void grow_contacts(size_t n, bool store);
+    void order_contacts(hipStream_t s, const DBuf<int2>& key, const int4* quad, long long n, int nfirst,
+                        DBuf<int2>& okey, DBuf<int4>* oquad);
+    void sort_near(hipStream_t s, long long n, int nfirst, int nsecond, DBuf<uint32_t>& hi, DBuf<uint32_t>& lo);
+    void ee_candidates(hipStream_t s, bool list, float th, unsigned cap);
 };
 void device_scan(hipStream_t s, const int* in, int* out, int n, int* tmp);
 // Broadphase build into caller device arrays with no allocation: the sort's
