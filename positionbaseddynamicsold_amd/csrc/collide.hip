@@ -16,6 +16,7 @@
 //   fixed point (integer sums are order independent, so the result does not
 //   depend on atomic ordering) and applied as the mean fix per vertex.
 // Paths are relative to PositionBasedDynamicsCUDA/PositionBasedDynamicsCUDA/.
+#include <climits>
 #include <mutex>
 
 #include "pbd_internal.hpp"
@@ -182,7 +183,7 @@ __global__ __launch_bounds__(256) void k_cell_ranges(const uint32_t* __restrict_
 // visited once per vertex, so a pair comes up once.  The form this replaces
 // made the pairs of every triangle (3.7 times as many on a folded 256 x 256
 // cloth), stored them, sorted them twice and compacted them: 2.6 ms per
-// detection there against 0.6 ms for the table, the visit and the narrowphase.
+// detection there against 0.3 ms for the table, the visit and the narrowphase.
 // ---------------------------------------------------------------------------
 constexpr int SWEPT_MAX_CELLS = 4096;  // cells of the caller's grid one box may span
 constexpr int ENTRY_MAX_CELLS = 64;    // cells of the table's own grid a face is entered in
@@ -225,15 +226,18 @@ __device__ __forceinline__ unsigned cell_slot(int x, int y, int z, unsigned mask
     return h & mask;
 }
 
-// A face as the visits read it, one cache line: its widened swept box, its
-// vertices, and whether the box may rule pairs out (face_cullable).
+// A face as the visits read it, half a cache line: its widened swept box, its
+// vertices, whether the box may rule pairs out (face_cullable), and its cell.
+// Centroid-cell tables hold the records themselves (one entry per face), so
+// that a visit reads a slot's faces side by side and nothing else of them.
 struct alignas(64) FaceRec {
     float lo[3];
     int v0;
     float hi[3];
     int v1;
-    int v2, cull;
-    int pad[6];
+    int v2, cull, face;
+    int cx, cy, cz;
+    int pad[2];
 };
 
 // Whether a vertex outside the face's swept box widened by 6 thickness cannot
@@ -256,10 +260,12 @@ __device__ __forceinline__ bool face_cullable(const float4* X, const float4* P, 
     return area >= 0.05f * (longest * longest) && th >= 4e-3f * longest;  // false for NaN
 }
 
-__device__ __forceinline__ void write_face(FaceRec* __restrict__ rec, int f, const float4* __restrict__ x,
-                                           const float4* __restrict__ p, const int* __restrict__ tris, float th,
-                                           float margin) {
+__device__ __forceinline__ FaceRec face_record(int f, const float4* __restrict__ x, const float4* __restrict__ p,
+                                               const int* __restrict__ tris, float th, float margin) {
     FaceRec r;
+    r.face = f;
+    r.cx = r.cy = r.cz = 0;
+    r.pad[0] = r.pad[1] = 0;
     r.v0 = tris[3 * f];
     r.v1 = tris[3 * f + 1];
     r.v2 = tris[3 * f + 2];
@@ -272,7 +278,7 @@ __device__ __forceinline__ void write_face(FaceRec* __restrict__ rec, int f, con
         r.hi[k] = widen_hi(b.hi[k], margin);
     }
     r.cull = face_cullable(X, P, th) ? 1 : 0;
-    rec[f] = r;
+    return r;
 }
 
 __device__ __forceinline__ bool box_misses(const SweptBox& b, const FaceRec& r) {
@@ -280,12 +286,12 @@ __device__ __forceinline__ bool box_misses(const SweptBox& b, const FaceRec& r) 
            r.lo[2] > b.hi[2];
 }
 
-// Centroid cells: the face's cell and place in its slot, and its record.
-// tcell[t] = (cell, slot), slot -1 outside a dense grid.
-__global__ __launch_bounds__(256) void k_face_cells(HashCfg g, const float4* __restrict__ x, const float4* __restrict__ p,
-                                                    const int* __restrict__ tris, int nt, float th, unsigned mask,
+// Centroid cells: the face's cell and place in its slot.  tcell[t] = (cell,
+// slot), slot -1 outside a dense grid.
+__global__ __launch_bounds__(256) void k_face_cells(HashCfg g, const float4* __restrict__ p,
+                                                    const int* __restrict__ tris, int nt, unsigned mask,
                                                     int* __restrict__ cnt, int4* __restrict__ tcell,
-                                                    int* __restrict__ rank, FaceRec* __restrict__ rec) {
+                                                    int* __restrict__ rank) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nt) return;
     int gp[3];
@@ -294,37 +300,63 @@ __global__ __launch_bounds__(256) void k_face_cells(HashCfg g, const float4* __r
     const unsigned slot = cell_slot(gp[0], gp[1], gp[2], mask);
     tcell[t] = make_int4(gp[0], gp[1], gp[2], in ? (int)slot : -1);
     rank[t] = in ? atomicAdd(&cnt[slot], 1) : 0;
-    write_face(rec, t, x, p, tris, th, 6.0f * th);
 }
 
 __global__ __launch_bounds__(256) void k_cell_fill(int nt, const int4* __restrict__ tcell, const int* __restrict__ rank,
                                                    const int* __restrict__ cnt, const int* __restrict__ end,
-                                                   int4* __restrict__ ent) {
+                                                   const float4* __restrict__ x, const float4* __restrict__ p,
+                                                   const int* __restrict__ tris, float th, FaceRec* __restrict__ ent) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nt) return;
     const int4 c = tcell[t];
-    if (c.w >= 0) ent[end[c.w] - cnt[c.w] + rank[t]] = make_int4(c.x, c.y, c.z, t);
+    if (c.w < 0) return;
+    FaceRec r = face_record(t, x, p, tris, th, 6.0f * th);
+    r.cx = c.x;
+    r.cy = c.y;
+    r.cz = c.z;
+    ent[end[c.w] - cnt[c.w] + rank[t]] = r;
 }
 
 // Each slot's place among the entries: end[slot] (END) or its start.  Order
-// among workgroups is whatever their atomics make it.
+// among workgroups is whatever their atomics make it: few workgroups, since
+// these are served one after the other (2^19 slots: 26 us with one per 256
+// slots).
+constexpr int PLACE_SLOTS = 4096;
 template <bool END>
-__global__ __launch_bounds__(256) void k_slot_places(const int* __restrict__ cnt, int nslots, int* __restrict__ place,
+__global__ __launch_bounds__(256) void k_slot_places(const int4* __restrict__ cnt, int nslots, int4* __restrict__ place,
                                                      unsigned* __restrict__ total) {
+    constexpr int Q = PLACE_SLOTS / 1024;
     __shared__ int wave[4], base;
-    const int i = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int c = i < nslots ? cnt[i] : 0;
-    int run = c;
-    for (int off = 1; off < 64; off <<= 1) {
-        const int o = __shfl_up(run, off);
-        if (lane >= off) run += o;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int i0 = blockIdx.x * (PLACE_SLOTS / 4) + wv * (Q * 64) + lane;  // in quads of slots
+    int4 c[Q];
+    int before[Q], run = 0;
+    for (int k = 0; k < Q; k++) {
+        c[k] = 4 * (i0 + 64 * k) < nslots ? cnt[i0 + 64 * k] : make_int4(0, 0, 0, 0);
+        int sum = c[k].x + c[k].y + c[k].z + c[k].w;
+        const int mine = sum;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(sum, off);
+            if (lane >= off) sum += o;
+        }
+        before[k] = run + sum - mine;
+        run += __shfl(sum, 63);
     }
-    if (lane == 63) wave[wv] = run;
+    if (lane == 0) wave[wv] = run;
     __syncthreads();
     if (threadIdx.x == 0) base = (int)atomicAdd(total, (unsigned)(wave[0] + wave[1] + wave[2] + wave[3]));
     __syncthreads();
-    for (int w = 0; w < wv; w++) run += wave[w];
-    if (i < nslots) place[i] = base + (END ? run : run - c);
+    int at = base;
+    for (int w = 0; w < wv; w++) at += wave[w];
+    for (int k = 0; k < Q; k++) {
+        if (4 * (i0 + 64 * k) >= nslots) break;
+        int4 r;
+        r.x = at + before[k] + (END ? c[k].x : 0);
+        r.y = r.x + (END ? c[k].y : c[k].x);
+        r.z = r.y + (END ? c[k].z : c[k].y);
+        r.w = r.z + (END ? c[k].w : c[k].z);
+        place[i0 + 64 * k] = r;
+    }
 }
 
 // Swept boxes: face records (their margin defines the candidate set), the
@@ -338,7 +370,7 @@ __global__ __launch_bounds__(256) void k_swept_faces(HashCfg g, HashCfg gi, cons
                                                      int* __restrict__ large, DetectCounts* __restrict__ c) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= nt) return;
-    write_face(rec, f, x, p, tris, th, 4.0f * th);
+    rec[f] = face_record(f, x, p, tris, th, 4.0f * th);
     const FaceRec& r = rec[f];
     int lo[3], hi[3];
     long long span = 1, n = 1;
@@ -383,23 +415,34 @@ __global__ __launch_bounds__(256) void k_swept_fill(int nt, const int4* __restri
             }
 }
 
-// Pairs a wave has found, appended to the global list in runs: one atomic on
-// the list's length per run.
+// Pairs a wave has found, appended in runs to the global list.  Atomics on one
+// address are served one after the other, about 13 ns each here, so one length
+// for the whole list bounded every visit (26,000 runs on the folded 256 x 256
+// cloth: 340 of 371 us).  The list is NEAR_BUCKETS lists of `cap` pairs, each
+// with its length in a line of its own; a wave goes on to another one after
+// every run, so that the lists fill evenly whatever wave finds the most.
 constexpr int VISIT_WAVES = 4, VISIT_BUF = 256;
 struct PairSink {
     int2* buf;       // this wave's LDS
     int n;           // wave-uniform
-    unsigned* len;
+    int bucket;      // wave-uniform
+    DetectCounts* c;
     int2* out;
-    unsigned cap;
+    unsigned cap;    // per bucket
     __device__ __forceinline__ void flush() {
         const int lane = threadIdx.x & 63;
         unsigned at = 0;
-        if (lane == 0) at = atomicAdd(len, (unsigned)n);
+        if (lane == 0) at = atomicAdd(&c->bucket[bucket].near, (unsigned)n);
         at = __shfl(at, 0);
+        int2* o = out + (size_t)bucket * cap;
         for (int i = lane; i < n; i += 64)
-            if (at + i < cap) out[at + i] = buf[i];
+            if (at + i < cap) o[at + i] = buf[i];
         n = 0;
+        bucket = (bucket + 17) % NEAR_BUCKETS;
+    }
+    __device__ __forceinline__ void count(int pairs) {
+        for (int off = 32; off > 0; off >>= 1) pairs += __shfl_xor(pairs, off);
+        if ((threadIdx.x & 63) == 0 && pairs) atomicAdd(&c->bucket[bucket].pairs, (unsigned long long)pairs);
     }
     // Called by all lanes of the wave.
     __device__ __forceinline__ void add(bool hit, int a, int b) {
@@ -447,54 +490,120 @@ __device__ __forceinline__ int3 around(int4 c, int l) {
     return make_int3(c.x + l % 3 - 1, c.y + l / 3 % 3 - 1, c.z + l / 9 - 1);
 }
 
-__device__ __forceinline__ unsigned long long wave_total(int n) {
-    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
-    return (unsigned long long)n;
-}
+// The cells around a group's own triangles, each once, 32 at a time: the cells
+// of the box of their cells that lie around one of them.  A group with more
+// than 32 triangles or a box of more than BOX_CELLS cells takes the 27 cells
+// around one triangle after the other instead, without those that lie around
+// an earlier one.
+constexpr int BOX_CELLS = 256;
+struct CellRounds {
+    int4* own;  // in LDS, 32 per group
+    const int* list;
+    const int4* tcell;
+    int deg, rounds;
+    bool boxed;
+    int3 lo, w;
+    // Called by all lanes of the wave, after the lanes are done with `own`.
+    __device__ __forceinline__ void start(int4* own_, const int* list_, int deg_, const int4* tcell_) {
+        own = own_;
+        list = list_;
+        tcell = tcell_;
+        deg = deg_;
+        const int l = threadIdx.x & 31;
+        const int4 c = l < deg ? tcell[list[l]] : make_int4(0, 0, 0, -1);
+        own[l] = c;
+        int m[3] = {c.w >= 0 ? c.x : INT_MAX, c.w >= 0 ? c.y : INT_MAX, c.w >= 0 ? c.z : INT_MAX};
+        int M[3] = {c.w >= 0 ? c.x : INT_MIN, c.w >= 0 ? c.y : INT_MIN, c.w >= 0 ? c.z : INT_MIN};
+        for (int off = 16; off > 0; off >>= 1)
+            for (int k = 0; k < 3; k++) {
+                m[k] = min(m[k], __shfl_xor(m[k], off, 32));
+                M[k] = max(M[k], __shfl_xor(M[k], off, 32));
+            }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        lo = make_int3(m[0] - 1, m[1] - 1, m[2] - 1);
+        long long n = 0;
+        if (M[0] >= m[0]) {
+            long long s[3];
+            for (int k = 0; k < 3; k++) s[k] = min((long long)M[k] - m[k] + 3, (long long)BOX_CELLS + 1);
+            w = make_int3((int)s[0], (int)s[1], (int)s[2]);
+            n = s[0] * s[1] * s[2];
+        }
+        boxed = deg <= 32 && n <= BOX_CELLS;
+        rounds = boxed ? ((int)n + 31) / 32 : deg;
+    }
+    // This lane's cell of round r, if it has one.
+    __device__ __forceinline__ bool cell(const HashCfg& g, int r, int3* q) const {
+        const int l = threadIdx.x & 31;
+        *q = make_int3(0, 0, 0);
+        if (r >= rounds) return false;
+        if (boxed) {
+            const int i = 32 * r + l, z = i / (w.x * w.y), y = (i - z * (w.x * w.y)) / w.x;
+            *q = make_int3(lo.x + i - (z * w.y + y) * w.x, lo.y + y, lo.z + z);
+            if (z >= w.z) return false;
+            bool in = false;
+            for (int j = 0; j < deg; j++) in |= near_cell(own[j], q->x, q->y, q->z);
+            return in && cell_key(g, q->x, q->y, q->z) >= 0;
+        }
+        const int4 tc = tcell[list[r]];
+        *q = around(tc, l);
+        if (tc.w < 0 || l >= 27) return false;
+        for (int j = 0; j < r; j++)
+            if (near_cell(tcell[list[j]], q->x, q->y, q->z)) return false;
+        return cell_key(g, q->x, q->y, q->z) >= 0;
+    }
+    // Whether c is a cell around one of the triangles.
+    __device__ __forceinline__ bool meets(int4 c) const {
+        if (c.w < 0) return false;
+        bool in = false;
+        if (boxed)
+            for (int j = 0; j < deg; j++) in |= near_cell(own[j], c.x, c.y, c.z);
+        else
+            for (int j = 0; j < deg && !in; j++) in = near_cell(tcell[list[j]], c.x, c.y, c.z);
+        return in;
+    }
+};
 
-// Vertex-face candidates by centroid cells.  Group = 32 lanes = one vertex:
-// for its triangles in turn, lanes 0..26 take the cells around the triangle's
-// own that no earlier triangle of the vertex has covered.  All candidates are
-// counted; listed are all of them (LIST) or those that no box rules out.
+// Vertex-face candidates by centroid cells.  Group = 32 lanes = one vertex.
+// All candidates are counted; listed are all of them (LIST) or those that no
+// box rules out.
 template <bool LIST>
 __global__ __launch_bounds__(64 * VISIT_WAVES) void k_vf_candidates(
     HashCfg g, const float4* __restrict__ x, const float4* __restrict__ p, int nv, const int* __restrict__ vtoff,
     const int* __restrict__ vtri, const int4* __restrict__ tcell, const int* __restrict__ cnt,
-    const int* __restrict__ end, unsigned mask, const int4* __restrict__ ent, const FaceRec* __restrict__ rec,
-    DetectCounts* __restrict__ c, int2* __restrict__ out, unsigned cap) {
+    const int* __restrict__ end, unsigned mask, const FaceRec* __restrict__ ent, DetectCounts* __restrict__ c,
+    int2* __restrict__ out, unsigned cap) {
     __shared__ int2 buf[VISIT_WAVES][VISIT_BUF];
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 31;
-    PairSink sink{buf[wv], 0, &c->near, out, cap};
+    __shared__ int4 own[VISIT_WAVES][2][32];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    PairSink sink{buf[wv], 0, (int)((blockIdx.x * VISIT_WAVES + wv) % NEAR_BUCKETS), c, out, cap};
     int pairs = 0;
     const int stride = (int)gridDim.x * VISIT_WAVES * 2;
     for (int v0 = ((int)blockIdx.x * VISIT_WAVES + wv) * 2; v0 < nv; v0 += stride) {
         const int v = v0 + (lane >> 5), at = min(v, nv - 1);
         const int o = vtoff[at], deg = v < nv ? vtoff[at + 1] - o : 0;
         const SweptBox b = vertex_box(x[at], p[at]);
-        const int most = max(deg, __shfl_xor(deg, 32));
-        for (int i = 0; i < most; i++) {
-            const int4 tc = i < deg ? tcell[vtri[o + i]] : make_int4(0, 0, 0, -1);
-            const int3 q = around(tc, l);
-            bool mine = tc.w >= 0 && l < 27 && cell_key(g, q.x, q.y, q.z) >= 0;
-            for (int j = 0; j < min(i, deg); j++)
-                if (near_cell(tcell[vtri[o + j]], q.x, q.y, q.z)) mine = false;
+        CellRounds cells;
+        __builtin_amdgcn_wave_barrier();  // the vertex before is done with `own`
+        cells.start(own[wv][lane >> 5], vtri + o, deg, tcell);
+        const int rounds = max(cells.rounds, __shfl_xor(cells.rounds, 32));
+        for (int r = 0; r < rounds; r++) {
+            int3 q;
+            const bool mine = cells.cell(g, r, &q);
             if (!__any(mine)) continue;
             const unsigned slot = cell_slot(q.x, q.y, q.z, mask);
             const int n = mine ? cnt[slot] : 0;
             visit_runs(n ? end[slot] - n : 0, n, [&](int e, int from) {
+                const int3 fq = make_int3(__shfl(q.x, from, 32), __shfl(q.y, from, 32), __shfl(q.z, from, 32));
                 bool hit = false;
                 int f = 0;
                 if (e >= 0) {
-                    const int4 ec = ent[e];
-                    const int3 fq = around(tc, from);
-                    f = ec.w;
+                    const FaceRec rec = ent[e];
+                    f = rec.face;
                     // a slot may hold other cells' faces too
-                    if (ec.x == fq.x && ec.y == fq.y && ec.z == fq.z) {
-                        const FaceRec r = rec[f];
-                        if (v != r.v0 && v != r.v1 && v != r.v2) {
-                            pairs++;
-                            hit = LIST || !(r.cull && box_misses(b, r));
-                        }
+                    if (rec.cx == fq.x && rec.cy == fq.y && rec.cz == fq.z && v != rec.v0 && v != rec.v1 && v != rec.v2) {
+                        pairs++;
+                        hit = LIST || !(rec.cull && box_misses(b, rec));
                     }
                 }
                 sink.add(hit, v, f);
@@ -502,8 +611,7 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_vf_candidates(
         }
     }
     if (sink.n) sink.flush();
-    const unsigned long long t = wave_total(pairs);
-    if (!LIST && lane == 0 && t) atomicAdd(&c->pairs, t);
+    if (!LIST) sink.count(pairs);
 }
 
 // Vertex-face candidates by swept boxes: the faces entered in the cells of the
@@ -516,7 +624,7 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_swept_candidates(
     DetectCounts* __restrict__ c, int2* __restrict__ out, unsigned cap) {
     __shared__ int2 buf[VISIT_WAVES][VISIT_BUF];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 31;
-    PairSink sink{buf[wv], 0, &c->near, out, cap};
+    PairSink sink{buf[wv], 0, (int)((blockIdx.x * VISIT_WAVES + wv) % NEAR_BUCKETS), c, out, cap};
     const int nlarge = (int)c->large;
     int pairs = 0;
     const int stride = (int)gridDim.x * VISIT_WAVES * 2;
@@ -567,31 +675,82 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_swept_candidates(
         for (int i = 0; i < nlarge; i += 32) test(used && !over && i + l < nlarge, large[min(i + l, nlarge - 1)]);
     }
     if (sink.n) sink.flush();
-    const unsigned long long t = wave_total(pairs);
-    if (lane == 0 && t) atomicAdd(&c->pairs, t);
-}
-
-// Swept boxes of the edges (four points each), not widened.
-__global__ __launch_bounds__(256) void k_edge_boxes(const int2* __restrict__ edges, int ne, const float4* __restrict__ x,
-                                                    const float4* __restrict__ p, float4* __restrict__ box) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= ne) return;
-    const int2 v = edges[e];
-    SweptBox b = vertex_box(x[v.x], p[v.x]);
-    box_add(b, x[v.y]);
-    box_add(b, p[v.y]);
-    box[2 * e] = make_float4(b.lo[0], b.lo[1], b.lo[2], 0.0f);
-    box[2 * e + 1] = make_float4(b.hi[0], b.hi[1], b.hi[2], 0.0f);
+    sink.count(pairs);
 }
 
 // Whether two edges' swept boxes lie further apart along an axis than the
 // contact distance and the rounding of the closest points' coordinates: every
 // point the narrowphase measures between lies in the boxes, so such a pair is
 // no contact.  (False for NaN.)
-__device__ __forceinline__ bool edges_apart(float4 alo, float4 ahi, float4 blo, float4 bhi, float th) {
+__device__ __forceinline__ bool edges_apart(const SweptBox& a, const SweptBox& b, float th) {
     auto apart = [&](float hi, float lo) { return lo - hi > 2.0f * th + 2e-6f * (fabsf(lo) + fabsf(hi)); };
-    return apart(ahi.x, blo.x) || apart(bhi.x, alo.x) || apart(ahi.y, blo.y) || apart(bhi.y, alo.y) ||
-           apart(ahi.z, blo.z) || apart(bhi.z, alo.z);
+    bool r = false;
+    for (int k = 0; k < 3; k++) r = r || apart(a.hi[k], b.lo[k]) || apart(b.hi[k], a.lo[k]);
+    return r;
+}
+
+// An entry of the edge table: an edge in one of the cells of its faces, with
+// its ends and the swept box of the four points, not widened.  `before`: none
+// (0), one (1: the cell o) or several (2) of the edge's other cells come first
+// in the order of its faces.
+struct alignas(64) EdgeRec {
+    int cx, cy, cz, edge;
+    int v0, v1, before, ox;
+    int oy, oz;
+    SweptBox box;
+};
+
+// Calls f(cell, before, other) for every distinct valid cell of e's faces.
+template <class F>
+__device__ __forceinline__ void edge_cells(int e, const int* __restrict__ etoff, const int* __restrict__ etri,
+                                           const int4* __restrict__ tcell, F&& f) {
+    const int o = etoff[e], deg = etoff[e + 1] - o;
+    int4 other = make_int4(0, 0, 0, 0);
+    int distinct = 0;
+    for (int j = 0; j < deg; j++) {
+        const int4 c = tcell[etri[o + j]];
+        bool fresh = c.w >= 0;
+        for (int m = 0; m < j && fresh; m++) {
+            const int4 d = tcell[etri[o + m]];
+            fresh = d.w < 0 || d.x != c.x || d.y != c.y || d.z != c.z;
+        }
+        if (!fresh) continue;
+        f(c, min(distinct, 2), other);
+        if (!distinct++) other = c;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_tri_cells(HashCfg g, const float4* __restrict__ p, const int* __restrict__ tris,
+                                                   int nt, unsigned mask, int4* __restrict__ tcell) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nt) return;
+    int gp[3];
+    tri_cell(g, p, tris, t, gp);
+    const bool in = cell_key(g, gp[0], gp[1], gp[2]) >= 0;
+    tcell[t] = make_int4(gp[0], gp[1], gp[2], in ? (int)cell_slot(gp[0], gp[1], gp[2], mask) : -1);
+}
+
+__global__ __launch_bounds__(256) void k_edge_count(int ne, const int* __restrict__ etoff, const int* __restrict__ etri,
+                                                    const int4* __restrict__ tcell, int* __restrict__ cnt) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < ne) edge_cells(e, etoff, etri, tcell, [&](int4 c, int, int4) { atomicAdd(&cnt[c.w], 1); });
+}
+
+// Each entry takes the next place of its slot, so that place[] ends at the
+// slots' ends.
+__global__ __launch_bounds__(256) void k_edge_fill(int ne, const int2* __restrict__ edges, const int* __restrict__ etoff,
+                                                   const int* __restrict__ etri, const int4* __restrict__ tcell,
+                                                   const float4* __restrict__ x, const float4* __restrict__ p,
+                                                   int* __restrict__ place, EdgeRec* __restrict__ ent) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= ne) return;
+    const int2 v = edges[e];
+    SweptBox b = vertex_box(x[v.x], p[v.x]);
+    box_add(b, x[v.y]);
+    box_add(b, p[v.y]);
+    edge_cells(e, etoff, etri, tcell, [&](int4 c, int before, int4 o) {
+        ent[atomicAdd(&place[c.w], 1)] = EdgeRec{c.x, c.y, c.z, e, v.x, v.y, before, o.x, o.y, o.z, b};
+    });
 }
 
 // Edge-edge candidates (new: the reference declares Contact::EE, CCD_Basic.h:14,
@@ -600,102 +759,95 @@ __device__ __forceinline__ bool edges_apart(float4 alo, float4 ahi, float4 blo, 
 // vertex and has no vertex that is a mesh neighbour of the other edge's (pairs
 // that close in the mesh are material neighbours, not contacts), once, as
 // (lower edge id, higher edge id).  Group = 32 lanes = the lower edge a: the
-// cells around its triangles, each once; a face found there offers its edges b
-// of higher id, and an edge b of several faces counts at the first of them (in
-// the order of b's list) that lies around a's triangles.
+// cells around its triangles, each once; an edge b entered in several of them
+// counts at the first in the order of its faces.
+// Edges have entries of their own, with all that the tests read: visiting the
+// faces' entries instead offered most edges twice and took four dependent
+// gathers to tell (fold of 96 x 96: 151 us against 84).
 constexpr int RING_MAX = 64;
 
 template <bool LIST>
 __global__ __launch_bounds__(64 * VISIT_WAVES) void k_ee_candidates(
     HashCfg g, int ne, const int2* __restrict__ edges, const int* __restrict__ etoff, const int* __restrict__ etri,
-    const int* __restrict__ tedge, const int* __restrict__ voff, const int* __restrict__ vnbr,
-    const int4* __restrict__ tcell, const int* __restrict__ cnt, const int* __restrict__ end, unsigned mask,
-    const int4* __restrict__ ent, const FaceRec* __restrict__ rec, const float4* __restrict__ box, float th,
-    DetectCounts* __restrict__ c, int2* __restrict__ out, unsigned cap) {
+    const int* __restrict__ voff, const int* __restrict__ vnbr, const float4* __restrict__ x,
+    const float4* __restrict__ p, const int4* __restrict__ tcell, const int* __restrict__ cnt,
+    const int* __restrict__ end, unsigned mask, const EdgeRec* __restrict__ ent, float th, DetectCounts* __restrict__ c,
+    int2* __restrict__ out, unsigned cap) {
     __shared__ int2 buf[VISIT_WAVES][VISIT_BUF];
-    __shared__ int ring_s[VISIT_WAVES][2][RING_MAX];
+    __shared__ int4 ring_s[VISIT_WAVES][2][RING_MAX / 4];
+    __shared__ int4 own[VISIT_WAVES][2][32];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 31;
-    int* ring = ring_s[wv][lane >> 5];
-    PairSink sink{buf[wv], 0, &c->ee_near, out, cap};
+    int4* ring = ring_s[wv][lane >> 5];
+    PairSink sink{buf[wv], 0, (int)((blockIdx.x * VISIT_WAVES + wv) % NEAR_BUCKETS), c, out, cap};
     int pairs = 0;
     const int stride = (int)gridDim.x * VISIT_WAVES * 2;
     for (int a0 = ((int)blockIdx.x * VISIT_WAVES + wv) * 2; a0 < ne; a0 += stride) {
         const int a = a0 + (lane >> 5), at = min(a, ne - 1);
         const int2 av = edges[at];
         const int o = etoff[at], deg = a < ne ? etoff[at + 1] - o : 0;
-        const float4 alo = box[2 * at], ahi = box[2 * at + 1];
+        SweptBox abox = vertex_box(x[av.x], p[av.x]);
+        box_add(abox, x[av.y]);
+        box_add(abox, p[av.y]);
         // a's vertices and their mesh neighbours: an edge with a vertex among them is no candidate
         const int r0 = voff[av.x], n0 = voff[av.x + 1] - r0, r1 = voff[av.y], n1 = voff[av.y + 1] - r1;
-        const bool fits = n0 + n1 + 2 <= RING_MAX;
-        __builtin_amdgcn_wave_barrier();  // the round before has read the lists
+        const int quads = (n0 + n1 + 5) / 4;
+        const bool fits = quads <= RING_MAX / 4;
+        __builtin_amdgcn_wave_barrier();  // the edge before is done with the lists
         if (fits)
-            for (int i = l; i < n0 + n1 + 2; i += 32)
-                ring[i] = i == 0 ? av.x : i == 1 ? av.y : i < n0 + 2 ? vnbr[r0 + i - 2] : vnbr[r1 + i - 2 - n0];
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        auto in_ring = [&](int u) {
+            for (int i = l; i < 4 * quads; i += 32)
+                reinterpret_cast<int*>(ring)[i] = i == 0            ? av.x
+                                                  : i == 1          ? av.y
+                                                  : i < n0 + 2      ? vnbr[r0 + i - 2]
+                                                  : i < n0 + n1 + 2 ? vnbr[r1 + i - 2 - n0]
+                                                                    : -1;
+        CellRounds cells;
+        cells.start(own[wv][lane >> 5], etri + o, deg, tcell);
+        auto ringed = [&](int u, int w) {
+            bool in = false;
             if (fits) {
-                bool in = false;
-                for (int i = 0; i < n0 + n1 + 2; i++) in |= ring[i] == u;
+                for (int i = 0; i < quads; i++) {
+                    const int4 r = ring[i];
+                    in |= r.x == u || r.y == u || r.z == u || r.w == u || r.x == w || r.y == w || r.z == w || r.w == w;
+                }
                 return in;
             }
-            bool in = u == av.x || u == av.y;
-            for (int i = 0; i < n0; i++) in |= vnbr[r0 + i] == u;
-            for (int i = 0; i < n1; i++) in |= vnbr[r1 + i] == u;
+            in = u == av.x || u == av.y || w == av.x || w == av.y;
+            for (int i = 0; i < n0; i++) in |= vnbr[r0 + i] == u || vnbr[r0 + i] == w;
+            for (int i = 0; i < n1; i++) in |= vnbr[r1 + i] == u || vnbr[r1 + i] == w;
             return in;
         };
-        const int most = max(deg, __shfl_xor(deg, 32));
-        for (int i = 0; i < most; i++) {
-            const int4 tc = i < deg ? tcell[etri[o + i]] : make_int4(0, 0, 0, -1);
-            const int3 q = around(tc, l);
-            bool mine = tc.w >= 0 && l < 27 && cell_key(g, q.x, q.y, q.z) >= 0;
-            for (int j = 0; j < min(i, deg); j++)
-                if (near_cell(tcell[etri[o + j]], q.x, q.y, q.z)) mine = false;
+        const int rounds = max(cells.rounds, __shfl_xor(cells.rounds, 32));
+        for (int r = 0; r < rounds; r++) {
+            int3 q;
+            const bool mine = cells.cell(g, r, &q);
             if (!__any(mine)) continue;
             const unsigned slot = cell_slot(q.x, q.y, q.z, mask);
             const int n = mine ? cnt[slot] : 0;
             visit_runs(n ? end[slot] - n : 0, n, [&](int e, int from) {
-                bool face = false, out_of[3] = {false, false, false};
-                int f = 0;
+                const int3 fq = make_int3(__shfl(q.x, from, 32), __shfl(q.y, from, 32), __shfl(q.z, from, 32));
+                bool hit = false;
+                int eb = 0;
                 if (e >= 0) {
-                    const int4 ec = ent[e];
-                    const int3 fq = around(tc, from);
-                    f = ec.w;
-                    face = ec.x == fq.x && ec.y == fq.y && ec.z == fq.z;
-                    if (face) {
-                        out_of[0] = !in_ring(rec[f].v0);
-                        out_of[1] = !in_ring(rec[f].v1);
-                        out_of[2] = !in_ring(rec[f].v2);
+                    const EdgeRec rec = ent[e];
+                    eb = rec.edge;
+                    if (eb > a && rec.cx == fq.x && rec.cy == fq.y && rec.cz == fq.z && !ringed(rec.v0, rec.v1)) {
+                        bool first = !rec.before || !cells.meets(make_int4(rec.ox, rec.oy, rec.oz, 0));
+                        if (rec.before == 2)
+                            for (int j = etoff[eb]; first; j++) {  // ends at a face of this cell
+                                const int4 d = tcell[etri[j]];
+                                if (d.w >= 0 && d.x == rec.cx && d.y == rec.cy && d.z == rec.cz) break;
+                                first = !cells.meets(d);
+                            }
+                        pairs += first;
+                        hit = first && (LIST || !edges_apart(abox, rec.box, th));
                     }
                 }
-                for (int k = 0; k < 3; k++) {
-                    bool hit = false;
-                    int eb = 0;
-                    if (face && out_of[k] && out_of[k == 2 ? 0 : k + 1]) {
-                        eb = tedge[3 * f + k];
-                        bool cand = eb > a;
-                        // a face with a repeated vertex has an edge twice
-                        for (int m = 0; m < k; m++) cand = cand && eb != tedge[3 * f + m];
-                        for (int j = etoff[eb]; cand && j < etoff[eb + 1]; j++) {
-                            const int f2 = etri[j];
-                            if (f2 == f) break;
-                            const int4 c2 = tcell[f2];
-                            for (int m = 0; c2.w >= 0 && m < deg; m++)
-                                if (near_cell(tcell[etri[o + m]], c2.x, c2.y, c2.z)) cand = false;
-                        }
-                        if (cand) {
-                            pairs++;
-                            hit = LIST || !edges_apart(alo, ahi, box[2 * eb], box[2 * eb + 1], th);
-                        }
-                    }
-                    sink.add(hit, a, eb);
-                }
+                sink.add(hit, a, eb);
             });
         }
     }
     if (sink.n) sink.flush();
-    const unsigned long long t = wave_total(pairs);
-    if (!LIST && lane == 0 && t) atomicAdd(&c->ee_pairs, t);
+    if (!LIST) sink.count(pairs);
 }
 
 // Vertex -> triangles (CSR, any order within a vertex).
@@ -708,12 +860,18 @@ __global__ __launch_bounds__(256) void k_vt_fill(const int* __restrict__ tris, i
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) vtri[off[tris[i]] + atomicSub(&cnt[tris[i]], 1) - 1] = i / 3;
 }
-__global__ __launch_bounds__(256) void k_unzip(const int2* __restrict__ a, int n, uint32_t* __restrict__ hi,
-                                               uint32_t* __restrict__ lo) {
+// The bucketed list as two arrays; at[b]: where bucket b's pairs go.
+struct BucketPlaces {
+    int at[NEAR_BUCKETS + 1];
+};
+__global__ __launch_bounds__(256) void k_unzip(const int2* __restrict__ a, unsigned cap, BucketPlaces b,
+                                               uint32_t* __restrict__ hi, uint32_t* __restrict__ lo) {
+    const int n = b.at[blockIdx.y + 1] - b.at[blockIdx.y];
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    hi[i] = (uint32_t)a[i].x;
-    lo[i] = (uint32_t)a[i].y;
+    const int2 q = a[(size_t)blockIdx.y * cap + i];
+    hi[b.at[blockIdx.y] + i] = (uint32_t)q.x;
+    lo[b.at[blockIdx.y] + i] = (uint32_t)q.y;
 }
 
 // ---------------------------------------------------------------------------
@@ -854,6 +1012,20 @@ __device__ bool vf_ccd(V3 x0, V3 x1, V3 x2, V3 x3, V3 p0, V3 p1, V3 p2, V3 p3, f
     return false;
 }
 
+// This workgroup's share of the bucketed candidate list: bucket blockIdx.x %
+// NEAR_BUCKETS, pairs from `from` on in steps of `step`.
+struct NearRun {
+    const int2* pairs;
+    unsigned n, from, step;
+    __device__ __forceinline__ NearRun(const int2* near, unsigned cap, const DetectCounts* c) {
+        const unsigned b = blockIdx.x % NEAR_BUCKETS;
+        pairs = near + (size_t)b * cap;
+        n = min(c->bucket[b].near, cap);
+        from = blockIdx.x / NEAR_BUCKETS * 256;
+        step = gridDim.x / NEAR_BUCKETS * 256;
+    }
+};
+
 // The narrowphase over the listed pairs (their number is on the device), its
 // contacts appended in any order.  STORE: time, normal and weights too (the
 // response needs only the vertices).
@@ -864,17 +1036,18 @@ __global__ __launch_bounds__(256) void k_narrow(const int2* __restrict__ near, u
                                                 unsigned cap, int4* __restrict__ vquad, int2* __restrict__ vf,
                                                 float* __restrict__ ct, float* __restrict__ cn,
                                                 double* __restrict__ cw) {
-    const unsigned n = min(c->near, near_cap);
-    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        const int2 q = near[i];
-        const int a = tris[3 * q.y], b = tris[3 * q.y + 1], d = tris[3 * q.y + 2];
+    const NearRun run(near, near_cap, c);
+    for (unsigned i = run.from + threadIdx.x; i < run.n; i += run.step) {
+        const int2 q = run.pairs[i];
+        const int4 v = make_int4(q.x, tris[3 * q.y], tris[3 * q.y + 1], tris[3 * q.y + 2]);
         float t;
         V3 nr, wg;
-        if (!vf_ccd(v3(x[q.x]), v3(x[a]), v3(x[b]), v3(x[d]), v3(p[q.x]), v3(p[a]), v3(p[b]), v3(p[d]), th, &t, &nr, &wg))
+        if (!vf_ccd(v3(x[v.x]), v3(x[v.y]), v3(x[v.z]), v3(x[v.w]), v3(p[v.x]), v3(p[v.y]), v3(p[v.z]), v3(p[v.w]), th,
+                    &t, &nr, &wg))
             continue;
         const unsigned o = atomicAdd(&c->contacts, 1u);
         if (o >= cap) continue;
-        vquad[o] = make_int4(q.x, a, b, d);
+        vquad[o] = v;
         if (STORE) {
             vf[o] = q;
             ct[o] = t;
@@ -1045,16 +1218,16 @@ __global__ __launch_bounds__(256) void k_narrow_ee(const int2* __restrict__ near
                                                    unsigned cap, int2* __restrict__ ab, int4* __restrict__ quad,
                                                    float* __restrict__ ct, float* __restrict__ cn,
                                                    double* __restrict__ cw) {
-    const unsigned n = min(c->ee_near, near_cap);
-    for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        const int2 q = near[i];
+    const NearRun run(near, near_cap, c);
+    for (unsigned i = run.from + threadIdx.x; i < run.n; i += run.step) {
+        const int2 q = run.pairs[i];
         const int2 ea = edges[q.x], eb = edges[q.y];
         float t, w[4];
         V3 nr;
         if (!ee_ccd(v3(x[ea.x]), v3(x[ea.y]), v3(x[eb.x]), v3(x[eb.y]), v3(p[ea.x]), v3(p[ea.y]), v3(p[eb.x]),
                     v3(p[eb.y]), th, &t, &nr, w))
             continue;
-        const unsigned o = atomicAdd(&c->ee_contacts, 1u);
+        const unsigned o = atomicAdd(&c->contacts, 1u);
         if (o >= cap) continue;
         quad[o] = make_int4(ea.x, ea.y, eb.x, eb.y);
         if (STORE) {
@@ -1323,7 +1496,7 @@ void Broadphase::build(hipStream_t s, const HashCfg& g, const float4* p, const i
 }
 
 void Broadphase::set_edges(hipStream_t s, const std::vector<int>& te, const std::vector<int2>& ed) {
-    tedge.upload(te, s);
+    edge_tris = te.size() / 3;
     edges.upload(ed, s);
     nedges = (int)ed.size();
     // edge -> triangles (CSR)
@@ -1387,12 +1560,24 @@ static DetectCounts* counts_of(const DBuf<int>& table) { return reinterpret_cast
 static int* slots_of(const DBuf<int>& table) { return table.ptr + sizeof(DetectCounts) / sizeof(int); }
 
 // The counters as of this point of the stream (waits).
-DetectCounts Broadphase::read_counts(hipStream_t s) {
+DetectTotals Broadphase::read_counts(hipStream_t s) {
     if (!counts_h) PBD_HIP(hipHostMalloc(&counts_h, sizeof(DetectCounts), hipHostMallocDefault));
     PBD_HIP(hipMemcpyAsync(counts_h, table.ptr, sizeof(DetectCounts), hipMemcpyDeviceToHost, s));
     PBD_HIP(hipStreamSynchronize(s));
-    return *reinterpret_cast<DetectCounts*>(counts_h);
+    const DetectCounts& c = *static_cast<const DetectCounts*>(counts_h);
+    DetectTotals t{0, 0, 0, c.contacts, c.entries, c.face_span, c.vertex_span};
+    for (int b = 0; b < NEAR_BUCKETS; b++) {
+        near_n[b] = c.bucket[b].near;
+        t.pairs += c.bucket[b].pairs;
+        t.near += near_n[b];
+        t.near_most = std::max(t.near_most, near_n[b]);
+    }
+    return t;
 }
+
+// Room for n candidates per bucket of the list.
+void Broadphase::grow_near(size_t n) { grow(near_, n * NEAR_BUCKETS); }
+unsigned Broadphase::near_cap() const { return (unsigned)std::min<size_t>(near_.n / NEAR_BUCKETS, 0x7fffffff); }
 
 // Workgroups of the candidate visits: each wave takes two vertices (edges) at
 // a time, and enough waves to fill the GPU take them in turn.
@@ -1406,16 +1591,15 @@ void Broadphase::cells(hipStream_t s, const HashCfg& g, const float4* x, const f
     grow(tcell, std::max(1, nt));
     grow(raw_rank, std::max(1, nt));
     grow(rec, (size_t)std::max(1, nt) * sizeof(FaceRec));
-    grow(ent, 2 * (size_t)std::max(1, nt));
     const int bits = table_bits_for(2ll * nt);
     clear_table(s, bits);
     const unsigned mask = (1u << table_bits) - 1;
-    hipLaunchKernelGGL(k_face_cells, dim3(blocks(nt)), dim3(256), 0, s, g, x, p, tris, nt, th, mask, slots_of(table),
-                       tcell.ptr, raw_rank.ptr, (FaceRec*)rec.ptr);
-    hipLaunchKernelGGL(k_slot_places<true>, dim3((1 << table_bits) / 256), dim3(256), 0, s, slots_of(table),
-                       1 << table_bits, place.ptr, &counts_of(table)->entries);
+    hipLaunchKernelGGL(k_face_cells, dim3(blocks(nt)), dim3(256), 0, s, g, p, tris, nt, mask, slots_of(table), tcell.ptr,
+                       raw_rank.ptr);
+    hipLaunchKernelGGL(k_slot_places<true>, dim3(((1 << table_bits) + PLACE_SLOTS - 1) / PLACE_SLOTS), dim3(256), 0, s,
+                       (const int4*)slots_of(table), 1 << table_bits, (int4*)place.ptr, &counts_of(table)->entries);
     hipLaunchKernelGGL(k_cell_fill, dim3(blocks(nt)), dim3(256), 0, s, nt, tcell.ptr, raw_rank.ptr, slots_of(table),
-                       place.ptr, (int4*)ent.ptr);
+                       place.ptr, x, p, tris, th, (FaceRec*)rec.ptr);
     PBD_HIP(hipGetLastError());
 }
 
@@ -1433,11 +1617,11 @@ void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, c
     nt = nt_;
     by_box = swept != nullptr;
     if (nt <= 0 || nv <= 0) return;
-    grow(near_, std::max<size_t>(1 << 16, (size_t)nv));
+    grow_near(std::max<size_t>(1 << 10, (size_t)nv / NEAR_BUCKETS));
     grow_contacts(std::max<size_t>(1 << 14, (size_t)nv / 4), store);
-    DetectCounts c{};
+    DetectTotals c{};
     for (;;) {
-        const unsigned near_cap = (unsigned)std::min<size_t>(near_.n, 0x7fffffff), cap = (unsigned)vquad.n;
+        const unsigned near_cap = this->near_cap(), cap = (unsigned)vquad.n;
         if (swept) {
             swept_table(s, g, *swept, x, p, tris, th);
             hipLaunchKernelGGL(k_swept_candidates, dim3(visit_blocks(nv)), dim3(64 * VISIT_WAVES), 0, s, g, *swept, x, p,
@@ -1448,7 +1632,7 @@ void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, c
             cells(s, g, x, p, tris, nt, th);
             hipLaunchKernelGGL(k_vf_candidates<false>, dim3(visit_blocks(nv)), dim3(64 * VISIT_WAVES), 0, s, g, x, p, nv,
                                vtoff.ptr, vtri.ptr, tcell.ptr, slots_of(table), place.ptr, (1u << table_bits) - 1,
-                               (const int4*)ent.ptr, (const FaceRec*)rec.ptr, counts_of(table), near_.ptr,
+                               (const FaceRec*)rec.ptr, counts_of(table), near_.ptr,
                                near_cap);
         }
         auto* narrow = store ? k_narrow<true> : k_narrow<false>;
@@ -1466,9 +1650,9 @@ void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, c
                       "a vertex's swept box spans more than 4096 cells: use a larger cell");
             check_pairs(c.pairs, "candidate pair count");
         }
-        if (!table_short && c.near <= near_cap && c.contacts <= cap) break;
+        if (!table_short && c.near_most <= near_cap && c.contacts <= cap) break;
         if (table_short) grow(ent, (size_t)c.entries + c.entries / 4);
-        else if (c.near > near_cap) grow(near_, (size_t)c.near + c.near / 4);
+        else if (c.near_most > near_cap) grow_near((size_t)c.near_most + c.near_most / 4);
         else grow_contacts((size_t)c.contacts + c.contacts / 4, store);
     }
     npairs = (long long)c.pairs;
@@ -1492,8 +1676,8 @@ void Broadphase::swept_table(hipStream_t s, const HashCfg& g, const HashCfg& gi,
     const unsigned mask = (1u << table_bits) - 1;
     hipLaunchKernelGGL(k_swept_faces, dim3(blocks(nt)), dim3(256), 0, s, g, gi, x, p, tris, nt, th, mask,
                        slots_of(table), sw_cell.ptr, (FaceRec*)rec.ptr, large.ptr, counts_of(table));
-    hipLaunchKernelGGL(k_slot_places<false>, dim3((1 << table_bits) / 256), dim3(256), 0, s, slots_of(table),
-                       1 << table_bits, place.ptr, &counts_of(table)->entries);
+    hipLaunchKernelGGL(k_slot_places<false>, dim3(((1 << table_bits) + PLACE_SLOTS - 1) / PLACE_SLOTS), dim3(256), 0, s,
+                       (const int4*)slots_of(table), 1 << table_bits, (int4*)place.ptr, &counts_of(table)->entries);
     hipLaunchKernelGGL(k_swept_fill, dim3(blocks(nt)), dim3(256), 0, s, nt, sw_cell.ptr, mask, place.ptr,
                        ent.ptr, (int)std::min<size_t>(ent.n, 0x7fffffff));
     PBD_HIP(hipGetLastError());
@@ -1535,15 +1719,23 @@ void Broadphase::order_contacts(hipStream_t s, const DBuf<int2>& key, const int4
     PBD_HIP(hipGetLastError());
 }
 
-// Sorts the n pairs in `near` by (first, second) into hi / lo.
-void Broadphase::sort_near(hipStream_t s, long long n, int nfirst, int nsecond, DBuf<uint32_t>& hi, DBuf<uint32_t>& lo) {
+// Sorts the listed pairs by (first, second) into hi / lo.
+void Broadphase::sort_near(hipStream_t s, int nfirst, int nsecond, DBuf<uint32_t>& hi, DBuf<uint32_t>& lo) {
+    BucketPlaces b{};
+    unsigned most = 0;
+    for (int i = 0; i < NEAR_BUCKETS; i++) {
+        b.at[i + 1] = b.at[i] + (int)near_n[i];
+        most = std::max(most, near_n[i]);
+    }
+    const long long n = b.at[NEAR_BUCKETS];
     grow(hi, (size_t)std::max(1ll, n));
     grow(lo, (size_t)std::max(1ll, n));
     if (n <= 0) return;
     grow(k2, n);
     grow(v2, n);
     grow(hist, radix_hist_ints(n));
-    hipLaunchKernelGGL(k_unzip, dim3(blocks(n)), dim3(256), 0, s, near_.ptr, (int)n, hi.ptr, lo.ptr);
+    hipLaunchKernelGGL(k_unzip, dim3(blocks(most), NEAR_BUCKETS), dim3(256), 0, s, near_.ptr, near_cap(), b, hi.ptr,
+                       lo.ptr);
     int fb = 1, vb = 1;
     while (fb < 31 && (1ll << fb) < nsecond) fb++;
     while (vb < 31 && (1ll << vb) < nfirst) vb++;
@@ -1557,20 +1749,20 @@ long long Broadphase::list_pairs(hipStream_t s, const HashCfg& g, const float4* 
     nt = nt_;
     npairs = 0;
     if (nt <= 0 || nv <= 0) return 0;
-    if (!near_.n) grow(near_, 1 << 16);
+    if (!near_.n) grow_near(1 << 10);
     for (;;) {
-        const unsigned cap = (unsigned)std::min<size_t>(near_.n, 0x7fffffff);
+        const unsigned cap = near_cap();
         cells(s, g, p, p, tris, nt, 0.0f);
         hipLaunchKernelGGL(k_vf_candidates<true>, dim3(visit_blocks(nv)), dim3(64 * VISIT_WAVES), 0, s, g, p, p, nv,
                            vtoff.ptr, vtri.ptr, tcell.ptr, slots_of(table), place.ptr, (1u << table_bits) - 1,
-                           (const int4*)ent.ptr, (const FaceRec*)rec.ptr, counts_of(table), near_.ptr, cap);
-        const DetectCounts c = read_counts(s);
+                           (const FaceRec*)rec.ptr, counts_of(table), near_.ptr, cap);
+        const DetectTotals c = read_counts(s);
         check_pairs(c.near, "candidate pair count");
-        npairs = c.near;
-        if (c.near <= cap) break;
-        grow(near_, c.near);
+        npairs = (long long)c.near;
+        if (c.near_most <= cap) break;
+        grow_near(c.near_most);
     }
-    sort_near(s, npairs, nv, nt, uv, uf);
+    sort_near(s, nv, nt, uv, uf);
     return npairs;
 }
 
@@ -1579,17 +1771,32 @@ long long Broadphase::list_pairs(hipStream_t s, const HashCfg& g, const float4* 
 void Broadphase::list_detected(hipStream_t s, const float4* p, const int* tris, int nv) {
     if (listed) return;
     const long long n = npairs;
-    if (by_box) sort_near(s, n, nv, nt, uv, uf);
+    if (by_box) sort_near(s, nv, nt, uv, uf);
     else if (n > 0) list_pairs(s, cfg, p, tris, nt, nv);
     npairs = n;
     listed = true;
 }
 
-void Broadphase::ee_candidates(hipStream_t s, bool list, float th, unsigned cap) {
+// The edge table of the faces' centroid cells at p, and its candidates.
+void Broadphase::ee_candidates(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris,
+                               int nt_, bool list, float th, unsigned cap) {
+    cfg = g;
+    nt = nt_;
+    grow(tcell, std::max(1, nt));
+    grow(rec, 3 * (size_t)std::max(1, nt) * sizeof(EdgeRec));
+    clear_table(s, table_bits_for(2ll * nt));
+    const unsigned mask = (1u << table_bits) - 1;
+    EdgeRec* ent = reinterpret_cast<EdgeRec*>(rec.ptr);
+    hipLaunchKernelGGL(k_tri_cells, dim3(blocks(nt)), dim3(256), 0, s, g, p, tris, nt, mask, tcell.ptr);
+    hipLaunchKernelGGL(k_edge_count, dim3(blocks(nedges)), dim3(256), 0, s, nedges, etoff.ptr, etri.ptr, tcell.ptr,
+                       slots_of(table));
+    hipLaunchKernelGGL(k_slot_places<false>, dim3(((1 << table_bits) + PLACE_SLOTS - 1) / PLACE_SLOTS), dim3(256), 0, s,
+                       (const int4*)slots_of(table), 1 << table_bits, (int4*)place.ptr, &counts_of(table)->entries);
+    hipLaunchKernelGGL(k_edge_fill, dim3(blocks(nedges)), dim3(256), 0, s, nedges, edges.ptr, etoff.ptr, etri.ptr,
+                       tcell.ptr, x, p, place.ptr, ent);
     auto* k = list ? k_ee_candidates<true> : k_ee_candidates<false>;
-    hipLaunchKernelGGL(k, dim3(visit_blocks(nedges)), dim3(64 * VISIT_WAVES), 0, s, cfg, nedges, edges.ptr, etoff.ptr,
-                       etri.ptr, tedge.ptr, voff.ptr, vnbr.ptr, tcell.ptr, slots_of(table), place.ptr,
-                       (1u << table_bits) - 1, (const int4*)ent.ptr, (const FaceRec*)rec.ptr, ebox.ptr, th,
+    hipLaunchKernelGGL(k, dim3(visit_blocks(nedges)), dim3(64 * VISIT_WAVES), 0, s, g, nedges, edges.ptr, etoff.ptr,
+                       etri.ptr, voff.ptr, vnbr.ptr, x, p, tcell.ptr, slots_of(table), place.ptr, mask, ent, th,
                        counts_of(table), near_.ptr, cap);
     PBD_HIP(hipGetLastError());
 }
@@ -1600,9 +1807,8 @@ void Broadphase::detect_ee(hipStream_t s, const HashCfg& g, const float4* x, con
     ee_npairs = ee_ncontacts = 0;
     ee_listed = false;
     if (nt_ <= 0 || nedges <= 0) return;
-    PBD_CHECK(tedge.n >= (size_t)3 * nt_, PBD_ERR_STATE, "internal: edge table does not match the triangles");
-    grow(near_, std::max<size_t>(1 << 16, (size_t)nedges));
-    grow(ebox, 2 * (size_t)nedges);
+    PBD_CHECK(edge_tris >= (size_t)nt_, PBD_ERR_STATE, "internal: edge table does not match the triangles");
+    grow_near(std::max<size_t>(1 << 10, (size_t)nedges / NEAR_BUCKETS));
     auto grow_ee = [&](size_t n) {
         grow(quad, n);
         if (!store) return;
@@ -1612,24 +1818,22 @@ void Broadphase::detect_ee(hipStream_t s, const HashCfg& g, const float4* x, con
         grow(rw, 4 * quad.n);
     };
     grow_ee(std::max<size_t>(1 << 14, (size_t)nedges / 8));
-    DetectCounts c{};
+    DetectTotals c{};
     for (;;) {
-        const unsigned near_cap = (unsigned)std::min<size_t>(near_.n, 0x7fffffff), cap = (unsigned)quad.n;
-        cells(s, g, x, p, tris, nt_, th);
-        hipLaunchKernelGGL(k_edge_boxes, dim3(blocks(nedges)), dim3(256), 0, s, edges.ptr, nedges, x, p, ebox.ptr);
-        ee_candidates(s, false, th, near_cap);
+        const unsigned near_cap = this->near_cap(), cap = (unsigned)quad.n;
+        ee_candidates(s, g, x, p, tris, nt_, false, th, near_cap);
         auto* narrow = store ? k_narrow_ee<true> : k_narrow_ee<false>;
         hipLaunchKernelGGL(narrow, dim3(1024), dim3(256), 0, s, near_.ptr, near_cap, edges.ptr, x, p, th,
                            counts_of(table), cap, eab.ptr, quad.ptr, rt.ptr, rn.ptr, rw.ptr);
         PBD_HIP(hipGetLastError());
         c = read_counts(s);
-        check_pairs(c.ee_pairs, "edge-edge candidate count");
-        if (c.ee_near <= near_cap && c.ee_contacts <= cap) break;
-        if (c.ee_near > near_cap) grow(near_, (size_t)c.ee_near + c.ee_near / 4);
-        else grow_ee((size_t)c.ee_contacts + c.ee_contacts / 4);
+        check_pairs(c.pairs, "edge-edge candidate count");
+        if (c.near_most <= near_cap && c.contacts <= cap) break;
+        if (c.near_most > near_cap) grow_near((size_t)c.near_most + c.near_most / 4);
+        else grow_ee((size_t)c.contacts + c.contacts / 4);
     }
-    ee_npairs = (long long)c.ee_pairs;
-    ee_ncontacts = c.ee_contacts;
+    ee_npairs = (long long)c.pairs;
+    ee_ncontacts = c.contacts;
     st_ee_raw += ee_npairs;
     st_ee_pairs += ee_npairs;
     st_ee_contacts += ee_ncontacts;
@@ -1641,10 +1845,13 @@ void Broadphase::list_detected_ee(hipStream_t s, const HashCfg& g, const float4*
                                   float th) {
     if (ee_listed) return;
     if (ee_npairs > 0) {
-        grow(near_, (size_t)ee_npairs);
-        cells(s, g, x, p, tris, nt, th);
-        ee_candidates(s, true, th, (unsigned)std::min<size_t>(near_.n, 0x7fffffff));
-        sort_near(s, ee_npairs, nedges, nedges, eua, eub);
+        for (;;) {
+            ee_candidates(s, g, x, p, tris, nt, true, th, near_cap());
+            const DetectTotals c = read_counts(s);
+            if (c.near_most <= near_cap()) break;
+            grow_near(c.near_most);
+        }
+        sort_near(s, nedges, nedges, eua, eub);
     }
     ee_listed = true;
 }

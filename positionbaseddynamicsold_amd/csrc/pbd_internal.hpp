@@ -234,12 +234,22 @@ struct HashCfg {
 };
 
 // Counters of a detection, cleared with the table's slot counts.
+constexpr int NEAR_BUCKETS = 64;
+struct DetectBucket {
+    unsigned long long pairs;  // distinct candidates
+    unsigned near;             // candidates that go to the narrowphase
+    unsigned pad[29];
+};
 struct DetectCounts {
-    unsigned long long pairs, ee_pairs;  // distinct candidates
-    unsigned near, ee_near;              // candidates that go to the narrowphase
-    unsigned contacts, ee_contacts;
-    unsigned entries, large;             // table entries; faces kept out of the table
-    unsigned face_span, vertex_span;     // 1: a box over the allowed cells of the caller's grid
+    unsigned contacts;
+    unsigned entries, large;          // table entries; faces kept out of the table
+    unsigned face_span, vertex_span;  // 1: a box over the allowed cells of the caller's grid
+    unsigned pad[27];
+    DetectBucket bucket[NEAR_BUCKETS];  // a line each
+};
+struct DetectTotals {
+    unsigned long long pairs, near;
+    unsigned near_most, contacts, entries, face_span, vertex_span;
 };
 
 // Broadphase + CCD working set (device buffers reused between calls).
@@ -257,8 +267,8 @@ struct Broadphase {
     DBuf<int> cnt, off, scan_tmp, idx;
     // vertex -> triangles of the current triangle list
     DBuf<int> vtoff, vtri;
-    // unsorted table of the faces by cell: counters and slot counts, slot
-    // places, entries (int4 cell and face, or int2 face and cell code), face
+    // unsorted table of the faces (edges) by cell: counters and slot counts, slot
+    // places, entries by swept box (face and cell code), face or edge
     // records, per-face cells
     DBuf<int> table, place, raw_rank, large;
     int table_bits = 0;
@@ -269,6 +279,7 @@ struct Broadphase {
     // candidates that go to the narrowphase; contacts in any order (the
     // response reads these) and, when asked for, in ascending order
     DBuf<int2> near_;
+    unsigned near_n[NEAR_BUCKETS] = {};
     DBuf<int4> vquad;
     DBuf<int2> vf, ckey;
     DBuf<float> rt, rn, ct, cn;
@@ -281,13 +292,13 @@ struct Broadphase {
     int few_slots = 0;  // LDS table of the response in one workgroup, 0 before the first use
     // running counts: detections, triangles, cell entries, raw pairs, distinct pairs, contacts
     long long st_dets = 0, st_tris = 0, st_entries = 0, st_raw = 0, st_pairs = 0, st_contacts = 0, st_resolved = 0;
-    // edge-edge: per-triangle edge ids, edge endpoints (lower, higher), edge ->
-    // triangles, vertex -> mesh neighbours, swept boxes, and the contacts
+    // edge-edge: edge endpoints (lower, higher), edge ->
+    // triangles, vertex -> mesh neighbours, and the contacts
     // (a0, a1, b0, b1) with their edge ids
-    DBuf<int> tedge, etoff, etri, voff, vnbr;
+    DBuf<int> etoff, etri, voff, vnbr;
+    size_t edge_tris = 0;
     DBuf<int2> edges;
     int nedges = 0;
-    DBuf<float4> ebox;
     DBuf<int4> quad, ecq;
     DBuf<int2> eab, eabs;
     DBuf<float> ect, ecn;
@@ -315,7 +326,9 @@ struct Broadphase {
 
 private:
     void clear_table(hipStream_t s, int bits);
-    DetectCounts read_counts(hipStream_t s);
+    DetectTotals read_counts(hipStream_t s);
+    void grow_near(size_t n);
+    unsigned near_cap() const;
     void cells(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt, float th);
     void swept_table(hipStream_t s, const HashCfg& g, const HashCfg& gi, const float4* x, const float4* p,
                      const int* tris, float th);
@@ -323,8 +336,9 @@ private:
     void grow_contacts(size_t n, bool store);
     void order_contacts(hipStream_t s, const DBuf<int2>& key, const int4* quad, long long n, int nfirst,
                         DBuf<int2>& okey, DBuf<int4>* oquad);
-    void sort_near(hipStream_t s, long long n, int nfirst, int nsecond, DBuf<uint32_t>& hi, DBuf<uint32_t>& lo);
-    void ee_candidates(hipStream_t s, bool list, float th, unsigned cap);
+    void sort_near(hipStream_t s, int nfirst, int nsecond, DBuf<uint32_t>& hi, DBuf<uint32_t>& lo);
+    void ee_candidates(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt, bool list,
+                       float th, unsigned cap);
 };
 void device_scan(hipStream_t s, const int* in, int* out, int n, int* tmp);
 // Broadphase build into caller device arrays with no allocation: the sort's
