@@ -9,12 +9,9 @@ namespace pbd {
 
 #define PBD_HD __host__ __device__ __forceinline__
 
-PBD_HD float atan2_hd(float y, float x) {
+// The angle of (x, y) from a, the smaller of |x| and |y| over the larger.
+PBD_HD float atan2_of(float a, float y, float x) {
     float ax = fabsf(x), ay = fabsf(y);
-    float mx = ax > ay ? ax : ay;
-    float mn = ax > ay ? ay : ax;
-    if (mx == 0.0f) return 0.0f;
-    float a = mn / mx;
     float s = a * a;
     float r = -0x1.09b858p-8f;
     r = r * s + 0x1.6633e4p-6f;
@@ -29,6 +26,14 @@ PBD_HD float atan2_hd(float y, float x) {
     if (x < 0.0f) r = 3.14159274f - r;
     if (y < 0.0f) r = -r;
     return r;
+}
+
+PBD_HD float atan2_hd(float y, float x) {
+    float ax = fabsf(x), ay = fabsf(y);
+    float mx = ax > ay ? ax : ay;
+    float mn = ax > ay ? ay : ax;
+    if (mx == 0.0f) return 0.0f;
+    return atan2_of(mn / mx, y, x);
 }
 
 struct V3 {
@@ -63,6 +68,23 @@ __device__ __forceinline__ float rcp_rn(float d) {
     const float e = __builtin_fmaf(-d, r, 1.0f);
     return __builtin_fmaf(e, r, r);
 }
+
+// Quotients a / b in the same b, correctly rounded: the double product of a and
+// 1/b (Newton steps on the hardware reciprocal, relative error below 2^-51) is
+// rounded once.  A quotient of two 24-bit significands is at least 2^-49 away
+// from the midpoint of two floats (relatively), so that rounding is the right
+// one unless the quotient is denormal.  For b in [2^-100, 2^100].  Three
+// operations a quotient and seven for b, against eleven a quotient; a single
+// correction step on a * RN(1/b) would take as few but is not always right.
+struct Reciprocal {
+    double y;
+    __device__ __forceinline__ explicit Reciprocal(float b) {
+        const double d = b, r = __builtin_amdgcn_rcpf(b);
+        const double r1 = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+        y = __builtin_fma(r1, __builtin_fma(-d, r1, 1.0), r1);
+    }
+    __device__ __forceinline__ float over(float a) const { return (float)((double)a * y); }
+};
 
 // Distance projection on two (x, y, z, w) records: the reference's CPU
 // formula r = normalize(p0-p1), dp0 = -w0/(w0+w1)(d-L) r, dp1 = +w1/(w0+w1)(d-L) r
@@ -157,21 +179,35 @@ PBD_HD float dihedral_hd(V3 e0, V3 e1, V3 o0, V3 o1) {
     return dih_angle(d);
 }
 
+// The quotients of a bending projection: IEEE division, or shared reciprocals
+// (Reciprocal) where their conditions hold.
+struct DivideBy {
+    float b;
+    PBD_HD explicit DivideBy(float v) : b(v) {}
+    PBD_HD float over(float a) const { return a / b; }
+};
+
 // Bending projection: C = theta - theta0, dp_i = -k w_i C / sum_j w_j |u_j|^2 u_i
 // with u = grad theta (Mueller et al. 2007 generic step; gradient from
-// Bridson et al. 2003).
-PBD_HD void project_bending(float4& q0, float4& q1, float4& q2, float4& q3, float rest, float k) {
-    V3 e0 = mk(q0.x, q0.y, q0.z), e1 = mk(q1.x, q1.y, q1.z);
-    V3 o0 = mk(q2.x, q2.y, q2.z), o1 = mk(q3.x, q3.y, q3.z);
-    Dih d = dih_terms(e0, e1, o0, o1);
-    if (!d.ok) return;
-    float th = dih_angle(d);
-    float s1 = d.elen / d.n1sq;
-    float s2 = d.elen / d.n2sq;
-    float a1 = (dot(sub(o0, e1), d.E) / d.elen) / d.n1sq;
-    float a2 = (dot(sub(o1, e1), d.E) / d.elen) / d.n2sq;
-    float b1 = (dot(sub(o0, e0), d.E) / d.elen) / d.n1sq;
-    float b2 = (dot(sub(o1, e0), d.E) / d.elen) / d.n2sq;
+// Bridson et al. 2003).  ok(den, th - rest, sin, cos, dots) decides whether the
+// quotients are to be trusted; returns false, with nothing changed, where not.
+template <class Over, class Ok>
+PBD_HD bool bending_step(const Dih& d, V3 e0, V3 e1, V3 o0, V3 o1, float4& q0, float4& q1, float4& q2, float4& q3,
+                         float rest, float k, Ok&& ok) {
+    const Over elen(d.elen), n1sq(d.n1sq), n2sq(d.n2sq);
+    const V3 c = cross(d.n2, d.n1);
+    const float num[5] = {dot(c, d.E), dot(sub(o0, e1), d.E), dot(sub(o1, e1), d.E), dot(sub(o0, e0), d.E),
+                          dot(sub(o1, e0), d.E)};
+    const float sn = elen.over(num[0]), cs = dot(d.n1, d.n2);
+    const float ax = fabsf(cs), ay = fabsf(sn);
+    const float mx = ax > ay ? ax : ay, mn = ax > ay ? ay : ax;
+    const float th = mx == 0.0f ? 0.0f : atan2_of(Over(mx).over(mn), sn, cs);
+    float s1 = n1sq.over(d.elen);
+    float s2 = n2sq.over(d.elen);
+    float a1 = n1sq.over(elen.over(num[1]));
+    float a2 = n2sq.over(elen.over(num[2]));
+    float b1 = n1sq.over(elen.over(num[3]));
+    float b2 = n2sq.over(elen.over(num[4]));
     V3 u0 = V3{a1 * d.n1.x + a2 * d.n2.x, a1 * d.n1.y + a2 * d.n2.y, a1 * d.n1.z + a2 * d.n2.z};
     V3 u1 = V3{-(b1 * d.n1.x) - b2 * d.n2.x, -(b1 * d.n1.y) - b2 * d.n2.y, -(b1 * d.n1.z) - b2 * d.n2.z};
     V3 u2 = scale(s1, d.n1);
@@ -181,8 +217,9 @@ PBD_HD void project_bending(float4& q0, float4& q1, float4& q2, float4& q3, floa
     den = den + q1.w * dot(u1, u1);
     den = den + q2.w * dot(u2, u2);
     den = den + q3.w * dot(u3, u3);
-    if (!(den > 1e-20f)) return;
-    float s = ((th - rest) / den) * k;
+    if (!ok(den, mx, cs, th - rest, num)) return false;
+    if (!(den > 1e-20f)) return true;
+    float s = Over(den).over(th - rest) * k;
     float f;
     f = s * q0.w;
     q0.x = q0.x - f * u0.x; q0.y = q0.y - f * u0.y; q0.z = q0.z - f * u0.z;
@@ -192,6 +229,50 @@ PBD_HD void project_bending(float4& q0, float4& q1, float4& q2, float4& q3, floa
     q2.x = q2.x - f * u2.x; q2.y = q2.y - f * u2.y; q2.z = q2.z - f * u2.z;
     f = s * q3.w;
     q3.x = q3.x - f * u3.x; q3.y = q3.y - f * u3.y; q3.z = q3.z - f * u3.z;
+    return true;
+}
+
+PBD_HD void project_bending(float4& q0, float4& q1, float4& q2, float4& q3, float rest, float k) {
+    V3 e0 = mk(q0.x, q0.y, q0.z), e1 = mk(q1.x, q1.y, q1.z);
+    V3 o0 = mk(q2.x, q2.y, q2.z), o1 = mk(q3.x, q3.y, q3.z);
+    Dih d = dih_terms(e0, e1, o0, o1);
+    if (!d.ok) return;
+    bending_step<DivideBy>(d, e0, e1, o0, o1, q0, q1, q2, q3, rest, k,
+                           [](float, float, float, float, const float*) { return true; });
+}
+
+// The same with shared reciprocals, equal to project_bending on every input:
+// squared lengths up to 2^32, denominators in Reciprocal's range, and
+// numerators that are zero or so large that no quotient is denormal; anything
+// else divides.  The chain of one projection bounds a tile's phase: 1730
+// cycles with divisions, 1390 so (5470 and 4080 with 16 waves on a CU).
+__device__ __forceinline__ void project_bending_fast(float4& q0, float4& q1, float4& q2, float4& q3, float rest,
+                                                     float k) {
+    V3 e0 = mk(q0.x, q0.y, q0.z), e1 = mk(q1.x, q1.y, q1.z);
+    V3 o0 = mk(q2.x, q2.y, q2.z), o1 = mk(q3.x, q3.y, q3.z);
+    Dih d;
+    d.E = sub(e1, e0);
+    d.n1 = cross(sub(o0, e0), sub(o0, e1));
+    d.n2 = cross(sub(o1, e1), sub(o1, e0));
+    d.n1sq = dot(d.n1, d.n1);
+    d.n2sq = dot(d.n2, d.n2);
+    const float e2 = dot(d.E, d.E);
+    bool fast = fmaxf(fmaxf(d.n1sq, d.n2sq), e2) <= 0x1p32f && e2 >= 0x1p-96f;
+    d.elen = sqrt_rn(e2);
+    d.ok = (d.n1sq > 1e-24f) && (d.n2sq > 1e-24f) && (d.elen > 1e-12f);
+    if (fast) {
+        if (!d.ok) return;
+        fast = bending_step<Reciprocal>(
+            d, e0, e1, o0, o1, q0, q1, q2, q3, rest, k,
+            [](float den, float mx, float cs, float c, const float* num) {
+                // |v| as an integer, zero as the largest
+                auto size = [](float v) { return (__float_as_uint(v) << 1) - 1u; };
+                unsigned least = min(size(cs), size(c));
+                for (int i = 0; i < 5; i++) least = min(least, size(num[i]));
+                return least >= (__float_as_uint(0x1p-76f) << 1) - 1u && mx >= 0x1p-90f && den <= 0x1p50f;
+            });
+    }
+    if (!fast) project_bending(q0, q1, q2, q3, rest, k);
 }
 
 // Analytic colliders.  Sphere: SolverPBD::ColliWithShpGrd / ColliderSphere /

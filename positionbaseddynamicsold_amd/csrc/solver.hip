@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void k_project_colour(const int4* __restrict__
         if (cap && sweep >= cap[__float_as_int(rc.y)]) return;
         float k = ktab_b[__float_as_int(rc.y) * kmax + ks];
         float4 q0 = p[q.x], q1 = p[q.y], q2 = p[q.z], q3 = p[q.w];
-        project_bending(q0, q1, q2, q3, rc.x, k);
+        project_bending_fast(q0, q1, q2, q3, rc.x, k);
         p[q.x] = q0;
         p[q.y] = q1;
         p[q.z] = q2;
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(256) void k_jacobi(JacobiDev J, const ClothDev* __r
             int4 q = J.bent[j];
             int2 m = J.bmeta[j];
             float4 q0 = pin[q.x], q1 = pin[q.y], q2 = pin[q.z], q3 = pin[q.w];
-            project_bending(q0, q1, q2, q3, __int_as_float(m.x), kb);
+            project_bending_fast(q0, q1, q2, q3, __int_as_float(m.x), kb);
             float4 r = m.y == 0 ? q0 : m.y == 1 ? q1 : m.y == 2 ? q2 : q3;
             sx = sx + (r.x - pi.x);
             sy = sy + (r.y - pi.y);
@@ -1037,7 +1037,7 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
                         const int i0 = br[u].x & 0xffffu, i1 = br[u].x >> 16, i2 = br[u].y & 0xffffu,
                                   i3 = br[u].y >> 16;
                         float4 q0 = P[i0], q1 = P[i1], q2 = P[i2], q3 = P[i3];
-                        project_bending(q0, q1, q2, q3, __uint_as_float(br[u].z), kb);
+                        project_bending_fast(q0, q1, q2, q3, __uint_as_float(br[u].z), kb);
                         P[i0] = q0;
                         P[i1] = q1;
                         P[i2] = q2;
