@@ -87,7 +87,8 @@ typedef struct {
     int path;               /* PBD_PATH_* */
     int tile_sweeps;        /* sweeps per launch for multi-tile cloths (0 = check_every, or up to four for grid
                                cloths of distance prims when check_every is 1 and neither a tolerance, the warm
-                               start nor collisions are in use; results are identical) */
+                               start nor collisions are in use; grid cloths with bending run one per launch where
+                               neither a tolerance nor the warm start is in use; results are identical) */
     int tile_max_verts;     /* most LDS vertices per tile (0 = from the device's LDS size); tiles are smaller where
                                the cloths would otherwise not fill the GPU */
     int block_threads;      /* threads per workgroup of the tile kernel (0 = by the tiles' sizes, at most 1024) */
@@ -107,7 +108,8 @@ typedef struct {
     int split_whole;        /* 1: a cloth that fits one LDS tile is stepped tile_sweeps sweeps per launch like a
                                multi-tile cloth (its one tile loads the whole cloth, no halo) instead of all its
                                sweeps in one launch, so that no launch waits on one cloth's whole budget
-                               (0 = one launch; results are identical either way) */
+                               (0 = one launch, except that a few larger grid cloths that leave most of the GPU
+                               idle, or collide, are stepped in several tiles; results are identical either way) */
     int per_chunk_launches; /* under per-cloth budgets (the warm start) with fixed sweeps: 0 = the substep's
                                tile work is one launch whose workgroups take (chunk, tile) items from a queue
                                built on the device after a residual kernel has made the keep decision, a

@@ -49,6 +49,7 @@ struct pbd_ctx {
     TilePlan plan;
     int plan_sweeps = 0, plan_max_load = 0, plan_split = 0;
     bool plan_small = false;  // planned with tiles smaller than the budget on offer
+    int plan_whole = 0;       // most vertices of a grid planned as one tile
     DBuf<TileDev> tiles;
     // launch orders: single-tile cloths' tiles, multi-tile cloths' tiles, and
     // both (the first launch of a substep runs them side by side)
@@ -250,8 +251,26 @@ bool distance_grids(const pbd_ctx* c) {
     return true;
 }
 
+// Sweeps are counted by nobody but the substep: no tolerance, no per-cloth budgets.
+bool free_sweeps(const pbd_ctx* c) { return !has_tolerance(c) && !c->ws.enabled; }
+
+// Every cloth is a grid, or has no prims, and at least one bends.
+bool bending_grids(const pbd_ctx* c) {
+    bool bends = false;
+    for (auto& k : c->cloths) {
+        if (k.np() > 0 && !plain_grid(k)) return false;
+        bends |= k.nb > 0;
+    }
+    return bends;
+}
+
 int effective_tile_sweeps(const pbd_ctx* c) {
     if (c->coll.enabled) return 1;  // contacts are resolved after every sweep
+    // Fixed sweeps: the result does not depend on the split, and with bending
+    // prims one sweep per launch is faster whatever was asked for (20 sweeps
+    // of 128^2 / 256^2 / 512^2 vertices: 648 / 692 / 985 us at one sweep per
+    // launch, 684 / 817 / 1328 us at two, at the best tile size of each).
+    if (c->sp.tile_sweeps > 1 && free_sweeps(c) && bending_grids(c)) return 1;
     if (c->sp.tile_sweeps > 0) return c->sp.tile_sweeps;
     // Unset and free to choose (fixed sweeps, no per-cloth budgets): four
     // sweeps per launch for distance prims.  Bending prims touch four vertices
@@ -261,7 +280,7 @@ int effective_tile_sweeps(const pbd_ctx* c) {
     // sweeps per launch, a 256 x 256 cloth with bending 721 us at 1 and 923 at 2.
     // Meshes are tiled by vertex id, whose cones may grow faster than a grid's:
     // they keep one.
-    if (c->sp.check_every <= 1 && !has_tolerance(c) && !c->ws.enabled && distance_grids(c))
+    if (c->sp.check_every <= 1 && free_sweeps(c) && distance_grids(c))
         return std::min(4, std::max(1, c->sp.iterations));
     return std::max(1, c->sp.check_every);
 }
@@ -385,8 +404,29 @@ TileShape tile_shape(const pbd_ctx* c, int ntiles) {
     return t;
 }
 
+// Most vertices of a grid that is stepped as one tile.  One workgroup per
+// cloth keeps the rest of the GPU idle, so a few grids that would fit a tile
+// are split where that is faster.  With collisions every sweep is a launch of
+// its own, which takes as long as its largest tile (96 x 96 vertices: 22 us as
+// one tile, 9 us in tiles).  Otherwise, 20 sweeps as one tile against tiles
+// at 4 / 2 / 1 sweeps per launch: 64 x 64 98 against 90 / - / -, 72 x 72
+// 159 against 88 / 117 / 160, 100 x 100 266 against 88 / 120 / 170; with
+// bending (one sweep per launch) 40 x 40 574 against 640, 48 x 48 680 against
+// 640, 80 x 80 1038 against 640.  As many grids as an eighth of the CUs
+// already fill their tiles well enough.
+int whole_grid_load(const pbd_ctx* c, int sweeps, int ml) {
+    if (c->sp.split_whole || has_tolerance(c)) return ml;
+    int load = 1024;
+    if (!c->coll.enabled) load = bending_grids(c) ? 2048 : sweeps >= 4 ? 4096 : sweeps >= 2 ? 4608 : 5632;
+    if (load >= ml) return ml;
+    int split = 0;
+    for (auto& k : c->cloths) split += plain_grid(k) && k.nv > load && k.nv <= ml;
+    return split > 0 && split <= c->num_cu / 8 ? load : ml;
+}
+
 void replan_if_needed(pbd_ctx* c) {
     int s = effective_tile_sweeps(c), ml = effective_max_load(c), sp = c->sp.split_whole ? 1 : 0;
+    const WholeLoad whole{whole_grid_load(c, s, ml), ml};
     // Tiles smaller than the budget where the multi-tile cloths would not fill
     // the GPU: a launch takes as long as its largest tile, so the smallest
     // tile size of at most one tile per CU is the fastest (a 389 x 211 cloth at
@@ -396,37 +436,39 @@ void replan_if_needed(pbd_ctx* c) {
     long long multi = 0;
     bool grids = true;
     for (auto& k : c->cloths)
-        if (k.nv > ml) {
+        if (!one_tile(k, whole)) {
             multi += k.nv;
-            grids &= k.rx > 0 && !k.has_user_pairs;
+            grids &= plain_grid(k);
         }
     std::vector<int> loads;
     if (multi > 0 && grids && !c->ws.enabled)
         for (int load : {512, 768, 1024, 1280, 1536, 2048, 2560, 3072, 3584, 4096, 4608})
             if (load < ml && (long long)load * c->num_cu > multi) loads.push_back(load);
     const bool small = !loads.empty();
-    if (s == c->plan_sweeps && ml == c->plan_max_load && sp == c->plan_split && small == c->plan_small) return;
+    if (s == c->plan_sweeps && ml == c->plan_max_load && sp == c->plan_split && small == c->plan_small &&
+        whole.grid == c->plan_whole)
+        return;
     // a failed plan leaves no valid one behind: the next call plans again
     c->plan_sweeps = 0;
     c->plan_max_load = 0;
     bool planned = false;
     if (small) {
-        loads = fitting_loads(c->cloths, ml, loads, s, c->num_cu);
+        loads = fitting_loads(c->cloths, whole, loads, s, c->num_cu);
         for (size_t i = 0; i < loads.size() && !planned; i++) {
             try {
-                plan_tiles(c->cloths, ml, loads[i], s, sp != 0, c->plan);
+                planned = plan_tiles(c->cloths, whole, loads[i], s, sp != 0, c->plan, c->num_cu);
             } catch (const Error& e) {
                 if (e.code != PBD_ERR_LIMIT) throw;
                 continue;  // some cone does not fit tiles of this size
             }
-            planned = (int)c->plan.tiles.size() <= c->num_cu;
         }
     }
-    if (!planned) plan_tiles(c->cloths, ml, ml, s, sp != 0, c->plan);
+    if (!planned) plan_tiles(c->cloths, whole, ml, s, sp != 0, c->plan);
     c->plan_sweeps = s;
     c->plan_max_load = ml;
     c->plan_split = sp;
     c->plan_small = small;
+    c->plan_whole = whole.grid;
     upload_plan(c);
     fill_cloth_dev(c);
 }
@@ -484,15 +526,23 @@ void do_init(pbd_ctx* c, int color_rounds) {
         std::vector<int> minus1(np, -1);
         d_color.upload(minus1, s);
         d_prd.upload(minus1, s);
-        d_unc.alloc(1);
-        int unc = np;
-        while (unc > 0) {
+        // Rounds in groups, each with its own count of prims left: one wait per
+        // group (a round after the last changes nothing).
+        constexpr int GROUP = 16;
+        d_unc.alloc(GROUP);
+        for (bool left = true; left;) {
             PBD_CHECK(rounds < color_rounds, PBD_ERR_COLOR, "colouring did not converge in the allowed rounds");
-            PBD_HIP(hipMemsetAsync(d_unc.ptr, 0, sizeof(int), s));
-            launch_color_round(s, d_npts.ptr, d_sn.ptr, d_adj.ptr, d_color.ptr, d_prd.ptr, d_unc.ptr, np);
-            PBD_HIP(hipMemcpyAsync(&unc, d_unc.ptr, sizeof(int), hipMemcpyDeviceToHost, s));
+            const int n = std::min(GROUP, color_rounds - rounds);
+            int unc[GROUP];
+            PBD_HIP(hipMemsetAsync(d_unc.ptr, 0, sizeof(int) * GROUP, s));
+            for (int r = 0; r < n; r++)
+                launch_color_round(s, d_npts.ptr, d_sn.ptr, d_adj.ptr, d_color.ptr, d_prd.ptr, d_unc.ptr + r, np);
+            PBD_HIP(hipMemcpyAsync(unc, d_unc.ptr, sizeof(int) * n, hipMemcpyDeviceToHost, s));
             PBD_HIP(hipStreamSynchronize(s));
-            rounds++;
+            for (int r = 0; r < n && left; r++) {
+                left = unc[r] > 0;
+                rounds++;
+            }
         }
         // ---- device stable colour sort (SortEdgesColors, PBD_cuda.cu:546-587)
         std::vector<uint32_t> ids(np);

@@ -569,11 +569,13 @@ static bool plan_block(const Cloth& c, const ClothTopo& topo, Block first, int m
     return true;
 }
 
-std::vector<int> fitting_loads(const std::vector<Cloth>& cloths, int whole_load, const std::vector<int>& loads, int sweeps,
-                               int max_tiles) {
+bool one_tile(const Cloth& c, const WholeLoad& whole) { return c.nv <= (plain_grid(c) ? whole.grid : whole.mesh); }
+
+std::vector<int> fitting_loads(const std::vector<Cloth>& cloths, const WholeLoad& whole, const std::vector<int>& loads,
+                               int sweeps, int max_tiles) {
     const Cloth* big = nullptr;
     for (const Cloth& c : cloths)
-        if (c.nv > whole_load && (!big || c.nv > big->nv)) big = &c;
+        if (!one_tile(c, whole) && (!big || c.nv > big->nv)) big = &c;
     if (!big || big->rx == 0) return {};
     ClothTopo topo;
     build_topo(*big, topo);
@@ -585,7 +587,7 @@ std::vector<int> fitting_loads(const std::vector<Cloth>& cloths, int whole_load,
             const int T = grid_block_side(*big, topo, load, std::max(1, sweeps) * big->ncolors, mark, entry, stamp);
             long long n = 0;
             for (const Cloth& c : cloths)
-                n += c.nv <= whole_load ? 1 : (long long)((c.rx + T - 1) / T) * ((c.ry + T - 1) / T);
+                n += one_tile(c, whole) ? 1 : (long long)((c.rx + T - 1) / T) * ((c.ry + T - 1) / T);
             seen = n <= max_tiles;
         }
         if (seen) fit.push_back(load);
@@ -593,7 +595,8 @@ std::vector<int> fitting_loads(const std::vector<Cloth>& cloths, int whole_load,
     return fit;
 }
 
-void plan_tiles(std::vector<Cloth>& cloths, int whole_load, int max_load, int sweeps, bool split_whole, TilePlan& plan) {
+bool plan_tiles(std::vector<Cloth>& cloths, const WholeLoad& whole, int max_load, int sweeps, bool split_whole,
+                TilePlan& plan, int max_tiles) {
     plan = TilePlan();
     struct Pending { int cloth; std::vector<TileOut> outs; };
     std::vector<Pending> per(cloths.size());
@@ -604,7 +607,7 @@ void plan_tiles(std::vector<Cloth>& cloths, int whole_load, int max_load, int sw
     for (size_t ci = 0; ci < cloths.size(); ci++) {
         Cloth& c = cloths[ci];
         per[ci].cloth = (int)ci;
-        const bool fits = c.nv <= whole_load;
+        const bool fits = one_tile(c, whole);
         c.whole = fits && !split_whole;
         c.max_loaded = 0;
         if (fits) {
@@ -628,6 +631,8 @@ void plan_tiles(std::vector<Cloth>& cloths, int whole_load, int max_load, int sw
     }
     // Many cloths are planned side by side, few cloths block by block.
     std::atomic_bool failed{false};
+    std::atomic<int> ntiles{(int)(cloths.size() - work.size())};
+    auto too_many = [&] { return max_tiles > 0 && ntiles > max_tiles; };
     const unsigned outer = work.size() >= hw ? hw : 1, inner = work.size() >= hw ? 1 : hw;
     parallel_for(work.size(), outer, [&](size_t w) {
         const int ci = work[w];
@@ -640,6 +645,7 @@ void plan_tiles(std::vector<Cloth>& cloths, int whole_load, int max_load, int sw
             std::vector<int> mark((size_t)c.nv, -1), entry((size_t)c.nv, 0);
             int stamp = 0;
             blocks = nominal_blocks(c, topo, max_load, phases, mark, entry, stamp);
+            ntiles += (int)blocks.size();
         }
         std::vector<std::vector<TileOut>> outs(blocks.size());
         // runs of blocks share one set of marks
@@ -647,9 +653,12 @@ void plan_tiles(std::vector<Cloth>& cloths, int whole_load, int max_load, int sw
         parallel_for((blocks.size() + run - 1) / run, inner, [&](size_t r) {
             std::vector<int> mark((size_t)c.nv, -1), entry((size_t)c.nv, 0);
             int stamp = 0;
-            for (size_t k = r * run; k < std::min(blocks.size(), (r + 1) * run); k++)
+            for (size_t k = r * run; k < std::min(blocks.size(), (r + 1) * run) && !too_many(); k++) {
                 if (!plan_block(c, topo, blocks[k], max_load, phases, mark, entry, stamp, outs[k])) failed = true;
+                ntiles += (int)outs[k].size() - 1;
+            }
         });
+        if (too_many()) return;
         auto& all = per[ci].outs;
         for (auto& o : outs)
             for (auto& t : o) all.push_back(std::move(t));
@@ -659,6 +668,7 @@ void plan_tiles(std::vector<Cloth>& cloths, int whole_load, int max_load, int sw
     });
     PBD_CHECK(!failed, PBD_ERR_LIMIT,
               "a single vertex's dependency cone exceeds the tile budget; lower the sweeps per launch");
+    if (too_many()) return false;
 
     // Flatten: offsets first, then the tiles' records side by side.
     struct Place { const Cloth* c; const TileOut* o; int own_at, vert_at, dist_at, bend_at; };
@@ -848,6 +858,7 @@ void plan_tiles(std::vector<Cloth>& cloths, int whole_load, int max_load, int sw
     for (int i = 0; i < (int)plan.tiles.size(); i++) (plan.tiles[i].whole ? whole_ids : part_ids).push_back(i);
     plan.whole_order = xcd_order(whole_ids);
     plan.partial_order = xcd_order(part_ids);
+    return true;
 }
 
 }  // namespace pbd

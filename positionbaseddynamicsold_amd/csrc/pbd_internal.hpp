@@ -434,15 +434,22 @@ struct TilePlan {
     // and distance prim updates of one launch of `sweeps` sweeps
     long long stat_loaded = 0, stat_interior = 0, stat_dist_loaded = 0, stat_dist_phase_needed = 0;
 };
+// Most vertices of a cloth that is one tile: grids with their own prims, meshes.
+struct WholeLoad {
+    int grid, mesh;
+};
+inline bool plain_grid(const Cloth& c) { return c.rx > 0 && !c.has_user_pairs; }
+bool one_tile(const Cloth& c, const WholeLoad& whole);
 // The budgets of `loads` (ascending) from the first at which a batch of grid
 // cloths takes about max_tiles tiles or fewer.
-std::vector<int> fitting_loads(const std::vector<Cloth>& cloths, int whole_load, const std::vector<int>& loads,
+std::vector<int> fitting_loads(const std::vector<Cloth>& cloths, const WholeLoad& whole, const std::vector<int>& loads,
                                int sweeps_per_launch, int max_tiles);
-// A cloth of at most whole_load vertices is one tile; the others' tiles load
-// at most max_load.  split_whole: a cloth that fits one tile still gets a
-// (single, halo-free) multi-launch tile instead of a whole tile.
-void plan_tiles(std::vector<Cloth>& cloths, int whole_load, int max_load, int sweeps_per_launch, bool split_whole,
-                TilePlan& plan);
+// A cloth within the whole load is one tile; the others' tiles load at most
+// max_load.  split_whole: a cloth that fits one tile still gets a (single,
+// halo-free) multi-launch tile instead of a whole tile.  With max_tiles > 0,
+// false and no plan once there would be more tiles.
+bool plan_tiles(std::vector<Cloth>& cloths, const WholeLoad& whole, int max_load, int sweeps_per_launch,
+                bool split_whole, TilePlan& plan, int max_tiles = 0);
 
 // ---------------------------------------------------------------------------
 // Kernel launchers (implemented in the .hip files)
