@@ -5,6 +5,8 @@
 #include <cmath>
 #include <cstring>
 #include <functional>
+#include <system_error>
+#include <thread>
 
 #include "pbd_internal.hpp"
 
@@ -133,7 +135,11 @@ struct pbd_ctx {
     pbd_profile prof{};
     std::vector<hipEvent_t> ev_pool;
     int ev_used = 0;
+    // pinned memory that state is read back through, and its bytes
+    void* readback = nullptr;
+    size_t readback_n = 0;
     ~pbd_ctx() {
+        if (readback) (void)hipHostFree(readback);
         for (auto e : ev_pool) (void)hipEventDestroy(e);
         for (auto& g : graph)
             if (g) (void)hipGraphExecDestroy(g);
@@ -2917,6 +2923,80 @@ int pbd_bench_copy(pbd_ctx* ctx, long long bytes, int reps, double* ms) {
     });
 }
 
+namespace {
+
+// Packed xyz of up to two arrays of n records to the caller's memory.  The GPU
+// packs chunks into pinned memory, which threads copy on, each with two chunks
+// in turn; pageable copies of the 16-byte records and unpacking them took 7 ms
+// for 2 x 1.4 million vertices (48 cloths), 1 ms so.
+constexpr int READ_CHUNK = 43520, READ_THREADS = 8;  // records per chunk (510 KiB)
+
+void read_xyz(pbd_ctx* c, const float4* const src[2], float* const dst[2], int n) {
+    struct Job { const float4* from; float* to; int n; };
+    std::vector<Job> jobs;
+    for (int a = 0; a < 2; a++)
+        for (int i = 0; dst[a] && i < n; i += READ_CHUNK)
+            jobs.push_back({src[a] + i, dst[a] + 3 * (size_t)i, std::min(READ_CHUNK, n - i)});
+    if (jobs.empty()) return;
+    const int threads = jobs.size() <= 2 ? 1 : std::min<int>(READ_THREADS, (int)(jobs.size() + 1) / 2);
+    const size_t room = ((size_t)12 * std::min(n, READ_CHUNK) + 63) / 64 * 64;  // of one chunk
+    const size_t need = room * 2 * threads;
+    if (c->readback_n < need) {
+        if (c->readback) (void)hipHostFree(c->readback);
+        c->readback = nullptr;
+        c->readback_n = 0;
+        PBD_HIP(hipHostMalloc(&c->readback, need, hipHostMallocDefault));
+        c->readback_n = need;
+    }
+    auto pinned = [&](int t, int half) { return (float*)((char*)c->readback + room * (2 * t + half)); };
+    if (threads == 1) {
+        for (size_t k = 0; k < jobs.size(); k++) launch_pack_xyz(c->stream, jobs[k].from, pinned(0, (int)k), jobs[k].n);
+        PBD_HIP(hipStreamSynchronize(c->stream));
+        for (size_t k = 0; k < jobs.size(); k++) memcpy(jobs[k].to, pinned(0, (int)k), (size_t)12 * jobs[k].n);
+        return;
+    }
+    std::vector<std::string> failed(threads);
+    auto work = [&](int t) {
+        hipEvent_t ev[2] = {nullptr, nullptr};
+        try {
+            set_device(c);
+            for (auto& e : ev) PBD_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            auto issue = [&](size_t k, int half) {
+                if (k >= jobs.size()) return;
+                launch_pack_xyz(c->stream, jobs[k].from, pinned(t, half), jobs[k].n);
+                PBD_HIP(hipEventRecord(ev[half], c->stream));
+            };
+            issue(t, 0);
+            issue((size_t)t + threads, 1);
+            int half = 0;
+            for (size_t k = t; k < jobs.size(); k += threads, half ^= 1) {
+                PBD_HIP(hipEventSynchronize(ev[half]));
+                memcpy(jobs[k].to, pinned(t, half), (size_t)12 * jobs[k].n);
+                issue(k + 2 * (size_t)threads, half);
+            }
+        } catch (const std::exception& e) {
+            failed[t] = e.what();
+        }
+        for (auto e : ev)
+            if (e) (void)hipEventDestroy(e);
+    };
+    std::vector<std::thread> pool;
+    try {
+        for (int t = 1; t < threads; t++) pool.emplace_back(work, t);
+    } catch (const std::system_error&) {
+        // fewer threads than asked for: this one does their share
+    }
+    const int started = (int)pool.size() + 1;
+    work(0);
+    for (int t = started; t < threads; t++) work(t);
+    for (auto& t : pool) t.join();
+    PBD_HIP(hipStreamSynchronize(c->stream));
+    for (auto& f : failed)
+        if (!f.empty()) throw Error(PBD_ERR_HIP, f);
+}
+
+}  // namespace
+
 int pbd_cloth_get_state(pbd_ctx* ctx, int id, int which, float* xyz) {
     return guard([&] {
         Cloth& c = cloth_of(ctx, id);
@@ -2926,14 +3006,9 @@ int pbd_cloth_get_state(pbd_ctx* ctx, int id, int which, float* xyz) {
         set_device(ctx);
         if (which == PBD_STATE_P) consolidate(ctx);
         DBuf<float4>& b = which == PBD_STATE_X ? ctx->x : which == PBD_STATE_V ? ctx->v : ctx->pbuf[ctx->pcur];
-        std::vector<float4> h(c.nv);
-        PBD_HIP(hipMemcpyAsync(h.data(), b.ptr + c.vbase, sizeof(float4) * c.nv, hipMemcpyDeviceToHost, ctx->stream));
-        PBD_HIP(hipStreamSynchronize(ctx->stream));
-        for (int i = 0; i < c.nv; i++) {
-            xyz[3 * i] = h[i].x;
-            xyz[3 * i + 1] = h[i].y;
-            xyz[3 * i + 2] = h[i].z;
-        }
+        const float4* const src[2] = {b.ptr + c.vbase, nullptr};
+        float* const dst[2] = {xyz, nullptr};
+        read_xyz(ctx, src, dst, c.nv);
     });
 }
 
@@ -3011,14 +3086,10 @@ int pbd_state_save(pbd_ctx* ctx, float* x, float* v) {
     return guard([&] {
         PBD_CHECK(ctx && ctx->inited, PBD_ERR_STATE, "call pbd_init first");
         set_device(ctx);
-        std::vector<float4> X, V;
-        ctx->x.download(X, ctx->stream);
-        ctx->v.download(V, ctx->stream);
+        const float4* const src[2] = {ctx->x.ptr, ctx->v.ptr};
+        float* const dst[2] = {x, v};
+        read_xyz(ctx, src, dst, ctx->nv_total);
         PBD_HIP(hipStreamSynchronize(ctx->stream));
-        for (int i = 0; i < ctx->nv_total; i++) {
-            if (x) { x[3 * i] = X[i].x; x[3 * i + 1] = X[i].y; x[3 * i + 2] = X[i].z; }
-            if (v) { v[3 * i] = V[i].x; v[3 * i + 1] = V[i].y; v[3 * i + 2] = V[i].z; }
-        }
     });
 }
 

@@ -619,5 +619,7 @@ void launch_fill_u64(hipStream_t s, unsigned long long* p, size_t n, unsigned lo
 void launch_fill_int(hipStream_t s, int* p, size_t n, int v);
 void launch_min_sweeps(hipStream_t s, int* sweeps, const int* cap, int sw, int n);
 void launch_copy(hipStream_t s, const float4* a, float4* b, size_t n);
+// xyz of n records, packed; out has room for a multiple of four floats.
+void launch_pack_xyz(hipStream_t s, const float4* a, float* out, int n);
 
 }  // namespace pbd

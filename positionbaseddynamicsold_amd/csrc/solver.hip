@@ -353,6 +353,25 @@ void launch_copy(hipStream_t s, const float4* a, float4* b, size_t n) {
     PBD_HIP(hipGetLastError());
 }
 
+// Four packed floats a thread, so that a wave writes 1 KiB in a row: `out` is
+// host memory, and the link to it bounds this kernel.
+__global__ __launch_bounds__(256) void k_pack_xyz(const float4* __restrict__ a, float4* __restrict__ out, int n) {
+    const int j = blockIdx.x * 256 + threadIdx.x;
+    if (4 * j >= 3 * n) return;
+    const int v = 4 * j / 3, k = 4 * j - 3 * v;
+    const float4 p = a[v], q = a[min(v + 1, n - 1)];
+    const float f[6] = {p.x, p.y, p.z, q.x, q.y, q.z};
+    out[j] = k == 0 ? make_float4(f[0], f[1], f[2], f[3])
+                    : k == 1 ? make_float4(f[1], f[2], f[3], f[4]) : make_float4(f[2], f[3], f[4], f[5]);
+}
+
+void launch_pack_xyz(hipStream_t s, const float4* a, float* out, int n) {
+    if (n <= 0) return;
+    const int quads = (int)((3ll * n + 3) / 4);
+    hipLaunchKernelGGL(k_pack_xyz, dim3((quads + 255) / 256), dim3(256), 0, s, a, (float4*)out, n);
+    PBD_HIP(hipGetLastError());
+}
+
 __global__ void k_fill_u64(unsigned long long* p, size_t n, unsigned long long v) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
