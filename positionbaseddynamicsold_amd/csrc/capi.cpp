@@ -2,6 +2,7 @@
 // solver orchestration.  Exceptions never cross this file's functions.
 #include <algorithm>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <functional>
@@ -52,6 +53,7 @@ struct pbd_ctx {
     int plan_sweeps = 0, plan_max_load = 0, plan_split = 0;
     bool plan_small = false;  // planned with tiles smaller than the budget on offer
     int plan_whole = 0;       // most vertices of a grid planned as one tile
+    int plan_steps = 0;       // and of a cloth planned for all its sweeps in one launch
     DBuf<TileDev> tiles;
     // launch orders: single-tile cloths' tiles, multi-tile cloths' tiles, and
     // both (the first launch of a substep runs them side by side)
@@ -432,7 +434,7 @@ int whole_grid_load(const pbd_ctx* c, int sweeps, int ml) {
 
 void replan_if_needed(pbd_ctx* c) {
     int s = effective_tile_sweeps(c), ml = effective_max_load(c), sp = c->sp.split_whole ? 1 : 0;
-    const WholeLoad whole{whole_grid_load(c, s, ml), ml};
+    WholeLoad whole{whole_grid_load(c, s, ml), ml, INT_MAX};
     // Tiles smaller than the budget where the multi-tile cloths would not fill
     // the GPU: a launch takes as long as its largest tile, so the smallest
     // tile size of at most one tile per CU is the fastest (a 389 x 211 cloth at
@@ -446,13 +448,22 @@ void replan_if_needed(pbd_ctx* c) {
             multi += k.nv;
             grids &= plain_grid(k);
         }
+    // Beside multi-tile cloths, a single-tile cloth's whole budget in the first
+    // launch holds up all the others unless the cloth is small (48 cloths of
+    // 240 to 87,000 vertices: 675 us per substep, 555 with no cloth whole).
+    // With bending even the smallest takes as long as the launches it holds up.
+    if (multi > 0 && !has_tolerance(c)) {
+        whole.steps = 2048;
+        for (auto& k : c->cloths)
+            if (k.nb > 0) whole.steps = 0;
+    }
     std::vector<int> loads;
     if (multi > 0 && grids && !c->ws.enabled)
         for (int load : {512, 768, 1024, 1280, 1536, 2048, 2560, 3072, 3584, 4096, 4608})
             if (load < ml && (long long)load * c->num_cu > multi) loads.push_back(load);
     const bool small = !loads.empty();
     if (s == c->plan_sweeps && ml == c->plan_max_load && sp == c->plan_split && small == c->plan_small &&
-        whole.grid == c->plan_whole)
+        whole.grid == c->plan_whole && whole.steps == c->plan_steps)
         return;
     // a failed plan leaves no valid one behind: the next call plans again
     c->plan_sweeps = 0;
@@ -475,6 +486,7 @@ void replan_if_needed(pbd_ctx* c) {
     c->plan_split = sp;
     c->plan_small = small;
     c->plan_whole = whole.grid;
+    c->plan_steps = whole.steps;
     upload_plan(c);
     fill_cloth_dev(c);
 }
@@ -1180,7 +1192,12 @@ bool project(pbd_ctx* c, int iterations, bool fused_whole, float dt, const int* 
                   "internal: the residuals were left to a launch that does not decide");
         if (!fold) ws_decide(s, dec->rs, ncl, dec->rule, dec->warm_sweeps, dec->full_sweeps, dec->cap, dec->keep);
     }
-    if (!fold) launch_fill_int(s, c->sweeps.ptr, ncl, 0);
+    // Fixed sweeps (no tolerance, no budgets): nothing reads the sweep counts
+    // or residual slots, and every cloth's result ends in the same buffer, so
+    // the substep is its tile launches alone (a 389 x 211 sheet: three small
+    // kernels of 4 us less beside five of 20).
+    const bool fixed = !any_tol && !cap;
+    if (!fold && !fixed) launch_fill_int(s, c->sweeps.ptr, ncl, 0);
     if (c->sp.path == PBD_PATH_JACOBI) {
         PBD_CHECK(!fused_whole && !delta, PBD_ERR_STATE, "internal: the Jacobi path is never fused");
         int sw = project_jacobi(c, iterations, cap, 0, c->nv_total, tol, -1);
@@ -1239,7 +1256,7 @@ bool project(pbd_ctx* c, int iterations, bool fused_whole, float dt, const int* 
     const bool int_store =
         integrate_end && !any_tol && !(fused_whole && c->any_partial && (nchunks < 2 || cap != nullptr));
     ensure_slots(c, nchunks);
-    if (!fold) launch_fill_u64(s, c->res_slots.ptr, (size_t)c->nslots * ncl, 0ull);
+    if (!fold && !fixed) launch_fill_u64(s, c->res_slots.ptr, (size_t)c->nslots * ncl, 0ull);
     const size_t lds = (size_t)std::max(1, c->plan.max_loaded) * sizeof(float4);
     const TileShape shape = tile_shape(c, (int)c->plan.tiles.size());
     const int threads = c->sp.block_threads > 0 ? c->sp.block_threads : 1024;
@@ -1286,6 +1303,8 @@ bool project(pbd_ctx* c, int iterations, bool fused_whole, float dt, const int* 
     // a fused substep advects every cloth in its first launch
     a.advect_load = fused_whole ? 1 : 0;
     a.integrate_end = int_store ? 1 : 0;
+    // with fixed sweeps they store into the buffer where the last chunk ends
+    if (fixed && c->any_partial && nchunks % 2 == 0) a.whole_out = c->pbuf[cur].ptr;
     if (c->any_whole && !c->any_partial) {
         a.sweep_base = 0;
         a.nsweeps = iterations;
@@ -1420,10 +1439,10 @@ bool project(pbd_ctx* c, int iterations, bool fused_whole, float dt, const int* 
     } else {
         cur ^= 1;
     }
-    if (!fold)  // the folded schedule kernel recorded them
+    if (!fold && !fixed)  // the folded schedule kernel recorded them
         launch_final_buffers(s, c->cl.ptr, ncl, start, launched, ts, iterations, any_tol ? nullptr : cap,
                              c->pfinal.ptr);
-    c->pfinal_valid = true;
+    c->pfinal_valid = !fixed;
     c->pcur = cur;
     if (any_tol || cap) {
         // per-cloth counts live on the device; read them now only if needed

@@ -608,7 +608,7 @@ bool plan_tiles(std::vector<Cloth>& cloths, const WholeLoad& whole, int max_load
         Cloth& c = cloths[ci];
         per[ci].cloth = (int)ci;
         const bool fits = one_tile(c, whole);
-        c.whole = fits && !split_whole;
+        c.whole = fits && !split_whole && c.nv <= whole.steps;
         c.max_loaded = 0;
         if (fits) {
             TileOut o;

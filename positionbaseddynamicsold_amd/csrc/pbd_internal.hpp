@@ -144,6 +144,7 @@ struct SolveArgs {
     int coherent_load;   // 1: p_in was written earlier in this launch by other workgroups (a queued
                          //    later chunk): loaded past every cache
     int substeps;        // fused single-tile cloths: substeps this launch runs
+    float4* whole_out;   // where single-tile cloths store p (nullptr: p_out)
     int lds_slots;       // vertices of dynamic LDS before the tail (set by the launch functions)
     int queue_ts;        // queued launches: sweeps per chunk; a tile whose cloth has a further chunk
                          //    stores p_out write-through for it (0: not queued)
@@ -434,9 +435,10 @@ struct TilePlan {
     // and distance prim updates of one launch of `sweeps` sweeps
     long long stat_loaded = 0, stat_interior = 0, stat_dist_loaded = 0, stat_dist_phase_needed = 0;
 };
-// Most vertices of a cloth that is one tile: grids with their own prims, meshes.
+// Most vertices of a cloth that is one tile: grids with their own prims,
+// meshes; and of one whose tile runs all its sweeps in one launch.
 struct WholeLoad {
-    int grid, mesh;
+    int grid, mesh, steps;
 };
 inline bool plain_grid(const Cloth& c) { return c.rx > 0 && !c.has_user_pairs; }
 bool one_tile(const Cloth& c, const WholeLoad& whole);
@@ -445,8 +447,8 @@ bool one_tile(const Cloth& c, const WholeLoad& whole);
 std::vector<int> fitting_loads(const std::vector<Cloth>& cloths, const WholeLoad& whole, const std::vector<int>& loads,
                                int sweeps_per_launch, int max_tiles);
 // A cloth within the whole load is one tile; the others' tiles load at most
-// max_load.  split_whole: a cloth that fits one tile still gets a (single,
-// halo-free) multi-launch tile instead of a whole tile.  With max_tiles > 0,
+// max_load.  split_whole: a cloth that fits one tile (or exceeds the steps)
+// still gets a (single, halo-free) multi-launch tile instead of a whole tile.  With max_tiles > 0,
 // false and no plan once there would be more tiles.
 bool plan_tiles(std::vector<Cloth>& cloths, const WholeLoad& whole, int max_load, int sweeps_per_launch,
                 bool split_whole, TilePlan& plan, int max_tiles = 0);

@@ -1105,6 +1105,7 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
     const bool integ = (td.whole && a.fused) || (a.integrate_end && a.sweep_base + nsweeps >= budget);
     // a queued chunk with a further chunk of its cloth after it hands its stores on
     const bool handoff = a.queue_ts > 0 && !td.whole && budget_c > a.sweep_base + a.queue_ts;
+    float4* const out = td.whole && a.whole_out ? a.whole_out : p_out;
     for (int i0 = tid; i0 < td.n_int; i0 += VERT_PREFETCH * T) {
         int g[VERT_PREFETCH];
 #pragma unroll
@@ -1119,7 +1120,7 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
                     const float4 Q = P[i0 + u * T];
                     v[g[u]] = make_float4((Q.x - X[u].x) / a.dt, (Q.y - X[u].y) / a.dt, (Q.z - X[u].z) / a.dt, 0.0f);
                     x[g[u]] = make_float4(Q.x, Q.y, Q.z, X[u].w);
-                    if (ss == nsub - 1) p_out[g[u]] = Q;
+                    if (ss == nsub - 1) out[g[u]] = Q;
                 }
         } else if (handoff) {
 #pragma unroll
@@ -1128,7 +1129,7 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
         } else {
 #pragma unroll
             for (int u = 0; u < VERT_PREFETCH; u++)
-                if (g[u] >= 0) p_out[g[u]] = P[i0 + u * T];
+                if (g[u] >= 0) out[g[u]] = P[i0 + u * T];
         }
     }
     }  // substeps
