@@ -401,6 +401,16 @@ TileShape tile_shape(const pbd_ctx* c, int ntiles) {
     t.threads = c->sp.block_threads > 0 ? c->sp.block_threads : 1024;
     t.regs = 0;
     t.lds = (size_t)std::max(1, c->plan.max_loaded) * sizeof(float4);
+    // Bending: a phase of a small tile has a few waves' work, and the waves
+    // without any still take issue slots and hold up the barrier (20 sweeps of
+    // 128^2 / 256^2 / 400^2 / 512^2 vertices: 591 / 639 / 830 / 992 us with 512
+    // threads, 609 / 657 / 818 / 960 with 768, 642 / 685 / 834 / 973 with 1024).
+    if (!c->plan.bend.empty() && c->sp.block_threads == 0) {
+        int most = 0;
+        for (auto& k : c->cloths)
+            if (k.np() > 0) most = std::max(most, k.max_loaded);
+        t.threads = most <= 2560 ? 512 : 768;
+    }
     if (!c->plan.bend.empty() || c->ncolors_max > REG_COLORS || ntiles > c->num_cu) return t;
     const int m = c->plan.max_phase;
     if (c->sp.block_threads == 0 && m <= 1024) t.threads = std::max(256, (m + 63) / 64 * 64);
