@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256) void k_cell_ranges(const uint32_t* __restrict_
 // visited once per vertex, so a pair comes up once.  The form this replaces
 // made the pairs of every triangle (3.7 times as many on a folded 256 x 256
 // cloth), stored them, sorted them twice and compacted them: 2.6 ms per
-// detection there against 0.3 ms for the table, the visit and the narrowphase.
+// detection there against 0.15 ms for the table, the visit and the narrowphase.
 // ---------------------------------------------------------------------------
 constexpr int SWEPT_MAX_CELLS = 4096;  // cells of the caller's grid one box may span
 constexpr int ENTRY_MAX_CELLS = 64;    // cells of the table's own grid a face is entered in
@@ -240,7 +240,7 @@ struct alignas(64) FaceRec {
     int pad[2];
 };
 
-// Whether a vertex outside the face's swept box widened by 6 thickness cannot
+// Whether a vertex outside the face's swept box widened by 4.5 thickness cannot
 // pass the narrowphase's floating-point tests: the face keeps a good shape
 // over the whole step (doubled area at least 0.05 of its longest edge squared,
 // bounded below from the start's area and the edges' changes), so barycentric
@@ -258,6 +258,88 @@ __device__ __forceinline__ bool face_cullable(const float4* X, const float4* P, 
     const float longest = fmaxf(fmaxf(l1, l2), sqrtf(dot(e3, e3))) + m1 + m2;
     const float area = sqrtf(dot(c, c)) - (l1 * m2 + l2 * m1 + m1 * m2);
     return area >= 0.05f * (longest * longest) && th >= 4e-3f * longest;  // false for NaN
+}
+
+// Half-spaces that hold every vertex that can touch a face (cullable faces;
+// others: all of space).  The narrowphase accepts a vertex at a time t whose
+// distance from the face's plane is at most 2 thickness and whose barycentric
+// coordinates are at least -e, e = thickness / mean edge length.  Along a
+// direction m such a point lies below the extended corners
+// (1 + 3 e) m.c_k - e sum(m.c), which are linear in t, plus 2 thickness
+// |m.n(t)|.  m are the outward normals of the edges in the face's plane at
+// t = 1/2, for which |m.n(t)| is bounded by the change of the edges, and the
+// plane's normal, both ways.  The slack covers the rounding of the
+// narrowphase's coordinates (relative to their size) and of its barycentric
+// coordinates (1e-4 for cullable faces).  Coordinates are relative to a corner.
+struct FaceAxes {
+    float4 edge[3];  // m, highest m.c
+    float4 plane;    // n, highest n.c
+    float4 origin;   // the corner, lowest n.c
+};
+
+__device__ __forceinline__ FaceAxes face_axes(const float4* X, const float4* P, float th) {
+    V3 c[2][3];
+    float size = 0.0f;
+    for (int k = 0; k < 3; k++) {
+        c[0][k] = mk(X[k].x - X[0].x, X[k].y - X[0].y, X[k].z - X[0].z);
+        c[1][k] = mk(P[k].x - X[0].x, P[k].y - X[0].y, P[k].z - X[0].z);
+        size = fmaxf(size, fmaxf(fmaxf(fabsf(X[k].x), fabsf(X[k].y)), fabsf(X[k].z)));
+        size = fmaxf(size, fmaxf(fmaxf(fabsf(P[k].x), fabsf(P[k].y)), fabsf(P[k].z)));
+    }
+    const V3 e1 = c[0][1], e2 = c[0][2], e3 = sub(e2, e1);
+    const V3 d1 = sub(sub(c[1][1], c[1][0]), e1), d2 = sub(sub(c[1][2], c[1][0]), e2), d3 = sub(d2, d1);
+    auto len = [](V3 a) { return sqrtf(dot(a, a)); };
+    const float l1 = len(e1), l2 = len(e2), l3 = len(e3), m1 = len(d1), m2 = len(d2), m3 = len(d3);
+    const float area = len(cross(e1, e2)) - (l1 * m2 + l2 * m1 + m1 * m2);  // lowest over the step
+    const float mean = (l1 + l2 + l3 - (m1 + m2 + m3)) / 3.0f;
+    const float e = 1.001f * th / mean;
+    const float turn = fminf(1.0f, 1e-3f + (0.5f * (l1 * m2 + l2 * m1) + 0.75f * m1 * m2) / area);
+    const float slack = 0.5f * th + 4e-6f * size;
+    FaceAxes r;
+    r.origin = make_float4(X[0].x, X[0].y, X[0].z, -INFINITY);
+    r.plane = r.edge[0] = r.edge[1] = r.edge[2] = make_float4(0.0f, 0.0f, 0.0f, INFINITY);
+    if (!(mean >= 0.25f * fmaxf(fmaxf(l1, l2), l3)) || !face_cullable(X, P, th)) return r;
+    V3 h[3];
+    for (int k = 0; k < 3; k++) h[k] = scale(0.5f, mk(c[0][k].x + c[1][k].x, c[0][k].y + c[1][k].y, c[0][k].z + c[1][k].z));
+    const V3 big = cross(sub(h[1], h[0]), sub(h[2], h[0]));
+    const V3 n = scale(1.0f / len(big), big);
+    auto range = [&](V3 m, float* lo, float* hi) {
+        *lo = INFINITY;
+        *hi = -INFINITY;
+        for (int t = 0; t < 2; t++) {
+            const float a = dot(m, c[t][0]), b = dot(m, c[t][1]), d = dot(m, c[t][2]), s = e * (a + b + d);
+            *hi = fmaxf(*hi, fmaxf(fmaxf(a, b), d) * (1.0f + 3.0f * e) - s);
+            *lo = fminf(*lo, fminf(fminf(a, b), d) * (1.0f + 3.0f * e) - s);
+        }
+    };
+    float lo, hi;
+    for (int k = 0; k < 3; k++) {
+        const V3 along = sub(h[k == 2 ? 0 : k + 1], h[k]), o = cross(along, n);
+        const V3 m = scale(1.0f / len(o), o);
+        range(m, &lo, &hi);
+        r.edge[k] = make_float4(m.x, m.y, m.z, hi + 2.0f * th * turn + slack);
+    }
+    range(n, &lo, &hi);
+    r.plane = make_float4(n.x, n.y, n.z, hi + 2.0f * th + slack);
+    r.origin.w = lo - 2.0f * th - slack;
+    return r;
+}
+
+// Whether the vertex stays outside one of the half-spaces (false for NaN).
+__device__ __forceinline__ bool axes_miss(const FaceAxes& f, float4 x, float4 p) {
+    const V3 a = mk(x.x - f.origin.x, x.y - f.origin.y, x.z - f.origin.z);
+    const V3 b = mk(p.x - f.origin.x, p.y - f.origin.y, p.z - f.origin.z);
+    // the rounding of the vertex's own coordinates along its way
+    const float own = 2e-6f * fmaxf(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fabsf(x.z)),
+                                    fmaxf(fmaxf(fabsf(p.x), fabsf(p.y)), fabsf(p.z)));
+    bool out = false;
+    for (int k = 0; k < 3; k++) {
+        const V3 m = mk(f.edge[k].x, f.edge[k].y, f.edge[k].z);
+        out = out || fminf(dot(m, a), dot(m, b)) - own > f.edge[k].w;
+    }
+    const V3 n = mk(f.plane.x, f.plane.y, f.plane.z);
+    const float na = dot(n, a), nb = dot(n, b);
+    return out || fminf(na, nb) - own > f.plane.w || fmaxf(na, nb) + own < f.origin.w;
 }
 
 __device__ __forceinline__ FaceRec face_record(int f, const float4* __restrict__ x, const float4* __restrict__ p,
@@ -305,12 +387,18 @@ __global__ __launch_bounds__(256) void k_face_cells(HashCfg g, const float4* __r
 __global__ __launch_bounds__(256) void k_cell_fill(int nt, const int4* __restrict__ tcell, const int* __restrict__ rank,
                                                    const int* __restrict__ cnt, const int* __restrict__ end,
                                                    const float4* __restrict__ x, const float4* __restrict__ p,
-                                                   const int* __restrict__ tris, float th, FaceRec* __restrict__ ent) {
+                                                   const int* __restrict__ tris, float th, FaceRec* __restrict__ ent,
+                                                   FaceAxes* __restrict__ axes) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nt) return;
     const int4 c = tcell[t];
     if (c.w < 0) return;
-    FaceRec r = face_record(t, x, p, tris, th, 6.0f * th);
+    if (axes) {
+        const int3 v = make_int3(tris[3 * t], tris[3 * t + 1], tris[3 * t + 2]);
+        const float4 X[3] = {x[v.x], x[v.y], x[v.z]}, P[3] = {p[v.x], p[v.y], p[v.z]};
+        axes[t] = face_axes(X, P, th);
+    }
+    FaceRec r = face_record(t, x, p, tris, th, 4.5f * th);
     r.cx = c.x;
     r.cy = c.y;
     r.cz = c.z;
@@ -455,31 +543,87 @@ struct PairSink {
     }
 };
 
-// One round of a group's visit: lane l (of 32) of the group holds a run of
-// `mine` entries starting at `start` (0 entries: none); calls f(e, l) for every
-// entry e of every lane l's run, the lanes taking them in turn, and f(-1, l)
-// for the lanes left over.  Both groups of a wave stay in the loop until the
-// longer is done, so f may use wave-wide operations.
+// Data parallel primitives over the 32 lanes of a group.
+template <int CTRL>
+__device__ __forceinline__ int dpp(int v, int old) {
+    return __builtin_amdgcn_update_dpp(old, v, CTRL, 0xf, 0xf, false);
+}
+template <class Op>
+__device__ __forceinline__ int group_reduce(int v, Op&& op) {
+    v = op(v, dpp<0xb1>(v, v));   // lanes xor 1
+    v = op(v, dpp<0x4e>(v, v));   // lanes xor 2
+    v = op(v, dpp<0x141>(v, v));  // half rows mirrored: the other four of eight
+    v = op(v, dpp<0x140>(v, v));  // rows mirrored: the other eight of sixteen
+    return op(v, __builtin_amdgcn_ds_swizzle(v, 0x401f));  // lanes xor 16
+}
+// Sum of the lanes up to and including this one.
+__device__ __forceinline__ int group_scan(int v) {
+    v += dpp<0x111>(v, 0);  // one lane up the row, then 2, 4, 8
+    v += dpp<0x112>(v, 0);
+    v += dpp<0x114>(v, 0);
+    v += dpp<0x118>(v, 0);
+    // the last lane of rows 0 and 2 to all of rows 1 and 3
+    return v + __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+}
+__device__ __forceinline__ void lds_ready() {  // this wave's LDS writes, to its own lanes
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// LDS of a group of 32 lanes.
+constexpr int BOX_CELLS = 256, RUN_WINDOW = 1024;
+struct GroupLds {
+    unsigned cover[BOX_CELLS / 32];     // the cells of a box that are visited
+    unsigned starts[RUN_WINDOW / 32];   // entries of the window that start a run
+    int4 run[64];                       // cell, and where its entries lie less those of the runs before
+};
+
+// One round of a group's visit: every lane brings two cells q with n entries
+// from `start` on (0: none); calls f(e, cell) for every entry, the lanes taking
+// them in turn, and f(-1, cell) for the lanes left over.  An entry finds its
+// run by counting the starts before it: a bit per entry in LDS, and one LDS
+// read of the run (a binary search by shuffles took 14 LDS operations an
+// entry; with it the visit of the folded 256 x 256 cloth took 119 us, 105 so).
+// Both groups of a wave stay in the loops until the longer is done, so f may
+// use wave-wide operations.
 template <class F>
-__device__ __forceinline__ void visit_runs(int start, int mine, F&& f) {
-    const int l = threadIdx.x & 31;
-    int sum = mine;
-    for (int off = 1; off < 32; off <<= 1) {
-        const int o = __shfl_up(sum, off, 32);
-        if (l >= off) sum += o;
-    }
+__device__ __forceinline__ void visit_runs(GroupLds& lds, const int3* q, const int* start, const int* n, F&& f) {
+    const int lane = threadIdx.x & 63, l = lane & 31;
+    const int sum = group_scan(n[0] + n[1]);
     const int total = __shfl(sum, 31, 32);
-    const int before = sum - mine;
+    const int before[2] = {sum - n[0] - n[1], sum - n[1]};
+    const unsigned below = (1u << l) - 1u;
+    unsigned has[2];
+    for (int c = 0; c < 2; c++) {
+        const unsigned long long m = __ballot(n[c] > 0);
+        has[c] = lane < 32 ? (unsigned)m : (unsigned)(m >> 32);
+    }
+    int id = __popc(has[0] & below) + __popc(has[1] & below);
+    __builtin_amdgcn_wave_barrier();  // the round before is done with the lists
+    for (int c = 0; c < 2; c++)
+        if (n[c] > 0) lds.run[id++] = make_int4(q[c].x, q[c].y, q[c].z, start[c] - before[c]);
     const int longest = max(total, __shfl_xor(total, 32));
-    for (int b = 0; b < longest; b += 32) {
-        const int i = b + l;
-        int at = 0;  // the last lane whose runs before it do not exceed i
-        for (int step = 16; step > 0; step >>= 1)
-            if (__shfl(before, at + step, 32) <= i) at += step;
-        const int e = __shfl(start, at, 32) + i - __shfl(before, at, 32);
-        f(i < total ? e : -1, at);
+    int runs = 0;  // that start before the current entries
+    for (int w0 = 0; w0 < longest; w0 += RUN_WINDOW) {
+        __builtin_amdgcn_wave_barrier();
+        lds.starts[l] = 0;
+        lds_ready();
+        for (int c = 0; c < 2; c++) {
+            const int at = before[c] - w0;
+            if (n[c] > 0 && at >= 0 && at < RUN_WINDOW) atomicOr(&lds.starts[at >> 5], 1u << (at & 31));
+        }
+        lds_ready();
+        const int w1 = min(longest, w0 + RUN_WINDOW);
+        for (int b = w0; b < w1; b += 32) {
+            const unsigned word = lds.starts[(b - w0) >> 5];
+            const int i = b + l;
+            const int4 r = lds.run[i < total ? runs + __popc(word & (0xffffffffu >> (31 - l))) - 1 : 0];
+            runs += __popc(word);
+            f(i < total ? i + r.w : -1, make_int3(r.x, r.y, r.z));
+        }
     }
 }
+static_assert(RUN_WINDOW == 32 * 32, "a lane clears one word of the window");
 
 // Whether c is a valid cell and (x, y, z) is within one cell of it.
 __device__ __forceinline__ bool near_cell(int4 c, int x, int y, int z) {
@@ -490,111 +634,141 @@ __device__ __forceinline__ int3 around(int4 c, int l) {
     return make_int3(c.x + l % 3 - 1, c.y + l / 3 % 3 - 1, c.z + l / 9 - 1);
 }
 
-// The cells around a group's own triangles, each once, 32 at a time: the cells
-// of the box of their cells that lie around one of them.  A group with more
-// than 32 triangles or a box of more than BOX_CELLS cells takes the 27 cells
-// around one triangle after the other instead, without those that lie around
-// an earlier one.
-constexpr int BOX_CELLS = 256;
+// The cells around a group's own triangles, each once, two per lane and round
+// (most boxes have 27 to 64 cells, which then take one round of memory
+// latencies): the cells of the box of their cells that lie around one of them.
+// A group with more than 32 triangles or a box of more than BOX_CELLS cells
+// takes the 27 cells around one triangle after the other instead, without
+// those that lie around an earlier one.
 struct CellRounds {
-    int4* own;  // in LDS, 32 per group
+    const GroupLds* lds;
     const int* list;
     const int4* tcell;
     int deg, rounds;
     bool boxed;
     int3 lo, w;
-    // Called by all lanes of the wave, after the lanes are done with `own`.
-    __device__ __forceinline__ void start(int4* own_, const int* list_, int deg_, const int4* tcell_) {
-        own = own_;
+    // Called by all lanes of the wave.
+    __device__ __forceinline__ void start(GroupLds& g, const int* list_, int deg_, const int4* tcell_) {
+        lds = &g;
         list = list_;
         tcell = tcell_;
         deg = deg_;
         const int l = threadIdx.x & 31;
         const int4 c = l < deg ? tcell[list[l]] : make_int4(0, 0, 0, -1);
-        own[l] = c;
-        int m[3] = {c.w >= 0 ? c.x : INT_MAX, c.w >= 0 ? c.y : INT_MAX, c.w >= 0 ? c.z : INT_MAX};
-        int M[3] = {c.w >= 0 ? c.x : INT_MIN, c.w >= 0 ? c.y : INT_MIN, c.w >= 0 ? c.z : INT_MIN};
-        for (int off = 16; off > 0; off >>= 1)
-            for (int k = 0; k < 3; k++) {
-                m[k] = min(m[k], __shfl_xor(m[k], off, 32));
-                M[k] = max(M[k], __shfl_xor(M[k], off, 32));
-            }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        lo = make_int3(m[0] - 1, m[1] - 1, m[2] - 1);
+        const bool valid = c.w >= 0;
+        auto least = [](int a, int b) { return min(a, b); };
+        auto most = [](int a, int b) { return max(a, b); };
+        lo = make_int3(group_reduce(valid ? c.x : INT_MAX, least), group_reduce(valid ? c.y : INT_MAX, least),
+                       group_reduce(valid ? c.z : INT_MAX, least));
+        const int3 hi = make_int3(group_reduce(valid ? c.x : INT_MIN, most), group_reduce(valid ? c.y : INT_MIN, most),
+                                  group_reduce(valid ? c.z : INT_MIN, most));
         long long n = 0;
-        if (M[0] >= m[0]) {
-            long long s[3];
-            for (int k = 0; k < 3; k++) s[k] = min((long long)M[k] - m[k] + 3, (long long)BOX_CELLS + 1);
-            w = make_int3((int)s[0], (int)s[1], (int)s[2]);
-            n = s[0] * s[1] * s[2];
+        w = make_int3(1, 1, 1);
+        if (hi.x >= lo.x) {
+            const long long top = BOX_CELLS + 1;
+            w = make_int3((int)min((long long)hi.x - lo.x + 3, top), (int)min((long long)hi.y - lo.y + 3, top),
+                          (int)min((long long)hi.z - lo.z + 3, top));
+            n = (long long)w.x * w.y * w.z;
         }
+        lo = make_int3(lo.x - 1, lo.y - 1, lo.z - 1);
         boxed = deg <= 32 && n <= BOX_CELLS;
-        rounds = boxed ? ((int)n + 31) / 32 : deg;
+        rounds = boxed ? ((int)n + 63) / 64 : deg;
+        // mark the 27 cells around each triangle
+        __builtin_amdgcn_wave_barrier();  // the group before is done with `cover`
+        if (l < BOX_CELLS / 32) g.cover[l] = 0;
+        lds_ready();
+        const int at = valid ? ((c.z - lo.z) * w.y + c.y - lo.y) * w.x + c.x - lo.x : -1;
+        const int off = ((l / 9 - 1) * w.y + l / 3 % 3 - 1) * w.x + l % 3 - 1;
+        const int m = boxed ? deg : 0, longest = max(m, __shfl_xor(m, 32));
+        for (int j = 0; j < longest; j++) {
+            const int a = __shfl(at, j, 32);
+            if (j < m && l < 27 && a >= 0) atomicOr(&g.cover[(a + off) >> 5], 1u << ((a + off) & 31));
+        }
+        lds_ready();
     }
-    // This lane's cell of round r, if it has one.
-    __device__ __forceinline__ bool cell(const HashCfg& g, int r, int3* q) const {
+    // This lane's cell c of round r, if it has one.
+    __device__ __forceinline__ bool cell(const HashCfg& g, int r, int c, int3* q) const {
         const int l = threadIdx.x & 31;
         *q = make_int3(0, 0, 0);
         if (r >= rounds) return false;
         if (boxed) {
-            const int i = 32 * r + l, z = i / (w.x * w.y), y = (i - z * (w.x * w.y)) / w.x;
-            *q = make_int3(lo.x + i - (z * w.y + y) * w.x, lo.y + y, lo.z + z);
-            if (z >= w.z) return false;
-            bool in = false;
-            for (int j = 0; j < deg; j++) in |= near_cell(own[j], q->x, q->y, q->z);
-            return in && cell_key(g, q->x, q->y, q->z) >= 0;
+            const int i = 64 * r + 32 * c + l;
+            if (i >= BOX_CELLS || !(lds->cover[i >> 5] >> (i & 31) & 1)) return false;
+            // i is small: the quotients of i + 1/2 are far enough from whole numbers
+            const int z = (int)(((float)i + 0.5f) * __builtin_amdgcn_rcpf((float)(w.x * w.y))), j = i - z * (w.x * w.y);
+            const int y = (int)(((float)j + 0.5f) * __builtin_amdgcn_rcpf((float)w.x));
+            *q = make_int3(lo.x + j - y * w.x, lo.y + y, lo.z + z);
+            return cell_key(g, q->x, q->y, q->z) >= 0;
         }
         const int4 tc = tcell[list[r]];
         *q = around(tc, l);
-        if (tc.w < 0 || l >= 27) return false;
+        if (tc.w < 0 || l >= 27 || c) return false;
         for (int j = 0; j < r; j++)
             if (near_cell(tcell[list[j]], q->x, q->y, q->z)) return false;
         return cell_key(g, q->x, q->y, q->z) >= 0;
     }
+    // The entries of this lane's cells q of round r; whether there are any.
+    __device__ __forceinline__ bool runs(const HashCfg& g, int r, const int* __restrict__ cnt,
+                                         const int* __restrict__ end, unsigned mask, int3* q, int* start, int* n) const {
+        for (int c = 0; c < 2; c++) {
+            const bool mine = cell(g, r, c, &q[c]);
+            const unsigned slot = mine ? cell_slot(q[c].x, q[c].y, q[c].z, mask) : 0u;
+            const int k = cnt[slot], e = end[slot];
+            n[c] = mine ? k : 0;
+            start[c] = e - k;
+        }
+        return n[0] + n[1] > 0;
+    }
     // Whether c is a cell around one of the triangles.
     __device__ __forceinline__ bool meets(int4 c) const {
         if (c.w < 0) return false;
+        if (boxed) {
+            const unsigned x = c.x - lo.x, y = c.y - lo.y, z = c.z - lo.z;
+            if (x >= (unsigned)w.x || y >= (unsigned)w.y || z >= (unsigned)w.z) return false;
+            const int i = ((int)z * w.y + (int)y) * w.x + (int)x;
+            return rounds && (lds->cover[i >> 5] >> (i & 31) & 1);
+        }
         bool in = false;
-        if (boxed)
-            for (int j = 0; j < deg; j++) in |= near_cell(own[j], c.x, c.y, c.z);
-        else
-            for (int j = 0; j < deg && !in; j++) in = near_cell(tcell[list[j]], c.x, c.y, c.z);
+        for (int j = 0; j < deg && !in; j++) in = near_cell(tcell[list[j]], c.x, c.y, c.z);
         return in;
     }
 };
 
 // Vertex-face candidates by centroid cells.  Group = 32 lanes = one vertex.
 // All candidates are counted; listed are all of them (LIST) or those that no
-// box rules out.
+// box rules out.  Memory latency bounds it (71% of the wave cycles wait), so
+// registers are held to 64 for eight waves per SIMD: 81 us against 95 with
+// seven on the folded 256 x 256 cloth (5 million pairs).
 template <bool LIST>
-__global__ __launch_bounds__(64 * VISIT_WAVES) void k_vf_candidates(
+__global__ __launch_bounds__(64 * VISIT_WAVES, 8) void k_vf_candidates(
     HashCfg g, const float4* __restrict__ x, const float4* __restrict__ p, int nv, const int* __restrict__ vtoff,
     const int* __restrict__ vtri, const int4* __restrict__ tcell, const int* __restrict__ cnt,
     const int* __restrict__ end, unsigned mask, const FaceRec* __restrict__ ent, DetectCounts* __restrict__ c,
     int2* __restrict__ out, unsigned cap) {
     __shared__ int2 buf[VISIT_WAVES][VISIT_BUF];
-    __shared__ int4 own[VISIT_WAVES][2][32];
+    __shared__ GroupLds group[VISIT_WAVES][2];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    GroupLds& lds = group[wv][lane >> 5];
     PairSink sink{buf[wv], 0, (int)((blockIdx.x * VISIT_WAVES + wv) % NEAR_BUCKETS), c, out, cap};
     int pairs = 0;
     const int stride = (int)gridDim.x * VISIT_WAVES * 2;
     for (int v0 = ((int)blockIdx.x * VISIT_WAVES + wv) * 2; v0 < nv; v0 += stride) {
         const int v = v0 + (lane >> 5), at = min(v, nv - 1);
         const int o = vtoff[at], deg = v < nv ? vtoff[at + 1] - o : 0;
-        const SweptBox b = vertex_box(x[at], p[at]);
+        SweptBox b = vertex_box(x[at], p[at]);
+        for (int k = 0; k < 3; k++) {  // the rounding of positions between the two
+            const float m = 1e-6f * fmaxf(fabsf(b.lo[k]), fabsf(b.hi[k]));
+            b.lo[k] -= m;
+            b.hi[k] += m;
+        }
         CellRounds cells;
-        __builtin_amdgcn_wave_barrier();  // the vertex before is done with `own`
-        cells.start(own[wv][lane >> 5], vtri + o, deg, tcell);
+        cells.start(lds, vtri + o, deg, tcell);
         const int rounds = max(cells.rounds, __shfl_xor(cells.rounds, 32));
         for (int r = 0; r < rounds; r++) {
-            int3 q;
-            const bool mine = cells.cell(g, r, &q);
-            if (!__any(mine)) continue;
-            const unsigned slot = cell_slot(q.x, q.y, q.z, mask);
-            const int n = mine ? cnt[slot] : 0;
-            visit_runs(n ? end[slot] - n : 0, n, [&](int e, int from) {
-                const int3 fq = make_int3(__shfl(q.x, from, 32), __shfl(q.y, from, 32), __shfl(q.z, from, 32));
+            int3 q[2];
+            int start[2], n[2];
+            if (!__any(cells.runs(g, r, cnt, end, mask, q, start, n))) continue;
+            visit_runs(lds, q, start, n, [&](int e, int3 fq) {
                 bool hit = false;
                 int f = 0;
                 if (e >= 0) {
@@ -623,6 +797,7 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_swept_candidates(
     const int2* __restrict__ ent, int ent_cap, const FaceRec* __restrict__ rec, const int* __restrict__ large,
     DetectCounts* __restrict__ c, int2* __restrict__ out, unsigned cap) {
     __shared__ int2 buf[VISIT_WAVES][VISIT_BUF];
+    __shared__ GroupLds group[VISIT_WAVES][2];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 31;
     PairSink sink{buf[wv], 0, (int)((blockIdx.x * VISIT_WAVES + wv) % NEAR_BUCKETS), c, out, cap};
     const int nlarge = (int)c->large;
@@ -653,18 +828,22 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_swept_candidates(
             sink.add(hit, v, f);
         };
         const int most = max(cells, __shfl_xor(cells, 32));
-        for (int c0 = 0; c0 < most; c0 += 32) {
-            const int3 q = cell_of(c0 + l);
-            const unsigned slot = cell_slot(q.x, q.y, q.z, mask);
-            int n = c0 + l < cells ? cnt[slot] : 0;
-            const int e1 = n ? end[slot] : 0;
-            if (e1 > ent_cap) n = 0;  // the table did not fit: the caller starts over
-            visit_runs(e1 - n, n, [&](int e, int from) {
+        for (int c0 = 0; c0 < most; c0 += 64) {
+            int3 q[2];
+            int start[2], n[2];
+            for (int c = 0; c < 2; c++) {
+                const bool mine = c0 + 32 * c + l < cells;
+                q[c] = cell_of(c0 + 32 * c + l);
+                const unsigned slot = mine ? cell_slot(q[c].x, q[c].y, q[c].z, mask) : 0u;
+                const int m = cnt[slot], e1 = end[slot];
+                n[c] = mine && e1 <= ent_cap ? m : 0;  // beyond: the table did not fit, the caller starts over
+                start[c] = e1 - m;
+            }
+            visit_runs(group[wv][lane >> 5], q, start, n, [&](int e, int3 fq) {
                 bool in = false;
                 int f = 0;
                 if (e >= 0) {
                     const int2 en = ent[e];
-                    const int3 fq = cell_of(c0 + from);
                     f = en.x;
                     in = (en.y & 0x7ffffff) == cell_code(fq.x, fq.y, fq.z) && ((en.y >> 27 & 1) || fq.x == lo[0]) &&
                          ((en.y >> 28 & 1) || fq.y == lo[1]) && ((en.y >> 29 & 1) || fq.z == lo[2]);
@@ -775,8 +954,9 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_ee_candidates(
     int2* __restrict__ out, unsigned cap) {
     __shared__ int2 buf[VISIT_WAVES][VISIT_BUF];
     __shared__ int4 ring_s[VISIT_WAVES][2][RING_MAX / 4];
-    __shared__ int4 own[VISIT_WAVES][2][32];
+    __shared__ GroupLds group[VISIT_WAVES][2];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 31;
+    GroupLds& lds = group[wv][lane >> 5];
     int4* ring = ring_s[wv][lane >> 5];
     PairSink sink{buf[wv], 0, (int)((blockIdx.x * VISIT_WAVES + wv) % NEAR_BUCKETS), c, out, cap};
     int pairs = 0;
@@ -801,7 +981,7 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_ee_candidates(
                                                   : i < n0 + n1 + 2 ? vnbr[r1 + i - 2 - n0]
                                                                     : -1;
         CellRounds cells;
-        cells.start(own[wv][lane >> 5], etri + o, deg, tcell);
+        cells.start(lds, etri + o, deg, tcell);
         auto ringed = [&](int u, int w) {
             bool in = false;
             if (fits) {
@@ -818,13 +998,10 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_ee_candidates(
         };
         const int rounds = max(cells.rounds, __shfl_xor(cells.rounds, 32));
         for (int r = 0; r < rounds; r++) {
-            int3 q;
-            const bool mine = cells.cell(g, r, &q);
-            if (!__any(mine)) continue;
-            const unsigned slot = cell_slot(q.x, q.y, q.z, mask);
-            const int n = mine ? cnt[slot] : 0;
-            visit_runs(n ? end[slot] - n : 0, n, [&](int e, int from) {
-                const int3 fq = make_int3(__shfl(q.x, from, 32), __shfl(q.y, from, 32), __shfl(q.z, from, 32));
+            int3 q[2];
+            int start[2], n[2];
+            if (!__any(cells.runs(g, r, cnt, end, mask, q, start, n))) continue;
+            visit_runs(lds, q, start, n, [&](int e, int3 fq) {
                 bool hit = false;
                 int eb = 0;
                 if (e >= 0) {
@@ -1028,25 +1205,32 @@ struct NearRun {
 
 // The narrowphase over the listed pairs (their number is on the device), its
 // contacts appended in any order.  STORE: time, normal and weights too (the
-// response needs only the vertices).
+// response needs only the vertices).  axes (may be null): pairs outside the
+// face's half-spaces are dropped first, and the workgroup gathers the others
+// until it has one for every thread, since the cubic is some 3000 instructions
+// (folded 256 x 256 cloth: 17,000 of 1.1 million pairs are left; 160 us
+// without the half-spaces, 33 with them).
 template <bool STORE>
 __global__ __launch_bounds__(256) void k_narrow(const int2* __restrict__ near, unsigned near_cap,
-                                                const int* __restrict__ tris, const float4* __restrict__ x,
-                                                const float4* __restrict__ p, float th, DetectCounts* __restrict__ c,
-                                                unsigned cap, int4* __restrict__ vquad, int2* __restrict__ vf,
-                                                float* __restrict__ ct, float* __restrict__ cn,
+                                                const int* __restrict__ tris, const FaceAxes* __restrict__ axes,
+                                                const float4* __restrict__ x, const float4* __restrict__ p, float th,
+                                                DetectCounts* __restrict__ c, unsigned cap, int4* __restrict__ vquad,
+                                                int2* __restrict__ vf, float* __restrict__ ct, float* __restrict__ cn,
                                                 double* __restrict__ cw) {
+    __shared__ int2 left[512];
+    __shared__ unsigned left_n;
+    if (threadIdx.x == 0) left_n = 0;
+    __syncthreads();
     const NearRun run(near, near_cap, c);
-    for (unsigned i = run.from + threadIdx.x; i < run.n; i += run.step) {
-        const int2 q = run.pairs[i];
+    auto solve = [&](int2 q) {
         const int4 v = make_int4(q.x, tris[3 * q.y], tris[3 * q.y + 1], tris[3 * q.y + 2]);
         float t;
         V3 nr, wg;
         if (!vf_ccd(v3(x[v.x]), v3(x[v.y]), v3(x[v.z]), v3(x[v.w]), v3(p[v.x]), v3(p[v.y]), v3(p[v.z]), v3(p[v.w]), th,
                     &t, &nr, &wg))
-            continue;
+            return;
         const unsigned o = atomicAdd(&c->contacts, 1u);
-        if (o >= cap) continue;
+        if (o >= cap) return;
         vquad[o] = v;
         if (STORE) {
             vf[o] = q;
@@ -1059,6 +1243,25 @@ __global__ __launch_bounds__(256) void k_narrow(const int2* __restrict__ near, u
             cw[4 * o + 2] = wg.y;
             cw[4 * o + 3] = wg.z;
         }
+    };
+    for (unsigned i0 = run.from; i0 < run.n; i0 += run.step) {
+        const unsigned i = i0 + threadIdx.x;
+        const bool last = i0 + run.step >= run.n;
+        int2 q = make_int2(0, 0);
+        bool keep = i < run.n;
+        if (keep) {
+            q = run.pairs[i];
+            keep = !axes || !axes_miss(axes[q.y], x[q.x], p[q.x]);
+        }
+        if (keep) left[atomicAdd(&left_n, 1u)] = q;
+        __syncthreads();
+        const unsigned n = left_n;
+        __syncthreads();  // every thread has read it before it changes
+        if (n < 256 && !last) continue;
+        for (unsigned k = threadIdx.x; k < n; k += 256) solve(left[k]);
+        __syncthreads();
+        if (threadIdx.x == 0) left_n = 0;
+        __syncthreads();
     }
 }
 
@@ -1585,9 +1788,10 @@ static int visit_blocks(int n) { return std::max(1, std::min(2048, (n + 2 * VISI
 
 // The centroid-cell table of the faces at p.
 void Broadphase::cells(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt_,
-                       float th) {
+                       float th, bool culled) {
     cfg = g;
     nt = nt_;
+    if (culled) grow(axes, (size_t)std::max(1, nt) * sizeof(FaceAxes));
     grow(tcell, std::max(1, nt));
     grow(raw_rank, std::max(1, nt));
     grow(rec, (size_t)std::max(1, nt) * sizeof(FaceRec));
@@ -1599,7 +1803,7 @@ void Broadphase::cells(hipStream_t s, const HashCfg& g, const float4* x, const f
     hipLaunchKernelGGL(k_slot_places<true>, dim3(((1 << table_bits) + PLACE_SLOTS - 1) / PLACE_SLOTS), dim3(256), 0, s,
                        (const int4*)slots_of(table), 1 << table_bits, (int4*)place.ptr, &counts_of(table)->entries);
     hipLaunchKernelGGL(k_cell_fill, dim3(blocks(nt)), dim3(256), 0, s, nt, tcell.ptr, raw_rank.ptr, slots_of(table),
-                       place.ptr, x, p, tris, th, (FaceRec*)rec.ptr);
+                       place.ptr, x, p, tris, th, (FaceRec*)rec.ptr, culled ? (FaceAxes*)axes.ptr : nullptr);
     PBD_HIP(hipGetLastError());
 }
 
@@ -1629,14 +1833,14 @@ void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, c
                                (int)std::min<size_t>(ent.n, 0x7fffffff), (const FaceRec*)rec.ptr, large.ptr,
                                counts_of(table), near_.ptr, near_cap);
         } else {
-            cells(s, g, x, p, tris, nt, th);
+            cells(s, g, x, p, tris, nt, th, true);
             hipLaunchKernelGGL(k_vf_candidates<false>, dim3(visit_blocks(nv)), dim3(64 * VISIT_WAVES), 0, s, g, x, p, nv,
                                vtoff.ptr, vtri.ptr, tcell.ptr, slots_of(table), place.ptr, (1u << table_bits) - 1,
-                               (const FaceRec*)rec.ptr, counts_of(table), near_.ptr,
-                               near_cap);
+                               (const FaceRec*)rec.ptr, counts_of(table), near_.ptr, near_cap);
         }
         auto* narrow = store ? k_narrow<true> : k_narrow<false>;
-        hipLaunchKernelGGL(narrow, dim3(1024), dim3(256), 0, s, near_.ptr, near_cap, tris, x, p, th,
+        hipLaunchKernelGGL(narrow, dim3(1024), dim3(256), 0, s, near_.ptr, near_cap, tris,
+                           swept ? nullptr : (const FaceAxes*)axes.ptr, x, p, th,
                            counts_of(table), cap, vquad.ptr, vf.ptr, rt.ptr, rn.ptr, rw.ptr);
         PBD_HIP(hipGetLastError());
         c = read_counts(s);
@@ -1752,7 +1956,7 @@ long long Broadphase::list_pairs(hipStream_t s, const HashCfg& g, const float4* 
     if (!near_.n) grow_near(1 << 10);
     for (;;) {
         const unsigned cap = near_cap();
-        cells(s, g, p, p, tris, nt, 0.0f);
+        cells(s, g, p, p, tris, nt, 0.0f, false);
         hipLaunchKernelGGL(k_vf_candidates<true>, dim3(visit_blocks(nv)), dim3(64 * VISIT_WAVES), 0, s, g, p, p, nv,
                            vtoff.ptr, vtri.ptr, tcell.ptr, slots_of(table), place.ptr, (1u << table_bits) - 1,
                            (const FaceRec*)rec.ptr, counts_of(table), near_.ptr, cap);

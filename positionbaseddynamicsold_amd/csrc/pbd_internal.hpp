@@ -274,7 +274,7 @@ struct Broadphase {
     DBuf<int> table, place, raw_rank, large;
     int table_bits = 0;
     DBuf<int2> ent;
-    DBuf<unsigned char> rec;
+    DBuf<unsigned char> rec, axes;
     DBuf<int4> tcell, sw_cell;
     void* counts_h = nullptr;  // pinned
     // candidates that go to the narrowphase; contacts in any order (the
@@ -330,7 +330,8 @@ private:
     DetectTotals read_counts(hipStream_t s);
     void grow_near(size_t n);
     unsigned near_cap() const;
-    void cells(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt, float th);
+    void cells(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt, float th,
+               bool culled);
     void swept_table(hipStream_t s, const HashCfg& g, const HashCfg& gi, const float4* x, const float4* p,
                      const int* tris, float th);
     void check_pairs(unsigned long long n, const char* what);

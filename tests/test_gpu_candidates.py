@@ -98,3 +98,29 @@ def test_response_equals_the_oracle_around_one_workgroup(orc, n, low, high):
         for passes in (1, 3):
             assert np.array_equal(ctx.ccd_resolve(p, w, 0.01, passes),
                                   orc.ccd_resolve(arr, count, tris, x, p, w, 0.01, passes))
+
+
+@pytest.mark.parametrize("th", [1e-4, 1e-3, 0.01, 0.06])
+@pytest.mark.parametrize("move", [0.0, 0.004, 0.03, 0.2])
+@pytest.mark.parametrize("shift,scale", [(0.0, 1.0), (300.0, 1.0), (0.0, 1e-4)])
+def test_culled_candidates_keep_every_contact(orc, th, move, shift, scale):
+    # well-shaped triangles, which boxes and half-spaces may rule out, from
+    # thicknesses far below their size to above it, still and tumbling, near
+    # the origin and far from it
+    print(f"culling th={th} move={move} shift={shift} scale={scale}", flush=True)
+    rng = np.random.default_rng(11)
+    nt = 300
+    a = rng.uniform(0, 2 * np.pi, (nt, 1)) + np.array([0.0, 2.1, 4.2]) + 0.3 * rng.standard_normal((nt, 3))
+    u, v = np.linalg.qr(rng.standard_normal((nt, 3, 3)))[0][:, :2].transpose(1, 0, 2)
+    corner = rng.uniform(0, 0.25, (nt, 1, 3)) + 0.03 * (np.cos(a)[..., None] * u[:, None] + np.sin(a)[..., None] * v[:, None])
+    x = ((corner.reshape(-1, 3) + shift) * scale).astype(np.float32)
+    p = x + scale * move * (rng.standard_normal((nt, 1, 3)) + 0.2 * rng.standard_normal((nt, 3, 3))).reshape(-1, 3)
+    p = p.astype(np.float32)
+    tris = np.arange(3 * nt, dtype=np.int32).reshape(nt, 3)
+    th = np.float32(th * scale)
+    desc = dict(cell=(0.3 * scale,) * 3, table_bits=8)
+    arr, n = orc.ccd_detect(orc.grid(1, **desc), x, p, tris, th)
+    assert n > 0 or move == 0.0 or th < 1e-3
+    with capi.Context() as ctx:
+        for a, b in zip(ctx.ccd_detect(capi.hash_desc(1, **desc), x, p, tris, th), orc.contacts_arrays(arr, n)):
+            assert np.array_equal(a, b)
