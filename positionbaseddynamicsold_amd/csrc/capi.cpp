@@ -2263,12 +2263,7 @@ int pbd_sh_get(pbd_ctx* ctx, int* keys, int* ids, int* raw, int* cstart, int* ce
         ctx->sh_stale = false;
         int nt = b.nt;
         if (nt > 0) {
-            std::vector<uint32_t> k1;
-            if (keys) {
-                b.keys.download(k1, s);
-                PBD_HIP(hipStreamSynchronize(s));
-                for (int i = 0; i < nt; i++) keys[i] = (int)k1[i] - 1;
-            }
+            if (keys) PBD_HIP(hipMemcpyAsync(keys, b.keys.ptr, sizeof(int) * nt, hipMemcpyDeviceToHost, s));
             if (ids) PBD_HIP(hipMemcpyAsync(ids, b.ids.ptr, sizeof(int) * nt, hipMemcpyDeviceToHost, s));
             if (raw) PBD_HIP(hipMemcpyAsync(raw, b.raw.ptr, sizeof(int) * nt, hipMemcpyDeviceToHost, s));
         }

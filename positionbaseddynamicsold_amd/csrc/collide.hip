@@ -127,35 +127,93 @@ __device__ __forceinline__ void tri_cell(const HashCfg& g, const P* __restrict__
     gp[2] = (int)floorf((cz - g.start[2]) / g.cell[2]);
 }
 
-__global__ __launch_bounds__(256) void k_tri_keys(HashCfg g, const float4* __restrict__ p,
-                                                  const int* __restrict__ tris, int nt,
-                                                  uint32_t* __restrict__ keys1, uint32_t* __restrict__ ids,
-                                                  int* __restrict__ raw) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nt) return;
-    int gp[3];
-    tri_cell(g, p, tris, t, gp);
-    int k = cell_key(g, gp[0], gp[1], gp[2]);
-    keys1[t] = (uint32_t)(k + 1);  // -1 sorts first, as the reference's signed sort
-    ids[t] = (uint32_t)t;
-    raw[t] = k;
-}
+// Keys of the triangles, one workgroup per sort tile, which also counts the
+// first digit; the workgroups behind the tiles set the cell ranges to -1.
+// Keys are stored plus 1, so that -1 (outside the grid) sorts first, as in the
+// reference's signed sort.  BOUNDED: a triangle with a vertex index outside
+// [0, nv) is given key -1 instead of being read.
+constexpr int KEY_THREADS = 1024, FILL_INTS = 16384;
 
-__global__ __launch_bounds__(256) void k_fill_i32(int* __restrict__ a, int n, int v) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = v;
+template <bool BOUNDED, typename P>
+__global__ __launch_bounds__(KEY_THREADS) void k_tri_keys(HashCfg g, const P* __restrict__ p, int nv,
+                                                          const int* __restrict__ tris, int nt, int ntiles,
+                                                          uint32_t* __restrict__ keys1, int* __restrict__ raw,
+                                                          int* __restrict__ counts, int* __restrict__ cstart,
+                                                          int* __restrict__ cend, int quads) {
+    const int tid = threadIdx.x;
+    if ((int)blockIdx.x >= ntiles) {
+        const int per = (g.ncells + FILL_INTS - 1) / FILL_INTS, f = blockIdx.x - ntiles;
+        int* a = f < per ? cstart : cend;
+        const long long from = (long long)(f < per ? f : f - per) * FILL_INTS;
+        const int n = (int)min((long long)FILL_INTS, g.ncells - from);
+        a += from;
+        int i = 0;
+        if (quads) {  // both arrays are 16-byte aligned
+            for (int j = tid; j < n / 4; j += KEY_THREADS) reinterpret_cast<int4*>(a)[j] = make_int4(-1, -1, -1, -1);
+            i = n & ~3;
+        }
+        for (i += tid; i < n; i += KEY_THREADS) a[i] = -1;
+        return;
+    }
+    __shared__ int h[256];
+    if (tid < 256) h[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RADIX_TILE / KEY_THREADS; r++) {
+        const int t = blockIdx.x * RADIX_TILE + r * KEY_THREADS + tid;
+        if (t >= nt) break;
+        int k = -1;
+        bool read = true;
+        if (BOUNDED) {
+            const int a = tris[3 * t], b = tris[3 * t + 1], c = tris[3 * t + 2];
+            read = a >= 0 && a < nv && b >= 0 && b < nv && c >= 0 && c < nv;
+        }
+        if (read) {
+            int gp[3];
+            tri_cell(g, p, tris, t, gp);
+            k = cell_key(g, gp[0], gp[1], gp[2]);
+        }
+        keys1[t] = (uint32_t)(k + 1);
+        raw[t] = k;
+        atomicAdd(&h[(k + 1) & 255], 1);
+    }
+    __syncthreads();
+    if (tid < 256) counts[blockIdx.x * 256 + tid] = h[tid];
 }
 
 // Correct ranges of each key in the sorted array (the reference's
 // findCellStartCPU misses some starts, SpatialHashSystem.cpp:357-387).
-__global__ __launch_bounds__(256) void k_cell_ranges(const uint32_t* __restrict__ keys1, int n,
-                                                     int* __restrict__ cstart, int* __restrict__ cend) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_cell_ranges(const int* __restrict__ keys, int n, int* __restrict__ cstart,
+                                                     int* __restrict__ cend) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    int k = (int)keys1[i] - 1;
+    const int k = keys[i];
     if (k < 0) return;
-    if (i == 0 || keys1[i - 1] != keys1[i]) cstart[k] = i;
-    if (i == n - 1 || keys1[i + 1] != keys1[i]) cend[k] = i;
+    if (i == 0 || keys[i - 1] != k) cstart[k] = i;
+    if (i == n - 1 || keys[i + 1] != k) cend[k] = i;
+}
+
+// The sorted table: keys (signed) and triangle ids in key order, unsorted
+// keys, cell ranges.  tk / tv: room for nt, hist: radix_hist_ints(nt).
+// Launches: keys with the first digit's counts and the ranges' fill, two per
+// digit less one, the ranges (522,000 triangles, 2^22 cells: 128 us before,
+// 53 us so).
+template <bool BOUNDED, typename P>
+static void build_sorted(hipStream_t s, const HashCfg& g, const P* p, int nv, const int* tris, int nt, uint32_t* ok,
+                         uint32_t* ov, int* raw, int* cstart, int* cend, uint32_t* tk, uint32_t* tv, int* hist) {
+    int bits = 1;
+    while (bits < 32 && ((1ll << bits) < (long long)g.ncells + 1)) bits++;
+    uint32_t* src = radix_passes(bits) % 2 ? tk : ok;
+    const int tiles = radix_tiles(nt);
+    const long long fill = 2ll * ((g.ncells + (long long)FILL_INTS - 1) / FILL_INTS);
+    const int quads = ((uintptr_t)cstart | (uintptr_t)cend) % 16 == 0;
+    if (tiles + fill > 0)
+        hipLaunchKernelGGL((k_tri_keys<BOUNDED, P>), dim3((unsigned)(tiles + fill)), dim3(KEY_THREADS), 0, s, g, p, nv, tris,
+                           nt, tiles, src, raw, hist, cstart, cend, quads);
+    radix_sort(s, src, nullptr, tk, tv, ok, ov, nt, bits, hist, true, 1u);
+    if (nt > 0)
+        hipLaunchKernelGGL(k_cell_ranges, dim3((nt + 255) / 256), dim3(256), 0, s, (const int*)ok, nt, cstart, cend);
+    PBD_HIP(hipGetLastError());
 }
 
 // ---------------------------------------------------------------------------
@@ -1688,14 +1746,7 @@ void Broadphase::build(hipStream_t s, const HashCfg& g, const float4* p, const i
     grow(hist, radix_hist_ints(nt));
     grow(cstart, std::max(1, g.ncells));
     grow(cend, std::max(1, g.ncells));
-    if (nt > 0) hipLaunchKernelGGL(k_tri_keys, dim3(blocks(nt)), dim3(256), 0, s, g, p, tris, nt, keys.ptr, ids.ptr, raw.ptr);
-    int bits = 1;
-    while (bits < 32 && ((1ll << bits) < (long long)g.ncells + 1)) bits++;
-    radix_sort_pairs(s, keys.ptr, ids.ptr, k2.ptr, v2.ptr, nt, bits, hist.ptr);
-    hipLaunchKernelGGL(k_fill_i32, dim3(blocks(g.ncells)), dim3(256), 0, s, cstart.ptr, g.ncells, -1);
-    hipLaunchKernelGGL(k_fill_i32, dim3(blocks(g.ncells)), dim3(256), 0, s, cend.ptr, g.ncells, -1);
-    if (nt > 0) hipLaunchKernelGGL(k_cell_ranges, dim3(blocks(nt)), dim3(256), 0, s, keys.ptr, nt, cstart.ptr, cend.ptr);
-    PBD_HIP(hipGetLastError());
+    build_sorted<false>(s, g, p, 0, tris, nt, keys.ptr, ids.ptr, raw.ptr, cstart.ptr, cend.ptr, k2.ptr, v2.ptr, hist.ptr);
 }
 
 void Broadphase::set_edges(hipStream_t s, const std::vector<int>& te, const std::vector<int2>& ed) {
@@ -2107,8 +2158,7 @@ void Broadphase::resolve(hipStream_t s, const float4* x, float4* p, int nv, floa
 // nothing carries over between calls; calls that overlap on one GPU race on
 // it.
 // ---------------------------------------------------------------------------
-constexpr size_t SH_NOALLOC_HIST_INTS = 2 * ((size_t)256 * (SH_NOALLOC_MAX_TRIS / 4096)) +
-                                        ((size_t)256 * (SH_NOALLOC_MAX_TRIS / 4096) + 1023) / 1024 + 2;
+constexpr size_t SH_NOALLOC_HIST_INTS = (size_t)256 * (2 * (SH_NOALLOC_MAX_TRIS / RADIX_TILE) + 1);
 constexpr size_t SH_NOALLOC_WORDS = 2 * (size_t)SH_NOALLOC_MAX_TRIS + SH_NOALLOC_HIST_INTS;
 static __device__ __align__(256) uint32_t scratch[SH_NOALLOC_WORDS];
 
@@ -2131,32 +2181,6 @@ static void* scratch_address(int device) {
     return addr[device];
 }
 
-// k_tri_keys on 3-float positions; a triangle with a vertex index outside
-// [0, nv) is given key -1 (outside the grid) instead of being read.
-__global__ __launch_bounds__(256) void k_tri_keys_noalloc(HashCfg g, const float* __restrict__ p, int nv,
-                                                          const int* __restrict__ tris, int nt,
-                                                          uint32_t* __restrict__ keys1, uint32_t* __restrict__ ids,
-                                                          int* __restrict__ raw) {
-    int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nt) return;
-    const int a = tris[3 * t], b = tris[3 * t + 1], c = tris[3 * t + 2];
-    int k = -1;
-    if (a >= 0 && a < nv && b >= 0 && b < nv && c >= 0 && c < nv) {
-        int gp[3];
-        tri_cell(g, p, tris, t, gp);
-        k = cell_key(g, gp[0], gp[1], gp[2]);
-    }
-    keys1[t] = (uint32_t)(k + 1);
-    ids[t] = (uint32_t)t;
-    raw[t] = k;
-}
-
-// keys1 (key + 1, the sort's unsigned form) -> key, in place.
-__global__ __launch_bounds__(256) void k_keys_signed(uint32_t* __restrict__ keys1, int n) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) keys1[i] = (uint32_t)((int)keys1[i] - 1);
-}
-
 void sh_build_noalloc(hipStream_t s, int device, const HashCfg& g, const float* pos, int nv, const int* tris, int nt,
                       int* sorted_keys, int* sorted_ids, int* raw_keys, int* cell_start, int* cell_end) {
     PBD_CHECK(nt <= SH_NOALLOC_MAX_TRIS, PBD_ERR_LIMIT,
@@ -2166,20 +2190,8 @@ void sh_build_noalloc(hipStream_t s, int device, const HashCfg& g, const float* 
     uint32_t* k2 = scr;
     uint32_t* v2 = scr + SH_NOALLOC_MAX_TRIS;
     int* hist = (int*)(scr + 2 * (size_t)SH_NOALLOC_MAX_TRIS);
-    uint32_t* k = (uint32_t*)sorted_keys;
-    uint32_t* v = (uint32_t*)sorted_ids;
-    if (nt > 0)
-        hipLaunchKernelGGL(k_tri_keys_noalloc, dim3(blocks(nt)), dim3(256), 0, s, g, pos, nv, tris, nt, k, v, raw_keys);
-    int bits = 1;
-    while (bits < 32 && ((1ll << bits) < (long long)g.ncells + 1)) bits++;
-    radix_sort_pairs(s, k, v, k2, v2, nt, bits, hist);
-    hipLaunchKernelGGL(k_fill_i32, dim3(blocks(g.ncells)), dim3(256), 0, s, cell_start, g.ncells, -1);
-    hipLaunchKernelGGL(k_fill_i32, dim3(blocks(g.ncells)), dim3(256), 0, s, cell_end, g.ncells, -1);
-    if (nt > 0) {
-        hipLaunchKernelGGL(k_cell_ranges, dim3(blocks(nt)), dim3(256), 0, s, k, nt, cell_start, cell_end);
-        hipLaunchKernelGGL(k_keys_signed, dim3(blocks(nt)), dim3(256), 0, s, k, nt);
-    }
-    PBD_HIP(hipGetLastError());
+    build_sorted<true>(s, g, pos, nv, tris, nt, (uint32_t*)sorted_keys, (uint32_t*)sorted_ids, raw_keys, cell_start,
+                       cell_end, k2, v2, hist);
 }
 
 }  // namespace pbd

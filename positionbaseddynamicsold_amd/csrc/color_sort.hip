@@ -87,97 +87,207 @@ int launch_color_round(hipStream_t s, const int* npts, const int* adj_sn, const 
 }
 
 // ---------------------------------------------------------------------------
-// Stable LSD radix pass over (key, value) uint32 pairs, 8-bit digits.
-// Blocks own 4096 consecutive elements.  hist[d * nb + b] counts digit d in
-// block b; an exclusive scan over that digit-major array gives every
-// (digit, block) its first output slot, and the scatter ranks equal digits
-// inside a block in input order (wave match + per-wave counts), so the pass
-// is stable.
+// Stable LSD radix sort of (key, value) uint32 pairs, 8-bit digits.  A pass is
+// two launches over tiles of 4096 consecutive elements: k_radix_hist counts
+// digit d of tile b into counts[b * 256 + d]; k_radix_scatter sums the rows of
+// the tiles before its own (and of all tiles, for the digits before) itself,
+// ranks equal digits of its tile in input order (wave match, per-wave counts)
+// and writes.  With more than RADIX_ROWS tiles the sums come from a launch of
+// their own (k_radix_rows).  Launches and their latencies bound the sort: half
+// a million pairs are 4 MB, a microsecond of bandwidth, per pass, which took
+// 37 us with a scan of three launches and a workgroup barrier per 256
+// elements, TIME us so.
 // ---------------------------------------------------------------------------
-constexpr int RB = 4096;
+constexpr int RB = RADIX_TILE, RT = 1024, RW = RT / 64, RR = RB / RT;
+constexpr int RADIX_ROWS = 256;
 
-__global__ __launch_bounds__(256) void k_radix_hist(const uint32_t* __restrict__ keys, int n,
-                                                    int shift, int* __restrict__ hist, int nb) {
+__global__ __launch_bounds__(RT) void k_radix_hist(const uint32_t* __restrict__ keys, int n, int shift,
+                                                   int* __restrict__ counts) {
     __shared__ int h[256];
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    int base = blockIdx.x * RB;
-    for (int i = threadIdx.x; i < RB; i += 256) {
-        int g = base + i;
-        if (g < n) atomicAdd(&h[(keys[g] >> shift) & 255u], 1);
+    const int t = threadIdx.x;
+    if (t < 256) h[t] = 0;
+    uint32_t k[RR];
+    for (int r = 0; r < RR; r++) {
+        const int i = blockIdx.x * RB + r * RT + t;
+        k[r] = i < n ? keys[i] : 0u;
     }
     __syncthreads();
-    hist[threadIdx.x * nb + blockIdx.x] = h[threadIdx.x];
+    for (int r = 0; r < RR; r++)
+        if (blockIdx.x * RB + r * RT + t < n) atomicAdd(&h[(k[r] >> shift) & 255u], 1);
+    __syncthreads();
+    if (t < 256) counts[blockIdx.x * 256 + t] = h[t];
 }
 
-__global__ __launch_bounds__(256) void k_radix_scatter(const uint32_t* __restrict__ kin,
-                                                       const uint32_t* __restrict__ vin,
-                                                       uint32_t* __restrict__ kout,
-                                                       uint32_t* __restrict__ vout, int n, int shift,
-                                                       const int* __restrict__ offs, int nb) {
-    __shared__ int base[256];
-    __shared__ int wcnt[4][256];
-    int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    base[t] = offs[t * nb + blockIdx.x];
+// rows[b][d] = digit d's count in the tiles before b, rows[nb][d] in all; one
+// workgroup per digit.
+__global__ __launch_bounds__(256) void k_radix_rows(const int* __restrict__ counts, int nb, int* __restrict__ rows) {
+    __shared__ int wave[4];
+    const int d = blockIdx.x, t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    int carry = 0;
+    for (int b0 = 0; b0 < nb; b0 += 256) {
+        const int b = b0 + t, c = b < nb ? counts[(size_t)b * 256 + d] : 0;
+        int run = c;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(run, off);
+            if (lane >= off) run += o;
+        }
+        if (lane == 63) wave[wv] = run;
+        __syncthreads();
+        for (int w = 0; w < wv; w++) run += wave[w];
+        if (b < nb) rows[(size_t)b * 256 + d] = carry + run - c;
+        carry += wave[0] + wave[1] + wave[2] + wave[3];
+        __syncthreads();
+    }
+    if (t == 0) rows[(size_t)nb * 256 + d] = carry;
+}
+
+// rows: from k_radix_rows, or nullptr: summed from counts here.  vin nullptr:
+// the values are the positions.  Keys are written less `less`.
+__global__ __launch_bounds__(RT) void k_radix_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
+                                                      uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, int n,
+                                                      int shift, const int* __restrict__ counts,
+                                                      const int* __restrict__ rows, int nb, uint32_t less) {
+    __shared__ int wcnt[RW][256];
+    __shared__ int before[RT / 256][256], all[RT / 256][256], start[256], base[256], wave[4], here[4];
+    __shared__ uint2 tile[RB];
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, b = blockIdx.x;
+    // this wave's elements, in order
+    const int i0 = b * RB + wv * (RB / RW) + lane;
+    uint32_t k[RR], v[RR];
+    for (int r = 0; r < RR; r++) {
+        const int i = i0 + 64 * r;
+        k[r] = i < n ? kin[i] : 0u;
+        v[r] = i < n ? (vin ? vin[i] : (uint32_t)i) : 0u;
+    }
+    {
+        const int d = t & 255, part = t >> 8;
+        int pre = 0, sum = 0;
+        if (rows) {
+            if (part == 0) {
+                pre = rows[(size_t)b * 256 + d];
+                sum = rows[(size_t)nb * 256 + d];
+            }
+        } else {
+            for (int q0 = part; q0 < nb; q0 += 16 * (RT / 256)) {
+                int c[16];  // in flight together
+#pragma unroll
+                for (int u = 0; u < 16; u++) c[u] = counts[min(q0 + u * (RT / 256), nb - 1) * 256 + d];
+#pragma unroll
+                for (int u = 0; u < 16; u++) {
+                    const int q = q0 + u * (RT / 256);
+                    sum += q < nb ? c[u] : 0;
+                    pre += q < b ? c[u] : 0;
+                }
+            }
+        }
+        before[part][d] = pre;
+        all[part][d] = sum;
+        for (int j = t; j < RW * 256; j += RT) (&wcnt[0][0])[j] = 0;
+    }
     __syncthreads();
-    for (int r = 0; r < RB / 256; r++) {
-        int i = blockIdx.x * RB + r * 256 + t;
-        bool valid = i < n;
-        uint32_t k = valid ? kin[i] : 0u, v = valid ? vin[i] : 0u;
-        int d = valid ? (int)((k >> shift) & 255u) : -1;
-        for (int j = lane; j < 256; j += 64) wcnt[wv][j] = 0;
+    int rank[RR];
+    for (int r = 0; r < RR; r++) {
+        const bool valid = i0 + 64 * r < n;
+        const int d = (k[r] >> shift) & 255u;
         // lanes with this lane's digit: one ballot per digit bit, so the cost
         // does not depend on how many distinct digits the wave holds
         unsigned long long m = __ballot(valid);
 #pragma unroll
-        for (int b = 0; b < 8; b++) {
-            const bool bit = (d >> b) & 1;
-            const unsigned long long bb = __ballot(valid && bit);
-            m &= bit ? bb : ~bb;
+        for (int bit = 0; bit < 8; bit++) {
+            const bool set = (d >> bit) & 1;
+            const unsigned long long bb = __ballot(valid && set);
+            m &= set ? bb : ~bb;
         }
-        int rank = 0;
+        const int below = __popcll(m & __lanemask_lt());
         if (valid) {
-            rank = __popcll(m & __lanemask_lt());
-            if (rank == 0) wcnt[wv][d] = __popcll(m);  // the digit's first lane
+            rank[r] = wcnt[wv][d] + below;
+            __builtin_amdgcn_wave_barrier();  // read before the digit's first lane adds
+            if (below == 0) wcnt[wv][d] = rank[r] + __popcll(m);
         }
-        __syncthreads();
-        if (valid) {
-            int pos = base[d] + rank;
-            for (int w2 = 0; w2 < wv; w2++) pos += wcnt[w2][d];
-            kout[pos] = k;
-            vout[pos] = v;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    // digit starts, and each wave's place within its digit
+    int pre = 0, sum = 0, incl = 0, mine = 0, upto = 0;  // digit t in all tiles and in this one
+    if (t < 256) {
+        for (int q = 0; q < RT / 256; q++) {
+            pre += before[q][t];
+            sum += all[q][t];
         }
-        __syncthreads();
-        base[t] += wcnt[0][t] + wcnt[1][t] + wcnt[2][t] + wcnt[3][t];
-        __syncthreads();
+        incl = sum;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(incl, off);
+            if (lane >= off) incl += o;
+        }
+        if (lane == 63) wave[wv] = incl;
+        for (int w = 0; w < RW; w++) {
+            const int c = wcnt[w][t];
+            wcnt[w][t] = mine;
+            mine += c;
+        }
+        upto = mine;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(upto, off);
+            if (lane >= off) upto += o;
+        }
+        if (lane == 63) here[wv] = upto;
+    }
+    __syncthreads();
+    if (t < 256) {
+        for (int w = 0; w < wv; w++) {
+            incl += wave[w];
+            upto += here[w];
+        }
+        start[t] = upto - mine;
+        base[t] = incl - sum + pre - start[t];
+    }
+    __syncthreads();
+    // in order in LDS first, so that the stores of a wave run over a few digits' places
+    for (int r = 0; r < RR; r++)
+        if (i0 + 64 * r < n) {
+            const int d = (k[r] >> shift) & 255u;
+            tile[start[d] + wcnt[wv][d] + rank[r]] = make_uint2(k[r], v[r]);
+        }
+    __syncthreads();
+    const int m = min(RB, n - b * RB);
+    for (int i = t; i < m; i += RT) {
+        const uint2 e = tile[i];
+        const int pos = base[(e.x >> shift) & 255u] + i;
+        kout[pos] = e.x - less;
+        vout[pos] = e.y;
     }
 }
 
-// Stable sort of (key, value) pairs on bits [0, bits) of the key.  Uses
-// (k2, v2) as the ping-pong buffer; the result ends in (k, v).  `hist` holds
-// radix_hist_ints(n) ints: digit counts | their exclusive scan (multi-block)
-// | the scan's block sums.
-void radix_sort_pairs(hipStream_t s, uint32_t* k, uint32_t* v, uint32_t* k2, uint32_t* v2, int n,
-                      int bits, int* hist) {
+// Stable sort of n (key, value) pairs on bits [0, bits) of the key from src
+// into out by way of tmp; src may be tmp when radix_passes(bits) is odd, out
+// when it is even.  sv == nullptr: the values are 0 .. n - 1.  counted: the
+// first digit's counts are in hist.  Keys come out less `less`.
+void radix_sort(hipStream_t s, const uint32_t* sk, const uint32_t* sv, uint32_t* tk, uint32_t* tv, uint32_t* ok,
+                uint32_t* ov, int n, int bits, int* hist, bool counted, uint32_t less) {
     if (n <= 0) return;
-    int nb = (n + RB - 1) / RB;
-    int passes = (bits + 7) / 8;
-    int* counts = hist;
-    int* offs = hist + (size_t)256 * nb;
-    int* sums = hist + (size_t)512 * nb;
-    uint32_t *ki = k, *vi = v, *ko = k2, *vo = v2;
+    const int nb = radix_tiles(n), passes = radix_passes(bits);
+    int* rows = nb > RADIX_ROWS ? hist + (size_t)256 * nb : nullptr;
     for (int ps = 0; ps < passes; ps++) {
-        hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(256), 0, s, ki, n, ps * 8, counts, nb);
-        device_scan(s, counts, offs, 256 * nb, sums);
-        hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(256), 0, s, ki, vi, ko, vo, n, ps * 8, offs, nb);
-        std::swap(ki, ko);
-        std::swap(vi, vo);
-    }
-    if (ki != k) {
-        PBD_HIP(hipMemcpyAsync(k, ki, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
-        PBD_HIP(hipMemcpyAsync(v, vi, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
+        const bool last = ps + 1 == passes, to_out = (passes - 1 - ps) % 2 == 0;
+        if (ps > 0 || !counted) hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(RT), 0, s, sk, n, ps * 8, hist);
+        if (rows) hipLaunchKernelGGL(k_radix_rows, dim3(256), dim3(256), 0, s, hist, nb, rows);
+        uint32_t *k = to_out ? ok : tk, *v = to_out ? ov : tv;
+        hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(RT), 0, s, sk, sv, k, v, n, ps * 8, hist, rows, nb,
+                           last ? less : 0u);
+        sk = k;
+        sv = v;
     }
     PBD_HIP(hipGetLastError());
+}
+
+// In place, with (k2, v2) as the other buffer.
+void radix_sort_pairs(hipStream_t s, uint32_t* k, uint32_t* v, uint32_t* k2, uint32_t* v2, int n, int bits, int* hist) {
+    if (n <= 0) return;
+    if (radix_passes(bits) % 2 == 0) return radix_sort(s, k, v, k2, v2, k, v, n, bits, hist, false, 0u);
+    radix_sort(s, k, v, k, v, k2, v2, n, bits, hist, false, 0u);
+    PBD_HIP(hipMemcpyAsync(k, k2, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
+    PBD_HIP(hipMemcpyAsync(v, v2, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
 }
 
 }  // namespace pbd

@@ -461,15 +461,15 @@ bool plan_tiles(std::vector<Cloth>& cloths, const WholeLoad& whole, int max_load
 // counted into *uncolored.
 int launch_color_round(hipStream_t s, const int* prim_npts, const int* adj_sn, const int* adj, int* color,
                        int* prd, int* uncolored, int np);
-// Ints of `hist` that radix_sort_pairs needs for n keys: the per-block digit
-// counts (256 x ceil(n / 4096)), their exclusive scan, and the block sums of
-// that scan.
-inline size_t radix_hist_ints(long long n) {
-    const size_t h = (size_t)256 * (size_t)((std::max(1ll, n) + 4095) / 4096);
-    return 2 * h + (h + 1023) / 1024 + 2;
-}
-void radix_sort_pairs(hipStream_t s, uint32_t* k, uint32_t* v, uint32_t* k2, uint32_t* v2, int n,
-                      int bits, int* hist);
+// Ints of `hist` that a sort of n keys needs: digit counts per tile, and their
+// sums over the tiles before.
+constexpr int RADIX_TILE = 4096;
+inline int radix_tiles(long long n) { return (int)((n + RADIX_TILE - 1) / RADIX_TILE); }
+inline int radix_passes(int bits) { return (bits + 7) / 8; }
+inline size_t radix_hist_ints(long long n) { return (size_t)256 * (2 * (size_t)radix_tiles(n) + 1); }
+void radix_sort(hipStream_t s, const uint32_t* sk, const uint32_t* sv, uint32_t* tk, uint32_t* tv, uint32_t* ok,
+                uint32_t* ov, int n, int bits, int* hist, bool counted, uint32_t less);
+void radix_sort_pairs(hipStream_t s, uint32_t* k, uint32_t* v, uint32_t* k2, uint32_t* v2, int n, int bits, int* hist);
 void launch_advect(hipStream_t s, const ClothDev* cloths, const int* vcloth, const float4* x,
                    float4* v, float4* p, int nv_begin, int nv_end, float dt, int skip_whole);
 void launch_integrate(hipStream_t s, const ClothDev* cloths, const int* vcloth, float4* x, float4* v,
