@@ -106,7 +106,7 @@ struct pbd_ctx {
     // learned warm start
     struct WarmStart {
         bool params_ready = false, enabled = false, nbr_built = false;
-        DBuf<float> prm, m, v, grad, partial, X, Y, norm;
+        DBuf<float> prm, m, v, grad, partial, losses, X, Y, norm;
         std::vector<float> norm_h;
         bool samples_normalized = false;
         DBuf<unsigned char> W;
@@ -2788,28 +2788,26 @@ int pbd_ws_train(pbd_ctx* ctx, int epochs, int batch, float lr, uint64_t seed, d
         W.partial.alloc((size_t)(((batch + 15) / 16 + 2) * (mlp_nparam() + 1)));
         double loss_sum = 0.0;
         long long loss_n = 0;
-        std::vector<float> g(1);
+        W.losses.alloc((size_t)std::max<long long>(1, n / batch + 1));  // of the last epoch's batches
         for (int e = 0; e < epochs; e++) {
             for (long long i = n - 1; i > 0; i--) {
                 long long j = (long long)(splitmix64(&st) % (uint64_t)(i + 1));
                 std::swap(perm[i], perm[j]);
             }
             W.perm.upload(perm, s);
-            loss_sum = 0.0;
-            loss_n = 0;
             for (long long b0 = 0; b0 + batch <= n || (b0 == 0 && n < batch); b0 += batch) {
                 int m = (int)std::min<long long>(batch, n - b0);
-                mlp_grad(s, W.W.ptr, W.X.ptr, W.Y.ptr, W.perm.ptr + b0, m, 1.0f / m, W.partial.ptr, W.grad.ptr);
-                mlp_adam(s, W.prm.ptr, W.grad.ptr, W.m.ptr, W.v.ptr, lr, 0.9f, 0.999f, 1e-8f, ++W.adam_step);
-                mlp_pack(s, W.prm.ptr, W.W.ptr);
-                if (e == epochs - 1) {
-                    float lv = 0.0f;
-                    PBD_HIP(hipMemcpyAsync(&lv, W.grad.ptr + mlp_nparam(), sizeof(float), hipMemcpyDeviceToHost, s));
-                    PBD_HIP(hipStreamSynchronize(s));
-                    loss_sum += lv;
-                    loss_n++;
-                }
+                float* loss = nullptr;
+                if (e == epochs - 1) loss = W.losses.ptr + loss_n++;
+                mlp_step(s, W.W.ptr, W.X.ptr, W.Y.ptr, W.perm.ptr + b0, m, 1.0f / m, W.partial.ptr, W.grad.ptr, W.prm.ptr,
+                         W.m.ptr, W.v.ptr, lr, 0.9f, 0.999f, 1e-8f, ++W.adam_step, loss);
             }
+        }
+        if (loss_n) {
+            std::vector<float> lv(loss_n);
+            PBD_HIP(hipMemcpyAsync(lv.data(), W.losses.ptr, sizeof(float) * loss_n, hipMemcpyDeviceToHost, s));
+            PBD_HIP(hipStreamSynchronize(s));
+            for (float l : lv) loss_sum += l;
         }
         PBD_HIP(hipStreamSynchronize(s));
         if (last_loss) *last_loss = loss_n ? loss_sum / loss_n : 0.0;

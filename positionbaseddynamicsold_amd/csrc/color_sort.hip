@@ -96,7 +96,7 @@ int launch_color_round(hipStream_t s, const int* npts, const int* adj_sn, const 
 // their own (k_radix_rows).  Launches and their latencies bound the sort: half
 // a million pairs are 4 MB, a microsecond of bandwidth, per pass, which took
 // 37 us with a scan of three launches and a workgroup barrier per 256
-// elements, TIME us so.
+// elements, 16 us so.
 // ---------------------------------------------------------------------------
 constexpr int RB = RADIX_TILE, RT = 1024, RW = RT / 64, RR = RB / RT;
 constexpr int RADIX_ROWS = 256;

@@ -214,183 +214,243 @@ __global__ __launch_bounds__(256) void k_mlp_forward(const MlpW* __restrict__ gW
 }
 
 // ---------------------------------------------------------------------------
-// training: forward + backward over 16 samples per wave; per-wave parameter
-// gradients written to partial[wave][NPARAM+1] (last slot: loss)
+// training: forward + backward over 16 samples per workgroup; their parameter
+// gradients written to partial[group][NPARAM+1] (last slot: loss)
+//
+// A batch of 4096 is 256 groups, one per CU, and the chain of layers bounds
+// the kernel: four waves share a group's columns (one 16-column tile each)
+// and its weight-gradient rows.  LDS rows are padded so that the 16 rows a
+// matrix operand reads fall on different banks (per batch 21 us with one wave
+// per group, 14 with four, 12 with padded rows).
 // ---------------------------------------------------------------------------
-struct alignas(16) BwdLds {
-    uint16_t xT[32 * 16];     // X^T [in][sample]
-    uint16_t a1T[64 * 16];    // A1^T
-    uint16_t a2T[64 * 16];    // A2^T
-    uint16_t dyT[16 * 16];    // dY^T [out16][sample]
-    uint16_t dh2[16 * 64];    // dH2 [sample][o]
-    uint16_t dh2T[64 * 16];   // dH2^T
-    uint16_t dh1T[64 * 16];   // dH1^T
-    float dh2f[16 * 64];
-    float dh1f[16 * 64];
-    float dy[16 * 4];
+constexpr int ROW64 = 68, ROW32 = 36, ROW16 = 20;  // row strides of 64, 32 and 16 columns
+
+struct alignas(16) TrainLds {
+    uint16_t w1[64 * ROW32], w2[64 * ROW64], w3[16 * ROW64], w2t[64 * ROW64];
+    float b1[64], b2[64], b3[16];
+    uint16_t xs[16 * ROW32], a1[16 * ROW64], a2[16 * ROW64], dh2[16 * ROW64];  // [sample][column]
+    uint16_t xT[32 * ROW16], a1T[64 * ROW16], a2T[64 * ROW16], dyT[16 * ROW16], dh2T[64 * ROW16], dh1T[64 * ROW16];
+    float dh1f[16 * ROW64], dh2f[16 * ROW64];
+    float y[16 * 16], dy[16 * 4];
 };
 
-constexpr int TRAIN_WAVES = 2;
+// n rows of `cols` (a multiple of 8) from packed global memory to padded LDS rows.
+template <int COLS, int ROW>
+__device__ __forceinline__ void load_rows(uint16_t* d, const uint16_t* __restrict__ g, int n) {
+    for (int i = threadIdx.x; i < n * (COLS / 8); i += blockDim.x) {
+        const uint4 v = ((const uint4*)g)[i];
+        uint2* o = (uint2*)(d + i / (COLS / 8) * ROW + i % (COLS / 8) * 8);
+        o[0] = make_uint2(v.x, v.y);
+        o[1] = make_uint2(v.z, v.w);
+    }
+}
 
-__global__ __launch_bounds__(128) void k_mlp_train(const MlpW* __restrict__ gW, const float* __restrict__ X,
-                                                   const float* __restrict__ T, const int* __restrict__ idx,
-                                                   int nbatch, float inv_total, float* __restrict__ partial) {
-    __shared__ MlpW W;
-    __shared__ FwdLds F[TRAIN_WAVES];
-    __shared__ BwdLds B[TRAIN_WAVES];
-    load_weights(&W, gW);
-    const int wv = threadIdx.x >> 6, l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-    FwdLds& f = F[wv];
-    BwdLds& b = B[wv];
-    const int gw = blockIdx.x * TRAIN_WAVES + wv;
-    const int base = gw * 16;
-    float* out = partial + (size_t)gw * (NPARAM + 1);
-    if (base >= nbatch) return;
+constexpr int TRAIN_THREADS = 256;
+
+__global__ __launch_bounds__(TRAIN_THREADS) void k_mlp_train(const MlpW* __restrict__ gW, const float* __restrict__ X,
+                                                             const float* __restrict__ T, const int* __restrict__ idx,
+                                                             int nbatch, float inv_total, float* __restrict__ partial) {
+    __shared__ TrainLds b;
+    const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, r = l & 15, q = l >> 4;
+    const int base = blockIdx.x * 16, col = 16 * wv + r;
+    float* out = partial + (size_t)blockIdx.x * (NPARAM + 1);
     // gather the 16 samples
-    for (int e = l; e < 16 * 32; e += 64) {
+    for (int e = tid; e < 16 * 32; e += TRAIN_THREADS) {
         int row = e / 32, k = e % 32, s = base + row;
         float v = (k < 22 && s < nbatch) ? X[(size_t)idx[s] * 22 + k] : 0.0f;
         uint16_t hv = f2bf(v);
-        f.xs[e] = hv;
-        b.xT[k * 16 + row] = hv;
+        b.xs[row * ROW32 + k] = hv;
+        b.xT[k * ROW16 + row] = hv;
     }
-    wave_sync();
-    forward16(W, f);
+    load_rows<32, ROW32>(b.w1, gW->w1, 64);
+    load_rows<64, ROW64>(b.w2, gW->w2, 64);
+    load_rows<64, ROW64>(b.w3, gW->w3, 16);
+    load_rows<64, ROW64>(b.w2t, gW->w2t, 64);
+    if (tid < 64) b.b1[tid] = gW->b1[tid];
+    else if (tid < 128) b.b2[tid - 64] = gW->b2[tid - 64];
+    else if (tid < 144) b.b3[tid - 128] = gW->b3[tid - 128];
+    float target = 0.0f;  // of sample l / 3, output l % 3
+    if (wv == 0 && l < 48 && base + l / 3 < nbatch) target = T[(size_t)idx[base + l / 3] * 3 + l % 3];
+    __syncthreads();
+    // forward: this wave's 16 columns of each layer; lane (q, r) has rows 4q .. 4q + 3
+    f32x4 acc[4];
+    float h1[4], h2[4];
+    mm16(b.xs, ROW32, b.w1 + wv * 16 * ROW32, ROW32, 32, 1, acc);
+    for (int i = 0; i < 4; i++) {
+        float a;
+        h1[i] = acc[0][i] + b.b1[col];
+        gelu(h1[i], &a, nullptr);
+        const uint16_t hv = f2bf(a);
+        b.a1[(4 * q + i) * ROW64 + col] = hv;
+        b.a1T[col * ROW16 + 4 * q + i] = hv;
+    }
+    __syncthreads();
+    mm16(b.a1, ROW64, b.w2 + wv * 16 * ROW64, ROW64, 64, 1, acc);
+    for (int i = 0; i < 4; i++) {
+        float a;
+        h2[i] = acc[0][i] + b.b2[col];
+        gelu(h2[i], &a, nullptr);
+        const uint16_t hv = f2bf(a);
+        b.a2[(4 * q + i) * ROW64 + col] = hv;
+        b.a2T[col * ROW16 + 4 * q + i] = hv;
+    }
+    __syncthreads();
     // dY = (y - t) / N (loss = sum 0.5 |y - t|^2 / N)
     float lossp = 0.0f;
-    if (l < 48) {
-        int row = l / 3, o = l % 3, s = base + row;
-        float dy = 0.0f;
-        if (s < nbatch) {
-            float e = f.y[row * 16 + o] - T[(size_t)idx[s] * 3 + o];
-            lossp = 0.5f * e * e * inv_total;
-            dy = e * inv_total;
+    if (wv == 0) {
+        mm16(b.a2, ROW64, b.w3, ROW64, 64, 1, acc);
+        for (int i = 0; i < 4; i++) b.y[(4 * q + i) * 16 + r] = acc[0][i] + b.b3[r];
+        wave_sync();
+        if (l < 48) {
+            int row = l / 3, o = l % 3;
+            float dy = 0.0f;
+            if (base + row < nbatch) {
+                float e = b.y[row * 16 + o] - target;
+                lossp = 0.5f * e * e * inv_total;
+                dy = e * inv_total;
+            }
+            b.dy[row * 4 + o] = dy;
         }
-        b.dy[row * 4 + o] = dy;
+        wave_sync();
+        for (int e = l; e < 16 * 16; e += 64) {
+            int o = e / 16, s = e % 16;
+            b.dyT[o * ROW16 + s] = o < 3 ? f2bf(b.dy[s * 4 + o]) : 0;
+        }
     }
-    wave_sync();
-    for (int e = l; e < 16 * 16; e += 64) {
-        int o = e / 16, s = e % 16;
-        b.dyT[e] = o < 3 ? f2bf(b.dy[s * 4 + o]) : 0;
-    }
-    // transposed activations for the weight-gradient products
-    for (int e = l; e < 16 * 64; e += 64) {
-        int row = e / 64, c = e % 64;
-        b.a1T[c * 16 + row] = f.a1[e];
-        b.a2T[c * 16 + row] = f.a2[e];
-    }
-    wave_sync();
+    __syncthreads();
     // dA2 = dY W3 (VALU, 3 terms), dH2 = dA2 * gelu'(H2)
-    for (int e = l; e < 16 * 64; e += 64) {
-        int row = e / 64, c = e % 64;
-        int s = base + row;
+    for (int i = 0; i < 4; i++) {
+        const int row = 4 * q + i;
         float da = 0.0f;
-        for (int o = 0; o < 3; o++) da += b.dy[row * 4 + o] * bf2f(W.w3[o * 64 + c]);
+        for (int o = 0; o < 3; o++) da += b.dy[row * 4 + o] * bf2f(b.w3[o * ROW64 + col]);
         float g, gd;
-        gelu(f.h2[e], &g, &gd);
-        float d = s < nbatch ? da * gd : 0.0f;
-        b.dh2f[e] = d;
+        gelu(h2[i], &g, &gd);
+        float d = base + row < nbatch ? da * gd : 0.0f;
+        b.dh2f[row * ROW64 + col] = d;
         uint16_t hv = f2bf(d);
-        b.dh2[e] = hv;
-        b.dh2T[c * 16 + row] = hv;
+        b.dh2[row * ROW64 + col] = hv;
+        b.dh2T[col * ROW16 + row] = hv;
     }
-    wave_sync();
+    __syncthreads();
     // dA1 = dH2 W2 (MFMA with B^T = W2^T stored as w2t), dH1 = dA1 * gelu'(H1)
-    {
-        f32x4 acc[4];
-        mm16(b.dh2, 64, W.w2t, 64, 64, 4, acc);
-        for (int t = 0; t < 4; t++)
-            for (int i = 0; i < 4; i++) {
-                int row = 4 * q + i, col = 16 * t + r;
-                float g, gd;
-                gelu(f.h1[row * 64 + col], &g, &gd);
-                float d = (base + row < nbatch) ? acc[t][i] * gd : 0.0f;
-                b.dh1f[row * 64 + col] = d;
-                b.dh1T[col * 16 + row] = f2bf(d);
-            }
+    mm16(b.dh2, ROW64, b.w2t + wv * 16 * ROW64, ROW64, 64, 1, acc);
+    for (int i = 0; i < 4; i++) {
+        const int row = 4 * q + i;
+        float g, gd;
+        gelu(h1[i], &g, &gd);
+        float d = (base + row < nbatch) ? acc[0][i] * gd : 0.0f;
+        b.dh1f[row * ROW64 + col] = d;
+        b.dh1T[col * ROW16 + row] = f2bf(d);
     }
-    wave_sync();
     // weight gradients: dW = dH^T A (MFMA, K = the 16 samples)
-    {
-        f32x4 acc[4];
-        // dW3 [3 x 64]
-        mm16(b.dyT, 16, b.a2T, 16, 16, 4, acc);
-        for (int t = 0; t < 4; t++)
-            for (int i = 0; i < 4; i++) {
-                int o = 4 * q + i, c = 16 * t + r;
-                if (o < 3) out[P_W3 + o * 64 + c] = acc[t][i];
-            }
-        // dW2 [64 x 64]: four row tiles of o
-        for (int ot = 0; ot < 4; ot++) {
-            mm16(b.dh2T + ot * 16 * 16, 16, b.a1T, 16, 16, 4, acc);
-            for (int t = 0; t < 4; t++)
-                for (int i = 0; i < 4; i++) {
-                    int o = ot * 16 + 4 * q + i, c = 16 * t + r;
-                    out[P_W2 + o * 64 + c] = acc[t][i];
-                }
-        }
-        // dW1 [64 x 22]: K padded 32
-        for (int ot = 0; ot < 4; ot++) {
-            mm16(b.dh1T + ot * 16 * 16, 16, b.xT, 16, 16, 2, acc);
-            for (int t = 0; t < 2; t++)
-                for (int i = 0; i < 4; i++) {
-                    int o = ot * 16 + 4 * q + i, c = 16 * t + r;
-                    if (c < 22) out[P_W1 + o * 22 + c] = acc[t][i];
-                }
-        }
+    // dW3 [3 x 64]: this wave's columns
+    mm16(b.dyT, ROW16, b.a2T + wv * 16 * ROW16, ROW16, 16, 1, acc);
+    for (int i = 0; i < 4; i++) {
+        int o = 4 * q + i;
+        if (o < 3) out[P_W3 + o * 64 + col] = acc[0][i];
     }
+    // dW2 [64 x 64]: this wave's rows
+    mm16(b.dh2T + wv * 16 * ROW16, ROW16, b.a1T, ROW16, 16, 4, acc);
+    for (int t = 0; t < 4; t++)
+        for (int i = 0; i < 4; i++) out[P_W2 + (16 * wv + 4 * q + i) * 64 + 16 * t + r] = acc[t][i];
+    __syncthreads();
+    // dW1 [64 x 22]: K padded 32
+    mm16(b.dh1T + wv * 16 * ROW16, ROW16, b.xT, ROW16, 16, 2, acc);
+    for (int t = 0; t < 2; t++)
+        for (int i = 0; i < 4; i++) {
+            int c = 16 * t + r;
+            if (c < 22) out[P_W1 + (16 * wv + 4 * q + i) * 22 + c] = acc[t][i];
+        }
     // bias gradients (FP32 sums over the 16 samples) and the loss
-    {
-        float s1 = 0.0f, s2 = 0.0f;
-        for (int row = 0; row < 16; row++) {
-            s1 += b.dh1f[row * 64 + l];
-            s2 += b.dh2f[row * 64 + l];
-        }
-        out[P_B1 + l] = s1;
-        out[P_B2 + l] = s2;
-        if (l < 3) {
-            float s3 = 0.0f;
-            for (int row = 0; row < 16; row++) s3 += b.dy[row * 4 + l];
-            out[P_B3 + l] = s3;
-        }
+    if (wv == 1 || wv == 2) {
+        const float* d = wv == 1 ? b.dh1f : b.dh2f;
+        float sum = 0.0f;
+        for (int row = 0; row < 16; row++) sum += d[row * ROW64 + l];
+        out[(wv == 1 ? P_B1 : P_B2) + l] = sum;
+    } else if (wv == 3 && l < 3) {
+        float s3 = 0.0f;
+        for (int row = 0; row < 16; row++) s3 += b.dy[row * 4 + l];
+        out[P_B3 + l] = s3;
+    } else if (wv == 0) {
         for (int off = 32; off > 0; off >>= 1) lossp += __shfl_xor(lossp, off);
         if (l == 0) out[NPARAM] = lossp;
     }
 }
 
-// Sum of the per-wave partials: a block takes 16 parameters x 16 wave
-// slices; slice j adds waves j, j + 16, ... in order and the 16 slice sums
-// are added in slice order (deterministic).
-__global__ __launch_bounds__(256) void k_mlp_reduce(const float* __restrict__ partial, int nw,
-                                                    float* __restrict__ grad) {
+// Adam (Kingma & Ba 2015) on the FP32 master parameters; c1 = 1 - b1^t, c2 = 1 - b2^t.
+struct AdamArgs {
+    float *w, *m, *v;
+    float lr, b1, b2, eps, c1, c2;
+};
+__device__ __forceinline__ float adam(const AdamArgs& a, int i, float gi) {
+    float mi = a.b1 * a.m[i] + (1.0f - a.b1) * gi;
+    float vi = a.b2 * a.v[i] + (1.0f - a.b2) * gi * gi;
+    a.m[i] = mi;
+    a.v[i] = vi;
+    float mh = mi / a.c1, vh = vi / a.c2;
+    return a.w[i] = a.w[i] - a.lr * mh / (sqrtf(vh) + a.eps);
+}
+
+// Parameter i in all of its places (the padding never changes).
+__device__ __forceinline__ void pack_param(MlpW* __restrict__ W, int i, float x) {
+    const uint16_t h = f2bf(x);
+    if (i < P_B1) {
+        const int o = i / 22, k = i % 22, st = k / 16, q = k % 16 / 4, j = k % 4;
+        W->w1[o * 32 + k] = h;
+        W->i1[o * 32 + 8 * q + 4 * st + j] = h;
+    } else if (i < P_W2) {
+        W->b1[i - P_B1] = x;
+    } else if (i < P_B2) {
+        const int o = (i - P_W2) / 64, k = (i - P_W2) % 64, st = k / 16, q = k % 16 / 4, j = k % 4;
+        W->w2[o * 64 + k] = h;
+        W->w2t[k * 64 + o] = h;
+        W->i2[o * 64 + 16 * q + 4 * st + j] = h;
+    } else if (i < P_W3) {
+        W->b2[i - P_B2] = x;
+    } else if (i < P_B3) {
+        const int o = (i - P_W3) / 64, k = (i - P_W3) % 64, st = k / 16, q = k % 16 / 4, j = k % 4;
+        W->w3[o * 64 + k] = h;
+        W->i3[o * 64 + 16 * q + 4 * st + j] = h;
+    } else {
+        W->b3[i - P_B3] = x;
+    }
+}
+
+// Sum of the groups' partials: a block takes 16 parameters x 16 slices of
+// groups; slice j adds groups j, j + 16, ... in order and the 16 slice sums
+// are added in slice order (deterministic).  STEP: each parameter's Adam step
+// and its packed copies follow in the thread that has the sum, instead of two
+// launches more.
+template <bool STEP>
+__global__ __launch_bounds__(256) void k_mlp_reduce(const float* __restrict__ partial, int nw, float* __restrict__ grad,
+                                                    AdamArgs a, MlpW* __restrict__ W, float* __restrict__ loss) {
     __shared__ float red[16][17];
     const int pi = threadIdx.x & 15, sl = threadIdx.x >> 4;
     const int i = blockIdx.x * 16 + pi;
     float acc = 0.0f;
     if (i <= NPARAM)
-        for (int w = sl; w < nw; w += 16) acc += partial[(size_t)w * (NPARAM + 1) + i];
+        for (int w0 = sl; w0 < nw; w0 += 16 * 16) {
+            float p[16];  // in flight together
+#pragma unroll
+            for (int u = 0; u < 16; u++) p[u] = partial[(size_t)min(w0 + 16 * u, nw - 1) * (NPARAM + 1) + i];
+#pragma unroll
+            for (int u = 0; u < 16; u++)
+                if (w0 + 16 * u < nw) acc += p[u];
+        }
     red[sl][pi] = acc;
     __syncthreads();
     if (sl == 0 && i <= NPARAM) {
         float t = 0.0f;
         for (int k = 0; k < 16; k++) t += red[k][pi];
         grad[i] = t;
+        if (STEP && i < NPARAM) pack_param(W, i, adam(a, i, t));
+        if (STEP && i == NPARAM && loss) *loss = t;
     }
 }
 
-// Adam (Kingma & Ba 2015) on the FP32 master parameters; c1 = 1 - b1^t, c2 = 1 - b2^t.
-__global__ __launch_bounds__(256) void k_adam(float* __restrict__ w, const float* __restrict__ g,
-                                              float* __restrict__ m, float* __restrict__ v, int n, float lr,
-                                              float b1, float b2, float eps, float c1, float c2) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float gi = g[i];
-    float mi = b1 * m[i] + (1.0f - b1) * gi;
-    float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    float mh = mi / c1, vh = vi / c2;
-    w[i] = w[i] - lr * mh / (sqrtf(vh) + eps);
+__global__ __launch_bounds__(256) void k_adam(AdamArgs a, const float* __restrict__ g, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) adam(a, i, g[i]);
 }
 
 // ---------------------------------------------------------------------------
@@ -869,23 +929,40 @@ void mlp_forward(hipStream_t s, const void* W, const float* X, int n, float* Y) 
     PBD_HIP(hipGetLastError());
 }
 
+static void train_groups(hipStream_t s, const void* W, const float* X, const float* T, const int* idx, int n,
+                         float inv_total, float* partial) {
+    hipLaunchKernelGGL(k_mlp_train, dim3((n + 15) / 16), dim3(TRAIN_THREADS), 0, s, (const MlpW*)W, X, T, idx, n,
+                       inv_total, partial);
+}
+
+static AdamArgs adam_args(float* w, float* m, float* v, float lr, float b1, float b2, float eps, int step) {
+    return {w, m, v, lr, b1, b2, eps, (float)(1.0 - std::pow((double)b1, step)), (float)(1.0 - std::pow((double)b2, step))};
+}
+
 // Gradient of the mean loss over samples idx[0..n) into grad[NPARAM]
 // (grad[NPARAM] = loss).  partial must hold ceil(n/16) * (NPARAM+1) floats.
 void mlp_grad(hipStream_t s, const void* W, const float* X, const float* T, const int* idx, int n, float inv_total,
               float* partial, float* grad) {
-    int waves = (n + 15) / 16;
-    int blocks = (waves + TRAIN_WAVES - 1) / TRAIN_WAVES;
-    PBD_HIP(hipMemsetAsync(partial, 0, sizeof(float) * (size_t)blocks * TRAIN_WAVES * (NPARAM + 1), s));
-    hipLaunchKernelGGL(k_mlp_train, dim3(blocks), dim3(64 * TRAIN_WAVES), 0, s, (const MlpW*)W, X, T, idx, n,
-                       inv_total, partial);
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((NPARAM + 1 + 15) / 16), dim3(256), 0, s, partial, waves, grad);
+    train_groups(s, W, X, T, idx, n, inv_total, partial);
+    hipLaunchKernelGGL(k_mlp_reduce<false>, dim3((NPARAM + 1 + 15) / 16), dim3(256), 0, s, partial, (n + 15) / 16, grad,
+                       AdamArgs{}, (MlpW*)nullptr, (float*)nullptr);
     PBD_HIP(hipGetLastError());
 }
 
 void mlp_adam(hipStream_t s, float* w, const float* g, float* m, float* v, float lr, float b1, float b2, float eps,
               int step) {
-    float c1 = (float)(1.0 - std::pow((double)b1, step)), c2 = (float)(1.0 - std::pow((double)b2, step));
-    hipLaunchKernelGGL(k_adam, dim3(nb256(NPARAM)), dim3(256), 0, s, w, g, m, v, NPARAM, lr, b1, b2, eps, c1, c2);
+    hipLaunchKernelGGL(k_adam, dim3(nb256(NPARAM)), dim3(256), 0, s, adam_args(w, m, v, lr, b1, b2, eps, step), g, NPARAM);
+    PBD_HIP(hipGetLastError());
+}
+
+// mlp_grad, mlp_adam and mlp_pack of one batch in two launches; the loss also
+// goes to *loss (device memory, may be null).
+void mlp_step(hipStream_t s, void* W, const float* X, const float* T, const int* idx, int n, float inv_total,
+              float* partial, float* grad, float* w, float* m, float* v, float lr, float b1, float b2, float eps, int step,
+              float* loss) {
+    train_groups(s, W, X, T, idx, n, inv_total, partial);
+    hipLaunchKernelGGL(k_mlp_reduce<true>, dim3((NPARAM + 1 + 15) / 16), dim3(256), 0, s, partial, (n + 15) / 16, grad,
+                       adam_args(w, m, v, lr, b1, b2, eps, step), (MlpW*)W, loss);
     PBD_HIP(hipGetLastError());
 }
 

@@ -359,6 +359,9 @@ void mlp_grad(hipStream_t s, const void* W, const float* X, const float* T, cons
               float* partial, float* grad);
 void mlp_adam(hipStream_t s, float* w, const float* g, float* m, float* v, float lr, float b1, float b2, float eps,
               int step);
+void mlp_step(hipStream_t s, void* W, const float* X, const float* T, const int* idx, int n, float inv_total,
+              float* partial, float* grad, float* w, float* m, float* v, float lr, float b1, float b2, float eps, int step,
+              float* loss);
 // Predicted corrections.  With vel, p is written: the advected positions of
 // x and vel (advect on load, no raw features); otherwise p is read.
 // rs_zero (fused form only): n_rs words the kernel clears on the way (the
