@@ -288,8 +288,9 @@ struct Broadphase {
     // sorted candidate lists, made when first asked for
     DBuf<uint32_t> uv, uf, eua, eub;
     bool by_box = false, listed = false, ee_listed = false;
-    DBuf<unsigned long long> acc;  // response sums and counts, zero between passes
+    DBuf<unsigned long long> acc;  // response sums, marks and counts, zero between responses
     DBuf<int> vcnt;
+    int sums_nv = 0, sums_chain = 0;  // what they are laid out for
     int few_slots = 0;  // LDS table of the response in one workgroup, 0 before the first use
     // running counts: detections, triangles, cell entries, raw pairs, distinct pairs, contacts
     long long st_dets = 0, st_tris = 0, st_entries = 0, st_raw = 0, st_pairs = 0, st_contacts = 0, st_resolved = 0;

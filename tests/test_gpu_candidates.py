@@ -95,7 +95,7 @@ def test_response_equals_the_oracle_around_one_workgroup(orc, n, low, high):
     assert low <= count <= high
     with capi.Context() as ctx:
         ctx.ccd_detect(capi.hash_desc(1, **desc), x, p, tris, 0.01)
-        for passes in (1, 3):
+        for passes in (1, 3, 4, 9):
             assert np.array_equal(ctx.ccd_resolve(p, w, 0.01, passes),
                                   orc.ccd_resolve(arr, count, tris, x, p, w, 0.01, passes))
 
