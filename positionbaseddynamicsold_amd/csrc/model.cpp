@@ -842,16 +842,32 @@ bool plan_tiles(std::vector<Cloth>& cloths, const WholeLoad& whole, int max_load
     }
     // XCD-aware launch order: consecutive (spatially adjacent) tiles go to the
     // same XCD.  Workgroups are dealt to the 8 XCDs round-robin by block id, so
-    // the j-th tile of group g gets block id j*8 + g.
-    auto xcd_order = [](const std::vector<int>& ids) {
-        const int X = 8;
-        int n = (int)ids.size();
-        int per_g = (n + X - 1) / X;
-        std::vector<int> ord((size_t)per_g * X, -1);
-        for (int i = 0; i < n; i++) {
-            int g = i / per_g, j = i % per_g;
-            ord[(size_t)j * X + g] = ids[i];
+    // the j-th tile of group g gets block id j*8 + g.  Up to one tile per CU
+    // the groups have equal counts.  Beyond, they have equal loads, and each
+    // starts with its largest tiles, so that small ones fill the end of a launch
+    // (48 cloths, 618 tiles on 512 places: 6.17 against 6.77 ms per frame; with
+    // equal loads 213 tiles of one sheet would crowd some XCDs, 1.53 against
+    // 1.17 ms).
+    auto xcd_order = [&](const std::vector<int>& ids) {
+        constexpr int X = 8, XCD_CUS = 32;
+        const bool loads = ids.size() > (size_t)X * XCD_CUS;
+        std::vector<std::vector<int>> group(X);
+        const size_t per = (ids.size() + X - 1) / X;
+        long long total = 0, before = 0;
+        for (int i : ids) total += plan.tiles[i].n_load;
+        for (size_t k = 0; k < ids.size(); k++) {
+            group[loads ? (size_t)std::min<long long>(X - 1, before * X / total) : k / per].push_back(ids[k]);
+            before += plan.tiles[ids[k]].n_load;
         }
+        size_t most = 0;
+        for (auto& g : group) {
+            if (loads)
+                std::stable_sort(g.begin(), g.end(), [&](int a, int b) { return plan.tiles[a].n_load > plan.tiles[b].n_load; });
+            most = std::max(most, g.size());
+        }
+        std::vector<int> ord(most * X, -1);
+        for (int g = 0; g < X; g++)
+            for (size_t j = 0; j < group[g].size(); j++) ord[j * X + g] = group[g][j];
         return ord;
     };
     std::vector<int> whole_ids, part_ids;
