@@ -516,8 +516,7 @@ __global__ __launch_bounds__(256) void k_swept_faces(HashCfg g, HashCfg gi, cons
                                                      int* __restrict__ large, DetectCounts* __restrict__ c) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= nt) return;
-    rec[f] = face_record(f, x, p, tris, th, 4.0f * th);
-    const FaceRec& r = rec[f];
+    const FaceRec r = face_record(f, x, p, tris, th, 4.0f * th);
     int lo[3], hi[3];
     long long span = 1, n = 1;
     for (int k = 0; k < 3; k++) {
@@ -527,6 +526,7 @@ __global__ __launch_bounds__(256) void k_swept_faces(HashCfg g, HashCfg gi, cons
         hi[k] = cell_coord(gi, r.hi[k], k);
         n *= (long long)min(hi[k] - lo[k] + 1, ENTRY_MAX_CELLS + 1);
     }
+    rec[f] = r;
     if (span > SWEPT_MAX_CELLS) c->face_span = 1;
     fcell[2 * f] = make_int4(lo[0], lo[1], lo[2], n > ENTRY_MAX_CELLS ? 1 : 0);
     fcell[2 * f + 1] = make_int4(hi[0], hi[1], hi[2], 0);
@@ -545,20 +545,23 @@ __global__ __launch_bounds__(256) void k_swept_faces(HashCfg g, HashCfg gi, cons
 __device__ __forceinline__ int cell_code(int x, int y, int z) { return (x & 511) | ((y & 511) << 9) | ((z & 511) << 18); }
 
 // place: each slot's start, moved up by every entry stored; it ends at the
-// slot's end.
+// slot's end.  FACE_LANES lanes share a face's cells, since every entry waits
+// for its atomic (128 x 128 drape, 118,000 to 198,000 entries: 17.4 us with a
+// thread per face, 14.4 so; counting waits for none and gains nothing by it).
+constexpr int FACE_LANES = 8;
 __global__ __launch_bounds__(256) void k_swept_fill(int nt, const int4* __restrict__ fcell, unsigned mask,
                                                     int* __restrict__ place, int2* __restrict__ ent, int cap) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
+    const int f = (blockIdx.x * blockDim.x + threadIdx.x) / FACE_LANES, lane = threadIdx.x % FACE_LANES;
     if (f >= nt) return;
     const int4 lo = fcell[2 * f], hi = fcell[2 * f + 1];
     if (lo.w) return;
-    for (int z = lo.z; z <= hi.z; z++)
-        for (int y = lo.y; y <= hi.y; y++)
-            for (int xx = lo.x; xx <= hi.x; xx++) {
-                const int at = atomicAdd(&place[cell_slot(xx, y, z, mask)], 1);
-                const int first = (xx == lo.x ? 1 << 27 : 0) | (y == lo.y ? 1 << 28 : 0) | (z == lo.z ? 1 << 29 : 0);
-                if (at < cap) ent[at] = make_int2(f, cell_code(xx, y, z) | first);
-            }
+    const int wx = hi.x - lo.x + 1, wy = hi.y - lo.y + 1, n = wx * wy * (hi.z - lo.z + 1);
+    for (int i = lane; i < n; i += FACE_LANES) {
+        const int z = i / (wx * wy), j = i - z * (wx * wy), y = j / wx, xx = j - y * wx;
+        const int at = atomicAdd(&place[cell_slot(lo.x + xx, lo.y + y, lo.z + z, mask)], 1);
+        const int first = (xx == 0 ? 1 << 27 : 0) | (y == 0 ? 1 << 28 : 0) | (z == 0 ? 1 << 29 : 0);
+        if (at < cap) ent[at] = make_int2(f, cell_code(lo.x + xx, lo.y + y, lo.z + z) | first);
+    }
 }
 
 // Pairs a wave has found, appended in runs to the global list.  Atomics on one
@@ -1666,7 +1669,9 @@ __global__ __launch_bounds__(256) void k_resolve_apply(const int4* __restrict__ 
     }
 }
 
-// Every pass of a few contacts in one workgroup, one contact per thread, with
+// Every pass of a few contacts in one workgroup, one contact per thread (350
+// contacts, two passes: 8.4 us; three launches take 12, and with sums in global
+// memory the workgroup took 30), with
 // the touched vertices' positions and sums in an LDS table (open addressing by
 // vertex id).  The contacts must have at most `slots` corners.
 // The sums are integers, so this order gives the bits of any other.
@@ -1966,7 +1971,7 @@ void Broadphase::swept_table(hipStream_t s, const HashCfg& g, const HashCfg& gi,
                        slots_of(table), sw_cell.ptr, (FaceRec*)rec.ptr, large.ptr, counts_of(table));
     hipLaunchKernelGGL(k_slot_places<false>, dim3(((1 << table_bits) + PLACE_SLOTS - 1) / PLACE_SLOTS), dim3(256), 0, s,
                        (const int4*)slots_of(table), 1 << table_bits, (int4*)place.ptr, &counts_of(table)->entries);
-    hipLaunchKernelGGL(k_swept_fill, dim3(blocks(nt)), dim3(256), 0, s, nt, sw_cell.ptr, mask, place.ptr,
+    hipLaunchKernelGGL(k_swept_fill, dim3(blocks((long long)FACE_LANES * nt)), dim3(256), 0, s, nt, sw_cell.ptr, mask, place.ptr,
                        ent.ptr, (int)std::min<size_t>(ent.n, 0x7fffffff));
     PBD_HIP(hipGetLastError());
 }
@@ -2158,9 +2163,11 @@ void Broadphase::resolve(hipStream_t s, const float4* x, float4* p, int nv, floa
         }
     }
     if (4 * n <= few_slots) {
-        // up to half of the slots stay free
-        const int slots = std::min(few_slots, std::max(64, 8 * n)), lds = slots * RESOLVE_SLOT_BYTES;
-        hipLaunchKernelGGL(k_resolve_few, dim3(1), dim3((n + 63) / 64 * 64), lds, s, vquad.ptr, nc, quad.ptr, ne, x, p,
+        // contacts share corners, so that half of the slots or more stay free; the threads without a contact
+        // help with the loops over the slots
+        const int slots = std::max(64, 4 * n), lds = slots * RESOLVE_SLOT_BYTES;
+        const int threads = std::min(RESOLVE_BLOCK, (std::max(n, slots / 2) + 63) / 64 * 64);
+        hipLaunchKernelGGL(k_resolve_few, dim3(1), dim3(threads), lds, s, vquad.ptr, nc, quad.ptr, ne, x, p,
                            th, min_n2, passes, slots);
         PBD_HIP(hipGetLastError());
         return;
