@@ -871,18 +871,19 @@ float mean_edge_length(const float* x, const int* tris, int nt) {
 }
 
 // Contact detection for the whole context (all cloths, global vertex ids).
-void detect_contacts(pbd_ctx* c, const float4* p) {
+// meanwhile queues the work that comes next and does not need the contacts.
+void detect_contacts(pbd_ctx* c, const float4* p, std::function<void()> meanwhile) {
     hipStream_t s = c->stream;
     HashCfg swept = c->ccfg;
     if (c->coll.broadphase == 1) swept = swept_cfg(c->ccfg, c->mean_edge, c->coll.thickness);
+    c->cbp.ee_npairs = 0;
+    c->cbp.ee_ncontacts = 0;
+    if (c->coll.edge_edge)
+        meanwhile = [c, s, p, next = std::move(meanwhile)] {
+            c->cbp.detect_ee(s, c->ccfg, c->x.ptr, p, c->gtris.ptr, c->gnt, c->coll.thickness, false, next);
+        };
     c->cbp.detect(s, c->ccfg, c->coll.broadphase == 1 ? &swept : nullptr, c->x.ptr, p, c->gtris.ptr, c->gnt,
-                  c->nv_total, c->coll.thickness, false);
-    if (c->coll.edge_edge) {
-        c->cbp.detect_ee(s, c->ccfg, c->x.ptr, p, c->gtris.ptr, c->gnt, c->coll.thickness, false);
-    } else {
-        c->cbp.ee_npairs = 0;
-        c->cbp.ee_ncontacts = 0;
-    }
+                  c->nv_total, c->coll.thickness, false, std::move(meanwhile));
 }
 
 // ---- learned warm start ------------------------------------------------------
@@ -1526,16 +1527,20 @@ void ccd_sweeps(pbd_ctx* c, int n, float dt, const int* cap) {
     c->pfinal_valid = false;
     for (int ii = 0; ii < n; ii++) {
         int cur = c->pcur;
-        if (ii % every == 0 || ii == n - 1) detect_contacts(c, c->pbuf[cur].ptr);
         a.sweep_base = ii;
-        if (c->order_first.n) {
+        // the sweep reads the p that contacts are detected at and writes the
+        // other one: it is queued before the host waits for the contacts
+        auto sweep = [&] {
+            if (!c->order_first.n) return;
             if (c->prof_on) PBD_HIP(hipEventRecord(next_event(c), s));
             launch_tiles(s, (int)c->order_first.n, c->order_first.ptr, c->tiles.ptr, c->tverts.ptr, c->tdist.ptr, c->tbend.ptr,
                      c->town.ptr, c->town_rest.ptr, c->tphases.ptr, c->tcounts.ptr, c->cl.ptr, c->ktab_d.ptr, c->ktab_b.ptr, c->x.ptr, c->v.ptr, c->pbuf[cur].ptr,
                          c->pbuf[cur ^ 1].ptr, c->res_slots.ptr, ncl, c->sweeps.ptr, cap, a, shape.threads,
                          shape.lds, !c->plan.bend.empty(), shape.regs);
             if (c->prof_on) PBD_HIP(hipEventRecord(next_event(c), s));
-        }
+        };
+        if (ii % every == 0 || ii == n - 1) detect_contacts(c, c->pbuf[cur].ptr, sweep);
+        else sweep();
         c->pcur = cur ^ 1;
         c->cbp.resolve(s, c->x.ptr, c->pbuf[c->pcur].ptr, c->nv_total, c->coll.thickness,
                        c->coll.resolve_passes, c->coll.min_normal2 > 0.0f ? c->coll.min_normal2 : 1e-6f);

@@ -1851,12 +1851,24 @@ void Broadphase::clear_table(hipStream_t s, int bits) {
 static DetectCounts* counts_of(const DBuf<int>& table) { return reinterpret_cast<DetectCounts*>(table.ptr); }
 static int* slots_of(const DBuf<int>& table) { return table.ptr + sizeof(DetectCounts) / sizeof(int); }
 
-// The counters as of this point of the stream (waits).
-DetectTotals Broadphase::read_counts(hipStream_t s) {
-    if (!counts_h) PBD_HIP(hipHostMalloc(&counts_h, sizeof(DetectCounts), hipHostMallocDefault));
-    PBD_HIP(hipMemcpyAsync(counts_h, table.ptr, sizeof(DetectCounts), hipMemcpyDeviceToHost, s));
-    PBD_HIP(hipStreamSynchronize(s));
-    const DetectCounts& c = *static_cast<const DetectCounts*>(counts_h);
+// The counters as of this point of the stream.  Waits for them only, after it
+// has queued what `meanwhile` queues (once), so that the GPU has work while the
+// host reads.  Slot: 0 vertex-face, 1 edge-edge (one may be read inside the
+// other's meanwhile).
+DetectTotals Broadphase::read_counts(hipStream_t s, int slot, std::function<void()>* meanwhile) {
+    if (!counts_h[slot]) {
+        PBD_HIP(hipHostMalloc(&counts_h[slot], sizeof(DetectCounts), hipHostMallocDefault));
+        PBD_HIP(hipEventCreateWithFlags(&counts_ready[slot], hipEventDisableTiming));
+    }
+    PBD_HIP(hipMemcpyAsync(counts_h[slot], table.ptr, sizeof(DetectCounts), hipMemcpyDeviceToHost, s));
+    PBD_HIP(hipEventRecord(counts_ready[slot], s));
+    if (meanwhile && *meanwhile) {
+        std::function<void()> queue;
+        queue.swap(*meanwhile);
+        queue();
+    }
+    PBD_HIP(hipEventSynchronize(counts_ready[slot]));
+    const DetectCounts& c = *static_cast<const DetectCounts*>(counts_h[slot]);
     DetectTotals t{0, 0, 0, c.contacts, c.entries, c.face_span, c.vertex_span};
     for (int b = 0; b < NEAR_BUCKETS; b++) {
         near_n[b] = c.bucket[b].near;
@@ -1903,13 +1915,16 @@ void Broadphase::check_pairs(unsigned long long n, const char* what) {
 // Vertex-face contacts of one substep: candidates, narrowphase.  Lists that
 // turn out too short are grown and the detection runs again.
 void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, const float4* x, const float4* p,
-                        const int* tris, int nt_, int nv, float th, bool store) {
+                        const int* tris, int nt_, int nv, float th, bool store, std::function<void()> meanwhile) {
     npairs = ncontacts = 0;
     listed = false;
     cfg = g;
     nt = nt_;
     by_box = swept != nullptr;
-    if (nt <= 0 || nv <= 0) return;
+    if (nt <= 0 || nv <= 0) {
+        if (meanwhile) meanwhile();
+        return;
+    }
     grow_near(std::max<size_t>(1 << 10, (size_t)nv / NEAR_BUCKETS));
     grow_contacts(std::max<size_t>(1 << 14, (size_t)nv / 4), store);
     DetectTotals c{};
@@ -1932,7 +1947,7 @@ void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, c
                            swept ? nullptr : (const FaceAxes*)axes.ptr, x, p, th,
                            counts_of(table), cap, vquad.ptr, vf.ptr, rt.ptr, rn.ptr, rw.ptr);
         PBD_HIP(hipGetLastError());
-        c = read_counts(s);
+        c = read_counts(s, 0, &meanwhile);
         if (swept) {
             PBD_CHECK(!c.face_span, PBD_ERR_LIMIT, "a face's swept box spans more than 4096 cells: use a larger cell");
             PBD_CHECK(c.entries < (1u << 31), PBD_ERR_LIMIT, "swept-box cell entries overflow int32");
@@ -2049,7 +2064,7 @@ long long Broadphase::list_pairs(hipStream_t s, const HashCfg& g, const float4* 
         hipLaunchKernelGGL(k_vf_candidates<true>, dim3(visit_blocks(nv)), dim3(64 * VISIT_WAVES), 0, s, g, p, p, nv,
                            vtoff.ptr, vtri.ptr, tcell.ptr, slots_of(table), place.ptr, (1u << table_bits) - 1,
                            (const FaceRec*)rec.ptr, counts_of(table), near_.ptr, cap);
-        const DetectTotals c = read_counts(s);
+        const DetectTotals c = read_counts(s, 0, nullptr);
         check_pairs(c.near, "candidate pair count");
         npairs = (long long)c.near;
         if (c.near_most <= cap) break;
@@ -2096,10 +2111,13 @@ void Broadphase::ee_candidates(hipStream_t s, const HashCfg& g, const float4* x,
 
 // Edge-edge contacts at p.
 void Broadphase::detect_ee(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt_,
-                           float th, bool store) {
+                           float th, bool store, std::function<void()> meanwhile) {
     ee_npairs = ee_ncontacts = 0;
     ee_listed = false;
-    if (nt_ <= 0 || nedges <= 0) return;
+    if (nt_ <= 0 || nedges <= 0) {
+        if (meanwhile) meanwhile();
+        return;
+    }
     PBD_CHECK(edge_tris >= (size_t)nt_, PBD_ERR_STATE, "internal: edge table does not match the triangles");
     grow_near(std::max<size_t>(1 << 10, (size_t)nedges / NEAR_BUCKETS));
     auto grow_ee = [&](size_t n) {
@@ -2119,7 +2137,7 @@ void Broadphase::detect_ee(hipStream_t s, const HashCfg& g, const float4* x, con
         hipLaunchKernelGGL(narrow, dim3(1024), dim3(256), 0, s, near_.ptr, near_cap, edges.ptr, x, p, th,
                            counts_of(table), cap, eab.ptr, quad.ptr, rt.ptr, rn.ptr, rw.ptr);
         PBD_HIP(hipGetLastError());
-        c = read_counts(s);
+        c = read_counts(s, 1, &meanwhile);
         check_pairs(c.pairs, "edge-edge candidate count");
         if (c.near_most <= near_cap && c.contacts <= cap) break;
         if (c.near_most > near_cap) grow_near((size_t)c.near_most + c.near_most / 4);
@@ -2140,7 +2158,7 @@ void Broadphase::list_detected_ee(hipStream_t s, const HashCfg& g, const float4*
     if (ee_npairs > 0) {
         for (;;) {
             ee_candidates(s, g, x, p, tris, nt, true, th, near_cap());
-            const DetectTotals c = read_counts(s);
+            const DetectTotals c = read_counts(s, 0, nullptr);
             if (c.near_most <= near_cap()) break;
             grow_near(c.near_most);
         }

@@ -2,6 +2,7 @@
 // (capi.cpp) and the HIP kernels (*.hip).
 #pragma once
 
+#include <functional>
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -257,7 +258,10 @@ struct DetectTotals {
 struct Broadphase {
     Broadphase() = default;
     ~Broadphase() {
-        if (counts_h) (void)hipHostFree(counts_h);
+        for (int i = 0; i < 2; i++) {
+            if (counts_h[i]) (void)hipHostFree(counts_h[i]);
+            if (counts_ready[i]) (void)hipEventDestroy(counts_ready[i]);
+        }
     }
     HashCfg cfg{};
     int nt = 0;
@@ -276,7 +280,8 @@ struct Broadphase {
     DBuf<int2> ent;
     DBuf<unsigned char> rec, axes;
     DBuf<int4> tcell, sw_cell;
-    void* counts_h = nullptr;  // pinned
+    void* counts_h[2] = {nullptr, nullptr};  // pinned
+    hipEvent_t counts_ready[2] = {nullptr, nullptr};
     // candidates that go to the narrowphase; contacts in any order (the
     // response reads these) and, when asked for, in ascending order
     DBuf<int2> near_;
@@ -313,12 +318,14 @@ struct Broadphase {
     // Vertex-face contacts (after set_triangles): candidates by the centroid
     // cells of g, or by swept boxes (swept: the table's own grid, whose ranges
     // contain g's).  store: contacts with time, normal and weights, in order.
+    // meanwhile: called once the detection is queued, before it is waited for;
+    // what it queues may write neither x, p nor this structure's buffers.
     void detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, const float4* x, const float4* p, const int* tris,
-                int nt, int nv, float th, bool store);
+                int nt, int nv, float th, bool store, std::function<void()> meanwhile = {});
     // Edge-edge contacts (after set_edges) by the centroid cells of g; the
     // response takes them with the vertex-face ones.
     void detect_ee(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt, float th,
-                   bool store);
+                   bool store, std::function<void()> meanwhile = {});
     long long list_pairs(hipStream_t s, const HashCfg& g, const float4* p, const int* tris, int nt, int nv);
     void list_detected(hipStream_t s, const float4* p, const int* tris, int nv);
     void list_detected_ee(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, float th);
@@ -328,7 +335,7 @@ struct Broadphase {
 
 private:
     void clear_table(hipStream_t s, int bits);
-    DetectTotals read_counts(hipStream_t s);
+    DetectTotals read_counts(hipStream_t s, int slot, std::function<void()>* meanwhile);
     void grow_near(size_t n);
     unsigned near_cap() const;
     void cells(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt, float th,
