@@ -384,11 +384,11 @@ typedef struct {
     long long ccd_detections;
     long long ccd_triangles;    /* triangles hashed */
     long long ccd_cell_entries; /* (cell, face) entries (swept-box candidates; one per triangle otherwise) */
-    long long ccd_raw_pairs;    /* candidate pairs emitted before de-duplication */
+    long long ccd_raw_pairs;    /* candidate pairs as met: each once, so equal to ccd_pairs */
     long long ccd_pairs;        /* distinct candidate pairs through the narrowphase */
     long long ccd_contacts;     /* contacts found */
     long long ccd_resolved;     /* contacts x passes evaluated by the response */
-    long long ccd_ee_raw_pairs; /* edge-edge candidates before de-duplication */
+    long long ccd_ee_raw_pairs; /* edge-edge candidates as met: equal to ccd_ee_pairs */
     long long ccd_ee_pairs;     /* distinct edge-edge candidates */
     long long ccd_ee_contacts;  /* edge-edge contacts found */
     /* bytes the LDS-tile launches must move as designed: per launched tile its

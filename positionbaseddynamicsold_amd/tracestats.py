@@ -9,11 +9,11 @@ for the two eager passes bench.py times with HIP events after its headline
 runs -- K warm-started substeps followed by K plain substeps, each preceded
 by one untimed substep, just before the copy-kernel calibration -- so the
 tile kernel's average launch duration can be compared with the bench's own
-figure.  Substeps are delimited by the per-substep k_final_buffers launch (the
-tile path's last kernel of a projection; integrate may run inside the tiles).
+figure.  A warm-started substep has one queued tile launch; a plain substep has
+the same number of tile launches each time (fixed sweeps launch nothing else).
 
 With counter files from `rocprofv3 --pmc FETCH_SIZE` and `--pmc WRITE_SIZE`
-runs (kernel filter "k_tiles|k_copy|k_final_buffers") of `bench.py
+runs (kernel filter "k_tiles|k_copy") of `bench.py
 --passes-only`, which repeats the same two passes, it prints the tile
 kernel's HBM traffic per launch in those passes, scaled by what the counters
 read for the calibration copy (1 GiB read + 1 GiB written per launch), next
@@ -22,9 +22,7 @@ printed, --passes).  With --collide (the JSON line of
 positionbaseddynamicsold_amd.collidework), it summarises that program's
 trace instead: every kernel's time and, with counter files of the same
 program, HBM bytes and GB/s per kernel, plus the algorithmic rate of the
-kernels whose bytes per unit are fixed (hash keys 56 B per triangle,
-narrowphase 104 B per candidate, edge-edge narrowphase 152 B per candidate,
-response 160 B per contact and pass).
+kernel whose bytes per unit are fixed (response 160 B per contact and pass).
 """
 from __future__ import annotations
 
@@ -55,14 +53,14 @@ def passes(seq, steps, name_of=lambda e: e[0], grid_of=lambda e: e[3]):
     c0 = max(i for i in copies if grid_of(seq[i]) == big)
     while c0 > 0 and name_of(seq[c0 - 1]) == "k_copy" and grid_of(seq[c0 - 1]) == big:
         c0 -= 1
-    # the last kernel of each substep: k_final_buffers (plain, per-chunk
-    # launches) or the queued tile launch (warm start, which records the
-    # final buffers in its schedule kernel)
-    ints = [i for i in range(c0) if name_of(seq[i]) in ("k_final_buffers", "k_tiles_queue")]
-    need = 2 * (steps + 1)
-    if len(ints) < need:
+    queued = [i for i in range(c0) if name_of(seq[i]).startswith("k_tiles_queue")]
+    if len(queued) < steps + 1:
         raise SystemExit("trace does not hold the two profiled passes")
-    ends = ints[-need:]
+    chunks = [i for i in range(queued[-1] + 1, c0) if name_of(seq[i]).startswith(("k_tiles", "void k_tiles"))]
+    per = len(chunks) // (steps + 1)
+    if per < 1 or per * (steps + 1) != len(chunks):
+        raise SystemExit("trace does not hold the plain pass")
+    ends = queued[-(steps + 1):] + chunks[per - 1::per]
     # pass = substeps 1..steps of each group of steps + 1 (the first is untimed)
     warm = (ends[0] + 1, ends[steps] + 1)
     plain = (ends[steps + 1] + 1, ends[2 * steps + 1] + 1)
@@ -111,7 +109,7 @@ def main():
         p = table(ev[pa:pb], f"profiled plain pass ({a.steps} substeps)")
         for label, per in (("warm", w), ("plain", p)):
             # the tile kernel in any of its forms (per-chunk launches, the queued launch, with bending)
-            t = [d for n, v in per.items() if n.startswith("k_tiles") for d in v]
+            t = [d for n, v in per.items() if n.removeprefix("void ").startswith("k_tiles") for d in v]
             if t:
                 print(f"k_tiles {label}: {len(t)} launches, average {statistics.fmean(t) / 1e3:.4f} ms")
     if a.fetch and a.write:
@@ -122,7 +120,7 @@ def main():
                 (wa2, wb2), (pa2, pb2), c0 = passes(seq, a.steps, grid_of=lambda e: e[2])
                 cal = statistics.fmean(v for n, v, g in seq[c0:] if n == "k_copy")
                 a2, b2 = (wa2, wb2) if rng == 0 else (pa2, pb2)
-                tiles = [v for n, v, _ in seq[a2:b2] if n.startswith("k_tiles")]
+                tiles = [v for n, v, _ in seq[a2:b2] if n.removeprefix("void ").startswith("k_tiles")]
                 vals.append((statistics.fmean(tiles), cal))
             (f, fc), (wr, wc) = vals
             scale_f = COPY_BYTES / (fc * 1024.0)
@@ -143,8 +141,7 @@ def main():
 HBM_PEAK = 8.0e12
 
 # algorithmic bytes per unit (work-file count) of the kernels with a fixed per-unit figure
-COLLIDE_ALG = {"k_tri_keys": (56, "triangles"), "k_narrow": (104, "pairs"), "k_resolve_acc": (160, "resolved"),
-               "k_narrow_ee": (152, "ee_pairs")}
+COLLIDE_ALG = {"k_resolve_acc": (160, "resolved")}
 
 
 def collide_summary(trace, work_path, fetch=None, write=None):
