@@ -508,15 +508,19 @@ __global__ __launch_bounds__(256) void k_slot_places(const int4* __restrict__ cn
 // Swept boxes: face records (their margin defines the candidate set), the
 // cells of the table's own grid gi they cover counted per slot.  A face over
 // more than ENTRY_MAX_CELLS of them goes to the list of large faces, which
-// every vertex tests.
+// every vertex tests.  The narrowphase's half-spaces are made here, where the
+// corners are loaded anyway (571,000 faces: 185 us without them, 193 with).
 __global__ __launch_bounds__(256) void k_swept_faces(HashCfg g, HashCfg gi, const float4* __restrict__ x,
                                                      const float4* __restrict__ p, const int* __restrict__ tris, int nt,
                                                      float th, unsigned mask, int* __restrict__ cnt,
                                                      int4* __restrict__ fcell, FaceRec* __restrict__ rec,
-                                                     int* __restrict__ large, DetectCounts* __restrict__ c) {
+                                                     FaceAxes* __restrict__ axes, int* __restrict__ large,
+                                                     DetectCounts* __restrict__ c) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= nt) return;
     const FaceRec r = face_record(f, x, p, tris, th, 4.0f * th);
+    const float4 X[3] = {x[r.v0], x[r.v1], x[r.v2]}, P[3] = {p[r.v0], p[r.v1], p[r.v2]};
+    axes[f] = face_axes(X, P, th);
     int lo[3], hi[3];
     long long span = 1, n = 1;
     for (int k = 0; k < 3; k++) {
@@ -1266,11 +1270,11 @@ struct NearRun {
 
 // The narrowphase over the listed pairs (their number is on the device), its
 // contacts appended in any order.  STORE: time, normal and weights too (the
-// response needs only the vertices).  axes (may be null): pairs outside the
-// face's half-spaces are dropped first, and the workgroup gathers the others
-// until it has one for every thread, since the cubic is some 3000 instructions
-// (folded 256 x 256 cloth: 17,000 of 1.1 million pairs are left; 160 us
-// without the half-spaces, 33 with them).
+// response needs only the vertices).  Pairs outside the face's half-spaces are
+// dropped first, and the workgroup gathers the others until it has one for
+// every thread, since the cubic is some 3000 instructions (folded 256 x 256
+// cloth: 17,000 of 1.1 million pairs are left; 160 us without the half-spaces,
+// 33 with them; 14.3 million swept-box pairs of a 512 x 512 one: 970 and 138).
 template <bool STORE>
 __global__ __launch_bounds__(256) void k_narrow(const int2* __restrict__ near, unsigned near_cap,
                                                 const int* __restrict__ tris, const FaceAxes* __restrict__ axes,
@@ -1312,7 +1316,7 @@ __global__ __launch_bounds__(256) void k_narrow(const int2* __restrict__ near, u
         bool keep = i < run.n;
         if (keep) {
             q = run.pairs[i];
-            keep = !axes || !axes_miss(axes[q.y], x[q.x], p[q.x]);
+            keep = !axes_miss(axes[q.y], x[q.x], p[q.x]);
         }
         if (keep) left[atomicAdd(&left_n, 1u)] = q;
         __syncthreads();
@@ -1944,7 +1948,7 @@ void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, c
         }
         auto* narrow = store ? k_narrow<true> : k_narrow<false>;
         hipLaunchKernelGGL(narrow, dim3(1024), dim3(256), 0, s, near_.ptr, near_cap, tris,
-                           swept ? nullptr : (const FaceAxes*)axes.ptr, x, p, th,
+                           (const FaceAxes*)axes.ptr, x, p, th,
                            counts_of(table), cap, vquad.ptr, vf.ptr, rt.ptr, rn.ptr, rw.ptr);
         PBD_HIP(hipGetLastError());
         c = read_counts(s, 0, &meanwhile);
@@ -1977,13 +1981,15 @@ void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, c
 void Broadphase::swept_table(hipStream_t s, const HashCfg& g, const HashCfg& gi, const float4* x, const float4* p,
                              const int* tris, float th) {
     grow(rec, (size_t)nt * sizeof(FaceRec));
+    grow(axes, (size_t)nt * sizeof(FaceAxes));
     grow(sw_cell, 2 * (size_t)nt);
     grow(large, nt);
     grow(ent, 12 * (size_t)nt);
     clear_table(s, table_bits_for(2ll * nt));
     const unsigned mask = (1u << table_bits) - 1;
     hipLaunchKernelGGL(k_swept_faces, dim3(blocks(nt)), dim3(256), 0, s, g, gi, x, p, tris, nt, th, mask,
-                       slots_of(table), sw_cell.ptr, (FaceRec*)rec.ptr, large.ptr, counts_of(table));
+                       slots_of(table), sw_cell.ptr, (FaceRec*)rec.ptr, (FaceAxes*)axes.ptr, large.ptr,
+                       counts_of(table));
     hipLaunchKernelGGL(k_slot_places<false>, dim3(((1 << table_bits) + PLACE_SLOTS - 1) / PLACE_SLOTS), dim3(256), 0, s,
                        (const int4*)slots_of(table), 1 << table_bits, (int4*)place.ptr, &counts_of(table)->entries);
     hipLaunchKernelGGL(k_swept_fill, dim3(blocks((long long)FACE_LANES * nt)), dim3(256), 0, s, nt, sw_cell.ptr, mask, place.ptr,

@@ -124,3 +124,29 @@ def test_culled_candidates_keep_every_contact(orc, th, move, shift, scale):
     with capi.Context() as ctx:
         for a, b in zip(ctx.ccd_detect(capi.hash_desc(1, **desc), x, p, tris, th), orc.contacts_arrays(arr, n)):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("th", [1e-3, 0.01, 0.06])
+@pytest.mark.parametrize("move", [0.0, 0.03, 0.2])
+@pytest.mark.parametrize("shift,scale", [(0.0, 1.0), (300.0, 1.0), (0.0, 1e-4)])
+def test_culled_swept_candidates_keep_every_contact(orc, th, move, shift, scale):
+    # the half-spaces over swept-box candidates: well-shaped triangles, some
+    # slivers and some with a repeated vertex between them
+    print(f"swept culling th={th} move={move} shift={shift} scale={scale}", flush=True)
+    rng = np.random.default_rng(12)
+    nt = 257
+    a = rng.uniform(0, 2 * np.pi, (nt, 1)) + np.array([0.0, 2.1, 4.2]) + 0.3 * rng.standard_normal((nt, 3))
+    a[::16, 1] = a[::16, 0] + 1e-3
+    u, v = np.linalg.qr(rng.standard_normal((nt, 3, 3)))[0][:, :2].transpose(1, 0, 2)
+    corner = rng.uniform(0, 0.25, (nt, 1, 3)) + 0.03 * (np.cos(a)[..., None] * u[:, None] + np.sin(a)[..., None] * v[:, None])
+    x = ((corner.reshape(-1, 3) + shift) * scale).astype(np.float32)
+    p = x + scale * move * (rng.standard_normal((nt, 1, 3)) + 0.2 * rng.standard_normal((nt, 3, 3))).reshape(-1, 3)
+    p = p.astype(np.float32)
+    tris = np.arange(3 * nt, dtype=np.int32).reshape(nt, 3)
+    tris[5::32, 2] = tris[5::32, 1]
+    th = np.float32(th * scale)
+    arr, n = orc.ccd_detect_swept(x, p, tris, th)
+    with capi.Context() as ctx:
+        got = ctx.ccd_detect(capi.hash_desc(1, cell=(0.3 * scale,) * 3, table_bits=8), x, p, tris, th, swept=True)
+        for g, b in zip(got, orc.contacts_arrays(arr, n)):
+            assert np.array_equal(g, b)
