@@ -816,10 +816,18 @@ uint64_t scene_fingerprint(const float* x, const float* p, int nv, const int* tr
     return h;
 }
 
+// Uploads a standalone scene.  What was found on an earlier one goes with it, so
+// that a call refused further on leaves empty lists and not ones whose vertices
+// and triangles are no longer there; keep: the vertex-face detection's stays if
+// this is its scene and settings.
 void upload_scene(pbd_ctx* c, const float* x, const float* p, const float* w, int nv, const int* tris, int nt,
-                  float th = 0.0f, const pbd_hash_desc* d = nullptr) {
+                  float th = 0.0f, const pbd_hash_desc* d = nullptr, bool keep = false) {
     PBD_CHECK(nv >= 0 && nt >= 0 && (x || !nv) && (p || !nv) && (tris || !nt), PBD_ERR_ARG, "bad scene arrays");
     for (long long i = 0; i < 3ll * nt; i++) PBD_CHECK(tris[i] >= 0 && tris[i] < nv, PBD_ERR_ARG, "triangle index out of range");
+    const uint64_t hash = scene_fingerprint(x, p, nv, tris, nt, th, d ? *d : pbd_hash_desc{});
+    if (!(keep && c->ccd_built && hash == c->scene_hash)) c->sbp.npairs = c->sbp.ncontacts = 0;
+    c->sbp.ee_npairs = c->sbp.ee_ncontacts = 0;
+    c->sh_stale = true;
     std::vector<float4> X(nv), P(nv);
     for (int i = 0; i < nv; i++) {
         float wi = w ? w[i] : 1.0f;
@@ -833,7 +841,7 @@ void upload_scene(pbd_ctx* c, const float* x, const float* p, const float* w, in
     c->snv = nv;
     c->snt = nt;
     c->s_th = th;
-    c->scene_hash = scene_fingerprint(x, p, nv, tris, nt, th, d ? *d : pbd_hash_desc{});
+    c->scene_hash = hash;
 }
 
 // The grid of the swept-box table: the caller's cells taken m at a time per
@@ -2308,10 +2316,7 @@ int pbd_ccd_detect(pbd_ctx* ctx, const pbd_hash_desc* d, const float* x, const f
         upload_scene(ctx, x, p, nullptr, nv, tris, nt, th, d);
         ctx->sbp.detect(s, g, nullptr, ctx->sx.ptr, ctx->sp4.ptr, ctx->stris.ptr, nt, nv, th, true);
         *nc = ctx->sbp.ncontacts;
-        ctx->sbp.ee_npairs = 0;
-        ctx->sbp.ee_ncontacts = 0;
         ctx->sh_built = true;
-        ctx->sh_stale = true;
         ctx->ccd_built = true;
     });
 }
@@ -2324,18 +2329,11 @@ int pbd_ccd_detect_ee(pbd_ctx* ctx, const pbd_hash_desc* d, const float* x, cons
         set_device(ctx);
         hipStream_t s = ctx->stream;
         HashCfg g = make_hash_cfg(*d);
-        const uint64_t prev_hash = ctx->scene_hash;
         // vertex-face contacts of an earlier detection on another scene, or
         // at another thickness or grid, do not carry over
-        upload_scene(ctx, x, p, nullptr, nv, tris, nt, th, d);
-        bool same = ctx->ccd_built && ctx->scene_hash == prev_hash;
-        if (same) {
-            // their list shares a buffer with the edge pairs
-            ctx->sbp.list_detected(s, ctx->sp4.ptr, ctx->stris.ptr, nv);
-        } else {
-            ctx->sbp.npairs = 0;
-            ctx->sbp.ncontacts = 0;
-        }
+        upload_scene(ctx, x, p, nullptr, nv, tris, nt, th, d, true);
+        // those of this one: their list shares a buffer with the edge pairs
+        ctx->sbp.list_detected(s, ctx->sp4.ptr, ctx->stris.ptr, nv);
         std::vector<int> te;
         std::vector<int2> ed;
         build_edge_table(tris, nt, te, ed);
@@ -2345,7 +2343,6 @@ int pbd_ccd_detect_ee(pbd_ctx* ctx, const pbd_hash_desc* d, const float* x, cons
         ctx->sbp.detect_ee(s, g, ctx->sx.ptr, ctx->sp4.ptr, ctx->stris.ptr, nt, th, true);
         if (npairs) *npairs = ctx->sbp.ee_npairs;
         *nc = ctx->sbp.ee_ncontacts;
-        ctx->sh_stale = true;
         ctx->sh_built = true;
         ctx->ccd_built = true;
     });
@@ -2410,8 +2407,6 @@ int pbd_ccd_detect_swept(pbd_ctx* ctx, const pbd_hash_desc* d, const float* x, c
         ctx->sbp.detect(s, g, &swept, ctx->sx.ptr, ctx->sp4.ptr, ctx->stris.ptr, nt, nv, th, true);
         if (npairs) *npairs = ctx->sbp.npairs;
         *nc = ctx->sbp.ncontacts;
-        ctx->sbp.ee_npairs = 0;
-        ctx->sbp.ee_ncontacts = 0;
         ctx->sh_built = false;  // the cell table holds swept entries, not centroid keys
         ctx->ccd_built = true;
     });

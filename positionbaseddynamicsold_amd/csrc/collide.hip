@@ -2085,7 +2085,7 @@ long long Broadphase::list_pairs(hipStream_t s, const HashCfg& g, const float4* 
 void Broadphase::list_detected(hipStream_t s, const float4* p, const int* tris, int nv) {
     if (listed) return;
     const long long n = npairs;
-    if (by_box) sort_near(s, nv, nt, uv, uf);
+    if (n > 0 && by_box) sort_near(s, nv, nt, uv, uf);
     else if (n > 0) list_pairs(s, cfg, p, tris, nt, nv);
     npairs = n;
     listed = true;
