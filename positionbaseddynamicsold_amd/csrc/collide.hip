@@ -16,8 +16,10 @@
 //   fixed point (integer sums are order independent, so the result does not
 //   depend on atomic ordering) and applied as the mean fix per vertex.
 // Paths are relative to PositionBasedDynamicsCUDA/PositionBasedDynamicsCUDA/.
+#include <algorithm>
 #include <climits>
 #include <mutex>
+#include <type_traits>
 
 #include "pbd_internal.hpp"
 #include "pbd_math.hpp"
@@ -690,6 +692,12 @@ __device__ __forceinline__ void visit_runs(GroupLds& lds, const int3* q, const i
 }
 static_assert(RUN_WINDOW == 32 * 32, "a lane clears one word of the window");
 
+// What a hub's unit visits (see HubRounds).
+struct HubItem {
+    const int* set;
+    int unit, place;
+};
+
 // Whether c is a valid cell and (x, y, z) is within one cell of it.
 __device__ __forceinline__ bool near_cell(int4 c, int x, int y, int z) {
     return c.w >= 0 && abs(c.x - x) <= 1 && abs(c.y - y) <= 1 && abs(c.z - z) <= 1;
@@ -699,12 +707,26 @@ __device__ __forceinline__ int3 around(int4 c, int l) {
     return make_int3(c.x + l % 3 - 1, c.y + l / 3 % 3 - 1, c.z + l / 9 - 1);
 }
 
-// The cells around a group's own triangles, each once, two per lane and round
-// (most boxes have 27 to 64 cells, which then take one round of memory
-// latencies): the cells of the box of their cells that lie around one of them.
-// A group with more than 32 triangles or a box of more than BOX_CELLS cells
-// takes the 27 cells around one triangle after the other instead, without
-// those that lie around an earlier one.
+// The entries of a lane's two cells q of round r of `cells`; whether there are any.
+template <class Cells>
+__device__ __forceinline__ bool cell_runs(const Cells& cells, const HashCfg& g, int r, const int* __restrict__ cnt,
+                                          const int* __restrict__ end, unsigned mask, int3* q, int* start, int* n) {
+    for (int c = 0; c < 2; c++) {
+        const bool mine = cells.cell(g, r, c, &q[c]);
+        const unsigned slot = mine ? cell_slot(q[c].x, q[c].y, q[c].z, mask) : 0u;
+        const int k = cnt[slot], e = end[slot];
+        n[c] = mine ? k : 0;
+        start[c] = e - k;
+    }
+    return n[0] + n[1] > 0;
+}
+
+// The cells around a group's own triangles (up to HUB_FACES), each once, two
+// per lane and round (most boxes have 27 to 64 cells, which then take one round
+// of memory latencies): the cells of the box of their cells that lie around one
+// of them.  A box of more than BOX_CELLS cells takes the 27 cells around one
+// triangle after the other instead, without those that lie around an earlier one.
+constexpr int HUB_FACES = 32;
 struct CellRounds {
     const GroupLds* lds;
     const int* list;
@@ -713,7 +735,7 @@ struct CellRounds {
     bool boxed;
     int3 lo, w;
     // Called by all lanes of the wave.
-    __device__ __forceinline__ void start(GroupLds& g, const int* list_, int deg_, const int4* tcell_) {
+    __device__ __forceinline__ void start(GroupLds& g, const int* list_, int deg_, const int4* tcell_, const HubItem&) {
         lds = &g;
         list = list_;
         tcell = tcell_;
@@ -736,7 +758,7 @@ struct CellRounds {
             n = (long long)w.x * w.y * w.z;
         }
         lo = make_int3(lo.x - 1, lo.y - 1, lo.z - 1);
-        boxed = deg <= 32 && n <= BOX_CELLS;
+        boxed = n <= BOX_CELLS;
         rounds = boxed ? ((int)n + 63) / 64 : deg;
         // mark the 27 cells around each triangle
         __builtin_amdgcn_wave_barrier();  // the group before is done with `cover`
@@ -772,18 +794,6 @@ struct CellRounds {
             if (near_cell(tcell[list[j]], q->x, q->y, q->z)) return false;
         return cell_key(g, q->x, q->y, q->z) >= 0;
     }
-    // The entries of this lane's cells q of round r; whether there are any.
-    __device__ __forceinline__ bool runs(const HashCfg& g, int r, const int* __restrict__ cnt,
-                                         const int* __restrict__ end, unsigned mask, int3* q, int* start, int* n) const {
-        for (int c = 0; c < 2; c++) {
-            const bool mine = cell(g, r, c, &q[c]);
-            const unsigned slot = mine ? cell_slot(q[c].x, q[c].y, q[c].z, mask) : 0u;
-            const int k = cnt[slot], e = end[slot];
-            n[c] = mine ? k : 0;
-            start[c] = e - k;
-        }
-        return n[0] + n[1] > 0;
-    }
     // Whether c is a cell around one of the triangles.
     __device__ __forceinline__ bool meets(int4 c) const {
         if (c.w < 0) return false;
@@ -799,17 +809,107 @@ struct CellRounds {
     }
 };
 
+// Hubs: vertices (edges) of more than HUB_FACES triangles, such as the poles of
+// a sphere or the tip of a cone.  Comparing the cells around one triangle with
+// those of all earlier ones, as above, is quadratic in a hub's triangles and
+// done by one group (a fan of 1024 triangles, 2 units wide: 118 ms a detection).  The cells
+// around a hub go into a set of its own instead, HUB_SLOTS slots per triangle
+// (27 cells at most), each slot holding 27 times the place of a triangle in the
+// hub's list plus a cell around it.  A unit is one triangle of one hub: 32 lanes
+// enter its cells, and later visit the HUB_SLOTS slots of the set at its place,
+// so that a hub's work spreads over as many groups as it has triangles (0.3 ms
+// for that fan).
+constexpr int HUB_SLOTS = 64;
+
+__device__ __forceinline__ unsigned hub_slot(int3 q, unsigned slots) {
+    return __umulhi(cell_slot(q.x, q.y, q.z, 0xffffffffu) * 0x9E3779B1u, slots);
+}
+__device__ __forceinline__ int3 hub_cell(int entry, const int* __restrict__ list, const int4* __restrict__ tcell) {
+    return around(tcell[list[entry / 27]], entry % 27);
+}
+__device__ __forceinline__ bool same_cell(int3 a, int3 b) { return a.x == b.x && a.y == b.y && a.z == b.z; }
+
+__global__ __launch_bounds__(256) void k_hub_count(const int* __restrict__ off, int n,
+                                                   unsigned long long* __restrict__ units) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int deg = off[i + 1] - off[i];
+    if (deg > HUB_FACES) atomicAdd(units, (unsigned long long)deg);
+}
+__global__ __launch_bounds__(256) void k_hub_units(const int* __restrict__ off, int n,
+                                                   unsigned long long* __restrict__ units, int2* __restrict__ unit) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int deg = off[i + 1] - off[i];
+    if (deg <= HUB_FACES) return;
+    const unsigned long long at = atomicAdd(units, (unsigned long long)deg);
+    for (int k = 0; k < deg; k++) unit[at + k] = make_int2(i, k);
+}
+// The sets of all hubs, from empty (-1) ones.
+__global__ __launch_bounds__(256) void k_hub_enter(const int2* __restrict__ unit, int nunits, const int* __restrict__ off,
+                                                   const int* __restrict__ tri, const int4* __restrict__ tcell,
+                                                   int* __restrict__ set) {
+    const int u = (int)(((long long)blockIdx.x * blockDim.x + threadIdx.x) / 32), l = threadIdx.x & 31;
+    if (u >= nunits || l >= 27) return;
+    const int2 h = unit[u];
+    const int* list = tri + off[h.x];
+    const unsigned slots = (unsigned)(off[h.x + 1] - off[h.x]) * HUB_SLOTS;
+    int* own = set + (size_t)(u - h.y) * HUB_SLOTS;
+    const int4 c = tcell[list[h.y]];
+    if (c.w < 0) return;
+    const int3 q = around(c, l);
+    for (unsigned s = hub_slot(q, slots);; s = s + 1 == slots ? 0 : s + 1) {  // ends: at most 27 of 64 slots fill
+        const int old = atomicCAS(&own[s], -1, h.y * 27 + l);
+        if (old == -1 || same_cell(hub_cell(old, list, tcell), q)) return;
+    }
+}
+
+// The cells in the slots of a unit, as CellRounds gives those of a group.
+struct HubRounds {
+    const int* list;
+    const int4* tcell;
+    const int* own;  // the hub's set
+    unsigned slots, at;
+    int rounds;
+    __device__ __forceinline__ void start(GroupLds&, const int* list_, int deg, const int4* tcell_, const HubItem& h) {
+        list = list_;
+        tcell = tcell_;
+        own = h.set + (size_t)(h.unit - h.place) * HUB_SLOTS;
+        slots = (unsigned)deg * HUB_SLOTS;
+        at = (unsigned)h.place * HUB_SLOTS;
+        rounds = deg ? 1 : 0;
+    }
+    __device__ __forceinline__ bool cell(const HashCfg& g, int r, int c, int3* q) const {
+        *q = make_int3(0, 0, 0);
+        const int i = r < rounds ? own[at + 32 * c + (threadIdx.x & 31)] : -1;
+        if (i < 0) return false;
+        *q = hub_cell(i, list, tcell);
+        return cell_key(g, q->x, q->y, q->z) >= 0;
+    }
+    __device__ __forceinline__ bool meets(int4 c) const {
+        if (c.w < 0) return false;
+        const int3 q = make_int3(c.x, c.y, c.z);
+        for (unsigned s = hub_slot(q, slots);; s = s + 1 == slots ? 0 : s + 1) {
+            const int i = own[s];
+            if (i < 0) return false;
+            if (same_cell(hub_cell(i, list, tcell), q)) return true;
+        }
+    }
+};
+static_assert(HUB_SLOTS == 64, "two slots per lane of a group");
+
 // Vertex-face candidates by centroid cells.  Group = 32 lanes = one vertex.
 // All candidates are counted; listed are all of them (LIST) or those that no
 // box rules out.  Memory latency bounds it (71% of the wave cycles wait), so
 // registers are held to 64 for eight waves per SIMD: 81 us against 95 with
-// seven on the folded 256 x 256 cloth (5 million pairs).
-template <bool LIST>
+// seven on the folded 256 x 256 cloth (5 million pairs).  Hubs are left out and
+// reported; HUBS: the units of hubs instead of the nv vertices.
+template <bool LIST, bool HUBS>
 __global__ __launch_bounds__(64 * VISIT_WAVES, 8) void k_vf_candidates(
     HashCfg g, const float4* __restrict__ x, const float4* __restrict__ p, int nv, const int* __restrict__ vtoff,
     const int* __restrict__ vtri, const int4* __restrict__ tcell, const int* __restrict__ cnt,
     const int* __restrict__ end, unsigned mask, const FaceRec* __restrict__ ent, DetectCounts* __restrict__ c,
-    int2* __restrict__ out, unsigned cap) {
+    int2* __restrict__ out, unsigned cap, const int2* __restrict__ unit, const int* __restrict__ hub_set) {
     __shared__ int2 buf[VISIT_WAVES][VISIT_BUF];
     __shared__ GroupLds group[VISIT_WAVES][2];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -818,21 +918,27 @@ __global__ __launch_bounds__(64 * VISIT_WAVES, 8) void k_vf_candidates(
     int pairs = 0;
     const int stride = (int)gridDim.x * VISIT_WAVES * 2;
     for (int v0 = ((int)blockIdx.x * VISIT_WAVES + wv) * 2; v0 < nv; v0 += stride) {
-        const int v = v0 + (lane >> 5), at = min(v, nv - 1);
-        const int o = vtoff[at], deg = v < nv ? vtoff[at + 1] - o : 0;
-        SweptBox b = vertex_box(x[at], p[at]);
+        const int item = v0 + (lane >> 5), last = min(item, nv - 1);
+        const int2 hub = HUBS ? unit[last] : make_int2(last, 0);
+        const int v = hub.x, o = vtoff[v];
+        int deg = item < nv ? vtoff[v + 1] - o : 0;
+        if (!HUBS && deg > HUB_FACES) {
+            c->hubs = 1;
+            deg = 0;
+        }
+        SweptBox b = vertex_box(x[v], p[v]);
         for (int k = 0; k < 3; k++) {  // the rounding of positions between the two
             const float m = 1e-6f * fmaxf(fabsf(b.lo[k]), fabsf(b.hi[k]));
             b.lo[k] -= m;
             b.hi[k] += m;
         }
-        CellRounds cells;
-        cells.start(lds, vtri + o, deg, tcell);
+        std::conditional_t<HUBS, HubRounds, CellRounds> cells;
+        cells.start(lds, vtri + o, deg, tcell, HubItem{hub_set, last, hub.y});
         const int rounds = max(cells.rounds, __shfl_xor(cells.rounds, 32));
         for (int r = 0; r < rounds; r++) {
             int3 q[2];
             int start[2], n[2];
-            if (!__any(cells.runs(g, r, cnt, end, mask, q, start, n))) continue;
+            if (!__any(cell_runs(cells, g, r, cnt, end, mask, q, start, n))) continue;
             visit_runs(lds, q, start, n, [&](int e, int3 fq) {
                 bool hit = false;
                 int f = 0;
@@ -936,7 +1042,10 @@ __device__ __forceinline__ bool edges_apart(const SweptBox& a, const SweptBox& b
 // An entry of the edge table: an edge in one of the cells of its faces, with
 // its ends and the swept box of the four points, not widened.  `before`: none
 // (0), one (1: the cell o) or several (2) of the edge's other cells come first
-// in the order of its faces.
+// in the order of its faces.  EDGE_HUB: an edge of more than HUB_FACES faces,
+// entered once per face, ox its place in etri; telling its distinct cells apart
+// one by one took 0.3 s for 1024 faces.
+constexpr int EDGE_HUB = 3;
 struct alignas(64) EdgeRec {
     int cx, cy, cz, edge;
     int v0, v1, before, ox;
@@ -944,11 +1053,24 @@ struct alignas(64) EdgeRec {
     SweptBox box;
 };
 
-// Calls f(cell, before, other) for every distinct valid cell of e's faces.
+// Calls f(e, cell, before, other) for every entry of this lane's edge e (0 <= e
+// < ne), a hub's by all lanes of the wave.  Called by all of them.
 template <class F>
-__device__ __forceinline__ void edge_cells(int e, const int* __restrict__ etoff, const int* __restrict__ etri,
+__device__ __forceinline__ void edge_cells(int e, int ne, const int* __restrict__ etoff, const int* __restrict__ etri,
                                            const int4* __restrict__ tcell, F&& f) {
-    const int o = etoff[e], deg = etoff[e + 1] - o;
+    int o = 0, deg = 0;
+    if (e < ne) {
+        o = etoff[e];
+        deg = etoff[e + 1] - o;
+    }
+    for (unsigned long long hubs = __ballot(deg > HUB_FACES); hubs; hubs &= hubs - 1) {
+        const int lane = __ffsll(hubs) - 1, h = __shfl(e, lane), h0 = __shfl(o, lane), h1 = h0 + __shfl(deg, lane);
+        for (int j = h0 + (int)(threadIdx.x & 63); j < h1; j += 64) {
+            const int4 c = tcell[etri[j]];
+            if (c.w >= 0) f(h, c, EDGE_HUB, make_int4(j, 0, 0, 0));
+        }
+    }
+    if (deg > HUB_FACES) return;
     int4 other = make_int4(0, 0, 0, 0);
     int distinct = 0;
     for (int j = 0; j < deg; j++) {
@@ -959,7 +1081,7 @@ __device__ __forceinline__ void edge_cells(int e, const int* __restrict__ etoff,
             fresh = d.w < 0 || d.x != c.x || d.y != c.y || d.z != c.z;
         }
         if (!fresh) continue;
-        f(c, min(distinct, 2), other);
+        f(e, c, min(distinct, 2), other);
         if (!distinct++) other = c;
     }
 }
@@ -977,7 +1099,7 @@ __global__ __launch_bounds__(256) void k_tri_cells(HashCfg g, const float4* __re
 __global__ __launch_bounds__(256) void k_edge_count(int ne, const int* __restrict__ etoff, const int* __restrict__ etri,
                                                     const int4* __restrict__ tcell, int* __restrict__ cnt) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < ne) edge_cells(e, etoff, etri, tcell, [&](int4 c, int, int4) { atomicAdd(&cnt[c.w], 1); });
+    edge_cells(e, ne, etoff, etri, tcell, [&](int, int4 c, int, int4) { atomicAdd(&cnt[c.w], 1); });
 }
 
 // Each entry takes the next place of its slot, so that place[] ends at the
@@ -986,13 +1108,12 @@ __global__ __launch_bounds__(256) void k_edge_fill(int ne, const int2* __restric
                                                    const int* __restrict__ etri, const int4* __restrict__ tcell,
                                                    const float4* __restrict__ x, const float4* __restrict__ p,
                                                    int* __restrict__ place, EdgeRec* __restrict__ ent) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= ne) return;
-    const int2 v = edges[e];
-    SweptBox b = vertex_box(x[v.x], p[v.x]);
-    box_add(b, x[v.y]);
-    box_add(b, p[v.y]);
-    edge_cells(e, etoff, etri, tcell, [&](int4 c, int before, int4 o) {
+    const int mine = blockIdx.x * blockDim.x + threadIdx.x;
+    edge_cells(mine, ne, etoff, etri, tcell, [&](int e, int4 c, int before, int4 o) {
+        const int2 v = edges[e];
+        SweptBox b = vertex_box(x[v.x], p[v.x]);
+        box_add(b, x[v.y]);
+        box_add(b, p[v.y]);
         ent[atomicAdd(&place[c.w], 1)] = EdgeRec{c.x, c.y, c.z, e, v.x, v.y, before, o.x, o.y, o.z, b};
     });
 }
@@ -1007,16 +1128,31 @@ __global__ __launch_bounds__(256) void k_edge_fill(int ne, const int2* __restric
 // counts at the first in the order of its faces.
 // Edges have entries of their own, with all that the tests read: visiting the
 // faces' entries instead offered most edges twice and took four dependent
-// gathers to tell (fold of 96 x 96: 151 us against 84).
+// gathers to tell (fold of 96 x 96: 151 us against 84).  Hubs are left out and
+// reported; HUBS: the units of hubs instead of the ne edges.
 constexpr int RING_MAX = 64;
 
-template <bool LIST>
+// Whether id is among n neighbours, which are in ascending order beyond RING_SORTED.
+constexpr int RING_SORTED = 16;
+__device__ __forceinline__ bool listed(const int* __restrict__ a, int n, int id) {
+    if (n > RING_SORTED) {
+        int lo = 0;  // the last one not above id, if any
+        for (int len = n; len > 1; len -= len / 2)
+            if (a[lo + len / 2] <= id) lo += len / 2;
+        return a[lo] == id;
+    }
+    bool in = false;
+    for (int i = 0; i < n; i++) in |= a[i] == id;
+    return in;
+}
+
+template <bool LIST, bool HUBS>
 __global__ __launch_bounds__(64 * VISIT_WAVES) void k_ee_candidates(
     HashCfg g, int ne, const int2* __restrict__ edges, const int* __restrict__ etoff, const int* __restrict__ etri,
     const int* __restrict__ voff, const int* __restrict__ vnbr, const float4* __restrict__ x,
     const float4* __restrict__ p, const int4* __restrict__ tcell, const int* __restrict__ cnt,
     const int* __restrict__ end, unsigned mask, const EdgeRec* __restrict__ ent, float th, DetectCounts* __restrict__ c,
-    int2* __restrict__ out, unsigned cap) {
+    int2* __restrict__ out, unsigned cap, const int2* __restrict__ unit, const int* __restrict__ hub_set) {
     __shared__ int2 buf[VISIT_WAVES][VISIT_BUF];
     __shared__ int4 ring_s[VISIT_WAVES][2][RING_MAX / 4];
     __shared__ GroupLds group[VISIT_WAVES][2];
@@ -1027,9 +1163,15 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_ee_candidates(
     int pairs = 0;
     const int stride = (int)gridDim.x * VISIT_WAVES * 2;
     for (int a0 = ((int)blockIdx.x * VISIT_WAVES + wv) * 2; a0 < ne; a0 += stride) {
-        const int a = a0 + (lane >> 5), at = min(a, ne - 1);
-        const int2 av = edges[at];
-        const int o = etoff[at], deg = a < ne ? etoff[at + 1] - o : 0;
+        const int item = a0 + (lane >> 5), last = min(item, ne - 1);
+        const int2 hub = HUBS ? unit[last] : make_int2(last, 0);
+        const int a = hub.x, o = etoff[a];
+        const int2 av = edges[a];
+        int deg = item < ne ? etoff[a + 1] - o : 0;
+        if (!HUBS && deg > HUB_FACES) {
+            c->hubs = 1;
+            deg = 0;
+        }
         SweptBox abox = vertex_box(x[av.x], p[av.x]);
         box_add(abox, x[av.y]);
         box_add(abox, p[av.y]);
@@ -1045,8 +1187,8 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_ee_candidates(
                                                   : i < n0 + 2      ? vnbr[r0 + i - 2]
                                                   : i < n0 + n1 + 2 ? vnbr[r1 + i - 2 - n0]
                                                                     : -1;
-        CellRounds cells;
-        cells.start(lds, etri + o, deg, tcell);
+        std::conditional_t<HUBS, HubRounds, CellRounds> cells;
+        cells.start(lds, etri + o, deg, tcell, HubItem{hub_set, last, hub.y});
         auto ringed = [&](int u, int w) {
             bool in = false;
             if (fits) {
@@ -1056,16 +1198,14 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_ee_candidates(
                 }
                 return in;
             }
-            in = u == av.x || u == av.y || w == av.x || w == av.y;
-            for (int i = 0; i < n0; i++) in |= vnbr[r0 + i] == u || vnbr[r0 + i] == w;
-            for (int i = 0; i < n1; i++) in |= vnbr[r1 + i] == u || vnbr[r1 + i] == w;
-            return in;
+            return u == av.x || u == av.y || w == av.x || w == av.y || listed(vnbr + r0, n0, u) ||
+                   listed(vnbr + r0, n0, w) || listed(vnbr + r1, n1, u) || listed(vnbr + r1, n1, w);
         };
         const int rounds = max(cells.rounds, __shfl_xor(cells.rounds, 32));
         for (int r = 0; r < rounds; r++) {
             int3 q[2];
             int start[2], n[2];
-            if (!__any(cells.runs(g, r, cnt, end, mask, q, start, n))) continue;
+            if (!__any(cell_runs(cells, g, r, cnt, end, mask, q, start, n))) continue;
             visit_runs(lds, q, start, n, [&](int e, int3 fq) {
                 bool hit = false;
                 int eb = 0;
@@ -1073,13 +1213,16 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_ee_candidates(
                     const EdgeRec rec = ent[e];
                     eb = rec.edge;
                     if (eb > a && rec.cx == fq.x && rec.cy == fq.y && rec.cz == fq.z && !ringed(rec.v0, rec.v1)) {
-                        bool first = !rec.before || !cells.meets(make_int4(rec.ox, rec.oy, rec.oz, 0));
+                        bool first = rec.before == 0 || rec.before == EDGE_HUB ||
+                                     !cells.meets(make_int4(rec.ox, rec.oy, rec.oz, 0));
                         if (rec.before == 2)
                             for (int j = etoff[eb]; first; j++) {  // ends at a face of this cell
                                 const int4 d = tcell[etri[j]];
                                 if (d.w >= 0 && d.x == rec.cx && d.y == rec.cy && d.z == rec.cz) break;
                                 first = !cells.meets(d);
                             }
+                        if (rec.before == EDGE_HUB)
+                            for (int j = etoff[eb]; first && j < rec.ox; j++) first = !cells.meets(tcell[etri[j]]);
                         pairs += first;
                         hit = first && (LIST || !edges_apart(abox, rec.box, th));
                     }
@@ -1793,6 +1936,7 @@ void Broadphase::build(hipStream_t s, const HashCfg& g, const float4* p, const i
 
 void Broadphase::set_edges(hipStream_t s, const std::vector<int>& te, const std::vector<int2>& ed) {
     edge_tris = te.size() / 3;
+    ehubs.forget();
     edges.upload(ed, s);
     nedges = (int)ed.size();
     // edge -> triangles (CSR)
@@ -1817,6 +1961,8 @@ void Broadphase::set_edges(hipStream_t s, const std::vector<int>& te, const std:
         nbr[fill[e.x]++] = e.y;
         nbr[fill[e.y]++] = e.x;
     }
+    for (int v = 0; v < nv; v++)
+        if (off[v + 1] - off[v] > RING_SORTED) std::sort(nbr.begin() + off[v], nbr.begin() + off[v + 1]);
     voff.upload(off, s);
     vnbr.upload(nbr, s);
     PBD_HIP(hipStreamSynchronize(s));
@@ -1824,6 +1970,7 @@ void Broadphase::set_edges(hipStream_t s, const std::vector<int>& te, const std:
 
 // Vertex -> triangles of a triangle list.
 void Broadphase::set_triangles(hipStream_t s, const int* tris, int nt_, int nv) {
+    vhubs.forget();
     grow(vtoff, (size_t)nv + 1);
     grow(vtri, (size_t)3 * std::max(1, nt_));
     grow(cnt, (size_t)nv + 1);
@@ -1873,7 +2020,7 @@ DetectTotals Broadphase::read_counts(hipStream_t s, int slot, std::function<void
     }
     PBD_HIP(hipEventSynchronize(counts_ready[slot]));
     const DetectCounts& c = *static_cast<const DetectCounts*>(counts_h[slot]);
-    DetectTotals t{0, 0, 0, c.contacts, c.entries, c.face_span, c.vertex_span};
+    DetectTotals t{0, 0, 0, c.contacts, c.entries, c.face_span, c.vertex_span, c.hubs};
     for (int b = 0; b < NEAR_BUCKETS; b++) {
         near_n[b] = c.bucket[b].near;
         t.pairs += c.bucket[b].pairs;
@@ -1889,7 +2036,52 @@ unsigned Broadphase::near_cap() const { return (unsigned)std::min<size_t>(near_.
 
 // Workgroups of the candidate visits: each wave takes two vertices (edges) at
 // a time, and enough waves to fill the GPU take them in turn.
-static int visit_blocks(int n) { return std::max(1, std::min(2048, (n + 2 * VISIT_WAVES - 1) / (2 * VISIT_WAVES))); }
+static int visit_blocks(long long n) { return (int)std::max(1ll, std::min(2048ll, (n + 2 * VISIT_WAVES - 1) / (2 * VISIT_WAVES))); }
+
+// The units of the hubs among n vertices (edges) with the CSR offsets off, asked
+// for once per triangle list (edge table), when a visit has reported a hub.
+void Broadphase::Hubs::find(hipStream_t s, const int* off, int n) {
+    DBuf<unsigned long long> total;
+    total.alloc(2);
+    PBD_HIP(hipMemsetAsync(total.ptr, 0, 2 * sizeof(unsigned long long), s));
+    hipLaunchKernelGGL(k_hub_count, dim3(blocks(n)), dim3(256), 0, s, off, n, total.ptr);
+    PBD_HIP(hipGetLastError());
+    unsigned long long u = 0;
+    PBD_HIP(hipMemcpyAsync(&u, total.ptr, sizeof u, hipMemcpyDeviceToHost, s));
+    PBD_HIP(hipStreamSynchronize(s));
+    PBD_CHECK(u < (1ull << 26), PBD_ERR_LIMIT, "too many triangles around hubs");  // HUB_SLOTS * u in 32 bits
+    grow(unit, (size_t)u);
+    grow(set, (size_t)u * HUB_SLOTS);
+    hipLaunchKernelGGL(k_hub_units, dim3(blocks(n)), dim3(256), 0, s, off, n, total.ptr + 1, unit.ptr);
+    PBD_HIP(hipGetLastError());
+    PBD_HIP(hipStreamSynchronize(s));  // `total` goes
+    units = (int)u;
+    known = true;
+}
+
+// Their sets at the triangles' current cells.
+void Broadphase::Hubs::enter(hipStream_t s, const int* off, const int* tri, const int4* tcell) {
+    PBD_HIP(hipMemsetAsync(set.ptr, 0xff, sizeof(int) * (size_t)units * HUB_SLOTS, s));
+    hipLaunchKernelGGL(k_hub_enter, dim3(blocks(32ll * units)), dim3(256), 0, s, unit.ptr, units, off, tri, tcell, set.ptr);
+    PBD_HIP(hipGetLastError());
+}
+
+// The visits of the vertices to the centroid-cell table.
+void Broadphase::vf_candidates(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, int nv, bool list,
+                               unsigned cap) {
+    const unsigned mask = (1u << table_bits) - 1;
+    auto visit = [&](auto* k, int n) {
+        hipLaunchKernelGGL(k, dim3(visit_blocks(n)), dim3(64 * VISIT_WAVES), 0, s, g, x, p, n, vtoff.ptr, vtri.ptr,
+                           tcell.ptr, slots_of(table), place.ptr, mask, (const FaceRec*)rec.ptr, counts_of(table), near_.ptr,
+                           cap, vhubs.unit.ptr, vhubs.set.ptr);
+    };
+    visit(list ? k_vf_candidates<true, false> : k_vf_candidates<false, false>, nv);
+    if (vhubs.units > 0) {
+        vhubs.enter(s, vtoff.ptr, vtri.ptr, tcell.ptr);
+        visit(list ? k_vf_candidates<true, true> : k_vf_candidates<false, true>, vhubs.units);
+    }
+    PBD_HIP(hipGetLastError());
+}
 
 // The centroid-cell table of the faces at p.
 void Broadphase::cells(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt_,
@@ -1942,9 +2134,7 @@ void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, c
                                counts_of(table), near_.ptr, near_cap);
         } else {
             cells(s, g, x, p, tris, nt, th, true);
-            hipLaunchKernelGGL(k_vf_candidates<false>, dim3(visit_blocks(nv)), dim3(64 * VISIT_WAVES), 0, s, g, x, p, nv,
-                               vtoff.ptr, vtri.ptr, tcell.ptr, slots_of(table), place.ptr, (1u << table_bits) - 1,
-                               (const FaceRec*)rec.ptr, counts_of(table), near_.ptr, near_cap);
+            vf_candidates(s, g, x, p, nv, false, near_cap);
         }
         auto* narrow = store ? k_narrow<true> : k_narrow<false>;
         hipLaunchKernelGGL(narrow, dim3(1024), dim3(256), 0, s, near_.ptr, near_cap, tris,
@@ -1952,6 +2142,10 @@ void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, c
                            counts_of(table), cap, vquad.ptr, vf.ptr, rt.ptr, rn.ptr, rw.ptr);
         PBD_HIP(hipGetLastError());
         c = read_counts(s, 0, &meanwhile);
+        if (c.hubs && !vhubs.known) {
+            vhubs.find(s, vtoff.ptr, nv);
+            continue;
+        }
         if (swept) {
             PBD_CHECK(!c.face_span, PBD_ERR_LIMIT, "a face's swept box spans more than 4096 cells: use a larger cell");
             PBD_CHECK(c.entries < (1u << 31), PBD_ERR_LIMIT, "swept-box cell entries overflow int32");
@@ -2067,10 +2261,12 @@ long long Broadphase::list_pairs(hipStream_t s, const HashCfg& g, const float4* 
     for (;;) {
         const unsigned cap = near_cap();
         cells(s, g, p, p, tris, nt, 0.0f, false);
-        hipLaunchKernelGGL(k_vf_candidates<true>, dim3(visit_blocks(nv)), dim3(64 * VISIT_WAVES), 0, s, g, p, p, nv,
-                           vtoff.ptr, vtri.ptr, tcell.ptr, slots_of(table), place.ptr, (1u << table_bits) - 1,
-                           (const FaceRec*)rec.ptr, counts_of(table), near_.ptr, cap);
+        vf_candidates(s, g, p, p, nv, true, cap);
         const DetectTotals c = read_counts(s, 0, nullptr);
+        if (c.hubs && !vhubs.known) {
+            vhubs.find(s, vtoff.ptr, nv);
+            continue;
+        }
         check_pairs(c.near, "candidate pair count");
         npairs = (long long)c.near;
         if (c.near_most <= cap) break;
@@ -2108,10 +2304,16 @@ void Broadphase::ee_candidates(hipStream_t s, const HashCfg& g, const float4* x,
                        (const int4*)slots_of(table), 1 << table_bits, (int4*)place.ptr, &counts_of(table)->entries);
     hipLaunchKernelGGL(k_edge_fill, dim3(blocks(nedges)), dim3(256), 0, s, nedges, edges.ptr, etoff.ptr, etri.ptr,
                        tcell.ptr, x, p, place.ptr, ent);
-    auto* k = list ? k_ee_candidates<true> : k_ee_candidates<false>;
-    hipLaunchKernelGGL(k, dim3(visit_blocks(nedges)), dim3(64 * VISIT_WAVES), 0, s, g, nedges, edges.ptr, etoff.ptr,
-                       etri.ptr, voff.ptr, vnbr.ptr, x, p, tcell.ptr, slots_of(table), place.ptr, mask, ent, th,
-                       counts_of(table), near_.ptr, cap);
+    auto visit = [&](auto* k, int n) {
+        hipLaunchKernelGGL(k, dim3(visit_blocks(n)), dim3(64 * VISIT_WAVES), 0, s, g, n, edges.ptr, etoff.ptr,
+                           etri.ptr, voff.ptr, vnbr.ptr, x, p, tcell.ptr, slots_of(table), place.ptr, mask, ent, th,
+                           counts_of(table), near_.ptr, cap, ehubs.unit.ptr, ehubs.set.ptr);
+    };
+    visit(list ? k_ee_candidates<true, false> : k_ee_candidates<false, false>, nedges);
+    if (ehubs.units > 0) {
+        ehubs.enter(s, etoff.ptr, etri.ptr, tcell.ptr);
+        visit(list ? k_ee_candidates<true, true> : k_ee_candidates<false, true>, ehubs.units);
+    }
     PBD_HIP(hipGetLastError());
 }
 
@@ -2144,6 +2346,10 @@ void Broadphase::detect_ee(hipStream_t s, const HashCfg& g, const float4* x, con
                            counts_of(table), cap, eab.ptr, quad.ptr, rt.ptr, rn.ptr, rw.ptr);
         PBD_HIP(hipGetLastError());
         c = read_counts(s, 1, &meanwhile);
+        if (c.hubs && !ehubs.known) {
+            ehubs.find(s, etoff.ptr, nedges);
+            continue;
+        }
         check_pairs(c.pairs, "edge-edge candidate count");
         if (c.near_most <= near_cap && c.contacts <= cap) break;
         if (c.near_most > near_cap) grow_near((size_t)c.near_most + c.near_most / 4);

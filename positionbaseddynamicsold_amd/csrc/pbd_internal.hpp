@@ -246,12 +246,13 @@ struct DetectCounts {
     unsigned contacts;
     unsigned entries, large;          // table entries; faces kept out of the table
     unsigned face_span, vertex_span;  // 1: a box over the allowed cells of the caller's grid
-    unsigned pad[27];
+    unsigned hubs;                    // 1: vertices (edges) of very many triangles were left out
+    unsigned pad[26];
     DetectBucket bucket[NEAR_BUCKETS];  // a line each
 };
 struct DetectTotals {
     unsigned long long pairs, near;
-    unsigned near_most, contacts, entries, face_span, vertex_span;
+    unsigned near_most, contacts, entries, face_span, vertex_span, hubs;
 };
 
 // Broadphase + CCD working set (device buffers reused between calls).
@@ -272,6 +273,21 @@ struct Broadphase {
     DBuf<int> cnt, off, scan_tmp, idx;
     // vertex -> triangles of the current triangle list
     DBuf<int> vtoff, vtri;
+    // vertices (edges) of very many triangles: their units and cell sets (the
+    // kernels' hubs); units 0 and not known until a visit has reported one
+    struct Hubs {
+        bool known = false;
+        int units = 0;
+        DBuf<int2> unit;
+        DBuf<int> set;
+        void forget() {
+            known = false;
+            units = 0;
+        }
+        void find(hipStream_t s, const int* off, int n);
+        void enter(hipStream_t s, const int* off, const int* tri, const int4* tcell);
+    };
+    Hubs vhubs, ehubs;
     // unsorted table of the faces (edges) by cell: counters and slot counts, slot
     // places, entries by swept box (face and cell code), face or edge
     // records, per-face cells
@@ -347,6 +363,7 @@ private:
     void order_contacts(hipStream_t s, const DBuf<int2>& key, const int4* quad, long long n, int nfirst,
                         DBuf<int2>& okey, DBuf<int4>* oquad);
     void sort_near(hipStream_t s, int nfirst, int nsecond, DBuf<uint32_t>& hi, DBuf<uint32_t>& lo);
+    void vf_candidates(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, int nv, bool list, unsigned cap);
     void ee_candidates(hipStream_t s, const HashCfg& g, const float4* x, const float4* p, const int* tris, int nt, bool list,
                        float th, unsigned cap);
 };
