@@ -824,9 +824,8 @@ void upload_scene(pbd_ctx* c, const float* x, const float* p, const float* w, in
                   float th = 0.0f, const pbd_hash_desc* d = nullptr, bool keep = false) {
     PBD_CHECK(nv >= 0 && nt >= 0 && (x || !nv) && (p || !nv) && (tris || !nt), PBD_ERR_ARG, "bad scene arrays");
     for (long long i = 0; i < 3ll * nt; i++) PBD_CHECK(tris[i] >= 0 && tris[i] < nv, PBD_ERR_ARG, "triangle index out of range");
-    const uint64_t hash = scene_fingerprint(x, p, nv, tris, nt, th, d ? *d : pbd_hash_desc{});
-    if (!(keep && c->ccd_built && hash == c->scene_hash)) c->sbp.npairs = c->sbp.ncontacts = 0;
-    c->sbp.ee_npairs = c->sbp.ee_ncontacts = 0;
+    const long long npairs = c->sbp.npairs, ncontacts = c->sbp.ncontacts;
+    c->sbp.npairs = c->sbp.ncontacts = c->sbp.ee_npairs = c->sbp.ee_ncontacts = 0;
     c->sh_stale = true;
     std::vector<float4> X(nv), P(nv);
     for (int i = 0; i < nv; i++) {
@@ -841,6 +840,12 @@ void upload_scene(pbd_ctx* c, const float* x, const float* p, const float* w, in
     c->snv = nv;
     c->snt = nt;
     c->s_th = th;
+    // last: the GPU has the uploads to do meanwhile
+    const uint64_t hash = scene_fingerprint(x, p, nv, tris, nt, th, d ? *d : pbd_hash_desc{});
+    if (keep && c->ccd_built && hash == c->scene_hash) {
+        c->sbp.npairs = npairs;
+        c->sbp.ncontacts = ncontacts;
+    }
     c->scene_hash = hash;
 }
 
