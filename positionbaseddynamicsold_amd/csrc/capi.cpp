@@ -850,9 +850,10 @@ void upload_scene(pbd_ctx* c, const float* x, const float* p, const float* w, in
 }
 
 // The grid of the swept-box table: the caller's cells taken m at a time per
-// axis so that they are about as large as a face's widened box.  Faces are then
-// entered in a few cells each and vertices look in one or two, whatever the
-// caller's cell (the candidates do not depend on it).
+// axis so that those of the lowest level are about as large as a widened face
+// at rest.  Together with the levels, faces are entered in a few cells each
+// whatever the caller's cell, their motion and their differences in size (the
+// candidates do not depend on it).
 HashCfg swept_cfg(const HashCfg& g, float mean_edge, float th) {
     HashCfg w = g;
     const float target = mean_edge + 8.0f * th;

@@ -246,13 +246,14 @@ static void build_sorted(hipStream_t s, const HashCfg& g, const P* p, int nv, co
 // detection there against 0.15 ms for the table, the visit and the narrowphase.
 // ---------------------------------------------------------------------------
 constexpr int SWEPT_MAX_CELLS = 4096;  // cells of the caller's grid one box may span
-constexpr int ENTRY_MAX_CELLS = 64;    // cells of the table's own grid a face is entered in
+constexpr int ENTRY_MAX_CELLS = 64;    // cells of one level of the table's grid a face is entered in (any at the last)
 
 __device__ __forceinline__ float widen_lo(float v, float m) { return v - (m + 1e-6f * fabsf(v)); }
 __device__ __forceinline__ float widen_hi(float v, float m) { return v + (m + 1e-6f * fabsf(v)); }
 
-__device__ __forceinline__ int cell_coord(const HashCfg& g, float v, int k) {
-    float c = floorf((v - g.start[k]) / g.cell[k]);
+// The cell of v along axis k, of cells `scale` times as long.
+__device__ __forceinline__ int cell_coord(const HashCfg& g, float v, int k, float scale = 1.0f) {
+    float c = floorf((v - g.start[k]) / (g.cell[k] * scale));
     c = fminf(fmaxf(c, -536870912.0f), 536870912.0f);  // keeps hi - lo + 1 within int
     int i = (int)c;
     if (g.mode == 0) i = min(max(i, 0), g.size[k] - 1);  // clamping keeps overlapping ranges overlapping
@@ -472,7 +473,7 @@ __global__ __launch_bounds__(256) void k_cell_fill(int nt, const int4* __restric
 constexpr int PLACE_SLOTS = 4096;
 template <bool END>
 __global__ __launch_bounds__(256) void k_slot_places(const int4* __restrict__ cnt, int nslots, int4* __restrict__ place,
-                                                     unsigned* __restrict__ total) {
+                                                     unsigned long long* __restrict__ total) {
     constexpr int Q = PLACE_SLOTS / 1024;
     __shared__ int wave[4], base;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -492,7 +493,7 @@ __global__ __launch_bounds__(256) void k_slot_places(const int4* __restrict__ cn
     }
     if (lane == 0) wave[wv] = run;
     __syncthreads();
-    if (threadIdx.x == 0) base = (int)atomicAdd(total, (unsigned)(wave[0] + wave[1] + wave[2] + wave[3]));
+    if (threadIdx.x == 0) base = (int)atomicAdd(total, (unsigned long long)(wave[0] + wave[1] + wave[2] + wave[3]));
     __syncthreads();
     int at = base;
     for (int w = 0; w < wv; w++) at += wave[w];
@@ -508,67 +509,83 @@ __global__ __launch_bounds__(256) void k_slot_places(const int4* __restrict__ cn
 }
 
 // Swept boxes: face records (their margin defines the candidate set), the
-// cells of the table's own grid gi they cover counted per slot.  A face over
-// more than ENTRY_MAX_CELLS of them goes to the list of large faces, which
-// every vertex tests.  The narrowphase's half-spaces are made here, where the
-// corners are loaded anyway (571,000 faces: 185 us without them, 193 with).
+// cells of the table's own grid they cover counted per slot.  The grid has
+// SWEPT_LEVELS levels, each of cells SWEPT_FACTOR times as long as those of the
+// one below: a face goes to the lowest where it covers at most ENTRY_MAX_CELLS
+// cells, and vertices look in every level that holds faces.  So neither faces
+// of very different size nor a motion over many cells make entries or visits
+// many (a folded 512 x 512 cloth moving 8 edges along each axis: 27 ms a
+// detection, 571 ms when faces over 64 cells went to a list that every vertex
+// tested).  The narrowphase's half-spaces are made here, where the corners are
+// loaded anyway (571,000 faces: 185 us without them, 193 with).
+__device__ __forceinline__ unsigned level_slot(int x, int y, int z, int level, unsigned mask) {
+    return (cell_slot(x, y, z, 0xffffffffu) + (unsigned)level * 0x9E3779B1u) & mask;
+}
+
 __global__ __launch_bounds__(256) void k_swept_faces(HashCfg g, HashCfg gi, const float4* __restrict__ x,
                                                      const float4* __restrict__ p, const int* __restrict__ tris, int nt,
                                                      float th, unsigned mask, int* __restrict__ cnt,
                                                      int4* __restrict__ fcell, FaceRec* __restrict__ rec,
-                                                     FaceAxes* __restrict__ axes, int* __restrict__ large,
-                                                     DetectCounts* __restrict__ c) {
+                                                     FaceAxes* __restrict__ axes, DetectCounts* __restrict__ c) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= nt) return;
     const FaceRec r = face_record(f, x, p, tris, th, 4.0f * th);
     const float4 X[3] = {x[r.v0], x[r.v1], x[r.v2]}, P[3] = {p[r.v0], p[r.v1], p[r.v2]};
     axes[f] = face_axes(X, P, th);
-    int lo[3], hi[3];
-    long long span = 1, n = 1;
-    for (int k = 0; k < 3; k++) {
-        // per-axis bounds first: the product of three spans of up to 2^31 overflows
+    long long span = 1;
+    // per-axis bounds first: the product of three spans of up to 2^31 overflows
+    for (int k = 0; k < 3; k++)
         span *= (long long)min(cell_coord(g, r.hi[k], k) - cell_coord(g, r.lo[k], k) + 1, SWEPT_MAX_CELLS + 1);
-        lo[k] = cell_coord(gi, r.lo[k], k);
-        hi[k] = cell_coord(gi, r.hi[k], k);
-        n *= (long long)min(hi[k] - lo[k] + 1, ENTRY_MAX_CELLS + 1);
-    }
     rec[f] = r;
-    if (span > SWEPT_MAX_CELLS) c->face_span = 1;
-    fcell[2 * f] = make_int4(lo[0], lo[1], lo[2], n > ENTRY_MAX_CELLS ? 1 : 0);
-    fcell[2 * f + 1] = make_int4(hi[0], hi[1], hi[2], 0);
-    if (n > ENTRY_MAX_CELLS) {
-        large[atomicAdd(&c->large, 1u)] = f;
-        return;
+    const bool over = span > SWEPT_MAX_CELLS;  // the detection is refused
+    if (over) c->face_span = 1;
+    int lo[3], hi[3], level = 0;
+    for (float scale = 1.0f;; level++, scale *= (float)SWEPT_FACTOR) {
+        long long n = 1;
+        for (int k = 0; k < 3; k++) {
+            lo[k] = cell_coord(gi, r.lo[k], k, scale);
+            hi[k] = over ? lo[k] : cell_coord(gi, r.hi[k], k, scale);
+            n *= (long long)min(hi[k] - lo[k] + 1, SWEPT_MAX_CELLS + 1);
+        }
+        if (n <= ENTRY_MAX_CELLS || level == SWEPT_LEVELS - 1) break;
     }
+    fcell[2 * f] = make_int4(lo[0], lo[1], lo[2], level);
+    fcell[2 * f + 1] = make_int4(hi[0], hi[1], hi[2], 0);
+    // read first, past the CU's cache: one store for most of the launch
+    if (!__hip_atomic_load(&c->level[level], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) c->level[level] = 1;
     for (int z = lo[2]; z <= hi[2]; z++)
         for (int y = lo[1]; y <= hi[1]; y++)
-            for (int xx = lo[0]; xx <= hi[0]; xx++) atomicAdd(&cnt[cell_slot(xx, y, z, mask)], 1);
+            for (int xx = lo[0]; xx <= hi[0]; xx++) atomicAdd(&cnt[level_slot(xx, y, z, level, mask)], 1);
 }
 
-// The cell of an entry, 9 bits per axis (a face covers at most ENTRY_MAX_CELLS
-// cells, so it cannot cover two that agree in them), and per axis whether it is
-// the face's lowest cell.
+// The cell of an entry, 9 bits per axis (a face covers fewer than CODE_SPAN
+// cells along each, so it cannot cover two that agree in them), per axis whether
+// it is the face's lowest cell, and the level.
+constexpr int CODE_SPAN = 512;
 __device__ __forceinline__ int cell_code(int x, int y, int z) { return (x & 511) | ((y & 511) << 9) | ((z & 511) << 18); }
 
 // place: each slot's start, moved up by every entry stored; it ends at the
 // slot's end.  FACE_LANES lanes share a face's cells, since every entry waits
 // for its atomic (128 x 128 drape, 118,000 to 198,000 entries: 17.4 us with a
 // thread per face, 14.4 so; counting waits for none and gains nothing by it).
+// Places past 2^31 compare as unsigned: such a detection is refused, and until
+// then nothing may be stored out of range.
 constexpr int FACE_LANES = 8;
 __global__ __launch_bounds__(256) void k_swept_fill(int nt, const int4* __restrict__ fcell, unsigned mask,
-                                                    int* __restrict__ place, int2* __restrict__ ent, int cap) {
+                                                    int* __restrict__ place, int2* __restrict__ ent, unsigned cap) {
     const int f = (blockIdx.x * blockDim.x + threadIdx.x) / FACE_LANES, lane = threadIdx.x % FACE_LANES;
     if (f >= nt) return;
     const int4 lo = fcell[2 * f], hi = fcell[2 * f + 1];
-    if (lo.w) return;
     const int wx = hi.x - lo.x + 1, wy = hi.y - lo.y + 1, n = wx * wy * (hi.z - lo.z + 1);
     for (int i = lane; i < n; i += FACE_LANES) {
         const int z = i / (wx * wy), j = i - z * (wx * wy), y = j / wx, xx = j - y * wx;
-        const int at = atomicAdd(&place[cell_slot(lo.x + xx, lo.y + y, lo.z + z, mask)], 1);
-        const int first = (xx == 0 ? 1 << 27 : 0) | (y == 0 ? 1 << 28 : 0) | (z == 0 ? 1 << 29 : 0);
-        if (at < cap) ent[at] = make_int2(f, cell_code(lo.x + xx, lo.y + y, lo.z + z) | first);
+        const unsigned at = (unsigned)atomicAdd(&place[level_slot(lo.x + xx, lo.y + y, lo.z + z, lo.w, mask)], 1);
+        const unsigned first = (xx == 0 ? 1u << 27 : 0) | (y == 0 ? 1u << 28 : 0) | (z == 0 ? 1u << 29 : 0);
+        if (at < cap)
+            ent[at] = make_int2(f, (int)((unsigned)cell_code(lo.x + xx, lo.y + y, lo.z + z) | first | (unsigned)lo.w << 30));
     }
 }
+static_assert(SWEPT_LEVELS <= 4, "two bits of an entry hold the level");
 
 // Pairs a wave has found, appended in runs to the global list.  Atomics on one
 // address are served one after the other, about 13 ns each here, so one length
@@ -960,69 +977,75 @@ __global__ __launch_bounds__(64 * VISIT_WAVES, 8) void k_vf_candidates(
 }
 
 // Vertex-face candidates by swept boxes: the faces entered in the cells of the
-// vertex's box, taken at the lowest cell that the two boxes' cell ranges share,
-// and the large faces.
+// vertex's box, level by level, taken at the lowest cell that the two boxes'
+// cell ranges share.
 __global__ __launch_bounds__(64 * VISIT_WAVES) void k_swept_candidates(
     HashCfg g, HashCfg gi, const float4* __restrict__ x, const float4* __restrict__ p, int nv,
     const int* __restrict__ vtoff, const int* __restrict__ cnt, const int* __restrict__ end, unsigned mask,
-    const int2* __restrict__ ent, int ent_cap, const FaceRec* __restrict__ rec, const int* __restrict__ large,
+    const int2* __restrict__ ent, unsigned ent_cap, const FaceRec* __restrict__ rec, const int4* __restrict__ fcell,
     DetectCounts* __restrict__ c, int2* __restrict__ out, unsigned cap) {
     __shared__ int2 buf[VISIT_WAVES][VISIT_BUF];
     __shared__ GroupLds group[VISIT_WAVES][2];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 31;
     PairSink sink{buf[wv], 0, (int)((blockIdx.x * VISIT_WAVES + wv) % NEAR_BUCKETS), c, out, cap};
-    const int nlarge = (int)c->large;
     int pairs = 0;
     const int stride = (int)gridDim.x * VISIT_WAVES * 2;
     for (int v0 = ((int)blockIdx.x * VISIT_WAVES + wv) * 2; v0 < nv; v0 += stride) {
         const int v = v0 + (lane >> 5), at = min(v, nv - 1);
         const bool used = v < nv && vtoff[at + 1] > vtoff[at];
         const SweptBox b = vertex_box(x[at], p[at]);
-        int lo[3], w[3];
         long long span = 1;
-        for (int k = 0; k < 3; k++) {
+        for (int k = 0; k < 3; k++)
             span *= (long long)min(cell_coord(g, b.hi[k], k) - cell_coord(g, b.lo[k], k) + 1, SWEPT_MAX_CELLS + 1);
-            lo[k] = cell_coord(gi, b.lo[k], k);
-            w[k] = min(cell_coord(gi, b.hi[k], k) - lo[k] + 1, SWEPT_MAX_CELLS + 1);
-        }
         const bool over = span > SWEPT_MAX_CELLS;
         if (used && over) c->vertex_span = 1;
-        const int cells = used && !over ? w[0] * w[1] * w[2] : 0;
-        auto cell_of = [&](int i) { return make_int3(lo[0] + i % w[0], lo[1] + i / w[0] % w[1], lo[2] + i / (w[0] * w[1])); };
-        auto test = [&](bool in, int f) {
-            bool hit = false;
-            if (in) {
-                const FaceRec r = rec[f];
-                hit = !box_misses(b, r) && v != r.v0 && v != r.v1 && v != r.v2;
-                pairs += hit;
+        float scale = 1.0f;
+        for (int level = 0; level < SWEPT_LEVELS; level++, scale *= (float)SWEPT_FACTOR) {
+            if (!c->level[level]) continue;  // the same for all
+            int lo[3], w[3];
+            for (int k = 0; k < 3; k++) {
+                lo[k] = cell_coord(gi, b.lo[k], k, scale);
+                w[k] = min(cell_coord(gi, b.hi[k], k, scale) - lo[k] + 1, SWEPT_MAX_CELLS + 1);
             }
-            sink.add(hit, v, f);
-        };
-        const int most = max(cells, __shfl_xor(cells, 32));
-        for (int c0 = 0; c0 < most; c0 += 64) {
-            int3 q[2];
-            int start[2], n[2];
-            for (int c = 0; c < 2; c++) {
-                const bool mine = c0 + 32 * c + l < cells;
-                q[c] = cell_of(c0 + 32 * c + l);
-                const unsigned slot = mine ? cell_slot(q[c].x, q[c].y, q[c].z, mask) : 0u;
-                const int m = cnt[slot], e1 = end[slot];
-                n[c] = mine && e1 <= ent_cap ? m : 0;  // beyond: the table did not fit, the caller starts over
-                start[c] = e1 - m;
-            }
-            visit_runs(group[wv][lane >> 5], q, start, n, [&](int e, int3 fq) {
-                bool in = false;
-                int f = 0;
-                if (e >= 0) {
-                    const int2 en = ent[e];
-                    f = en.x;
-                    in = (en.y & 0x7ffffff) == cell_code(fq.x, fq.y, fq.z) && ((en.y >> 27 & 1) || fq.x == lo[0]) &&
-                         ((en.y >> 28 & 1) || fq.y == lo[1]) && ((en.y >> 29 & 1) || fq.z == lo[2]);
+            const int cells = used && !over ? w[0] * w[1] * w[2] : 0;
+            // cells of the box may agree in their codes
+            const bool wide = w[0] >= CODE_SPAN || w[1] >= CODE_SPAN || w[2] >= CODE_SPAN;
+            auto cell_of = [&](int i) { return make_int3(lo[0] + i % w[0], lo[1] + i / w[0] % w[1], lo[2] + i / (w[0] * w[1])); };
+            const int most = max(cells, __shfl_xor(cells, 32));
+            for (int c0 = 0; c0 < most; c0 += 64) {
+                int3 q[2];
+                int start[2], n[2];
+                for (int c = 0; c < 2; c++) {
+                    const bool mine = c0 + 32 * c + l < cells;
+                    q[c] = cell_of(c0 + 32 * c + l);
+                    const unsigned slot = mine ? level_slot(q[c].x, q[c].y, q[c].z, level, mask) : 0u;
+                    const int m = cnt[slot], e1 = end[slot];
+                    n[c] = mine && (unsigned)e1 <= ent_cap ? m : 0;  // beyond: the table did not fit, the caller starts over
+                    start[c] = e1 - m;
                 }
-                test(in, f);
-            });
+                visit_runs(group[wv][lane >> 5], q, start, n, [&](int e, int3 fq) {
+                    bool hit = false;
+                    int f = 0;
+                    if (e >= 0) {
+                        const int2 en = ent[e];
+                        f = en.x;
+                        bool in = (en.y & 0x7ffffff) == cell_code(fq.x, fq.y, fq.z) &&
+                                  (int)((unsigned)en.y >> 30) == level && ((en.y >> 27 & 1) || fq.x == lo[0]) &&
+                                  ((en.y >> 28 & 1) || fq.y == lo[1]) && ((en.y >> 29 & 1) || fq.z == lo[2]);
+                        if (wide && in) {
+                            const int4 a = fcell[2 * f], z = fcell[2 * f + 1];
+                            in = fq.x >= a.x && fq.x <= z.x && fq.y >= a.y && fq.y <= z.y && fq.z >= a.z && fq.z <= z.z;
+                        }
+                        if (in) {
+                            const FaceRec r = rec[f];
+                            hit = !box_misses(b, r) && v != r.v0 && v != r.v1 && v != r.v2;
+                            pairs += hit;
+                        }
+                    }
+                    sink.add(hit, v, f);
+                });
+            }
         }
-        for (int i = 0; i < nlarge; i += 32) test(used && !over && i + l < nlarge, large[min(i + l, nlarge - 1)]);
     }
     if (sink.n) sink.flush();
     sink.count(pairs);
@@ -2020,7 +2043,7 @@ DetectTotals Broadphase::read_counts(hipStream_t s, int slot, std::function<void
     }
     PBD_HIP(hipEventSynchronize(counts_ready[slot]));
     const DetectCounts& c = *static_cast<const DetectCounts*>(counts_h[slot]);
-    DetectTotals t{0, 0, 0, c.contacts, c.entries, c.face_span, c.vertex_span, c.hubs};
+    DetectTotals t{0, 0, c.entries, 0, c.contacts, c.face_span, c.vertex_span, c.hubs};
     for (int b = 0; b < NEAR_BUCKETS; b++) {
         near_n[b] = c.bucket[b].near;
         t.pairs += c.bucket[b].pairs;
@@ -2130,7 +2153,7 @@ void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, c
             swept_table(s, g, *swept, x, p, tris, th);
             hipLaunchKernelGGL(k_swept_candidates, dim3(visit_blocks(nv)), dim3(64 * VISIT_WAVES), 0, s, g, *swept, x, p,
                                nv, vtoff.ptr, slots_of(table), place.ptr, (1u << table_bits) - 1, ent.ptr,
-                               (int)std::min<size_t>(ent.n, 0x7fffffff), (const FaceRec*)rec.ptr, large.ptr,
+                               (unsigned)std::min<size_t>(ent.n, 0x7fffffff), (const FaceRec*)rec.ptr, sw_cell.ptr,
                                counts_of(table), near_.ptr, near_cap);
         } else {
             cells(s, g, x, p, tris, nt, th, true);
@@ -2148,7 +2171,7 @@ void Broadphase::detect(hipStream_t s, const HashCfg& g, const HashCfg* swept, c
         }
         if (swept) {
             PBD_CHECK(!c.face_span, PBD_ERR_LIMIT, "a face's swept box spans more than 4096 cells: use a larger cell");
-            PBD_CHECK(c.entries < (1u << 31), PBD_ERR_LIMIT, "swept-box cell entries overflow int32");
+            PBD_CHECK(c.entries < (1ull << 31), PBD_ERR_LIMIT, "swept-box cell entries overflow int32");
         }
         const bool table_short = swept && c.entries > ent.n;
         if (!table_short) {
@@ -2177,17 +2200,15 @@ void Broadphase::swept_table(hipStream_t s, const HashCfg& g, const HashCfg& gi,
     grow(rec, (size_t)nt * sizeof(FaceRec));
     grow(axes, (size_t)nt * sizeof(FaceAxes));
     grow(sw_cell, 2 * (size_t)nt);
-    grow(large, nt);
     grow(ent, 12 * (size_t)nt);
     clear_table(s, table_bits_for(2ll * nt));
     const unsigned mask = (1u << table_bits) - 1;
     hipLaunchKernelGGL(k_swept_faces, dim3(blocks(nt)), dim3(256), 0, s, g, gi, x, p, tris, nt, th, mask,
-                       slots_of(table), sw_cell.ptr, (FaceRec*)rec.ptr, (FaceAxes*)axes.ptr, large.ptr,
-                       counts_of(table));
+                       slots_of(table), sw_cell.ptr, (FaceRec*)rec.ptr, (FaceAxes*)axes.ptr, counts_of(table));
     hipLaunchKernelGGL(k_slot_places<false>, dim3(((1 << table_bits) + PLACE_SLOTS - 1) / PLACE_SLOTS), dim3(256), 0, s,
                        (const int4*)slots_of(table), 1 << table_bits, (int4*)place.ptr, &counts_of(table)->entries);
     hipLaunchKernelGGL(k_swept_fill, dim3(blocks((long long)FACE_LANES * nt)), dim3(256), 0, s, nt, sw_cell.ptr, mask, place.ptr,
-                       ent.ptr, (int)std::min<size_t>(ent.n, 0x7fffffff));
+                       ent.ptr, (unsigned)std::min<size_t>(ent.n, 0x7fffffff));
     PBD_HIP(hipGetLastError());
 }
 

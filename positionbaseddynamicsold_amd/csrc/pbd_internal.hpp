@@ -235,6 +235,9 @@ struct HashCfg {
     int ncells;          // dense: size product; hashed: 1 << table_bits
 };
 
+// Levels of the swept-box table's own grid, each of cells SWEPT_FACTOR times as long.
+constexpr int SWEPT_LEVELS = 4, SWEPT_FACTOR = 4;
+
 // Counters of a detection, cleared with the table's slot counts.
 constexpr int NEAR_BUCKETS = 64;
 struct DetectBucket {
@@ -243,16 +246,17 @@ struct DetectBucket {
     unsigned pad[29];
 };
 struct DetectCounts {
+    unsigned long long entries;       // of the table
     unsigned contacts;
-    unsigned entries, large;          // table entries; faces kept out of the table
+    unsigned level[SWEPT_LEVELS];     // 1: the level holds faces
     unsigned face_span, vertex_span;  // 1: a box over the allowed cells of the caller's grid
     unsigned hubs;                    // 1: vertices (edges) of very many triangles were left out
-    unsigned pad[26];
+    unsigned pad[22];
     DetectBucket bucket[NEAR_BUCKETS];  // a line each
 };
 struct DetectTotals {
-    unsigned long long pairs, near;
-    unsigned near_most, contacts, entries, face_span, vertex_span, hubs;
+    unsigned long long pairs, near, entries;
+    unsigned near_most, contacts, face_span, vertex_span, hubs;
 };
 
 // Broadphase + CCD working set (device buffers reused between calls).
@@ -291,7 +295,7 @@ struct Broadphase {
     // unsorted table of the faces (edges) by cell: counters and slot counts, slot
     // places, entries by swept box (face and cell code), face or edge
     // records, per-face cells
-    DBuf<int> table, place, raw_rank, large;
+    DBuf<int> table, place, raw_rank;
     int table_bits = 0;
     DBuf<int2> ent;
     DBuf<unsigned char> rec, axes;
