@@ -294,7 +294,7 @@ int effective_tile_sweeps(const pbd_ctx* c) {
 }
 
 int effective_max_load(const pbd_ctx* c) {
-    int lim = (c->lds_max - TILE_STATIC_LDS) / 16;
+    int lim = (c->lds_max - TILE_TAIL_LDS) / 16;
     if (c->sp.tile_max_verts > 0) lim = std::min(lim, c->sp.tile_max_verts);
     return std::max(64, lim);
 }
@@ -449,7 +449,7 @@ void replan_if_needed(pbd_ctx* c) {
     // the GPU: a launch takes as long as its largest tile, so the smallest
     // tile size of at most one tile per CU is the fastest (a 389 x 211 cloth at
     // 4 sweeps per launch: 113 us per substep with 213 tiles of up to 2048
-    // vertices, 265 us with 18 of up to 10,208).
+    // vertices, 265 us with 18 of up to 10,224).
     // (Grids only: a mesh's tiles are id ranges, whose cones do not shrink with them.)
     long long multi = 0;
     bool grids = true;
@@ -1896,9 +1896,7 @@ int pbd_create(int device, pbd_ctx** out) {
             int lds = 0;
             PBD_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
             PBD_HIP(hipDeviceGetAttribute(&c->num_cu, hipDeviceAttributeMultiprocessorCount, device));
-            // the vertices' lds_max - TILE_STATIC_LDS and the tail are what a tile kernel's dynamic LDS may reach
-            const size_t dyn = tiles_lds_optin((size_t)std::max(lds, 65536) - (TILE_STATIC_LDS - TILE_TAIL_LDS));
-            c->lds_max = (int)dyn + (TILE_STATIC_LDS - TILE_TAIL_LDS);
+            c->lds_max = (int)tiles_lds_optin((size_t)std::max(lds, 65536));
         } catch (...) {
             delete c;
             throw;
@@ -3188,7 +3186,7 @@ int pbd_autotune(pbd_ctx* ctx, int trial_substeps, pbd_solver_params* best, int*
         const pbd_solver_params base = ctx->sp;
         const HashCfg hbase = ctx->ccfg;
         // tile sizes: the whole LDS, half of it (two workgroups per CU), and two fixed caps
-        const int half = (ctx->lds_max / 2 - TILE_STATIC_LDS) / 16;
+        const int half = (ctx->lds_max / 2 - TILE_TAIL_LDS) / 16;
         std::vector<int> threads = {256, 512, 1024}, sweeps, maxv = {0, 4096, 2048}, bits = {-1};
         if (half > 4096 && half < effective_max_load(ctx)) maxv.insert(maxv.begin() + 1, half);
         if (ctx->coll.enabled) {

@@ -640,13 +640,11 @@ int tiles_per_cu(bool with_bend, int threads, size_t lds_bytes);
 // returns what they may use (bytes, or 64 KiB if the runtime refuses).
 size_t tiles_lds_optin(size_t bytes);
 // A tile launch's dynamic LDS: the tile's vertices, then a tail of
-// TILE_TAIL_LDS bytes (16 doubles of block reductions, an idle vertex pair, a
-// word), so that vertex 0 sits at LDS address 0.  TILE_STATIC_LDS bytes of the
-// CU's LDS are kept from the vertices: the tail, and the few static words of
-// the deciding kernels.
+// TILE_TAIL_LDS bytes, so that vertex 0 sits at LDS address 0 (the kernels have
+// no static LDS).  The tail in float4 slots: 16 doubles of block reductions, an
+// idle vertex pair, the walks' words, the keep decision's sums and words.
 constexpr int TILE_TAIL_LDS = 256;
-constexpr int TILE_STATIC_LDS = 512;
-constexpr int TILE_IDLE_SLOT = 8, TILE_WORD_SLOT = 10;  // in float4 slots after the vertices
+constexpr int TILE_IDLE_SLOT = 8, TILE_WORD_SLOT = 10, TILE_DECIDE_SLOT = 11;
 // The launch form that keeps a tile's distance records in registers
 // (k_tiles_regs<R>): colours and records per thread and colour it holds.
 constexpr int REG_COLORS = 8;

@@ -684,9 +684,9 @@ __device__ __forceinline__ void record_decision(const TileQueue& q, const ClothD
 // thread of the workgroup calls this; all get the same answer.
 __device__ __forceinline__ bool cloth_decide(const TileQueue& q, const TileDev& td, const ClothDev& cd, int ncl,
                                              int* sweeps_out, double m0, double m1, unsigned long long sq0,
-                                             unsigned long long sq1) {
-    __shared__ unsigned long long acc[4];
-    __shared__ int s_flag, s_base;
+                                             unsigned long long sq1, float4* tail) {
+    unsigned long long* acc = (unsigned long long*)(tail + TILE_DECIDE_SLOT);
+    int &s_flag = ((int*)(tail + TILE_DECIDE_SLOT + 2))[0], &s_base = ((int*)(tail + TILE_DECIDE_SLOT + 2))[1];
     const int c = td.cloth;
     if (threadIdx.x == 0) acc[0] = acc[1] = acc[2] = acc[3] = 0ull;
     for (int off = 32; off > 0; off >>= 1) {
@@ -886,7 +886,7 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
         __syncthreads();
         own_resid_parts<PREFETCH>(P, own + td.own_off, own_rest + td.own_off, td.n_own, &m1, &sq1);
         // (its barriers come after every read of P above)
-        const bool k = cloth_decide(q, td, cd, ncl, sweeps_out, m0, m1, sq0, sq1);
+        const bool k = cloth_decide(q, td, cd, ncl, sweeps_out, m0, m1, sq0, sq1, P + a.lds_slots);
         budget_c = k ? q.warm_sweeps : q.full_sweeps;
         nsweeps = k ? nk : nd;
         if (!k) {
@@ -1324,7 +1324,8 @@ __global__ __launch_bounds__(1024) void k_tiles_queue_bend(TILE_PARAMS, TileQueu
 template <bool BEND>
 __device__ __forceinline__ void tiles_decide_walk(TILE_PARAMS, const TileQueue& q, float4* P) {
     double* red = (double*)(P + a.lds_slots);
-    __shared__ int s_slot, s_chunk;
+    int* words = (int*)(P + a.lds_slots + TILE_WORD_SLOT);
+    int &s_slot = words[0], &s_chunk = words[1];
     if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(q.launches, 1);
     for (;;) {
         if (threadIdx.x < 64) {
@@ -1561,7 +1562,7 @@ __global__ __launch_bounds__(1024) void k_queue_schedule_decide(
 // Dynamic LDS the tile kernel may use on the current device: opts in to
 // `bytes` and returns it, or returns the 64 KiB every launch may use without
 // an opt-in when the runtime refuses it.  Every context on a device asks for
-// the same amount (the device's per-workgroup maximum less the kernel's
+// the same amount (the device's per-workgroup maximum: the kernels have no
 // static LDS), so contexts never lower each other's limit.
 size_t tiles_lds_optin(size_t bytes) {
     if (bytes <= 65536) return bytes;
