@@ -15,6 +15,9 @@ using namespace pbd;
 
 static thread_local std::string g_err;
 
+// Most sweeps per launch that the library chooses by itself.
+constexpr int CHOSEN_SWEEPS = 4;
+
 struct pbd_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -54,6 +57,7 @@ struct pbd_ctx {
     bool plan_small = false;  // planned with tiles smaller than the budget on offer
     int plan_whole = 0;       // most vertices of a grid planned as one tile
     int plan_steps = 0;       // and of a cloth planned for all its sweeps in one launch
+    int refused_load[CHOSEN_SWEEPS + 1] = {};  // largest tile budget that chosen sweeps per launch had no plan for
     DBuf<TileDev> tiles;
     // launch orders: single-tile cloths' tiles, multi-tile cloths' tiles, and
     // both (the first launch of a substep runs them side by side)
@@ -272,6 +276,17 @@ bool bending_grids(const pbd_ctx* c) {
     return bends;
 }
 
+// Sweeps per launch that nobody asked for are the library's choice.
+bool chooses_sweeps(const pbd_ctx* c) {
+    return !c->coll.enabled && c->sp.tile_sweeps <= 0 && c->sp.check_every <= 1 && free_sweeps(c) && distance_grids(c);
+}
+
+int effective_max_load(const pbd_ctx* c) {
+    int lim = (c->lds_max - TILE_TAIL_LDS) / 16;
+    if (c->sp.tile_max_verts > 0) lim = std::min(lim, c->sp.tile_max_verts);
+    return std::max(64, lim);
+}
+
 int effective_tile_sweeps(const pbd_ctx* c) {
     if (c->coll.enabled) return 1;  // contacts are resolved after every sweep
     // Fixed sweeps: the result does not depend on the split, and with bending
@@ -288,15 +303,10 @@ int effective_tile_sweeps(const pbd_ctx* c) {
     // sweeps per launch, a 256 x 256 cloth with bending 721 us at 1 and 923 at 2.
     // Meshes are tiled by vertex id, whose cones may grow faster than a grid's:
     // they keep one.
-    if (c->sp.check_every <= 1 && free_sweeps(c) && distance_grids(c))
-        return std::min(4, std::max(1, c->sp.iterations));
-    return std::max(1, c->sp.check_every);
-}
-
-int effective_max_load(const pbd_ctx* c) {
-    int lim = (c->lds_max - TILE_TAIL_LDS) / 16;
-    if (c->sp.tile_max_verts > 0) lim = std::min(lim, c->sp.tile_max_verts);
-    return std::max(64, lim);
+    if (!chooses_sweeps(c)) return std::max(1, c->sp.check_every);
+    int s = std::min(CHOSEN_SWEEPS, std::max(1, c->sp.iterations));
+    while (s > 1 && effective_max_load(c) <= c->refused_load[s]) s--;
+    return s;
 }
 
 void upload_plan(pbd_ctx* c) {
@@ -442,8 +452,8 @@ int whole_grid_load(const pbd_ctx* c, int sweeps, int ml) {
     return split > 0 && split <= c->num_cu / 8 ? load : ml;
 }
 
-void replan_if_needed(pbd_ctx* c) {
-    int s = effective_tile_sweeps(c), ml = effective_max_load(c), sp = c->sp.split_whole ? 1 : 0;
+void replan_at(pbd_ctx* c, int s) {
+    int ml = effective_max_load(c), sp = c->sp.split_whole ? 1 : 0;
     WholeLoad whole{whole_grid_load(c, s, ml), ml, INT_MAX};
     // Tiles smaller than the budget where the multi-tile cloths would not fill
     // the GPU: a launch takes as long as its largest tile, so the smallest
@@ -499,6 +509,19 @@ void replan_if_needed(pbd_ctx* c) {
     c->plan_steps = whole.steps;
     upload_plan(c);
     fill_cloth_dev(c);
+}
+
+void replan_if_needed(pbd_ctx* c) {
+    for (;;) {
+        const int s = effective_tile_sweeps(c);
+        try {
+            return replan_at(c, s);
+        } catch (const Error& e) {
+            // a budget too small for the chosen sweeps' cones may do for fewer
+            if (e.code != PBD_ERR_LIMIT || !chooses_sweeps(c) || s <= 1) throw;
+            c->refused_load[s] = effective_max_load(c);
+        }
+    }
 }
 
 void ensure_slots(pbd_ctx* c, int nchunks) {
@@ -718,6 +741,7 @@ void do_init(pbd_ctx* c, int color_rounds) {
     fill_ktabs(c);
     c->plan_sweeps = 0;
     c->plan_max_load = 0;
+    for (int& l : c->refused_load) l = 0;
     // grids always have a plan: theirs waits for the solver parameters; a
     // mesh that has none is refused here
     bool mesh = false;

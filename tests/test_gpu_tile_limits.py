@@ -1,4 +1,5 @@
-"""The largest tile: 160 KiB of LDS less 256 bytes hold 10,224 vertices."""
+"""Limits of the tile plan.  The largest tile: 160 KiB of LDS less 256 bytes hold
+10,224 vertices."""
 import numpy as np
 import pytest
 
@@ -36,3 +37,29 @@ def test_one_vertex_more_is_not(orc):
     info, x = stepped(pos, tris, capi.PATH_AUTO, False)
     assert info.whole == 0 and 1 < info.ntiles and info.max_loaded <= LARGEST
     assert np.array_equal(x, stepped(pos, tris, capi.PATH_GLOBAL, False)[1])
+
+
+# budgets too small for the cones of the four sweeps that a launch runs by default
+@pytest.mark.parametrize("budget", [64, 100, 256, 512, 1024])
+@pytest.mark.parametrize("before_init", [False, True])
+def test_small_budgets_take_fewer_sweeps_per_launch(budget, before_init):
+    x = []
+    for path in (capi.PATH_AUTO, capi.PATH_GLOBAL):
+        with capi.Context() as ctx:
+            c = ctx.add_grid(46, 34, 1.0, 0.7, jitter=1e-4, seed=0)
+            ctx.set_constraint_option(c, capi.DISTANCE, (1.0, 1.0, 1.0))
+            ctx.set_pins(c, [0, 45])
+            if before_init:
+                ctx.set_solver(iterations=5, path=path, tile_max_verts=budget)
+                ctx.init()
+            else:
+                ctx.init()
+                ctx.set_solver(iterations=5, path=path, tile_max_verts=budget)
+            ctx.step(3)
+            assert path == capi.PATH_GLOBAL or ctx.info(c).max_loaded <= budget
+            x.append(ctx.get(c))
+            # a larger budget takes four again
+            ctx.set_solver(iterations=5, path=path)
+            ctx.step(3)
+            x.append(ctx.get(c))
+    assert np.array_equal(x[0], x[2]) and np.array_equal(x[1], x[3])
