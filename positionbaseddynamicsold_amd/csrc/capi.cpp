@@ -24,6 +24,7 @@ struct pbd_ctx {
     std::vector<Cloth> cloths;
     bool inited = false;
     pbd_solver_params sp{};
+    bool sp_set = false;  // by the caller
     int lds_max = 65536;
     // state
     DBuf<float4> x, v, pbuf[2];
@@ -742,11 +743,12 @@ void do_init(pbd_ctx* c, int color_rounds) {
     c->plan_sweeps = 0;
     c->plan_max_load = 0;
     for (int& l : c->refused_load) l = 0;
-    // grids always have a plan: theirs waits for the solver parameters; a
-    // mesh that has none is refused here
-    bool mesh = false;
-    for (auto& k : c->cloths) mesh |= k.np() > 0 && (k.rx == 0 || k.has_user_pairs);
-    if (mesh) replan_if_needed(c);
+    // cloths that have no plan are refused here; grids always have one at the
+    // default parameters, which mostly change before the first substep: theirs
+    // waits where no others were set
+    bool now = c->sp_set;
+    for (auto& k : c->cloths) now |= k.np() > 0 && (k.rx == 0 || k.has_user_pairs);
+    if (now) replan_if_needed(c);
     else fill_cloth_dev(c);
     PBD_HIP(hipStreamSynchronize(s));
     c->inited = true;
@@ -2172,6 +2174,7 @@ int pbd_set_solver_params(pbd_ctx* ctx, const pbd_solver_params* p) {
         PBD_CHECK(p->warm_rule == 0 || p->warm_rule == 1, PBD_ERR_ARG, "warm_rule must be 0 (max) or 1 (RMS)");
         PBD_CHECK(p->warm_gate >= 0.0f, PBD_ERR_ARG, "warm_gate must be >= 0");
         ctx->sp = *p;
+        ctx->sp_set = true;
         if (ctx->inited) {
             set_device(ctx);
             fill_ktabs(ctx);

@@ -63,3 +63,19 @@ def test_small_budgets_take_fewer_sweeps_per_launch(budget, before_init):
             ctx.step(3)
             x.append(ctx.get(c))
     assert np.array_equal(x[0], x[2]) and np.array_equal(x[1], x[3])
+
+
+@pytest.mark.parametrize("mesh", [False, True])
+def test_init_refuses_a_budget_that_no_plan_fits(orc, mesh):
+    pos, tris = orc.grid_mesh(20, 20, 1.0, 1.0, jitter=1e-4, seed=0)
+    with capi.Context() as ctx:
+        c = ctx.add_mesh(pos, tris) if mesh else ctx.add_grid(20, 20, jitter=1e-4)
+        ctx.set_constraint_option(c, capi.DISTANCE, (1.0, 1.0, 1.0))
+        ctx.set_solver(iterations=4, tile_sweeps=4, tile_max_verts=64)
+        with pytest.raises(capi.PbdError, match="tile budget") as e:
+            ctx.init()
+        assert e.value.code == capi.PBD_ERR_LIMIT
+        ctx.set_solver(iterations=4, tile_max_verts=1024)
+        ctx.init()
+        ctx.step(1)
+        assert np.isfinite(ctx.get(c)).all()
