@@ -11,6 +11,7 @@
 #include <thread>
 #include <unordered_map>
 
+#include "parallel.hpp"
 #include "pbd_internal.hpp"
 #include "pbd_math.hpp"
 
@@ -483,19 +484,6 @@ int plan_one(const ClothTopo& t, const std::vector<int>& interior, int phases, i
 struct Block { int x0, x1, y0, y1; };
 
 }  // namespace
-
-// Runs f(i) for i in [0, n) on `threads` threads (each index once).
-template <class F>
-static void parallel_for(size_t n, unsigned threads, F&& f) {
-    std::atomic_size_t next{0};
-    auto work = [&]() {
-        for (size_t i; (i = next.fetch_add(1)) < n;) f(i);
-    };
-    std::vector<std::thread> pool;
-    for (unsigned t = 1; t < threads && t < n; t++) pool.emplace_back(work);
-    work();
-    for (auto& th : pool) th.join();
-}
 
 // Side of a grid cloth's nominal square block: the largest (in steps of 0.85)
 // whose central cone fits the loaded budget.
