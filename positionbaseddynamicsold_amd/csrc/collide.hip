@@ -541,18 +541,17 @@ __global__ __launch_bounds__(256) void k_swept_faces(HashCfg g, HashCfg gi, cons
     if (over) c->face_span = 1;
     int lo[3], hi[3], level = 0;
     for (float scale = 1.0f;; level++, scale *= (float)SWEPT_FACTOR) {
-        long long n = 1;
+        int n = 1;
         for (int k = 0; k < 3; k++) {
             lo[k] = cell_coord(gi, r.lo[k], k, scale);
             hi[k] = over ? lo[k] : cell_coord(gi, r.hi[k], k, scale);
-            n *= (long long)min(hi[k] - lo[k] + 1, SWEPT_MAX_CELLS + 1);
+            n *= min(hi[k] - lo[k] + 1, ENTRY_MAX_CELLS + 1);
         }
         if (n <= ENTRY_MAX_CELLS || level == SWEPT_LEVELS - 1) break;
     }
     fcell[2 * f] = make_int4(lo[0], lo[1], lo[2], level);
     fcell[2 * f + 1] = make_int4(hi[0], hi[1], hi[2], 0);
-    // read first, past the CU's cache: one store for most of the launch
-    if (!__hip_atomic_load(&c->level[level], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) c->level[level] = 1;
+    c->level[level] = 1;
     for (int z = lo[2]; z <= hi[2]; z++)
         for (int y = lo[1]; y <= hi[1]; y++)
             for (int xx = lo[0]; xx <= hi[0]; xx++) atomicAdd(&cnt[level_slot(xx, y, z, level, mask)], 1);
@@ -989,6 +988,8 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_swept_candidates(
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, l = lane & 31;
     PairSink sink{buf[wv], 0, (int)((blockIdx.x * VISIT_WAVES + wv) % NEAR_BUCKETS), c, out, cap};
     int pairs = 0;
+    unsigned levels = 0;  // that hold faces, the same for all
+    for (int k = 0; k < SWEPT_LEVELS; k++) levels |= c->level[k] ? 1u << k : 0u;
     const int stride = (int)gridDim.x * VISIT_WAVES * 2;
     for (int v0 = ((int)blockIdx.x * VISIT_WAVES + wv) * 2; v0 < nv; v0 += stride) {
         const int v = v0 + (lane >> 5), at = min(v, nv - 1);
@@ -1001,7 +1002,7 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_swept_candidates(
         if (used && over) c->vertex_span = 1;
         float scale = 1.0f;
         for (int level = 0; level < SWEPT_LEVELS; level++, scale *= (float)SWEPT_FACTOR) {
-            if (!c->level[level]) continue;  // the same for all
+            if (!(levels >> level & 1)) continue;
             int lo[3], w[3];
             for (int k = 0; k < 3; k++) {
                 lo[k] = cell_coord(gi, b.lo[k], k, scale);
@@ -1068,7 +1069,7 @@ __device__ __forceinline__ bool edges_apart(const SweptBox& a, const SweptBox& b
 // in the order of its faces.  EDGE_HUB: an edge of more than HUB_FACES faces,
 // entered once per face, ox its place in etri; telling its distinct cells apart
 // one by one took 0.3 s for 1024 faces.
-constexpr int EDGE_HUB = 3;
+constexpr int EDGE_HUB = 4;
 struct alignas(64) EdgeRec {
     int cx, cy, cz, edge;
     int v0, v1, before, ox;
@@ -1236,16 +1237,15 @@ __global__ __launch_bounds__(64 * VISIT_WAVES) void k_ee_candidates(
                     const EdgeRec rec = ent[e];
                     eb = rec.edge;
                     if (eb > a && rec.cx == fq.x && rec.cy == fq.y && rec.cz == fq.z && !ringed(rec.v0, rec.v1)) {
-                        bool first = rec.before == 0 || rec.before == EDGE_HUB ||
-                                     !cells.meets(make_int4(rec.ox, rec.oy, rec.oz, 0));
-                        if (rec.before == 2)
-                            for (int j = etoff[eb]; first; j++) {  // ends at a face of this cell
+                        bool first = !(rec.before & 3) || !cells.meets(make_int4(rec.ox, rec.oy, rec.oz, 0));
+                        if (rec.before >= 2) {
+                            const int own = rec.before == EDGE_HUB ? rec.ox : INT_MAX;
+                            for (int j = etoff[eb]; first && j != own; j++) {  // ends at a face of this cell
                                 const int4 d = tcell[etri[j]];
-                                if (d.w >= 0 && d.x == rec.cx && d.y == rec.cy && d.z == rec.cz) break;
+                                if (own == INT_MAX && d.w >= 0 && d.x == rec.cx && d.y == rec.cy && d.z == rec.cz) break;
                                 first = !cells.meets(d);
                             }
-                        if (rec.before == EDGE_HUB)
-                            for (int j = etoff[eb]; first && j < rec.ox; j++) first = !cells.meets(tcell[etri[j]]);
+                        }
                         pairs += first;
                         hit = first && (LIST || !edges_apart(abox, rec.box, th));
                     }
