@@ -418,7 +418,9 @@ PBD_API int pbd_profile_read(pbd_ctx* ctx, pbd_profile* out, int reset);
  * and, with collisions enabled, the hash table size (table_bits - 2 ..
  * table_bits + 2 of the hashed grid), restoring x and v after every trial.
  * The fastest candidate becomes the solver configuration and is returned in
- * `best` (and `best_table_bits`, -1 without collisions).  No candidate
+ * `best` (and `best_table_bits`, -1 without collisions); the settings at hand
+ * stay where they are faster than every candidate.  Candidates that come to the
+ * same launches are timed once.  No candidate
  * changes results: tile plans keep the colour order, hashed candidate sets
  * do not depend on the table size, and with a residual tolerance only
  * tile_sweeps == check_every is tried. */
