@@ -266,6 +266,12 @@ bool distance_grids(const pbd_ctx* c) {
     return true;
 }
 
+// A warm substep's tile launch decides: a cloth's tiles wait for each other, so
+// more of them cost more than they spread (40 cloths of the benchmark's sizes, 6
+// substeps at 1 / 2 / 3 sweeps per chunk: 13.1 / 8.2 / 6.9 ms with cloths split
+// as for the other launches, 9.7 / 6.8 / 6.7 with all whole that fit a tile).
+bool decides_in_launch(const pbd_ctx* c) { return c->ws.enabled && c->sp.per_chunk_launches == 2; }
+
 // Sweeps are counted by nobody but the substep: no tolerance, no per-cloth budgets.
 bool free_sweeps(const pbd_ctx* c) { return !has_tolerance(c) && !c->ws.enabled; }
 
@@ -446,7 +452,7 @@ TileShape tile_shape(const pbd_ctx* c, int ntiles) {
 // 640, 80 x 80 1038 against 640.  As many grids as an eighth of the CUs
 // already fill their tiles well enough.
 int whole_grid_load(const pbd_ctx* c, int sweeps, int ml) {
-    if (c->sp.split_whole || has_tolerance(c)) return ml;
+    if (c->sp.split_whole || has_tolerance(c) || decides_in_launch(c)) return ml;
     int load = 1024;
     if (!c->coll.enabled) load = bending_grids(c) ? 2048 : sweeps >= 4 ? 4096 : sweeps >= 2 ? 4608 : 5632;
     if (load >= ml) return ml;
@@ -475,7 +481,7 @@ void replan_at(pbd_ctx* c, int s) {
     // launch holds up all the others unless the cloth is small (48 cloths of
     // 240 to 87,000 vertices: 675 us per substep, 555 with no cloth whole).
     // With bending even the smallest takes as long as the launches it holds up.
-    if (multi > 0 && !has_tolerance(c)) {
+    if (multi > 0 && !has_tolerance(c) && !decides_in_launch(c)) {
         whole.steps = 2048;
         for (auto& k : c->cloths)
             if (k.nb > 0) whole.steps = 0;

@@ -79,3 +79,20 @@ def test_init_refuses_a_budget_that_no_plan_fits(orc, mesh):
         ctx.init()
         ctx.step(1)
         assert np.isfinite(ctx.get(c)).all()
+
+
+@pytest.mark.parametrize("form,whole", [(0, 0), (1, 0), (2, 1)])
+def test_a_launch_that_decides_keeps_cloths_of_one_tile_whole(form, whole):
+    # the tiles of a cloth wait for each other there
+    with capi.Context() as ctx:
+        for n in (60, 130):
+            c = ctx.add_grid(n, n, 1.0, 1.0, jitter=1e-4, seed=n)
+            ctx.set_constraint_option(c, capi.DISTANCE, (1.0, 1.0, 1.0))
+            ctx.set_pins(c, [0])
+        ctx.init()
+        ctx.ws_init(0)
+        ctx.ws_enable(True)
+        ctx.set_solver(iterations=6, tile_sweeps=2, check_every=2, warm_iterations=2, per_chunk_launches=form)
+        assert (ctx.info(0).whole, ctx.info(0).ntiles, ctx.info(1).whole) == (whole, 1, 0)
+        ctx.step(2)
+        assert np.isfinite(ctx.get(0)).all()
