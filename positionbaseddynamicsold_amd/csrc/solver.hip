@@ -795,7 +795,12 @@ __device__ __forceinline__ bool cloth_decide(const TileQueue& q, const TileDev& 
 // registers for the whole launch, REGS per thread and colour.  A phase then
 // waits for nothing but LDS and runs no loop: with the few waves of a small
 // tile its time is the length of its instruction chain.
-template <bool BEND, bool DECIDE = false, int REGS = 0>
+//
+// STEPS: fused single-tile cloths run a.substeps substeps.  Launches of one have
+// a form of their own: what the loop keeps in registers across substeps cost
+// them two spilled ones and 5 to 8% (one-sweep launches of a 389 x 211 mesh 3.45
+// against 3.18 ms a frame, of a 256 x 256 cloth with bending 6.51 against 6.26).
+template <bool BEND, bool DECIDE = false, int REGS = 0, bool STEPS = false>
 __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, double* red,
                                           const TileQueue* qd = nullptr) {
     constexpr int PREFETCH = TileFetch<BEND>::dist;
@@ -930,7 +935,7 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
     // A context of single-tile cloths runs several substeps in one launch:
     // each thread stores and loads the same vertices, so x and v carry over
     // through memory without a barrier of their own.
-    const int nsub = (td.whole && a.fused) ? a.substeps : 1;
+    const int nsub = (STEPS && td.whole && a.fused) ? a.substeps : 1;
     int sw = 0;
     double resid = -1.0;
     for (int ss = 0; ss < nsub; ss++) {
@@ -1141,13 +1146,13 @@ __device__ __forceinline__ int tiles_body(TILE_PARAMS, int slot, float4* P, doub
 // workgroup takes entries blockIdx.x, blockIdx.x + gridDim.x, ... .  With
 // gridDim.x a multiple of 8 every entry a workgroup takes sits at its own
 // position mod 8, the XCD the list's layout meant it for.
-template <bool BEND, int REGS = 0>
+template <bool BEND, int REGS = 0, bool STEPS = false>
 __device__ __forceinline__ void tiles_walk(TILE_PARAMS, const int* __restrict__ n_items, float4* P) {
     double* red = (double*)(P + a.lds_slots);
     // one loop for both forms, so the body is inlined once
     const int n = n_items ? *n_items : (int)gridDim.x;
     for (int it = blockIdx.x; it < n; it += gridDim.x) {
-        tiles_body<BEND, false, REGS>(TILE_ARGS, order[it], P, red);
+        tiles_body<BEND, false, REGS, STEPS>(TILE_ARGS, order[it], P, red);
         __syncthreads();  // the tile's stores have read LDS before the next tile loads
     }
 }
@@ -1169,6 +1174,21 @@ template <int REGS>
 __global__ __launch_bounds__(1024) void k_tiles_regs(TILE_PARAMS, const int* __restrict__ n_items) {
     extern __shared__ float4 P[];
     tiles_walk<false, REGS>(TILE_ARGS, n_items, P);
+}
+
+// The same for several substeps in one launch.
+__global__ __launch_bounds__(1024, 8) void k_tiles_steps(TILE_PARAMS, const int* __restrict__ n_items) {
+    extern __shared__ float4 P[];
+    tiles_walk<false, 0, true>(TILE_ARGS, n_items, P);
+}
+__global__ __launch_bounds__(1024) void k_tiles_bend_steps(TILE_PARAMS, const int* __restrict__ n_items) {
+    extern __shared__ float4 P[];
+    tiles_walk<true, 0, true>(TILE_ARGS, n_items, P);
+}
+template <int REGS>
+__global__ __launch_bounds__(1024) void k_tiles_regs_steps(TILE_PARAMS, const int* __restrict__ n_items) {
+    extern __shared__ float4 P[];
+    tiles_walk<false, REGS, true>(TILE_ARGS, n_items, P);
 }
 
 // The tiles of a later chunk: the entries of `order` (the multi-tile launch
@@ -1568,8 +1588,9 @@ size_t tiles_lds_optin(size_t bytes) {
     if (bytes <= 65536) return bytes;
     for (const void* k : {(const void*)k_tiles, (const void*)k_tiles_bend, (const void*)k_tiles_queue,
                           (const void*)k_tiles_queue_bend, (const void*)k_tiles_decide,
-                          (const void*)k_tiles_decide_bend, (const void*)k_tiles_regs<1>,
-                          (const void*)k_tiles_regs<2>}) {
+                          (const void*)k_tiles_decide_bend, (const void*)k_tiles_regs<1>, (const void*)k_tiles_regs<2>,
+                          (const void*)k_tiles_steps, (const void*)k_tiles_bend_steps,
+                          (const void*)k_tiles_regs_steps<1>, (const void*)k_tiles_regs_steps<2>}) {
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
         if (e != hipSuccess) {
             (void)hipGetLastError();  // the refusal is handled by the smaller limit
@@ -1589,6 +1610,11 @@ void launch_tiles(hipStream_t s, int nblocks, const int* order, const TileDev* t
     SolveArgs a = args;
     a.lds_slots = (int)(lds_bytes / sizeof(float4));
     auto* kernel = with_bend ? k_tiles_bend : regs == 1 ? k_tiles_regs<1> : regs == 2 ? k_tiles_regs<2> : k_tiles;
+    if (a.substeps > 1)
+        kernel = with_bend   ? k_tiles_bend_steps
+                 : regs == 1 ? k_tiles_regs_steps<1>
+                 : regs == 2 ? k_tiles_regs_steps<2>
+                             : k_tiles_steps;
     hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(threads), lds_bytes + TILE_TAIL_LDS, s, order, tiles,
                        verts, dist, bend, own, own_rest, phases, counts, cloths, ktab_d, ktab_b, x, v,
                        p_in, p_out, res_slots, ncl, sweeps_out, sweep_cap, a, n_items);
