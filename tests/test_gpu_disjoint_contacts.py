@@ -1,0 +1,56 @@
+"""The response to contacts that share no corner, which fill the table of one
+workgroup as far as it goes."""
+import time
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from positionbaseddynamicsold_amd import capi
+
+TH, PASSES = 0.01, 2
+
+
+def disjoint(n):
+    """n faces with a vertex of another triangle pushed through each."""
+    k = int(np.ceil(np.sqrt(n)))
+    at = np.stack(np.meshgrid(np.arange(k), [0], np.arange(k), indexing="ij"), -1).reshape(-1, 1, 3)[:n]
+    face = [[0, 0, 0], [0.3, 0, 0], [0, 0, 0.3]]
+    other = [[0.08, 0.02, 0.08], [0.08, 0.4, 0.08], [0.12, 0.4, 0.08]]
+    x = (at + np.array(face + other)).reshape(-1, 3).astype(np.float32)
+    p = x + np.float32(0.002) * np.random.default_rng(n).standard_normal(x.shape).astype(np.float32)
+    p[3::6, 1] -= np.float32(0.03)
+    return x, p, np.arange(len(x), dtype=np.int32).reshape(-1, 3)
+
+
+@pytest.mark.parametrize("n", [1, 15, 64, 464, 742, 743, 928, 929])
+def test_disjoint_contacts_equal_the_oracle(orc, n):
+    x, p, tris = disjoint(n)
+    desc = dict(cell=(0.5, 0.5, 0.5), table_bits=12)
+    arr, count = orc.ccd_detect(orc.grid(1, **desc), x, p, tris, TH)
+    assert count == n
+    w = np.ones(len(x), np.float32)
+    w[::11] = 0.0
+    with capi.Context() as ctx:
+        ctx.ccd_detect(capi.hash_desc(1, **desc), x, p, tris, TH)
+        assert np.array_equal(ctx.ccd_resolve(p, w, TH, PASSES), orc.ccd_resolve(arr, count, tris, x, p, w, TH, PASSES))
+
+
+def test_few_disjoint_contacts_take_less_than_many():
+    # 464 in one workgroup: 160 us a call where they filled its table, 75 with
+    # slots to spare; 929, beyond it, take 97
+    best = {}
+    for n in (464, 929):
+        x, p, tris = disjoint(n)
+        w = np.ones(len(x), np.float32)
+        with capi.Context() as ctx:
+            ctx.ccd_detect(capi.hash_desc(1, cell=(0.5, 0.5, 0.5), table_bits=12), x, p, tris, TH)
+            times = []
+            for _ in range(40):
+                t0 = time.perf_counter()
+                ctx.ccd_resolve(p, w, TH, PASSES)
+                times.append(time.perf_counter() - t0)
+            best[n] = min(times)
+    print({n: f"{1e6 * t:.0f} us" for n, t in best.items()}, flush=True)
+    assert best[464] < best[929]
