@@ -300,16 +300,16 @@ int effective_tile_sweeps(const pbd_ctx* c) {
     if (c->coll.enabled) return 1;  // contacts are resolved after every sweep
     // Fixed sweeps: the result does not depend on the split, and with bending
     // prims one sweep per launch is faster whatever was asked for (20 sweeps
-    // of 128^2 / 256^2 / 512^2 vertices: 648 / 692 / 985 us at one sweep per
-    // launch, 684 / 817 / 1328 us at two, at the best tile size of each).
+    // of 128^2 / 256^2 / 512^2 vertices: 560 / 590 / 921 us at one sweep per
+    // launch; 684 / 817 / 1328 us at two when one took 648 / 692 / 985).
     if (c->sp.tile_sweeps > 1 && free_sweeps(c) && bending_grids(c)) return 1;
     if (c->sp.tile_sweeps > 0) return c->sp.tile_sweeps;
     // Unset and free to choose (fixed sweeps, no per-cloth budgets): four
     // sweeps per launch for distance prims.  Bending prims touch four vertices
     // and take three times the colours, so their cones grow too fast: one.
     // Measured per substep of 20 sweeps at the best tile size for each: a
-    // 389 x 211 cloth 152 / 133 / 117 / 113 / 133 us at 1 / 2 / 3 / 4 / 5
-    // sweeps per launch, a 256 x 256 cloth with bending 721 us at 1 and 923 at 2.
+    // 389 x 211 cloth 196 / 122 / 104 / 102 / 119 us at 1 / 2 / 3 / 4 / 5
+    // sweeps per launch.
     // Meshes are tiled by vertex id, whose cones may grow faster than a grid's:
     // they keep one.
     if (!chooses_sweeps(c)) return std::max(1, c->sp.check_every);
@@ -422,8 +422,8 @@ TileShape tile_shape(const pbd_ctx* c, int ntiles) {
     t.lds = (size_t)std::max(1, c->plan.max_loaded) * sizeof(float4);
     // Bending: a phase of a small tile has a few waves' work, and the waves
     // without any still take issue slots and hold up the barrier (20 sweeps of
-    // 128^2 / 256^2 / 400^2 / 512^2 vertices: 591 / 639 / 830 / 992 us with 512
-    // threads, 609 / 657 / 818 / 960 with 768, 642 / 685 / 834 / 973 with 1024).
+    // 128^2 / 256^2 / 400^2 / 512^2 vertices: 560 / 591 / 767 / 937 us with 512
+    // threads, 571 / 596 / 764 / 922 with 768, 596 / 618 / 786 / 919 with 1024).
     if (!c->plan.bend.empty() && c->sp.block_threads == 0) {
         int most = 0;
         for (auto& k : c->cloths)
@@ -446,10 +446,10 @@ TileShape tile_shape(const pbd_ctx* c, int ntiles) {
 // are split where that is faster.  With collisions every sweep is a launch of
 // its own, which takes as long as its largest tile (96 x 96 vertices: 22 us as
 // one tile, 9 us in tiles).  Otherwise, 20 sweeps as one tile against tiles
-// at 4 / 2 / 1 sweeps per launch: 64 x 64 98 against 90 / - / -, 72 x 72
-// 159 against 88 / 117 / 160, 100 x 100 266 against 88 / 120 / 170; with
-// bending (one sweep per launch) 40 x 40 574 against 640, 48 x 48 680 against
-// 640, 80 x 80 1038 against 640.  As many grids as an eighth of the CUs
+// at 4 / 2 / 1 sweeps per launch: 64 x 64 98 us whole, 72 x 72 162 against
+// 77 / 100 / 160, 100 x 100 271 against 79 / 103 / 157; with bending (one
+// sweep per launch) 45 x 45 562 whole, 48 x 48 723 against 561, 80 x 80 1120
+// against 561.  As many grids as an eighth of the CUs
 // already fill their tiles well enough.
 int whole_grid_load(const pbd_ctx* c, int sweeps, int ml) {
     if (c->sp.split_whole || has_tolerance(c) || decides_in_launch(c)) return ml;
